@@ -4,6 +4,8 @@ ends) against the CPU oracle on identical seeded inputs.
 Tolerances (written where used): rtol 1e-3 for fp32 I/O, 2e-2 for bf16/fp16
 I/O, each with an absolute floor of rtol * rms(reference tensor).  The oracle
 runs in fp32 on the already-rounded inputs."""
+import math
+
 import pytest
 import torch
 
@@ -301,6 +303,26 @@ def test_cumsum_decay_helper(chunk):
     w5 = O.decay_from_raw(raw[0, 0]).view(1, H, 1, K).expand(1, H, T, K)
     tab5 = O.cumsum_decay(w5, chunk, 64)
     assert_close(out5["incl"], tab5.incl.reshape(1, H, T, K).transpose(1, 2).reshape(1, T, C), 1e-5, "incl v5")
+
+
+@pytest.mark.parametrize("B,T,C", [(1, 128, 1), (2, 256, 63), (1, 128, 130), (1, 384, 129)])
+@pytest.mark.parametrize("precision", [64, 32])
+def test_decay_tables_of_128_token_chunks_ragged_widths(B, T, C, precision):
+    """Widths that do not fill the last workgroup, odd ones (one channel per lane) and even ones (two), against fp64.
+    fp32 sums of up to 128 terms bounded by 5.3: off by at most 128 * 2^-24 * 128 * 5.3 / 2 = 2.6e-3 in the worst case and
+    by some 1e-4 in practice, which an exponential turns into a relative error of the same size."""
+    import rwkv_wkv_hip as W
+    raw = torch.randn(B, T, C, generator=torch.Generator().manual_seed(C)) * 0.5 - 1.5
+    out = {n: x.double().cpu() for n, x in W.cumsum_decay(raw.to(dev()), 128, factors=True, precision=precision).items()}
+    lw = (-raw.double().exp()).clamp(min=math.log(0.005)).view(B, T // 128, 128, C)
+    incl = lw.cumsum(2)
+    total, intra = incl[:, :, -1:], incl - lw
+    mid = intra[:, :, 64:65]
+    ref = dict(log_w=lw, incl=incl, inter=total - incl, intra=intra, chunk_sum=total, ws_exp=total.exp(), inter_exp=(total - incl).exp(),
+               intra_exp=intra.exp(), r_decay=(intra - mid).exp(), k_inv_decay=(mid - incl).exp())
+    for n, x in ref.items():
+        x = x.reshape(out[n].shape)
+        torch.testing.assert_close(out[n], x, rtol=2e-4, atol=2e-4 if n in ("log_w", "incl", "inter", "intra", "chunk_sum") else 1e-37, msg=lambda m: f"{n}: {m}")
 
 
 # ------------------------------------------------- blocked matrix-core path --
