@@ -124,6 +124,12 @@ int wkv6_forward(void *stream, int B, int T, int C, int H, int dtype, unsigned f
                  const float *state_in, void *y, float *state_out,
                  void *workspace, size_t workspace_bytes);
 
+/* One token per sequence, the serving loop's call (RWKV-v6/src/module/rwkv_inner.py's single-token branch: no floor on
+ * the decay): wkv6_forward with T = 1 and flags 0, with the raw decay w (B, C) in fp32 or in `dtype` (w_dtype).
+ * state_out may be state_in.  (wkv5_forward with T = 1 runs the same kernel.) */
+int wkv6_decode(void *stream, int B, int C, int H, int dtype, int w_dtype, const void *r, const void *k, const void *v,
+                const void *w, const float *u, const float *state_in, void *y, float *state_out);
+
 /* wkv6_forward for callers that cannot allocate device memory and have no workspace to pass: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same
  * arguments and results as wkv6_forward with the chunked algorithm (bf16 r/k/v/y and WKV_FLOOR_DECAY required,

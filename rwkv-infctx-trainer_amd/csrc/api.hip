@@ -4,6 +4,7 @@
 #include "../../include/rwkv_wkv_hip.h"
 #include "common.h"
 #include "wkv56_recurrent.hip"
+#include "wkv56_decode.hip"
 #include "wkv56_chunked.hip"
 #include "wkv56_noalloc.hip"
 #include "wkv4.hip"
@@ -73,8 +74,10 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
                                                state_out, workspace, (flags & WKV_FLOOR_DECAY) ? 1 : 0);
         return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
     }
-    hipError_t e = recurrent_forward((hipStream_t)stream, dtype, per_token, B, T, C, H, r, k, v, (const float *)w, u, state_in, y,
-                                     state_out, (flags & WKV_FLOOR_DECAY) ? 1 : 0);
+    const int floor_decay = (flags & WKV_FLOOR_DECAY) ? 1 : 0;
+    hipError_t e = T == 1 ? decode_launch((hipStream_t)stream, dtype, WKV_F32, per_token, B * H, H, r, k, v, w, u, state_in, y, state_out, floor_decay)
+                          : recurrent_forward((hipStream_t)stream, dtype, per_token, B, T, C, H, r, k, v, (const float *)w, u, state_in, y,
+                                              state_out, floor_decay);
     return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
 }
 
@@ -223,6 +226,20 @@ int wkv5_forward(void *stream, int B, int T, int C, int H, int dtype, unsigned f
                  float *state_out, void *workspace, size_t workspace_bytes) {
     return forward56(false, stream, B, T, C, H, dtype, flags, algo, r, k, v, w, u, state_in, y, state_out, workspace,
                      workspace_bytes);
+}
+
+int wkv6_decode(void *stream, int B, int C, int H, int dtype, int w_dtype, const void *r, const void *k, const void *v,
+                const void *w, const float *u, const float *state_in, void *y, float *state_out) {
+    int st = check_dims56(B, 1, C, H, dtype);
+    if (st) return st;
+    if (w_dtype != WKV_F32 && w_dtype != dtype) return WKV_ERR_DTYPE;
+    if (!r || !k || !v || !w || !u || !state_in || !y || !state_out) return WKV_ERR_NULL;
+    for (const void *p : {r, k, v, w, (const void *)u, (const void *)state_in, (const void *)y, (const void *)state_out})
+        if (!aligned16(p)) return WKV_ERR_ALIGN;
+    st = check_state_alias(state_in, state_out, B, H, false);
+    if (st) return st;
+    hipError_t e = decode_launch((hipStream_t)stream, dtype, w_dtype, true, B * H, H, r, k, v, w, u, state_in, y, state_out, 0);
+    return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
 }
 
 int wkv6_forward_noalloc(void *stream, int B, int T, int C, int H, int dtype, unsigned flags, const void *r,

@@ -33,6 +33,7 @@ SIGNATURES = {
     "wkv_profile_end": (_I, [_P, _I]),
     "wkv6_forward_workspace": (c_size_t, [_I] * 6),
     "wkv6_forward": (_I, [_P, _I, _I, _I, _I, _I, c_uint, _I] + [_P] * 8 + [_P, c_size_t]),
+    "wkv6_decode": (_I, [_P] + [_I] * 5 + [_P] * 8),
     "wkv6_forward_noalloc": (_I, [_P, _I, _I, _I, _I, _I, c_uint] + [_P] * 8),
     "wkv6_backward_workspace": (c_size_t, [_I] * 6),
     "wkv6_backward": (_I, [_P, _I, _I, _I, _I, _I, c_uint, _I] + [_P] * 14 + [_P, c_size_t]),
@@ -90,6 +91,23 @@ def lib():
         except Exception:            # noqa: BLE001 - set-up then happens on the first call
             pass
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host side (csrc/host.cpp), bound to the kernel library."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise WKVError(f"the native host side is missing: build it first (make -C rwkv-infctx-trainer_amd/csrc): {e}") from e
+        module.bind(LIB_PATH, WKVError)
+        _host = module
+    return _host
 
 
 def check(status: int, what: str):
