@@ -13,7 +13,8 @@ new state is returned, and is differentiable); RUN_WKV5_CUDA /
 RUN_WKV6STATE_CUDA keep the reference's in-place convention on top of them.
 
 All tensors must live on the GPU; the work is done by librwkv_wkv_hip.so on the
-current HIP stream.
+current HIP stream.  The operators' host side (checks, allocation, autograd) is
+native: csrc/host.cpp.
 """
 from __future__ import annotations
 
@@ -50,25 +51,8 @@ def _on_gpu(*ts):
             raise WKVError("rwkv_wkv_hip operators need GPU tensors (there is no CPU path)")
 
 
-def _check_rkv(B, T, C, H, r, k, v):
-    dtype = r.dtype
-    if dtype not in _DT:
-        raise ValueError(f"Unsupported dtype {dtype} for WKV")
-    assert dtype == k.dtype and dtype == v.dtype
-    assert r.is_contiguous() and k.is_contiguous() and v.is_contiguous()
-    assert r.shape == (B, T, C) and k.shape == (B, T, C) and v.shape == (B, T, C)
-    return _DT[dtype]
-
-
 def _workspace(nbytes, device):
     return torch.empty(max(int(nbytes), 16), dtype=torch.uint8, device=device)
-
-
-def _blocked(version, B, T, C, H, dtype):
-    """True when a call with these arguments takes the blocked (matrix-core) algorithm."""
-    L = _lib.lib()
-    fq = L.wkv5_forward_workspace if version == 5 else L.wkv6_forward_workspace
-    return T > 1 and dtype in _DT and fq(B, T, C, H, _DT[dtype], _algo) > 0
 
 
 stats = {"forward_launches": 0, "forward_reused": 0}      # counters for tests and diagnostics
@@ -205,12 +189,11 @@ class call_key:
         return False
 
 
-def _forward56_cached(version, B, T, C, H, r, k, v, w32, u32, s32, need_grad, out_state=None):
-    """_forward56 behind the recompute cache (when one is installed)."""
+def _forward56_cached(version, B, T, C, H, r, k, v, w, u, s, need_grad, out_state):
+    """The operator's forward behind the recompute cache: y, the new state, the workspace with the state checkpoints and
+    the algorithm in force."""
     cache = _cache
-    if cache is None:
-        return _forward56(version, B, T, C, H, r, k, v, w32, u32, s32, need_grad, out_state)
-    sig = (version, B, T, C, H, r.dtype, w32.dtype, tuple(w32.shape), out_state is not None)
+    sig = (version, B, T, C, H, r.dtype, w.dtype, tuple(w.shape), out_state is not None)
     if need_grad:
         hit = cache.pop(_key, sig, r)
         if hit is not None:          # the recomputation of a forward run that kept its results
@@ -220,129 +203,62 @@ def _forward56_cached(version, B, T, C, H, r, k, v, w32, u32, s32, need_grad, ou
                 new_state = out_state
             stats["forward_reused"] += 1
             return y, new_state, ws, algo
-        return _forward56(version, B, T, C, H, r, k, v, w32, u32, s32, True, out_state)
-    y, new_state, ws, algo = _forward56(version, B, T, C, H, r, k, v, w32, u32, s32, True, out_state)    # keep checkpoints
-    cache.push(_key, sig, r, (y, new_state.clone() if out_state is not None else new_state, ws, algo))
-    return y, new_state, ws, algo
-
-
-def _forward56(version, B, T, C, H, r, k, v, w32, u32, s32, need_grad, out_state=None):
-    """Returns y, new_state and, when a backward call will follow, the
-    workspace in which the forward kernel left its state checkpoints (sized
-    for that backward call) together with the algorithm that was in force.
-    `w32` is fp32, or (WKV6, blocked algorithm) bf16 as it came."""
-    L = _lib.lib()
-    dt = _check_rkv(B, T, C, H, r, k, v)
-    _on_gpu(r, k, v, w32, u32, s32)
-    y = torch.empty_like(r)
-    new_state = torch.empty_like(s32) if out_state is None else out_state       # (must not overlap s32)
-    flags = _lib.FLOOR_DECAY if T > 1 else 0
-    if w32.dtype == torch.bfloat16:
-        flags |= _lib.W_BF16
     algo = _algo
-    fn, fq, bq = (L.wkv5_forward, L.wkv5_forward_workspace, L.wkv5_backward_workspace) if version == 5 else \
-                 (L.wkv6_forward, L.wkv6_forward_workspace, L.wkv6_backward_workspace)
-    ws = None
-    if need_grad and fq(B, T, C, H, dt, algo) > 0:
-        ws = _workspace(max(fq(B, T, C, H, dt, algo), bq(B, T, C, H, dt, algo)), r.device)
-    check(fn(_stream(), B, T, C, H, dt, flags, algo, _ptr(r), _ptr(k), _ptr(v), _ptr(w32), _ptr(u32), _ptr(s32),
-             _ptr(y), _ptr(new_state), _ptr(ws), 0 if ws is None else ws.numel()), f"wkv{version}_forward")
+    y, new_state, ws = _lib.host().forward56(version, algo, B, T, C, H, r, k, v, w, u, s, out_state)
     stats["forward_launches"] += 1
+    if not need_grad:
+        cache.push(_key, sig, r, (y, new_state.clone() if out_state is not None else new_state, ws, algo))
     return y, new_state, ws, algo
 
 
-def _backward56(version, B, T, C, H, r, k, v, w32, u32, s32, gy, gstate, ws, algo):
-    L = _lib.lib()
-    dt = _DT[r.dtype]
-    gr, gk, gv = torch.empty_like(r), torch.empty_like(k), torch.empty_like(v)
-    gw = torch.empty_like(w32)
-    gu = torch.empty_like(u32)
-    gs = torch.empty_like(s32)
-    flags = _lib.FLOOR_DECAY if T > 1 else 0
-    if w32.dtype == torch.bfloat16:
-        flags |= _lib.W_BF16           # gw comes back in bf16 too (torch.empty_like above)
-    fn, wsq = (L.wkv5_backward, L.wkv5_backward_workspace) if version == 5 else (L.wkv6_backward, L.wkv6_backward_workspace)
-    need = wsq(B, T, C, H, dt, algo)
-    if ws is not None and ws.numel() >= need:
-        flags |= _lib.CHECKPOINTS_VALID
-    else:           # no forward workspace, or one sized for another plan (wkv_tune changed in between): rebuild inside
-        ws = _workspace(need, r.device)
-    check(fn(_stream(), B, T, C, H, dt, flags, algo, _ptr(r), _ptr(k), _ptr(v), _ptr(w32), _ptr(u32), _ptr(s32),
-             _ptr(gy), _ptr(gstate), _ptr(gr), _ptr(gk), _ptr(gv), _ptr(gw), _ptr(gu), _ptr(gs), _ptr(ws), ws.numel()),
-          f"wkv{version}_backward")
-    return gr, gk, gv, gw, gu, gs
+class _Cached56(torch.autograd.Function):
+    """WKV5 / WKV6 while a recompute cache is installed (otherwise the native front, csrc/host.cpp, is called directly).
+    ``in_place``: the new state goes into ``s`` and no gradient flows through it, as in the reference
+    (RWKV-v5/src/module/TimeMix.py:60,139-140)."""
 
-
-class _WKV5Fn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, grad_mode, B, T, C, H, state, r, k, v, w, u):
-        assert state.dtype == torch.float32 and w.dtype == torch.float32
-        assert state.is_contiguous() and w.is_contiguous() and u.is_contiguous()
-        assert state.shape == (B, H, HEAD, HEAD) and H * HEAD == C
-        u32 = u.float().contiguous().view(H, HEAD)
-        w32 = w.view(H, HEAD)
+    def forward(ctx, version, in_place, grad_mode, B, T, C, H, r, k, v, w, u, s):
+        assert s.is_contiguous() and w.is_contiguous() and u.is_contiguous()
+        assert s.shape == (B, H, HEAD, HEAD) and H * HEAD == C and u.numel() == C
+        assert (s.dtype == w.dtype == torch.float32 and w.numel() == C) if version == 5 else w.shape == (B, T, C)
         need_grad = grad_mode and any(ctx.needs_input_grad)      # no checkpoints kept under torch.no_grad()
         with torch.no_grad():
-            y, new_state, ws, algo = _forward56_cached(5, B, T, C, H, r, k, v, w32, u32, state, need_grad)
-        ctx.dims = (B, T, C, H)
-        ctx.meta = (w.shape, u.shape, u.dtype)
-        ctx.ws, ctx.algo = ws, algo
-        ctx.save_for_backward(r, k, v, w32, u32, state)
-        return y, new_state
+            u32, s32 = u.float(), s.clone() if in_place else s.float()
+            w32 = w if version == 5 else _lib.host().decay_operand(_algo, B, T, C, H, r, w)
+            y, new_state, ws, algo = _forward56_cached(version, B, T, C, H, r, k, v, w32, u32, s32, need_grad, s if in_place else None)
+        ctx.set_materialize_grads(False)
+        ctx.call = (version, in_place, algo, B, T, C, H, w.dtype, u.dtype, s.dtype)
+        ctx.ws = ws
+        ctx.save_for_backward(r, k, v, w32, u32, s32)
+        return y if in_place else (y, new_state.to(s.dtype))
 
     @staticmethod
-    def backward(ctx, gy, gstate):
-        B, T, C, H = ctx.dims
-        r, k, v, w32, u32, state = ctx.saved_tensors
-        wshape, ushape, udtype = ctx.meta
-        gy = gy.contiguous()
+    def backward(ctx, gy, gstate=None):
+        version, in_place, algo, B, T, C, H, wdtype, udtype, sdtype = ctx.call
+        r, k, v, w32, u32, s32 = ctx.saved_tensors
+        gy = torch.zeros_like(r) if gy is None else gy.contiguous()
         assert gy.dtype == r.dtype
         gstate = None if gstate is None else gstate.float().contiguous()
-        with torch.no_grad():
-            gr, gk, gv, gw, gu, gs = _backward56(5, B, T, C, H, r, k, v, w32, u32, state, gy, gstate, ctx.ws, ctx.algo)
-        return (None, None, None, None, None, gs, gr, gk, gv, gw.view(wshape), gu.view(ushape).to(udtype))
+        gr, gk, gv, gw, gu, gs = _lib.host().backward56(version, algo, B, T, C, H, r, k, v, w32, u32, s32, gy, gstate, ctx.ws)
+        return (None,) * 7 + (gr, gk, gv, gw.to(wdtype), gu.to(udtype), None if in_place else gs.to(sdtype))
+
+
+def _op56(version, in_place, B, T, C, H, r, k, v, w, u, s):
+    if _cache is not None:
+        return _Cached56.apply(version, in_place, torch.is_grad_enabled(), B, T, C, H, r, k, v, w, u, s)
+    out = _lib.host().wkv56(version, _algo, in_place, B, T, C, H, r, k, v, w, u, s)
+    stats["forward_launches"] += 1
+    return out
 
 
 class WKV_5:
     """WKV5: per-channel decay.  ``WKV_5.apply(B, T, C, H, state, r, k, v, w, u) -> (y, new_state)`` with state
     (B,H,64,64) fp32 [key][value]; r,k,v (B,T,C) in one dtype; w (H,64) fp32 raw; u (H,64).  Differentiable in
-    everything, the state included.  (A thin front of the autograd Function: it notes whether autograd is recording,
-    which the Function itself cannot see, so that a call under torch.no_grad() keeps no checkpoints.)"""
+    everything, the state included; a call under torch.no_grad() keeps no checkpoints."""
 
     @staticmethod
     def apply(B, T, C, H, state, r, k, v, w, u):
-        return _WKV5Fn.apply(torch.is_grad_enabled(), B, T, C, H, state, r, k, v, w, u)
-
-
-class _WKV6Fn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, grad_mode, B, T, C, H, r, k, v, w, u, s):
-        assert s.is_contiguous() and w.is_contiguous() and u.is_contiguous()
-        assert s.shape == (B, H, HEAD, HEAD) and H * HEAD == C and w.shape == (B, T, C)
-        u32 = u.float().contiguous().view(H, HEAD)
-        native_w = w.dtype == torch.bfloat16 and r.dtype == torch.bfloat16 and _blocked(6, B, T, C, H, r.dtype)
-        w32 = w if native_w else w.float()
-        s32 = s.float()
-        need_grad = grad_mode and any(ctx.needs_input_grad)
-        with torch.no_grad():
-            y, new_state, ws, algo = _forward56_cached(6, B, T, C, H, r, k, v, w32, u32, s32, need_grad)
-        ctx.dims = (B, T, C, H)
-        ctx.meta = (w.dtype, u.shape, u.dtype, s.dtype)
-        ctx.ws, ctx.algo = ws, algo
-        ctx.save_for_backward(r, k, v, w32, u32, s32)
-        return y, new_state.to(s.dtype)
-
-    @staticmethod
-    def backward(ctx, gy, gstate):
-        B, T, C, H = ctx.dims
-        r, k, v, w32, u32, s32 = ctx.saved_tensors
-        wdtype, ushape, udtype, sdtype = ctx.meta
-        gy = gy.contiguous()
-        assert gy.dtype == r.dtype
-        gstate = None if gstate is None else gstate.float().contiguous()
-        with torch.no_grad():
-            gr, gk, gv, gw, gu, gs = _backward56(6, B, T, C, H, r, k, v, w32, u32, s32, gy, gstate, ctx.ws, ctx.algo)
-        return (None, None, None, None, None, gr, gk, gv, gw.to(wdtype), gu.view(ushape).to(udtype), gs.to(sdtype))
+        return _op56(5, False, B, T, C, H, r, k, v, w, u, state)
 
 
 class WKV_6:
@@ -353,60 +269,7 @@ class WKV_6:
 
     @staticmethod
     def apply(B, T, C, H, r, k, v, w, u, s):
-        return _WKV6Fn.apply(torch.is_grad_enabled(), B, T, C, H, r, k, v, w, u, s)
-
-
-class _RunInPlace5(torch.autograd.Function):
-    """WKV5 with the reference's in-place state convention: y is returned, the new state is written by the kernel
-    straight into the caller's buffer (e.g. one layer's slice of the trainer's (N_layer,B,H,64,64) tensor,
-    RWKV-v5/src/model.py:53-61), the incoming state survives in a private copy for backward (the reference's
-    ``state.clone()``, TimeMix.py:60).  No gradient flows through the state, as in the reference (:139-140)."""
-
-    @staticmethod
-    def forward(ctx, grad_mode, B, T, C, H, state, r, k, v, w, u):
-        u32, w32 = u.float().contiguous().view(H, HEAD), w.view(H, HEAD)
-        s_in = state.clone()
-        with torch.no_grad():
-            y, _, ws, algo = _forward56_cached(5, B, T, C, H, r, k, v, w32, u32, s_in, grad_mode and any(ctx.needs_input_grad),
-                                               out_state=state)
-        ctx.dims, ctx.meta, ctx.ws, ctx.algo = (B, T, C, H), (w.shape, u.shape, u.dtype), ws, algo
-        ctx.save_for_backward(r, k, v, w32, u32, s_in)
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        B, T, C, H = ctx.dims
-        r, k, v, w32, u32, s_in = ctx.saved_tensors
-        wshape, ushape, udtype = ctx.meta
-        with torch.no_grad():
-            gr, gk, gv, gw, gu, _ = _backward56(5, B, T, C, H, r, k, v, w32, u32, s_in, gy.contiguous(), None, ctx.ws, ctx.algo)
-        return (None, None, None, None, None, None, gr, gk, gv, gw.view(wshape), gu.view(ushape).to(udtype))
-
-
-class _RunInPlace6(torch.autograd.Function):
-    """WKV6 counterpart of ``_RunInPlace5`` (RWKV-v6/src/module/TimeMix.py:51,111-118)."""
-
-    @staticmethod
-    def forward(ctx, grad_mode, B, T, C, H, r, k, v, w, u, s):
-        u32 = u.float().contiguous().view(H, HEAD)
-        native_w = w.dtype == torch.bfloat16 and r.dtype == torch.bfloat16 and _blocked(6, B, T, C, H, r.dtype)
-        w32 = w if native_w else w.float()
-        s_in = s.clone()
-        with torch.no_grad():
-            y, _, ws, algo = _forward56_cached(6, B, T, C, H, r, k, v, w32, u32, s_in, grad_mode and any(ctx.needs_input_grad),
-                                               out_state=s)
-        ctx.dims, ctx.meta, ctx.ws, ctx.algo = (B, T, C, H), (w.dtype, u.shape, u.dtype), ws, algo
-        ctx.save_for_backward(r, k, v, w32, u32, s_in)
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        B, T, C, H = ctx.dims
-        r, k, v, w32, u32, s_in = ctx.saved_tensors
-        wdtype, ushape, udtype = ctx.meta
-        with torch.no_grad():
-            gr, gk, gv, gw, gu, _ = _backward56(6, B, T, C, H, r, k, v, w32, u32, s_in, gy.contiguous(), None, ctx.ws, ctx.algo)
-        return (None, None, None, None, None, gr, gk, gv, gw.to(wdtype), gu.view(ushape).to(udtype), None)
+        return _op56(6, False, B, T, C, H, r, k, v, w, u, s)
 
 
 def _direct_state(state, B, H):
@@ -415,10 +278,11 @@ def _direct_state(state, B, H):
 
 def RUN_WKV5_CUDA(B, T, C, H, state, r, k, v, w, u):
     """The reference's calling convention (RWKV-v5/src/module/TimeMix.py:145-154): returns y and leaves the new
-    state in ``state``.  An fp32 contiguous state buffer is written by the kernel directly (no copy afterwards);
-    anything else goes through the functional operator and a copy."""
+    state in ``state``.  An fp32 contiguous state buffer (e.g. one layer's slice of the trainer's (N_layer,B,H,64,64)
+    tensor, RWKV-v5/src/model.py:53-61) is written by the kernel directly, the incoming state surviving in a private copy
+    for backward; anything else goes through the functional operator and a copy."""
     if _direct_state(state, B, H) and w.dtype == torch.float32 and w.is_contiguous() and u.is_contiguous():
-        return _RunInPlace5.apply(torch.is_grad_enabled(), B, T, C, H, state, r, k, v, w, u)
+        return _op56(5, True, B, T, C, H, r, k, v, w, u, state)
     y, new_state = WKV_5.apply(B, T, C, H, state.clone(), r, k, v, w, u)
     with torch.no_grad():
         state.copy_(new_state)
@@ -429,57 +293,18 @@ def RUN_WKV6STATE_CUDA(B, T, C, H, r, k, v, w, u, s):
     """The reference's calling convention (RWKV-v6/src/module/TimeMix.py:111-118): returns y and leaves the new
     state in ``s`` (written by the kernel directly when ``s`` is an fp32 contiguous buffer)."""
     if _direct_state(s, B, H) and w.is_contiguous() and u.is_contiguous() and w.shape == (B, T, C):
-        return _RunInPlace6.apply(torch.is_grad_enabled(), B, T, C, H, r, k, v, w, u, s)
+        return _op56(6, True, B, T, C, H, r, k, v, w, u, s)
     y, new_state = WKV_6.apply(B, T, C, H, r, k, v, w, u, s.clone())
     with torch.no_grad():
         s.copy_(new_state)
     return y
 
 
-class _WKV4(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, grad_mode, time_decay, time_first, k, v, wkv_state):
-        L = _lib.lib()
-        assert k.dim() == 3 and v.shape == k.shape and k.dtype == v.dtype
-        B, T, C = k.shape
-        assert time_decay.shape == (C,) and time_first.shape == (C,) and wkv_state.shape == (B, C, 3)
-        if k.dtype not in _DT:
-            raise ValueError(f"Unsupported dtype {k.dtype} for WKV")
-        _on_gpu(time_decay, time_first, k, v, wkv_state)
-        td, tf = time_decay.float().contiguous(), time_first.float().contiguous()
-        k, v, st = k.contiguous(), v.contiguous(), wkv_state.float().contiguous()
-        y = torch.empty_like(k)
-        new_state = torch.empty_like(st)
-        need_grad = grad_mode and any(ctx.needs_input_grad)
-        ckpt = _workspace(L.wkv4_checkpoint_bytes(B, T, C), k.device) if need_grad else None
-        check(L.wkv4_forward(_stream(), B, T, C, _DT[k.dtype], _ptr(td), _ptr(tf), _ptr(k), _ptr(v), _ptr(st),
-                             _ptr(y), _ptr(new_state), _ptr(ckpt)), "wkv4_forward")
-        ctx.save_for_backward(td, tf, k, v, st, ckpt)
-        ctx.meta = (time_decay.dtype, time_first.dtype)
-        return y, new_state
-
-    @staticmethod
-    def backward(ctx, gy, gnew_state):
-        L = _lib.lib()
-        td, tf, k, v, st, ckpt = ctx.saved_tensors
-        B, T, C = k.shape
-        gy = gy.contiguous()
-        gns = None if gnew_state is None else gnew_state.float().contiguous()
-        gtd, gtf = torch.empty_like(td), torch.empty_like(tf)
-        gk, gv = torch.empty_like(k), torch.empty_like(v)
-        gst = torch.empty_like(st)
-        ws = _workspace(L.wkv4_backward_workspace(B, T, C, _DT[k.dtype]), k.device)
-        check(L.wkv4_backward(_stream(), B, T, C, _DT[k.dtype], _ptr(td), _ptr(tf), _ptr(k), _ptr(v), _ptr(st),
-                              _ptr(gy), _ptr(gns), _ptr(gtd), _ptr(gtf), _ptr(gk), _ptr(gv), _ptr(gst), _ptr(ckpt),
-                              _ptr(ws), ws.numel()), "wkv4_backward")
-        return None, gtd.to(ctx.meta[0]), gtf.to(ctx.meta[1]), gk, gv, gst
-
-
 def wkv_op(time_decay, time_first, k, v, wkv_state):
     """RWKV-v4 WKV with the signature of torch.ops.rwkv.wkv
     (RWKV-v4neo/src/model.py:130-132): time_decay, time_first (C); k, v (B,T,C);
     wkv_state (B,C,3) = (aa, bb, pp).  Returns (y, new_state)."""
-    return _WKV4.apply(torch.is_grad_enabled(), time_decay, time_first, k, v, wkv_state)
+    return _lib.host().wkv4(time_decay, time_first, k, v, wkv_state)
 
 
 def cumsum_decay(w, chunk_len=128, per_token=True, factors=False, precision=64):

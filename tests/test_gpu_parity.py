@@ -84,6 +84,29 @@ def test_recurrent_with_many_heads(version, dtype, B, T):
     compare(got, ref, RTOL[dtype], f"v{version}/{dtype}/B{B}T{T}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H", [(1, 1), (3, 5), (40, 7)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_single_token_with_decay_in_the_io_dtype(dtype, B, H, in_place):
+    """One token with the raw decay in the type of r, k, v (read as it is), the state returned or updated in place."""
+    import rwkv_wkv_hip as W
+    from rwkv_wkv_hip import configs
+    wl = configs.make(3, B=B, T=1, C=64 * H, H=H, dtype=dtype)
+    t = wl.tensors
+    w = t["w"].to(dtype)
+    y_ref, s_ref = O.wkv6_op(B, 1, wl.C, H, t["r"].float(), t["k"].float(), t["v"].float(), w.float(), t["u"], t["state"])
+    g = {n: x.to(dev()) for n, x in t.items()}
+    with torch.no_grad():
+        if in_place:
+            s = g["state"]
+            y = W.RUN_WKV6STATE_CUDA(B, 1, wl.C, H, g["r"], g["k"], g["v"], w.to(dev()), g["u"], s)
+        else:
+            y, s = W.WKV_6.apply(B, 1, wl.C, H, g["r"], g["k"], g["v"], w.to(dev()), g["u"], g["state"])
+    assert y.dtype == dtype
+    assert_close(y, y_ref, 1e-3 if dtype == torch.float32 else 2e-2, "y")
+    assert_close(s, s_ref, 1e-3, "state")
+
+
 @pytest.mark.parametrize("version", [5, 6])
 def test_floor_on_decay_and_its_zero_gradient(version):
     """Raw decays large enough that exp(-exp(w)) < 0.005: the operator uses
