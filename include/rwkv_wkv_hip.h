@@ -288,6 +288,35 @@ int wkv_sigmoid_mul_forward(void *stream, size_t n, int dtype, const void *r, co
 int wkv_sigmoid_mul_backward(void *stream, size_t n, int dtype, const void *r, const void *kv, const void *gout,
                              void *gr, void *gkv);
 
+/* ---- A layer for one token per sequence (a serving loop), bf16, at most 64 rows (sequences) at a time.
+ *
+ * Products of the rows with up to 8 weight matrices in one launch:  out = f(x' W),
+ *   w        [n][k] as torch.nn.Linear keeps it, or [k][n] (k_major)
+ *   x        (rows, k);  with mix (k) non-NULL  x' = x + (shift - x) d,  d = mix, or 1 - mix with lerp (the token shift and
+ *            mixing of RWKV-v6/src/module/ChannelMix.py:31-35, RWKV-v5/src/module/TimeMix.py:295-298)
+ *   act      0 none, 1 tanh, 2 relu(.)^2, 3 sigmoid(mul) * (.)   (RWKV-v5/src/module/ChannelMix.py:48-49); mul (rows, n)
+ * k a multiple of 64, every n of 16. */
+typedef struct {
+    const void *w, *x, *shift, *mix, *mul;
+    void *out;
+    int n, k_major, lerp, act;
+} wkv_rows_product;
+int wkv_rows_products(void *stream, int rows, int k, int count, const wkv_rows_product *products);
+
+/* The v6 data-dependent mixes for single tokens (RWKV-v6/src/module/TimeMix.py:264-276): as wkv_lora_mix_forward with
+ * x, shift (rows, C), maa = HOST array of the five time_maa parameters (bf16), act (rows, 5, 32), w2 (5, 32, C) as the
+ * reference keeps it, out (5, rows, C).  C a multiple of 16. */
+int wkv_lora_mix_rows(void *stream, int rows, int C, const void *x, const void *shift, const void *const *maa, const void *act,
+                      const void *w2, void *out);
+
+/* From the projections of one token to the input of the output projection: the operator's step, ln_x and the gate
+ * (RWKV-v6/src/module/TimeMix.py:280-298, RWKV-v5/src/module/TimeMix.py:309-320).  r, k, v, gate, out (B, C) bf16;
+ * time_decay, u, ln_weight, ln_bias (C) bf16; lora (B, 64) and w2 (64, C): the v6 decay is time_decay + lora @ w2;
+ * lora NULL: time_decay (v5).  state_out may be state_in. */
+int wkv_timemix_head(void *stream, int B, int C, int H, const void *r, const void *k, const void *v, const void *gate, const void *time_decay,
+                     const void *lora, const void *w2, const void *u, const void *ln_weight, const void *ln_bias, float scale, float eps,
+                     const float *state_in, float *state_out, void *out);
+
 /* Backward of L2Wrap (RWKV-v5/src/model.py:140-148): gy (rows, V) is zero except, in every row, at the first
  * position of the row's maximum, where it is factor * mask[row] * max (mask (rows) fp32 or NULL = ones). */
 int wkv_l2wrap_backward(void *stream, int rows, int V, int dtype, float factor, const void *y, const float *mask,

@@ -11,6 +11,7 @@
 #include "cumsum_decay.hip"
 #include "block_edges.hip"
 #include "lora_mix.hip"
+#include "layer_decode.hip"
 
 using namespace wkv;
 
@@ -461,6 +462,57 @@ int wkv_ln_gate_backward(void *stream, int rows, int C, int dtype, float scale, 
     hipError_t e = WKV_BY_DTYPE(dtype, CALL);
 #undef CALL
     return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
+}
+
+int wkv_rows_products(void *stream, int row_count, int k, int count, const wkv_rows_product *products) {
+    if (row_count <= 0 || row_count > rows::MAX_ROWS || k <= 0 || k % 64 != 0 || count <= 0 || count > rows::MAX_JOBS) return WKV_ERR_DIMS;
+    if (!products) return WKV_ERR_NULL;
+    rows::Jobs jobs{};
+    jobs.count = count;
+    for (int i = 0; i < count; i++) {
+        const wkv_rows_product &p = products[i];
+        if (p.n <= 0 || p.n % 16 != 0 || (size_t)p.n * k >= (1u << 31)) return WKV_ERR_DIMS;
+        if (p.act < rows::ACT_NONE || p.act > rows::ACT_SIGMOID_MUL) return WKV_ERR_ALGO;
+        if (!p.w || !p.x || !p.out || (p.mix && !p.shift) || (p.act == rows::ACT_SIGMOID_MUL && !p.mul)) return WKV_ERR_NULL;
+        for (const void *q : {p.w, p.x, p.shift, p.mix, p.mul, (const void *)p.out})
+            if (!aligned16(q)) return WKV_ERR_ALIGN;
+        jobs.j[i] = {(const bf16 *)p.w, (const bf16 *)p.x, (const bf16 *)p.shift, (const bf16 *)p.mix, (const bf16 *)p.mul, (bf16 *)p.out,
+                     p.n, p.k_major, p.lerp, p.act};
+    }
+    return rows::rows_products_launch((hipStream_t)stream, row_count, k, jobs) == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
+}
+
+int wkv_lora_mix_rows(void *stream, int row_count, int C, const void *x, const void *shift, const void *const *maa, const void *act,
+                      const void *w2, void *out) {
+    if (row_count <= 0 || C <= 0 || C % 16 != 0) return WKV_ERR_DIMS;
+    if (!x || !shift || !maa || !act || !w2 || !out) return WKV_ERR_NULL;
+    rows::Maa m;
+    for (int j = 0; j < 5; j++) {
+        if (!maa[j]) return WKV_ERR_NULL;
+        if (!aligned16(maa[j])) return WKV_ERR_ALIGN;
+        m.p[j] = (const bf16 *)maa[j];
+    }
+    for (const void *p : {x, shift, act, w2, (const void *)out})
+        if (!aligned16(p)) return WKV_ERR_ALIGN;
+    hipLaunchKernelGGL(rows::lora_mix_rows, dim3(C / 16), dim3(320), 0, (hipStream_t)stream, row_count, C, (const bf16 *)x, (const bf16 *)shift, m,
+                       (const bf16 *)act, (const bf16 *)w2, (bf16 *)out);
+    return hipGetLastError() == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
+}
+
+int wkv_timemix_head(void *stream, int B, int C, int H, const void *r, const void *k, const void *v, const void *gate, const void *time_decay,
+                     const void *lora, const void *w2, const void *u, const void *ln_weight, const void *ln_bias, float scale, float eps,
+                     const float *state_in, float *state_out, void *out) {
+    int st = check_dims56(B, 1, C, H, WKV_BF16);
+    if (st) return st;
+    if (!r || !k || !v || !gate || !time_decay || (lora && !w2) || !u || !ln_weight || !ln_bias || !state_in || !state_out || !out) return WKV_ERR_NULL;
+    for (const void *p : {r, k, v, gate, time_decay, lora, w2, u, ln_weight, ln_bias, (const void *)state_in, (const void *)state_out, (const void *)out})
+        if (!aligned16(p)) return WKV_ERR_ALIGN;
+    st = check_state_alias(state_in, state_out, B, H, false);
+    if (st) return st;
+    hipLaunchKernelGGL(rows::timemix_head, dim3(B * H), dim3(256), 0, (hipStream_t)stream, H, (const bf16 *)r, (const bf16 *)k, (const bf16 *)v,
+                       (const bf16 *)gate, (const bf16 *)time_decay, (const bf16 *)lora, (const bf16 *)w2, (const bf16 *)u,
+                       (const bf16 *)ln_weight, (const bf16 *)ln_bias, scale, eps, state_in, state_out, (bf16 *)out);
+    return hipGetLastError() == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
 }
 
 static int check_flat(size_t n, int dtype) {

@@ -60,6 +60,9 @@ SIGNATURES = {
     "wkv_relu_square_backward": (_I, [_P, c_size_t, _I, _P, _P, _P]),
     "wkv_sigmoid_mul_forward": (_I, [_P, c_size_t, _I, _P, _P, _P]),
     "wkv_sigmoid_mul_backward": (_I, [_P, c_size_t, _I] + [_P] * 5),
+    "wkv_rows_products": (_I, [_P, _I, _I, _I, _P]),
+    "wkv_lora_mix_rows": (_I, [_P, _I, _I] + [_P] * 6),
+    "wkv_timemix_head": (_I, [_P, _I, _I, _I] + [_P] * 10 + [c_float, c_float] + [_P] * 3),
     "wkv_l2wrap_backward": (_I, [_P, _I, _I, _I, c_float, _P, _P, _P]),
 }
 
@@ -105,7 +108,8 @@ def host():
             from . import _host as module
         except ImportError as e:
             raise WKVError(f"the native host side is missing: build it first (make -C rwkv-infctx-trainer_amd/csrc): {e}") from e
-        module.bind(LIB_PATH, WKVError)
+        import torch
+        module.bind(LIB_PATH, WKVError, torch.nn.Linear, torch.nn.GroupNorm)
         _host = module
     return _host
 

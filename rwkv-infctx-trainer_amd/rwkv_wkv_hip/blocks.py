@@ -273,9 +273,14 @@ class L2Wrap(torch.autograd.Function):
 
 
 # ---- block forwards on these kernels -------------------------------------------------------------------------------
+# One token per sequence without autograd (a serving loop) takes kernels of its own, csrc/layer_decode.hip, where module
+# and inputs are plain bf16; host().*_decode answers None for every other call.
 def timemix5_forward(self, x, last_state):
     """RWKV_TimeMix._forward_cuda of v5 (RWKV-v5/src/module/TimeMix.py:286-323): returns
     (out (B,T,C), (shift_state_out (B,C), wkv_state_out (B,H,64,64)))."""
+    out = _lib.host().timemix_decode(5, self, x, last_state)
+    if out is not None:
+        return out
     B, T, C = x.shape
     H = self.n_head
     xk, xv, xr, xg = token_shift_mix(x, last_state[0], (self.time_mix_k, self.time_mix_v, self.time_mix_r, self.time_mix_g),
@@ -288,6 +293,9 @@ def timemix5_forward(self, x, last_state):
 
 def timemix6_forward(self, x, last_state):
     """RWKV_TimeMix6_0._forward_cuda (RWKV-v6/src/module/TimeMix.py:253-302)."""
+    out = _lib.host().timemix_decode(6, self, x, last_state)
+    if out is not None:
+        return out
     B, T, C = x.shape
     H = self.n_head
     (xxx,) = token_shift_mix(x, last_state[0], (self.time_maa_x,))
@@ -310,6 +318,9 @@ def timemix6_forward(self, x, last_state):
 
 def channelmix5_forward(self, x, last_state):
     """RWKV_ChannelMix.forward of v5 (RWKV-v5/src/module/ChannelMix.py:35-49)."""
+    out = _lib.host().channelmix_decode(5, self, x, last_state)
+    if out is not None:
+        return out
     xk, xr = token_shift_mix(x, last_state, (self.time_mix_k, self.time_mix_r), lerp=True)
     kv = self.value(relu_square(self.key(xk)))
     return sigmoid_mul(self.receptance(xr), kv), x[:, -1]
@@ -317,6 +328,9 @@ def channelmix5_forward(self, x, last_state):
 
 def channelmix6_forward(self, x, last_state):
     """RWKV_ChannelMix6_0.forward (RWKV-v6/src/module/ChannelMix.py:30-37)."""
+    out = _lib.host().channelmix_decode(6, self, x, last_state)
+    if out is not None:
+        return out
     xk, xr = token_shift_mix(x, last_state, (self.time_maa_k, self.time_maa_r))
     kv = self.value(relu_square(self.key(xk)))
     return sigmoid_mul(self.receptance(xr), kv), x[:, -1]

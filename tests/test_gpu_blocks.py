@@ -274,6 +274,45 @@ def test_timemix_forward_on_the_kernels_bf16_module(version):
 
 
 @pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("B,H,ffn", [(1, 1, 64), (3, 2, 448), (16, 1, 192), (17, 3, 640), (33, 2, 256), (64, 9, 2016), (65, 1, 128)])
+def test_layer_of_single_tokens(version, B, H, ffn):
+    """A serving loop's layer (one token per sequence, no autograd, bf16): row counts at the edges of the 16-row tiles, widths
+    of fewer and of more 64-deep chunks than a workgroup has wavefronts; 65 rows and ffn = 2016 take the general way.
+    Against the fp32 modules on the same rounded parameters.  Six bf16 roundings (2^-9 each, added in squares: 4.8e-3) lie
+    between input and output: 1e-2 in norm over all rows.  In one row the operator's sum over 64 keys and ln_x's mean can
+    cancel, which divides by what is left: among 64 rows some lose a digit, 4.8e-2 (the general way's worst row: 2.1e-2)."""
+    from rwkv_wkv_hip import blocks as K
+    C = 64 * H
+    g = _g(B + 10 * H)
+    bf = lambda t: t.bfloat16().float()
+    x, shift, shift2 = (bf(torch.randn(B, *n, generator=g)) for n in ((1, C), (C,), (C,)))
+    state = torch.randn(B, H, 64, 64, generator=g) * 0.1
+    tm, cm = (TimeMix5 if version == 5 else TimeMix6)(C, H, seed=8), (ChannelMix5 if version == 5 else ChannelMix6)(C, ffn, seed=9)
+    for m in (tm, cm):
+        for p in m.parameters():
+            p.data = bf(p.data)
+    if version == 5:
+        wkv = lambda B, T, C, H, s, r, k, v, w, u: O.wkv5_op(B, T, C, H, s, r, k, v, w, u)
+    else:
+        wkv = lambda B, T, C, H, r, k, v, w, u, s: O.wkv6_op(B, T, C, H, r, k, v, w, u, s)
+    gtm, gcm = copy.deepcopy(tm).cuda().bfloat16(), copy.deepcopy(cm).cuda().bfloat16()
+    with torch.no_grad():
+        a_ref, (sh_ref, s_ref) = tm(x, (shift, state), wkv)
+        y_ref, sh2_ref = cm(a_ref, shift2)
+        timemix, channelmix = (K.timemix5_forward, K.channelmix5_forward) if version == 5 else (K.timemix6_forward, K.channelmix6_forward)
+        xg, states = x.cuda().bfloat16(), (shift.cuda().bfloat16(), state.cuda())
+        a, (sh, s) = timemix(gtm, xg, states)
+        y, sh2 = channelmix(gcm, a, shift2.cuda().bfloat16())
+    assert a.dtype == y.dtype == torch.bfloat16 and a.shape == y.shape == x.shape
+    assert torch.equal(sh.float().cpu(), sh_ref) and torch.equal(sh2, a[:, -1]) and s.dtype == torch.float32
+    for name, got, ref in (("timemix", a, a_ref), ("state", s, s_ref), ("layer", y, y_ref)):
+        got, ref = got.float().cpu().reshape(B, -1), ref.reshape(B, -1)
+        rel = (got - ref).norm(dim=1) / ref.norm(dim=1)
+        assert rel.max() < 4.8e-2, f"{name}: row {int(rel.argmax())} off by {rel.max():.2e}"
+        assert (got - ref).norm() < 1e-2 * ref.norm(), f"{name}: off by {((got - ref).norm() / ref.norm()).item():.2e}"
+
+
+@pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_channelmix_forward_on_the_kernels(version, dtype):
     from rwkv_wkv_hip import blocks as K
