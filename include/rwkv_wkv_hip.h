@@ -291,11 +291,13 @@ int wkv_sigmoid_mul_backward(void *stream, size_t n, int dtype, const void *r, c
 /* ---- A layer for one token per sequence (a serving loop), bf16, at most 64 rows (sequences) at a time.
  *
  * Products of the rows with up to 8 weight matrices in one launch:  out = f(x' W),
- *   w        [n][k] as torch.nn.Linear keeps it, or [k][n] (k_major)
+ *   w        [n][k] as torch.nn.Linear keeps it; k_major: [k][n] as the LoRA parameters are kept, and the result comes in
+ *            fp32 parts (WKV_LORA_PARTS, rows, n) that the two functions below add up
  *   x        (rows, k);  with mix (k) non-NULL  x' = x + (shift - x) d,  d = mix, or 1 - mix with lerp (the token shift and
  *            mixing of RWKV-v6/src/module/ChannelMix.py:31-35, RWKV-v5/src/module/TimeMix.py:295-298)
- *   act      0 none, 1 tanh, 2 relu(.)^2, 3 sigmoid(mul) * (.)   (RWKV-v5/src/module/ChannelMix.py:48-49); mul (rows, n)
+ *   act      0 none, 1 relu(.)^2, 2 sigmoid(mul) * (.)   (RWKV-v5/src/module/ChannelMix.py:48-49; not with k_major); mul (rows, n)
  * k a multiple of 64, every n of 16. */
+#define WKV_LORA_PARTS 8
 typedef struct {
     const void *w, *x, *shift, *mix, *mul;
     void *out;
@@ -304,14 +306,15 @@ typedef struct {
 int wkv_rows_products(void *stream, int rows, int k, int count, const wkv_rows_product *products);
 
 /* The v6 data-dependent mixes for single tokens (RWKV-v6/src/module/TimeMix.py:264-276): as wkv_lora_mix_forward with
- * x, shift (rows, C), maa = HOST array of the five time_maa parameters (bf16), act (rows, 5, 32), w2 (5, 32, C) as the
- * reference keeps it, out (5, rows, C).  C a multiple of 16. */
+ * x, shift (rows, C), maa = HOST array of the five time_maa parameters (bf16), act (WKV_LORA_PARTS, rows, 5, 32) fp32 =
+ * xxx @ time_maa_w1 in parts, before the tanh, w2 (5, 32, C) as the reference keeps it, out (5, rows, C).  C a multiple of 16. */
 int wkv_lora_mix_rows(void *stream, int rows, int C, const void *x, const void *shift, const void *const *maa, const void *act,
                       const void *w2, void *out);
 
 /* From the projections of one token to the input of the output projection: the operator's step, ln_x and the gate
  * (RWKV-v6/src/module/TimeMix.py:280-298, RWKV-v5/src/module/TimeMix.py:309-320).  r, k, v, gate, out (B, C) bf16;
- * time_decay, u, ln_weight, ln_bias (C) bf16; lora (B, 64) and w2 (64, C): the v6 decay is time_decay + lora @ w2;
+ * time_decay, u, ln_weight, ln_bias (C) bf16; lora (WKV_LORA_PARTS, B, 64) fp32 in parts and w2 (64, C): the v6
+ * decay is time_decay + tanh(lora) @ w2;
  * lora NULL: time_decay (v5).  state_out may be state_in. */
 int wkv_timemix_head(void *stream, int B, int C, int H, const void *r, const void *k, const void *v, const void *gate, const void *time_decay,
                      const void *lora, const void *w2, const void *u, const void *ln_weight, const void *ln_bias, float scale, float eps,

@@ -476,7 +476,7 @@ int wkv_rows_products(void *stream, int row_count, int k, int count, const wkv_r
         if (!p.w || !p.x || !p.out || (p.mix && !p.shift) || (p.act == rows::ACT_SIGMOID_MUL && !p.mul)) return WKV_ERR_NULL;
         for (const void *q : {p.w, p.x, p.shift, p.mix, p.mul, (const void *)p.out})
             if (!aligned16(q)) return WKV_ERR_ALIGN;
-        jobs.j[i] = {(const bf16 *)p.w, (const bf16 *)p.x, (const bf16 *)p.shift, (const bf16 *)p.mix, (const bf16 *)p.mul, (bf16 *)p.out,
+        jobs.j[i] = {(const bf16 *)p.w, (const bf16 *)p.x, (const bf16 *)p.shift, (const bf16 *)p.mix, (const bf16 *)p.mul, p.out,
                      p.n, p.k_major, p.lerp, p.act};
     }
     return rows::rows_products_launch((hipStream_t)stream, row_count, k, jobs) == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
@@ -495,7 +495,7 @@ int wkv_lora_mix_rows(void *stream, int row_count, int C, const void *x, const v
     for (const void *p : {x, shift, act, w2, (const void *)out})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
     hipLaunchKernelGGL(rows::lora_mix_rows, dim3(C / 16), dim3(320), 0, (hipStream_t)stream, row_count, C, (const bf16 *)x, (const bf16 *)shift, m,
-                       (const bf16 *)act, (const bf16 *)w2, (bf16 *)out);
+                       (const float *)act, (const bf16 *)w2, (bf16 *)out);
     return hipGetLastError() == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
 }
 
@@ -510,7 +510,7 @@ int wkv_timemix_head(void *stream, int B, int C, int H, const void *r, const voi
     st = check_state_alias(state_in, state_out, B, H, false);
     if (st) return st;
     hipLaunchKernelGGL(rows::timemix_head, dim3(B * H), dim3(256), 0, (hipStream_t)stream, H, (const bf16 *)r, (const bf16 *)k, (const bf16 *)v,
-                       (const bf16 *)gate, (const bf16 *)time_decay, (const bf16 *)lora, (const bf16 *)w2, (const bf16 *)u,
+                       (const bf16 *)gate, (const bf16 *)time_decay, (const float *)lora, (const bf16 *)w2, (const bf16 *)u,
                        (const bf16 *)ln_weight, (const bf16 *)ln_bias, scale, eps, state_in, state_out, (bf16 *)out);
     return hipGetLastError() == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
 }

@@ -448,15 +448,16 @@ PyObject *py_timemix_decode(PyObject *, PyObject *const *a, Py_ssize_t n) {
     void *stream = dev.stream();
     // scratch: r, k, v, gate, the head results; v6 also the five mixes and the two LoRAs' activations
     const int64_t rows = B * C;
-    Tensor scratch = at::empty({(version == 6 ? 10 : 5) * rows + B * 224}, x.options());
+    constexpr int64_t parts = 2 * WKV_LORA_PARTS;          // (fp32 counted in bf16)
+    Tensor scratch = at::empty({(version == 6 ? 10 : 5) * rows + (version == 6 ? parts * B * 224 : 0)}, x.options());
     at::BFloat16 *q = scratch.data_ptr<at::BFloat16>();
-    at::BFloat16 *r = q, *k = r + rows, *v = k + rows, *g = v + rows, *z = g + rows, *mixes = z + rows, *act = mixes + 5 * rows, *lora = act + B * 160;
+    at::BFloat16 *r = q, *k = r + rows, *v = k + rows, *g = v + rows, *z = g + rows, *mixes = z + rows, *act = mixes + 5 * rows, *lora = act + parts * B * 160;
     Tensor out = at::empty_like(x), new_state = at::empty_like(state);
     if (version == 6) {
-        const wkv_rows_product first{w1, px, ps, maa_x, nullptr, act, 160, 1, 0, 1};
+        const wkv_rows_product first{w1, px, ps, maa_x, nullptr, act, 160, 1, 0, 0};
         check(abi.wkv_rows_products(stream, B, C, 1, &first), "wkv_rows_products");
         check(abi.wkv_lora_mix_rows(stream, B, C, px, ps, maa, act, w2, mixes), "wkv_lora_mix_rows");
-        const wkv_rows_product proj[5] = {{dw1, mixes, nullptr, nullptr, nullptr, lora, 64, 1, 0, 1},
+        const wkv_rows_product proj[5] = {{dw1, mixes, nullptr, nullptr, nullptr, lora, 64, 1, 0, 0},
                                           {wk, mixes + rows, nullptr, nullptr, nullptr, k, (int)C, 0, 0, 0},
                                           {wvv, mixes + 2 * rows, nullptr, nullptr, nullptr, v, (int)C, 0, 0, 0},
                                           {wr, mixes + 3 * rows, nullptr, nullptr, nullptr, r, (int)C, 0, 0, 0},
@@ -497,9 +498,9 @@ PyObject *py_channelmix_decode(PyObject *, PyObject *const *a, Py_ssize_t n) {
     OnDevice dev(x);
     Tensor scratch = at::empty({B * (F + C)}, x.options()), out = at::empty_like(x);
     at::BFloat16 *k = scratch.data_ptr<at::BFloat16>(), *r = k + B * F;
-    const wkv_rows_product proj[2] = {{wk, px, ps, mk, nullptr, k, (int)F, 0, lerp, 2}, {wr, px, ps, mr, nullptr, r, (int)C, 0, lerp, 0}};
+    const wkv_rows_product proj[2] = {{wk, px, ps, mk, nullptr, k, (int)F, 0, lerp, 1}, {wr, px, ps, mr, nullptr, r, (int)C, 0, lerp, 0}};
     check(abi.wkv_rows_products(dev.stream(), B, C, 2, proj), "wkv_rows_products");
-    const wkv_rows_product last{wvv, k, nullptr, nullptr, r, ptr(out), (int)C, 0, 0, 3};
+    const wkv_rows_product last{wvv, k, nullptr, nullptr, r, ptr(out), (int)C, 0, 0, 2};
     check(abi.wkv_rows_products(dev.stream(), B, F, 1, &last), "wkv_rows_products");
     return tuple(out, x.select(1, 0));
     END_HANDLE_TH_ERRORS

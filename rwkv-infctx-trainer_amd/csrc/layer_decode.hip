@@ -1,6 +1,6 @@
 // The layer of a serving loop: one token per sequence, a few rows (sequences) at a time, bf16.  What a row costs is the
 // weights, read once; as library products, element-wise passes and dtype conversions a v6 layer of one row was some 45
-// launches (H32: 526 us, of which the weights need 22 us).  Here it is seven kernels:
+// launches (H32: 560 us, of which the weights need 22 us).  Here it is seven kernels, 47 us:
 //
 //   rows_products   any number of products  out = f(x' W)  of up to 64 rows with weights of their own, in one launch;
 //                   x' may be the token-shift mix of x, formed where it is read (RWKV-v5/src/module/TimeMix.py:295-298,
@@ -21,16 +21,16 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int MAX_ROWS = 64, MAX_JOBS = 8;
 struct Job {
-    const bf16 *w;          // k_major ? [K][N] : [N][K]
+    const bf16 *w;          // [N][K], k_major: [K][N]
     const bf16 *x;          // [rows][K]
     const bf16 *shift;      // [rows][K], with mix
     const bf16 *mix;        // [K], or NULL: x as it is
     const bf16 *mul;        // [rows][N], ACT_SIGMOID_MUL
-    bf16 *out;              // [rows][N]
+    void *out;              // bf16 [rows][N]; k_major: fp32 [SPLIT][rows][N], parts of the sum
     int n, k_major, lerp, act;
 };
 struct Jobs { Job j[MAX_JOBS]; int count; };
-enum { ACT_NONE = 0, ACT_TANH = 1, ACT_RELU_SQUARE = 2, ACT_SIGMOID_MUL = 3 };
+enum { ACT_NONE = 0, ACT_RELU_SQUARE = 1, ACT_SIGMOID_MUL = 2 };
 
 __device__ __forceinline__ f4 mma(s8 a, s8 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
@@ -51,71 +51,144 @@ __device__ __forceinline__ s8 mixed(s8 x, s8 xx, s8 c, int lerp) {
     return __builtin_bit_cast(s8, p);
 }
 
-// One wavefront's share of a 16-column tile: the 64-deep chunks wv, wv + WAVES, ... of the contraction.  The weights
-// are the A operand (their columns are the MFMA's rows), the rows of x the B operand: lane (kg = lane/16, n = lane%16)
-// supplies weight row n and x row n, eight consecutive k each.
-template <int MT, int WAVES, int U, bool MIX, bool K_MAJOR>
-__device__ __forceinline__ void accumulate(const Job &job, int tile, int rows, int K, int wv, int kg, int n, f4 (&acc)[MT]) {
-    const int chunks = K / 64;
-    const bf16 *w = job.w + (K_MAJOR ? (size_t)16 * tile + n + (size_t)(8 * kg) * job.n : (size_t)(16 * tile + n) * K + 8 * kg);
-    size_t xo[MT];
+// A workgroup per 16 columns; its wavefronts share the contraction and meet in LDS.  The weights are the A operand of the
+// MFMAs (their columns are the rows there), the rows of x the B operand: lane (kg = lane/16, n = lane%16) supplies
+// weight row n and x row n, eight consecutive k each.
+//
+// Bound by the weights, so by how they are fetched.  Read in the operand's own layout (16 rows x 64 bytes an instruction)
+// they come at 3.4 TB/s; read along the rows, 512 bytes each of two, at 5.  So a wavefront takes 16 rows x 256 k at a time
+// that way into registers (two such segments in flight, used in turn) and turns them in LDS that belongs to it alone;
+// the same for the rows of x, of which only those that exist are read, and mixed on the way.
+//
+// TN columns (16, or 8 where 16 would leave compute units without a workgroup) and XL fetches of x, each fetch 512
+// consecutive elements: two rows of a segment of 256 k, or one row of 512.
+template <int TN, int XL> struct Shape {
+    static constexpr int SEG = 4096 / TN, LD = SEG + 8, PER = TN / 8;     // k of a segment, padded row in LDS, rows per fetch
+    static constexpr int XROWS = PER * XL, MT = (XROWS + 15) / 16;
+    static __device__ int row(int lane) { return lane / (SEG / 8); }
+    static __device__ int k(int lane) { return 8 * (lane % (SEG / 8)); }
+};
+template <int TN, int XL> struct Turn { uint16_t w[TN * Shape<TN, XL>::LD], x[Shape<TN, XL>::XROWS * Shape<TN, XL>::LD]; };
+
+template <int XL, bool MIX> struct Segment { s8 w[8], x[XL], shift[MIX ? XL : 1], mix; };
+template <int TN, int XL, bool MIX>
+__device__ __forceinline__ void fetch(Segment<XL, MIX> &s, const Job &job, const bf16 *w, int row0, int rows, int K, int k0, int lane) {
+    typedef Shape<TN, XL> Sh;
+    const int k = min(k0 + Sh::k(lane), K - 8);              // (past the end: read again and not used)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) xo[mt] = (size_t)min(16 * mt + n, rows - 1) * K + 8 * kg;
-    for (int c0 = wv; c0 < chunks; c0 += U * WAVES) {
-        s8 a[U][2], b[U][2][MT], bs[MIX ? U : 1][2][MT], bc[MIX ? U : 1][2];
+    for (int i = 0; i < 8; i++) s.w[i] = *reinterpret_cast<const s8 *>(w + (size_t)(Sh::PER * i) * K + k);
 #pragma unroll
-        for (int i = 0; i < U; i++) {
-            const int c = min(c0 + i * WAVES, chunks - 1);           // (a chunk past the end is read again and not used)
-#pragma unroll
-            for (int hf = 0; hf < 2; hf++) {
-                const int k = 64 * c + 32 * hf;
-                if (K_MAJOR) {
-#pragma unroll
-                    for (int e = 0; e < 8; e++) a[i][hf][e] = (short)w[(size_t)(k + e) * job.n].bits;
-                } else {
-                    a[i][hf] = *reinterpret_cast<const s8 *>(w + k);
-                }
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-                    b[i][hf][mt] = *reinterpret_cast<const s8 *>(job.x + xo[mt] + k);
-                    if (MIX) bs[i][hf][mt] = *reinterpret_cast<const s8 *>(job.shift + xo[mt] + k);
-                }
-                if (MIX) bc[i][hf] = *reinterpret_cast<const s8 *>(job.mix + 8 * kg + k);
-            }
+    for (int i = 0; i < XL; i++)
+        if (row0 + Sh::PER * i < rows) {
+            const size_t o = (size_t)min(row0 + Sh::PER * i + Sh::row(lane), rows - 1) * K + k;
+            s.x[i] = *reinterpret_cast<const s8 *>(job.x + o);
+            if (MIX) s.shift[i] = *reinterpret_cast<const s8 *>(job.shift + o);
         }
+    if (MIX) s.mix = *reinterpret_cast<const s8 *>(job.mix + k);
+}
+template <int TN, int XL, bool MIX>
+__device__ __forceinline__ void turn(const Segment<XL, MIX> &s, Turn<TN, XL> &t, const Job &job, int row0, int rows, int lane) {
+    typedef Shape<TN, XL> Sh;
+    const int o = Sh::row(lane) * Sh::LD + Sh::k(lane);
 #pragma unroll
-        for (int i = 0; i < U; i++)
-            if (c0 + i * WAVES < chunks) {
+    for (int i = 0; i < 8; i++) *reinterpret_cast<s8 *>(&t.w[Sh::PER * i * Sh::LD + o]) = s.w[i];
 #pragma unroll
-                for (int hf = 0; hf < 2; hf++)
+    for (int i = 0; i < XL; i++)
+        if (row0 + Sh::PER * i < rows)
+            *reinterpret_cast<s8 *>(&t.x[Sh::PER * i * Sh::LD + o]) = MIX ? mixed(s.x[i], s.shift[MIX ? i : 0], s.mix, job.lerp) : s.x[i];
+}
+// (lanes whose row of x does not exist repeat the last one, and those beyond 8 weight rows repeat them: rows and columns
+// of the result that nobody reads)
+template <int TN, int XL>
+__device__ __forceinline__ void multiply(const Turn<TN, XL> &t, int steps, int live, int lane, f4 (&acc)[Shape<TN, XL>::MT]) {
+    typedef Shape<TN, XL> Sh;
+    const int n = lane & 15, k = 8 * (lane >> 4);
+    int xo[Sh::MT];
 #pragma unroll
-                    for (int mt = 0; mt < MT; mt++)
-                        acc[mt] = mma(a[i][hf], MIX ? mixed(b[i][hf][mt], bs[i][hf][mt], bc[i][hf], job.lerp) : b[i][hf][mt], acc[mt]);
-            }
+    for (int mt = 0; mt < Sh::MT; mt++) xo[mt] = min(16 * mt + n, live - 1) * Sh::LD + k;
+#pragma unroll
+    for (int i = 0; i < Sh::SEG / 32; i++)
+        if (i < steps) {
+            const s8 a = *reinterpret_cast<const s8 *>(&t.w[(n % TN) * Sh::LD + k + 32 * i]);
+#pragma unroll
+            for (int mt = 0; mt < Sh::MT; mt++) acc[mt] = mma(a, *reinterpret_cast<const s8 *>(&t.x[xo[mt] + 32 * i]), acc[mt]);
+        }
+}
+// the lanes of a wavefront exchange data through LDS: program order is enough for the hardware, the compiler is told
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <int TN, int XL, int WAVES, bool MIX>
+__device__ __forceinline__ void accumulate(const Job &job, Turn<TN, XL> &t, int tile, int row0, int rows, int K, int wv, int lane,
+                                           f4 (&acc)[Shape<TN, XL>::MT]) {
+    typedef Shape<TN, XL> Sh;
+    constexpr bool TWO = XL <= 8;                            // two segments in flight where the registers allow it
+    const bf16 *w = job.w + (size_t)(TN * tile + Sh::row(lane)) * K;
+    const int step = WAVES * Sh::SEG, live = min(rows - row0, Sh::XROWS);
+    Segment<XL, MIX> a, b;
+    auto use = [&](Segment<XL, MIX> &s, int k0, int ahead) __attribute__((always_inline)) {
+        wave_sync();
+        turn<TN>(s, t, job, row0, rows, lane);
+        if (k0 + ahead < K) fetch<TN>(s, job, w, row0, rows, K, k0 + ahead, lane);
+        wave_sync();
+        multiply(t, min(Sh::SEG, K - k0) / 32, live, lane, acc);
+    };
+    const int first = wv * Sh::SEG;
+    if (first >= K) return;
+    fetch<TN>(a, job, w, row0, rows, K, first, lane);
+    if (TWO && first + step < K) fetch<TN>(b, job, w, row0, rows, K, first + step, lane);
+    for (int k0 = first; k0 < K; k0 += (TWO ? 2 : 1) * step) {
+        use(a, k0, (TWO ? 2 : 1) * step);
+        if (TWO && k0 + step < K) use(b, k0 + step, 2 * step);
+    }
+}
+// The weights of the LoRAs are kept [k][n]: two bytes at a time in the operand's layout.  Their columns are few (160 and
+// 64), so the contraction is cut into SPLIT parts for workgroups of their own (10 workgroups took 6.6 us for the 160
+// columns of a row at K 2048); whoever reads the result adds the parts.
+constexpr int SPLIT = 8;
+template <int MT, int WAVES, bool MIX>
+__device__ __forceinline__ void accumulate_k_major(const Job &job, int tile, int part, int row0, int rows, int K, int wv, int lane, f4 (&acc)[MT]) {
+    const int kg = lane >> 4, n = lane & 15, last = (part + 1) * (K / 32) / SPLIT;
+    for (int step = part * (K / 32) / SPLIT + wv; step < last; step += WAVES) {
+        const int k = 32 * step + 8 * kg;
+        s8 a;
+        const bf16 *w = job.w + (size_t)k * job.n + 16 * tile + n;
+#pragma unroll
+        for (int e = 0; e < 8; e++) a[e] = (short)w[(size_t)e * job.n].bits;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const size_t o = (size_t)min(row0 + 16 * mt + n, rows - 1) * K + k;
+            const s8 x = *reinterpret_cast<const s8 *>(job.x + o);
+            acc[mt] = mma(a, MIX ? mixed(x, *reinterpret_cast<const s8 *>(job.shift + o), *reinterpret_cast<const s8 *>(job.mix + k), job.lerp) : x, acc[mt]);
+        }
     }
 }
 
-// A workgroup per 16 columns; its wavefronts share the contraction and meet in LDS.  Bound by the weights: every
-// wavefront keeps up to 8 KB of them in flight, and the chunks of a row are dealt out so that the wavefronts of a
-// workgroup read 64 WAVES consecutive elements of it together.  (x, up to 64 rows, comes out of the caches.)
-template <int MT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void rows_products(int rows, int K, Jobs jobs) {
-    __shared__ __align__(16) f4 part[WAVES][MT][64];
-    int tile = blockIdx.x, ji = 0;
-    while (tile >= jobs.j[ji].n / 16) tile -= jobs.j[ji++].n / 16;     // (the grid is the sum of all tiles)
+template <int TN> __host__ __device__ inline int workgroups(const Job &job) { return job.k_major ? job.n / 16 * SPLIT : job.n / TN; }
+
+template <int TN, int XL, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, XL <= 2 ? 4 : 2) void rows_products(int rows, int K, Jobs jobs) {
+    constexpr int MT = Shape<TN, XL>::MT;
+    __shared__ __align__(16) Turn<TN, XL> turned[WAVES];
+    f4 (*part)[MT][64] = reinterpret_cast<f4 (*)[MT][64]>(turned);       // (used after the contraction)
+    static_assert(sizeof(turned[0]) >= MT * 64 * sizeof(f4), "the sums fit where the weights were turned");
+    int wg = blockIdx.x, ji = 0;
+    const int row0 = Shape<TN, XL>::XROWS * blockIdx.y;
+    while (wg >= workgroups<TN>(jobs.j[ji])) wg -= workgroups<TN>(jobs.j[ji++]);     // (the grid is the sum over all jobs)
     const Job job = jobs.j[ji];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, n = lane & 15;
     f4 acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) acc[mt] = f4{0.f, 0.f, 0.f, 0.f};
-    constexpr int U = MT == 1 ? 4 : 2, UM = MT == 1 ? 2 : 1;
     if (job.k_major) {
-        if (job.mix) accumulate<MT, WAVES, UM, true, true>(job, tile, rows, K, wv, kg, n, acc);
-        else accumulate<MT, WAVES, UM, false, true>(job, tile, rows, K, wv, kg, n, acc);
+        if (job.mix) accumulate_k_major<MT, WAVES, true>(job, wg / SPLIT, wg % SPLIT, row0, rows, K, wv, lane, acc);
+        else accumulate_k_major<MT, WAVES, false>(job, wg / SPLIT, wg % SPLIT, row0, rows, K, wv, lane, acc);
     } else {
-        if (job.mix) accumulate<MT, WAVES, UM, true, false>(job, tile, rows, K, wv, kg, n, acc);
-        else accumulate<MT, WAVES, U, false, false>(job, tile, rows, K, wv, kg, n, acc);
+        if (job.mix) accumulate<TN, XL, WAVES, true>(job, turned[wv], wg, row0, rows, K, wv, lane, acc);
+        else accumulate<TN, XL, WAVES, false>(job, turned[wv], wg, row0, rows, K, wv, lane, acc);
     }
+    __syncthreads();
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) part[wv][mt][lane] = acc[mt];
     __syncthreads();
@@ -123,14 +196,16 @@ __global__ __launch_bounds__(64 * WAVES) void rows_products(int rows, int K, Job
     f4 s = part[0][wv][lane];
 #pragma unroll
     for (int i = 1; i < WAVES; i++) s += part[i][wv][lane];
-    const int m = 16 * wv + n;                          // the lane holds columns 16 tile + 4 kg .. +3 of row m
+    const int m = row0 + 16 * wv + n;                   // the lane holds four consecutive columns of row m
     if (m >= rows) return;
-    const size_t o = (size_t)m * job.n + 16 * tile + 4 * kg;
     float y[4] = {s[0], s[1], s[2], s[3]};
-    if (job.act == ACT_TANH) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = tanhf(y[e]);
-    } else if (job.act == ACT_RELU_SQUARE) {
+    if (job.k_major) {
+        store4((float *)job.out + ((size_t)(wg % SPLIT) * rows + m) * job.n + 16 * (wg / SPLIT) + 4 * kg, y);
+        return;
+    }
+    if (TN == 8 && kg >= 2) return;
+    const size_t o = (size_t)m * job.n + TN * wg + 4 * kg;
+    if (job.act == ACT_RELU_SQUARE) {
 #pragma unroll
         for (int e = 0; e < 4; e++) { const float p = fmaxf(round_bf16(y[e]), 0.f); y[e] = p * p; }
     } else if (job.act == ACT_SIGMOID_MUL) {
@@ -139,14 +214,14 @@ __global__ __launch_bounds__(64 * WAVES) void rows_products(int rows, int K, Job
 #pragma unroll
         for (int e = 0; e < 4; e++) y[e] = sigmoid(q[e]) * round_bf16(y[e]);
     }
-    store4(job.out + o, y);
+    store4((bf16 *)job.out + o, y);
 }
 
 // out[j] = x + (shift - x) (maa_j + act_j w2_j): a wavefront per mix and 16 channels, whose 32-deep product is one MFMA
-// per 16 rows.  act [rows][5][32]; w2 [5][32][C].
+// per 16 rows.  act [SPLIT][rows][5][32], parts of the first LoRA product, whose tanh is taken here; w2 [5][32][C].
 struct Maa { const bf16 *p[5]; };
 __global__ __launch_bounds__(320) void lora_mix_rows(int rows, int C, const bf16 *__restrict__ x, const bf16 *__restrict__ shift,
-        Maa maa, const bf16 *__restrict__ act, const bf16 *__restrict__ w2, bf16 *__restrict__ out)
+        Maa maa, const float *__restrict__ act, const bf16 *__restrict__ w2, bf16 *__restrict__ out)
 {
     const int lane = threadIdx.x & 63, j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, n = lane & 15;
     const int c0 = 16 * blockIdx.x;
@@ -158,7 +233,18 @@ __global__ __launch_bounds__(320) void lora_mix_rows(int rows, int C, const bf16
     load4(maa.p[j] + c0 + 4 * kg, d);
     for (int m0 = 0; m0 < rows; m0 += 16) {
         const int m = m0 + n, mc = min(m, rows - 1);
-        const s8 b = *reinterpret_cast<const s8 *>(act + ((size_t)mc * 5 + j) * 32 + 8 * kg);
+        float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < SPLIT; p++) {
+            const float *q = act + (((size_t)p * rows + mc) * 5 + j) * 32 + 8 * kg;
+            const float4 lo = *reinterpret_cast<const float4 *>(q), hi = *reinterpret_cast<const float4 *>(q + 4);
+            t[0] += lo.x; t[1] += lo.y; t[2] += lo.z; t[3] += lo.w;
+            t[4] += hi.x; t[5] += hi.y; t[6] += hi.z; t[7] += hi.w;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) t[e] = tanhf(t[e]);
+        const uint4 bp = make_uint4(bf16_pack2(t[0], t[1]), bf16_pack2(t[2], t[3]), bf16_pack2(t[4], t[5]), bf16_pack2(t[6], t[7]));
+        const s8 b = __builtin_bit_cast(s8, bp);
         const size_t o = (size_t)mc * C + c0 + 4 * kg;
         float xv[4], xx[4], y[4];
         load4(x + o, xv);
@@ -171,9 +257,9 @@ __global__ __launch_bounds__(320) void lora_mix_rows(int rows, int C, const bf16
 }
 
 // One workgroup per (row, head), lane (key group, four value columns) as in decode56.  lora != NULL (v6): the raw decay
-// of the head's channels is time_decay + lora[row] w2 (64 deep); NULL (v5): time_decay itself.
+// of the head's channels is time_decay + tanh(lora[row]) w2 (64 deep), lora [SPLIT][rows][64] in parts; NULL (v5): time_decay itself.
 __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restrict__ r, const bf16 *__restrict__ k, const bf16 *__restrict__ v,
-        const bf16 *__restrict__ gate, const bf16 *__restrict__ time_decay, const bf16 *__restrict__ lora, const bf16 *__restrict__ w2,
+        const bf16 *__restrict__ gate, const bf16 *__restrict__ time_decay, const float *__restrict__ lora, const bf16 *__restrict__ w2,
         const bf16 *__restrict__ u, const bf16 *__restrict__ ln_w, const bf16 *__restrict__ ln_b, float scale, float eps,
         const float *s_in, float *s_out, bf16 *__restrict__ out)
 {
@@ -185,11 +271,19 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
     for (int i = 0; i < 4; i++) S[i] = *reinterpret_cast<const float4 *>(s_in + so + (kq + 16 * i) * HEAD + c4);
     {
         const int ch = tid & 63, q = tid >> 6;
-        float a = 0.f;
+        float a = 0.f, w2v[16];
         if (lora) {
 #pragma unroll
-            for (int e = 0; e < 16; e++)
-                a = fmaf(to_float(lora[(size_t)row * 64 + 16 * q + e]), to_float(w2[(size_t)(16 * q + e) * C + h * HEAD + ch]), a);
+            for (int e = 0; e < 16; e++) w2v[e] = to_float(w2[(size_t)(16 * q + e) * C + h * HEAD + ch]);
+            if (tid < HEAD) {
+                float t = 0.f;
+#pragma unroll
+                for (int p = 0; p < SPLIT; p++) t += lora[((size_t)p * (gridDim.x / H) + row) * HEAD + tid];
+                dec[tid] = tanhf(t);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 16; e++) a = fmaf(dec[16 * q + e], w2v[e], a);
         }
         part[q][ch] = a;
         __syncthreads();
@@ -235,20 +329,20 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
     out[base + tid] = from_float<bf16>(z * g * sigmoid(g));
 }
 
-// Sixteen wavefronts per tile where the tiles do not fill the compute units, eight otherwise: the wavefronts' number is
-// what keeps memory requests in flight, and meeting in LDS costs more the more of them meet.
+// Eight wavefronts per workgroup where the workgroups do not fill the compute units twice over, four (of which several
+// share a compute unit) otherwise.  One or two rows: 8 columns per workgroup where 16 would leave compute units idle.
 static hipError_t rows_products_launch(hipStream_t s, int rows, int K, const Jobs &jobs) {
-    int tiles = 0;
-    for (int i = 0; i < jobs.count; i++) tiles += jobs.j[i].n / 16;
-    const bool wide = tiles < 2 * cu_count();
-#define WKV_ROWS(MT)                                                                                                  \
-    do {                                                                                                              \
-        if (wide) hipLaunchKernelGGL((rows_products<MT, 16>), dim3(tiles), dim3(1024), 0, s, rows, K, jobs);          \
-        else hipLaunchKernelGGL((rows_products<MT, 8>), dim3(tiles), dim3(512), 0, s, rows, K, jobs);                 \
-    } while (0)
-    if (rows <= 16) WKV_ROWS(1);
-    else if (rows <= 32) WKV_ROWS(2);
-    else WKV_ROWS(4);
+    int wgs16 = 0, wgs8 = 0;
+    for (int i = 0; i < jobs.count; i++) { wgs16 += workgroups<16>(jobs.j[i]); wgs8 += workgroups<8>(jobs.j[i]); }
+    const bool wide = wgs16 < 2 * cu_count();
+#define WKV_ROWS(TN, XL, WAVES)                                                                                        \
+    hipLaunchKernelGGL((rows_products<TN, XL, WAVES>), dim3(TN == 16 ? wgs16 : wgs8, (rows + TN * XL / 8 - 1) / (TN * XL / 8)), \
+                       dim3(64 * WAVES), 0, s, rows, K, jobs)
+    if (rows > 16) WKV_ROWS(16, 16, 4);    // (the LDS of more wavefronts does not fit; 33..64 rows: two workgroups read a tile's weights together)
+    else if (rows > 2) { if (wide) WKV_ROWS(16, 8, 8); else WKV_ROWS(16, 8, 4); }
+    else if (wgs16 < cu_count()) WKV_ROWS(8, 2, 8);
+    else if (wide) WKV_ROWS(16, 1, 8);
+    else WKV_ROWS(16, 1, 4);
 #undef WKV_ROWS
     return hipGetLastError();
 }
