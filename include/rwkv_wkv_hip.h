@@ -57,8 +57,15 @@ typedef enum { WKV_F32 = 0, WKV_BF16 = 1, WKV_F16 = 2 } wkv_dtype;
                                  the reference's w.float() does.  WKV_ERR_ALGO where the call would run token by
                                  token */
 
+#define WKV_NO_CHECKPOINTS 8u /* forward only: no backward call will follow, the workspace is one of at least
+                                 wkv56_forward_scratch() bytes that holds the summaries of the time split alone.
+                                 (Without any workspace a forward call runs every sequence in one piece.) */
+
+#define WKV_W_F16 16u         /* as WKV_W_BF16, for fp16 streams and WKV_ALGO_AUTO with two tokens or more */
+
 /* algorithm selector */
-#define WKV_ALGO_AUTO      0  /* chunked where it applies, else recurrent */
+#define WKV_ALGO_AUTO      0  /* blocked where it applies (with WKV_FLOOR_DECAY: bf16 streams as WKV_ALGO_CHUNKED, fp32
+                                 and fp16 streams with fp32 products), else recurrent */
 #define WKV_ALGO_RECURRENT 1  /* per-token fp32 recurrence, any T, any dtype */
 #define WKV_ALGO_CHUNKED   2  /* 64-token chunks on the matrix cores, bf16 operands */
 
@@ -109,16 +116,17 @@ int wkv_profile_end(float *ms, int capacity);
  * full state gradient).
  */
 /* Workspaces: forward needs none; if it is given one of at least
- * wkv6_forward_workspace() bytes (the chunked algorithm only) it leaves state
+ * wkv6_forward_workspace() bytes (the blocked algorithms only) it leaves state
  * checkpoints there.  Passing that same buffer, sized by
  * wkv6_backward_workspace() (>= the forward size), to backward together with
  * WKV_CHECKPOINTS_VALID saves backward one sweep over k, v, w. */
-/* state_out == state_in (the state updated in place) is accepted by the per-token algorithm and by the chunked one
+/* state_out == state_in (the state updated in place) is accepted for fp32 and fp16 streams, and by the chunked algorithm
  * whenever the plan cuts no sequence of the shape into time segments (B*H at least the number of compute units, or
  * WKV_TUNE_SEGMENTS 1); where it does (short batches, e.g. the 7B shape with B = 1), and for buffers that overlap
  * without being the same, the call returns WKV_ERR_ALIAS and the caller keeps two state buffers and alternates.
  * The same holds for wkv5_forward and wkv6_forward_noalloc. */
 size_t wkv6_forward_workspace(int B, int T, int C, int H, int dtype, int algo);
+size_t wkv56_forward_scratch(int B, int T, int C, int H, int dtype, int algo);      /* see WKV_NO_CHECKPOINTS; may be 0 */
 int wkv6_forward(void *stream, int B, int T, int C, int H, int dtype, unsigned flags, int algo,
                  const void *r, const void *k, const void *v, const void *w, const float *u,
                  const float *state_in, void *y, float *state_out,

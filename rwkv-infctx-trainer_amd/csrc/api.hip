@@ -6,6 +6,7 @@
 #include "wkv56_recurrent.hip"
 #include "wkv56_decode.hip"
 #include "wkv56_chunked.hip"
+#include "wkv56_f32.hip"
 #include "wkv56_noalloc.hip"
 #include "wkv4.hip"
 #include "cumsum_decay.hip"
@@ -28,15 +29,23 @@ int check_dims56(int B, int T, int C, int H, int dtype) {
     return WKV_OK;
 }
 
-// the blocked matrix-core path takes bf16 streams with the decay floor switched on
-// (whose range analysis relies on the decay floor); everything else goes token by token
-int pick_algo56(int algo, int T, int dtype, unsigned flags) {
-    (void)T;
+// The blocked kernels rely on the decay floor (whose range analysis they need).  With it bf16 streams take those of
+// wkv56_chunked.hip, fp32 and fp16 streams of two tokens or more those of wkv56_f32.hip (ALGO_F32, not a selector of the
+// ABI); everything else goes token by token.
+constexpr int ALGO_F32 = 3;
+int pick_algo56(int algo, int T, int C, int dtype, unsigned flags) {
+    // (the fp32 kernels' stores count on offsets of the last step's missing tokens not wrapping)
+    const bool can_f32 = T > 1 && (flags & WKV_FLOOR_DECAY) && (long long)(T + 64) * C < (1ll << 30);
     const bool can_chunk = dtype == WKV_BF16 && (flags & WKV_FLOOR_DECAY);
-    if (algo == WKV_ALGO_AUTO) return can_chunk ? WKV_ALGO_CHUNKED : WKV_ALGO_RECURRENT;
+    if (algo == WKV_ALGO_AUTO) return can_chunk ? WKV_ALGO_CHUNKED : can_f32 ? ALGO_F32 : WKV_ALGO_RECURRENT;
     if (algo == WKV_ALGO_RECURRENT) return algo;
     if (algo == WKV_ALGO_CHUNKED) return can_chunk ? algo : WKV_ERR_ALGO;
     return WKV_ERR_ALGO;
+}
+// whether the decay's type (flags) is one the algorithm reads
+bool decay_type_fits(int a, int dtype, bool per_token, unsigned flags) {
+    if ((flags & WKV_W_BF16) && (!per_token || a != WKV_ALGO_CHUNKED)) return false;
+    return !(flags & WKV_W_F16) || (per_token && a == ALGO_F32 && dtype == WKV_F16);
 }
 
 // state_out == state_in (the state updated in place, as a serving loop does) is fine whenever every workgroup reads
@@ -59,23 +68,27 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
     for (const void *p : {r, k, v, (const void *)w, (const void *)u, (const void *)state_in, (const void *)y,
                           (const void *)state_out})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
-    const int a = pick_algo56(algo, T, dtype, flags);
+    const int a = pick_algo56(algo, T, C, dtype, flags);
     if (a < 0) return a;
     st = check_state_alias(state_in, state_out, B, H, a == WKV_ALGO_CHUNKED && chunked::splits_time(B * H, T));
     if (st) return st;
-    const bool w16 = (flags & WKV_W_BF16) != 0;
-    if (w16 && (!per_token || a != WKV_ALGO_CHUNKED)) return WKV_ERR_ALGO;
-    if (a == WKV_ALGO_CHUNKED) {
+    if (!decay_type_fits(a, dtype, per_token, flags)) return WKV_ERR_ALGO;
+    const bool w16 = (flags & (WKV_W_BF16 | WKV_W_F16)) != 0;
+    const int floor_decay = (flags & WKV_FLOOR_DECAY) ? 1 : 0;
+    if (a != WKV_ALGO_RECURRENT) {
         // with a workspace the state at the start of every 64-token step is left there for backward
+        const bool keep = !(flags & WKV_NO_CHECKPOINTS);
         if (workspace) {
             if (!aligned16(workspace)) return WKV_ERR_ALIGN;
-            if (workspace_bytes < chunked::forward_workspace(B, T, H)) return WKV_ERR_WORKSPACE;
+            if (workspace_bytes < (keep ? chunked::forward_workspace(B, T, H) : chunked::forward_scratch(B, T, H))) return WKV_ERR_WORKSPACE;
         }
-        hipError_t e = chunked::forward_launch((hipStream_t)stream, per_token, w16, B, T, C, H, r, k, v, w, u, state_in, y,
-                                               state_out, workspace, (flags & WKV_FLOOR_DECAY) ? 1 : 0);
+        hipError_t e = a == WKV_ALGO_CHUNKED
+                           ? chunked::forward_launch((hipStream_t)stream, per_token, w16, B, T, C, H, r, k, v, w, u, state_in, y, state_out,
+                                                     workspace, keep, floor_decay)
+                           : f32::forward_launch((hipStream_t)stream, dtype, per_token, w16, B, T, C, H, r, k, v, w, u, state_in, y, state_out,
+                                                 workspace, keep, floor_decay);
         return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
     }
-    const int floor_decay = (flags & WKV_FLOOR_DECAY) ? 1 : 0;
     hipError_t e = T == 1 ? decode_launch((hipStream_t)stream, dtype, WKV_F32, per_token, B * H, H, r, k, v, w, u, state_in, y, state_out, floor_decay)
                           : recurrent_forward((hipStream_t)stream, dtype, per_token, B, T, C, H, r, k, v, (const float *)w, u, state_in, y,
                                               state_out, floor_decay);
@@ -85,15 +98,15 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
 // (sizes are for the larger of the two algorithms a call with these arguments can take)
 size_t forward56_workspace(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
-    return pick_algo56(algo, T, dtype, WKV_FLOOR_DECAY) == WKV_ALGO_CHUNKED ? chunked::forward_workspace(B, T, H) : 0;
+    const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
+    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_workspace(B, T, H) : 0;
 }
 
 size_t backward56_workspace(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
     const size_t rec = recurrent_backward_workspace(B, T, C);
-    if (pick_algo56(algo, T, dtype, WKV_FLOOR_DECAY) == WKV_ALGO_CHUNKED)
-        return std::max(rec, chunked::backward_workspace(B, T, C, H));
-    return rec;
+    const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
+    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? std::max(rec, chunked::backward_workspace(B, T, C, H)) : rec;
 }
 
 int backward56(bool per_token, void *stream, int B, int T, int C, int H, int dtype, unsigned flags, int algo,
@@ -107,13 +120,13 @@ int backward56(bool per_token, void *stream, int B, int T, int C, int H, int dty
                           (const void *)gstate_out, (const void *)gr, (const void *)gk, (const void *)gv,
                           (const void *)gw, (const void *)gu, (const void *)gstate_in, (const void *)workspace})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
-    const int a = pick_algo56(algo, T, dtype, flags);
+    const int a = pick_algo56(algo, T, C, dtype, flags);
     if (a < 0) return a;
-    const bool w16 = (flags & WKV_W_BF16) != 0;
-    if (w16 && (!per_token || a != WKV_ALGO_CHUNKED)) return WKV_ERR_ALGO;
+    if (!decay_type_fits(a, dtype, per_token, flags)) return WKV_ERR_ALGO;
+    const bool w16 = (flags & (WKV_W_BF16 | WKV_W_F16)) != 0;
     if (!workspace) return WKV_ERR_NULL;
-    if (workspace_bytes < (a == WKV_ALGO_CHUNKED ? chunked::backward_workspace(B, T, C, H)
-                                                 : recurrent_backward_workspace(B, T, C)))
+    if (workspace_bytes < (a == WKV_ALGO_RECURRENT ? recurrent_backward_workspace(B, T, C)
+                                                   : chunked::backward_workspace(B, T, C, H)))
         return WKV_ERR_WORKSPACE;
     if (gstate_in && gstate_out) {      // several workgroups share a head's state gradient: some read gstate_out after
                                         // others have written gstate_in, so the two are never the same memory
@@ -125,6 +138,11 @@ int backward56(bool per_token, void *stream, int B, int T, int C, int H, int dty
         hipError_t e = chunked::backward_launch((hipStream_t)stream, per_token, w16, B, T, C, H, r, k, v, w, u, state_in, gy,
                                                 gstate_out, gr, gk, gv, gw, gu, gstate_in, workspace,
                                                 (flags & WKV_CHECKPOINTS_VALID) != 0, (flags & WKV_FLOOR_DECAY) ? 1 : 0);
+        return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
+    }
+    if (a == ALGO_F32) {
+        hipError_t e = f32::backward_launch((hipStream_t)stream, dtype, per_token, w16, B, T, C, H, r, k, v, w, u, state_in, gy, gstate_out, gr, gk,
+                                            gv, gw, gu, gstate_in, workspace, (flags & WKV_CHECKPOINTS_VALID) != 0, 1);
         return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
     }
     hipError_t e = recurrent_backward((hipStream_t)stream, dtype, per_token, B, T, C, H, r, k, v, (const float *)w, u, state_in, gy,
@@ -162,7 +180,7 @@ const char *wkv_strerror(int status) {
 int wkv_abi_version(void) { return 2; }
 
 int wkv_init(void) {
-    if (chunked::init_kernels() != hipSuccess) return WKV_ERR_LAUNCH;
+    if (chunked::init_kernels() != hipSuccess || f32::init_kernels() != hipSuccess) return WKV_ERR_LAUNCH;
     return chunked::init_static_scratch() == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;      // (for the current device)
 }
 
@@ -212,6 +230,11 @@ int wkv_profile_end(float *ms, int capacity) {
 size_t wkv6_forward_workspace(int B, int T, int C, int H, int dtype, int algo) {
     return forward56_workspace(B, T, C, H, dtype, algo);
 }
+size_t wkv56_forward_scratch(int B, int T, int C, int H, int dtype, int algo) {
+    if (check_dims56(B, T, C, H, dtype)) return 0;
+    const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
+    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_scratch(B, T, H) : 0;
+}
 size_t wkv5_forward_workspace(int B, int T, int C, int H, int dtype, int algo) {
     return forward56_workspace(B, T, C, H, dtype, algo);
 }
@@ -252,7 +275,7 @@ int wkv6_forward_noalloc(void *stream, int B, int T, int C, int H, int dtype, un
     for (const void *p : {r, k, v, (const void *)w, (const void *)u, (const void *)state_in, (const void *)y,
                           (const void *)state_out})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
-    if (pick_algo56(WKV_ALGO_CHUNKED, T, dtype, flags) != WKV_ALGO_CHUNKED) return WKV_ERR_ALGO;
+    if (pick_algo56(WKV_ALGO_CHUNKED, T, C, dtype, flags) != WKV_ALGO_CHUNKED) return WKV_ERR_ALGO;
     st = check_state_alias(state_in, state_out, B, H, chunked::splits_time(B * H, T));
     if (st) return st;
     hipError_t e = chunked::forward_static_launch((hipStream_t)stream, true, (flags & WKV_W_BF16) != 0, B, T, C, H, r, k, v, w,

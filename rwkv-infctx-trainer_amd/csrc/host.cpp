@@ -26,7 +26,7 @@ namespace {
 
 #define WKV_ABI(X)                                                                                                          \
     X(wkv_strerror) X(wkv5_forward) X(wkv6_forward) X(wkv5_forward_workspace) X(wkv6_forward_workspace) X(wkv5_backward)      \
-    X(wkv6_backward) X(wkv5_backward_workspace) X(wkv6_backward_workspace) X(wkv6_decode) X(wkv4_forward) X(wkv4_backward)    \
+    X(wkv6_backward) X(wkv5_backward_workspace) X(wkv6_backward_workspace) X(wkv56_forward_scratch) X(wkv6_decode) X(wkv4_forward) X(wkv4_backward)    \
     X(wkv4_checkpoint_bytes) X(wkv4_backward_workspace) X(wkv_rows_products) X(wkv_lora_mix_rows) X(wkv_timemix_head)
 struct {
 #define X(name) decltype(&::name) name = nullptr;
@@ -90,7 +90,7 @@ size_t backward_bytes(int version, const Dims &d, int dt, int algo) {
     return (version == 5 ? abi.wkv5_backward_workspace : abi.wkv6_backward_workspace)(d.B, d.T, d.C, d.H, dt, algo);
 }
 unsigned flags_of(const Dims &d, const Tensor &w) {
-    return (d.T > 1 ? WKV_FLOOR_DECAY : 0u) | (w.scalar_type() == at::kBFloat16 ? WKV_W_BF16 : 0u);
+    return (d.T > 1 ? WKV_FLOOR_DECAY : 0u) | (w.scalar_type() == at::kBFloat16 ? WKV_W_BF16 : w.scalar_type() == at::kHalf ? WKV_W_F16 : 0u);
 }
 
 struct Forward56 { Tensor y, state, ws; };
@@ -110,17 +110,20 @@ Forward56 forward56(int version, const Dims &d, int algo, const Tensor &r, const
         return o;
     }
     size_t n = 0;
-    if (keep && (n = forward_bytes(version, d, dt, algo)) > 0) {
-        n = std::max(n, backward_bytes(version, d, dt, algo));
-        o.ws = bytes(n, r);
+    unsigned flags = flags_of(d, w);
+    Tensor scratch;
+    if (keep) {
+        if ((n = forward_bytes(version, d, dt, algo)) > 0) o.ws = scratch = bytes(std::max(n, backward_bytes(version, d, dt, algo)), r);
+    } else if ((n = abi.wkv56_forward_scratch(d.B, d.T, d.C, d.H, dt, algo)) > 0 && !out_state.is_same(s)) {
+        flags |= WKV_NO_CHECKPOINTS;          // the time split's summaries; none where no sequence is cut
+        scratch = bytes(n, r);
     }
-    const unsigned flags = flags_of(d, w);
     if (version == 5)
         check(abi.wkv5_forward(dev.stream(), d.B, d.T, d.C, d.H, dt, flags, algo, ptr(r), ptr(k), ptr(v), fptr(w), fptr(u), fptr(s),
-                               ptr(o.y), fptr(o.state), ptr(o.ws), o.ws.defined() ? o.ws.numel() : 0), "wkv5_forward");
+                               ptr(o.y), fptr(o.state), ptr(scratch), scratch.defined() ? scratch.numel() : 0), "wkv5_forward");
     else
         check(abi.wkv6_forward(dev.stream(), d.B, d.T, d.C, d.H, dt, flags, algo, ptr(r), ptr(k), ptr(v), ptr(w), fptr(u), fptr(s),
-                               ptr(o.y), fptr(o.state), ptr(o.ws), o.ws.defined() ? o.ws.numel() : 0), "wkv6_forward");
+                               ptr(o.y), fptr(o.state), ptr(scratch), scratch.defined() ? scratch.numel() : 0), "wkv6_forward");
     return o;
 }
 
@@ -146,14 +149,14 @@ Backward56 backward56(int version, const Dims &d, int algo, const Tensor &r, con
     return g;
 }
 
-// The raw decay in the type the kernels take: WKV5's is fp32; WKV6's is read as it is where the call takes the blocked
-// algorithm in bf16 (as the reference widens it inside, RWKV-v6/src/module/TimeMix.py:50), or is one token without a
-// backward, and is widened here otherwise.
+// The raw decay in the type the kernels take: WKV5's is fp32; WKV6's is read as it is, in the type of the streams, where
+// the call takes a blocked algorithm (the reference widens it, RWKV-v6/src/module/TimeMix.py:50), or is one token without
+// a backward, and is widened here otherwise.
 Tensor decay_operand(int version, const Dims &d, int algo, const Tensor &r, const Tensor &w, bool keep) {
     if (version == 5 || w.scalar_type() == at::kFloat) return w;
     if (w.scalar_type() == r.scalar_type()) {
         if (d.T == 1 && !keep) return w;
-        if (d.T > 1 && w.scalar_type() == at::kBFloat16 && forward_bytes(6, d, WKV_BF16, algo) > 0) return w;
+        if (d.T > 1 && forward_bytes(6, d, dtype_code(r), algo) > 0) return w;
     }
     return w.to(at::kFloat);
 }

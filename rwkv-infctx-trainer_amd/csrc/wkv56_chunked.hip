@@ -1440,21 +1440,28 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     }
 }
 
-// Sums the per-(batch, segment) partial sums of gu (gw) in a fixed order.  The (batch, head) pairs below nA ran as
-// one segment and left theirs in `one` [b][C]; the others ran as nseg segments and left theirs in `many`
-// [(b*nseg + seg)][C].
-__global__ void sum_partials(int B, int H, int nA, int nseg, const float *__restrict__ one, const float *__restrict__ many,
-                             float *__restrict__ out) {
+// Sums the per-(batch, segment) partial sums of gu (grid row 0) and gw (row 1, time-invariant decay only) in a fixed
+// order.  The (batch, head) pairs below nA ran as one segment and left theirs in `one` [b][C]; the others ran as nseg
+// segments and left theirs in `many` [(b*nseg + seg)][C].
+struct Partials { const float *one, *many; float *out; };
+__global__ void sum_partials(int B, int H, int nA, int nseg, Partials gu, Partials gw) {
+    const Partials p = blockIdx.y ? gw : gu;
     const int c = blockIdx.x * blockDim.x + threadIdx.x, C = H * HEAD;
     if (c >= C) return;
     const int h = c / HEAD;
     float sum = 0.f;
     for (int b = 0; b < B; b++) {
-        if (b * H + h < nA) sum += one[(size_t)b * C + c];
+        if (b * H + h < nA) sum += p.one[(size_t)b * C + c];
         else
-            for (int x = 0; x < nseg; x++) sum += many[(size_t)(b * nseg + x) * C + c];
+            for (int x = 0; x < nseg; x++) sum += p.many[(size_t)(b * nseg + x) * C + c];
     }
-    out[c] = sum;
+    p.out[c] = sum;
+}
+static hipError_t sum_partials_launch(hipStream_t s, int B, int C, int H, int nA, int nseg, const float *gu_one, const float *gu_many, float *gu,
+                                      const float *gw_one, const float *gw_many, float *gw) {      // gw_one == nullptr: gu alone
+    hipLaunchKernelGGL(sum_partials, dim3((C + 255) / 256, gw_one ? 2 : 1), dim3(256), 0, s, B, H, nA, nseg, Partials{gu_one, gu_many, gu},
+                       Partials{gw_one, gw_many, gw});
+    return hipGetLastError();
 }
 
 // ------------------------------------------------------------------ launchers --
@@ -1550,6 +1557,7 @@ static Layout layout(int B, int Tlen, int C, int H, const GroupPlan &gp) {
 // true when the plan in force cuts some sequence of this shape into time segments
 bool splits_time(int BH, int Tlen) { return plan_groups(BH, Tlen).b.nseg > 1; }
 size_t forward_workspace(int B, int Tlen, int H) { return layout(B, Tlen, H * HEAD, H, plan_groups(B * H, Tlen)).forward_total; }
+size_t forward_scratch(int B, int Tlen, int H) { return part_bytes(B * H, plan_groups(B * H, Tlen)); }
 size_t backward_workspace(int B, int Tlen, int C, int H) { return layout(B, Tlen, C, H, plan_groups(B * H, Tlen)).total; }
 
 // The 16-wavefront kernels use more LDS than a kernel gets by default.  Raising the limit is a property of the loaded
@@ -1623,15 +1631,16 @@ hipError_t forward_launch(hipStream_t s, bool per_token, bool w16, int B, int Tl
     return hipGetLastError();
 }
 
-// forward with a caller's workspace (or none: one piece per sequence, no checkpoints)
+// forward with a caller's workspace (or none: one piece per sequence, no checkpoints); keep: the workspace takes the
+// checkpoints too, else the piece summaries alone
 hipError_t forward_launch(hipStream_t s, bool per_token, bool w16, int B, int Tlen, int C, int H, const void *r, const void *k,
                           const void *v, const void *w, const float *u, const float *s_in, void *y, float *s_out,
-                          void *workspace, int floor_decay) {
+                          void *workspace, bool keep, int floor_decay) {
     const GroupPlan gp = plan_groups(B * H, Tlen);
     const Layout L = layout(B, Tlen, C, H, gp);
     char *ws = (char *)workspace;
-    return forward_launch(s, per_token, w16, B, Tlen, C, H, r, k, v, w, u, s_in, y, s_out, ws ? (float *)(ws + L.ckpt) : nullptr,
-                          (ws && gp.b.nseg > 1) ? (float *)(ws + L.part) : nullptr, gp, floor_decay);
+    return forward_launch(s, per_token, w16, B, Tlen, C, H, r, k, v, w, u, s_in, y, s_out, ws && keep ? (float *)(ws + L.ckpt) : nullptr,
+                          (ws && gp.b.nseg > 1) ? (float *)(ws + (keep ? L.part : 0)) : nullptr, gp, floor_decay);
 }
 
 hipError_t backward_launch(hipStream_t s, bool per_token, bool w16, int B, int Tlen, int C, int H, const void *r, const void *k,
@@ -1696,11 +1705,7 @@ hipError_t backward_launch(hipStream_t s, bool per_token, bool w16, int B, int T
     prof_end(KID_CHUNK_BACKWARD, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sum_partials, dim3((C + 255) / 256), dim3(256), 0, s, B, H, gp.nA, pl.nseg, gu_one, gu_many, gu);
-    if (!per_token)
-        hipLaunchKernelGGL(sum_partials, dim3((C + 255) / 256), dim3(256), 0, s, B, H, gp.nA, pl.nseg, gw_one, gw_many,
-                           (float *)gw);
-    return hipGetLastError();
+    return sum_partials_launch(s, B, C, H, gp.nA, pl.nseg, gu_one, gu_many, gu, per_token ? nullptr : gw_one, gw_many, (float *)gw);
 }
 
 }  // namespace chunked

@@ -32,6 +32,7 @@ SIGNATURES = {
     "wkv_profile_begin": (_I, [_I, _I]),
     "wkv_profile_end": (_I, [_P, _I]),
     "wkv6_forward_workspace": (c_size_t, [_I] * 6),
+    "wkv56_forward_scratch": (c_size_t, [_I] * 6),
     "wkv6_forward": (_I, [_P, _I, _I, _I, _I, _I, c_uint, _I] + [_P] * 8 + [_P, c_size_t]),
     "wkv6_decode": (_I, [_P] + [_I] * 5 + [_P] * 8),
     "wkv6_forward_noalloc": (_I, [_P, _I, _I, _I, _I, _I, c_uint] + [_P] * 8),

@@ -642,3 +642,70 @@ def test_chunked_random_sweep(case):
     if regime == "floor":
         hit_gw = got["gw"].float().cpu()[hit]
         assert (hit_gw == 0).all(), "no gradient where the floor holds"
+
+
+# --------------------------------------------- blocked path with fp32 products --
+@pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("B,H,T,nseg,pps,regime", [
+    (1, 1, 2, 0, 0, "fast"), (2, 3, 15, 0, 0, "slow"), (1, 2, 63, 0, 0, "floor"), (3, 1, 64, 0, 0, "fast"), (1, 3, 65, 1, 0, "floor"),
+    (2, 2, 200, 2, 0, "fast"), (1, 2, 1000, 3, 0, "slow"), (1, 5, 832, 5, 1, "fast"), (2, 1, 1344, 4, 3, "slow"), (1, 2, 700, 0, 0, "floor")])
+def test_f32_blocked(version, dtype, B, H, T, nseg, pps, regime):
+    """fp32 and fp16 streams of two tokens or more: one step and several, ragged lengths, time splits with early stops and
+    without, decays at the floor; the outputs that stay fp32 also within 1e-4 of the token-by-token kernels, which do the
+    same multiply-adds in another order (fp32 sums over T <= 1344 tokens: 2^-24 sqrt(T) = 2e-6 of the rms on average, the
+    decay gradient a difference of sums some ten times its size, the worst of 10^5 elements five times the average)."""
+    from rwkv_wkv_hip import _lib, configs
+    L = _lib.lib()
+    wl = configs.make(1 if version == 5 else 3, B=B, T=T, C=64 * H, H=H, dtype=dtype, seed=6000 + T)
+    w = wl.tensors["w"]
+    if regime == "slow" and version == 6:
+        w -= 4.0
+    elif regime == "floor":
+        hit = torch.rand(w.shape, generator=torch.Generator().manual_seed(T)) < 0.3
+        w[hit] = 2.5
+    assert L.wkv_tune(_lib.TUNE_SEGMENTS, nseg) == 0 and L.wkv_tune(_lib.TUNE_PIECE_STEPS, pps) == 0
+    try:
+        got = run_gpu56(version, wl)
+    finally:
+        assert L.wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0 and L.wkv_tune(_lib.TUNE_PIECE_STEPS, 0) == 0
+    compare(got, run_oracle56(version, wl), 1e-3 if dtype == torch.float32 else 2e-2, f"f32 blocked {regime}")
+    tokens = run_gpu56(version, wl, algo="recurrent")
+    for n in NAMES:
+        if got[n].dtype == torch.float32:
+            assert_close(got[n], tokens[n], 1e-4, f"against token by token: {n}")
+    if regime == "floor":
+        assert (got["gw"].cpu()[hit] == 0).all(), "no gradient where the floor holds"
+
+
+@pytest.mark.parametrize("T,nseg", [(50, 0), (520, 3)])
+def test_f32_blocked_fp16_decay_and_scratch(T, nseg):
+    """fp16 raw decay read as it is (its gradient comes back in fp16), and a forward call that keeps no checkpoints: the
+    same y and state whether its sequences are cut in time (with scratch for the summaries) or not (state in place)."""
+    import rwkv_wkv_hip as W
+    from rwkv_wkv_hip import _lib, configs
+    L = _lib.lib()
+    wl = configs.make(3, B=1, T=T, C=192, H=3, dtype=torch.float16, seed=77)
+    wl.tensors["w"] = wl.tensors["w"].half()
+    ref = run_oracle56(6, _with(wl, w=wl.tensors["w"].float()))
+    assert L.wkv_tune(_lib.TUNE_SEGMENTS, nseg) == 0
+    try:
+        got = run_gpu56(6, wl)
+        g = {n: x.to(dev()) for n, x in wl.tensors.items()}
+        with torch.no_grad():
+            y, s = W.WKV_6.apply(1, T, 192, 3, g["r"], g["k"], g["v"], g["w"], g["u"], g["state"])
+            st = g["state"].clone()
+            y2 = W.RUN_WKV6STATE_CUDA(1, T, 192, 3, g["r"], g["k"], g["v"], g["w"], g["u"], st)
+    finally:
+        assert L.wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0
+    assert got["gw"].dtype == torch.float16
+    compare(got, ref, 2e-2, "fp16 decay")
+    for name, a, b in (("y", y, ref["y"]), ("state", s, ref["state"]), ("y in place", y2, ref["y"]), ("state in place", st, ref["state"])):
+        assert_close(a, b, 2e-2, name)
+
+
+def _with(wl, **tensors):
+    import copy
+    other = copy.copy(wl)
+    other.tensors = dict(wl.tensors, **tensors)
+    return other
