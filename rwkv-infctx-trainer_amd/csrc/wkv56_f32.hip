@@ -100,39 +100,50 @@ __device__ __forceinline__ float half_exponents(const float (&lw)[N], float (&x)
     }
     return s;          // log2 of the half's decay
 }
-// sums over the 64 lanes of eight per-token values, left as four partial sums per token
-__device__ __forceinline__ void store_row_sums(const float (&p)[8], float (*out)[4], int lane) {
+// sums over the 64 lanes of eight per-token values, left as the four partial sums of the lane groups: part[group][token]
+__device__ __forceinline__ void store_row_sums(const float (&p)[8], float (*part)[8], int lane) {
+    float s[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float s = chunked::row_prefix_sum(p[i]);
-        if ((lane & 15) == 15) out[i][lane >> 4] = s;
+    for (int i = 0; i < 8; i++) s[i] = chunked::row_prefix_sum(p[i]);
+    if ((lane & 15) == 15) {
+        *reinterpret_cast<f4 *>(&part[lane >> 4][0]) = f4{s[0], s[1], s[2], s[3]};
+        *reinterpret_cast<f4 *>(&part[lane >> 4][4]) = f4{s[4], s[5], s[6], s[7]};
     }
+}
+__device__ __forceinline__ float row_sum(const float (*part)[4][8], int tok) {       // part[half block][group][token]
+    const float (*p)[8] = part[tok >> 3];
+    return (p[0][tok & 7] + p[1][tok & 7]) + (p[2][tok & 7] + p[3][tok & 7]);
 }
 
 // ------------------------------------------------------------------------------------------------------------ forward --
-// Eight wavefronts, two per SIMD, one barrier per 64-token step.  Wavefronts 0-3 walk the state (values 16 w .. +15, all
-// keys) over the step's four blocks and write y; wavefronts 4-7 meanwhile prepare one block each of the NEXT step in
-// the other buffer: the scaled copies, and the masked matrix of the block from them.  Bound by the matrix pipe: 160
-// instructions of 32 clocks per SIMD and step.
+// Twelve wavefronts, one barrier per 64-token step.  Wavefronts 0-3 walk the state (values 16 w .. +15, all keys) over
+// the step's four blocks.  Wavefronts 4-11 meanwhile build the masked matrices of the step and prepare half a block each
+// of the NEXT step in the other buffer; after the barrier the first four add the matrices' products to the y they hold
+// in registers.  Bound by the matrix pipe: 160 instructions of 32 clocks per SIMD and step.  (With the eight wavefronts
+// that fill two per SIMD, a whole block's preparation per wavefront took 12 k clocks a step, the walk 7 k.)
+constexpr int NT_FWD = 768;
 struct FwdTiles {
     float rm[SB * LD], km[SB * LD], v[SB * LD];
     float em[4][HEAD], eb[4][HEAD];      // e^{m}, e^{b-m} per block and key
-    f4 at[4][64];                        // masked matrix of each block: rows s, columns t
-    float rho[SB][4];
+    float rho[8][4][8];                  // r . (u o k) per token, in parts
+};
+struct FwdShared {
+    FwdTiles step[2];
+    f4 at[2][4][64];                     // masked matrix of each block of a step: rows s, columns t
 };
 
 template <class T, class W, bool PER_TOKEN_W>
-__global__ __launch_bounds__(NT) void forward_f32(int bh0, int Tlen, int C, int H, int nseg, int sps, int m,
+__global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, int H, int nseg, int sps, int m,
         const T *__restrict__ r, const T *__restrict__ k, const T *__restrict__ v, const W *__restrict__ wraw,
         const float *__restrict__ u, const float *s_in, T *__restrict__ y, float *s_out, float *__restrict__ ckpt,
         const float *__restrict__ part, int floor_decay)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    FwdTiles *const buf = reinterpret_cast<FwdTiles *>(smem_raw);
+    FwdShared &sh = *reinterpret_cast<FwdShared *>(smem_raw);
     const int bh = bh0 + blockIdx.x / nseg, seg = blockIdx.x % nseg, b = bh / H, h = bh % H;
     const int lane = threadIdx.x & 63, w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, n = lane & 15;
     const bool chain = w8 < 4;
-    const int q = w8 & 3;
+    const int q = chain ? w8 : (w8 - 4) >> 1, hf = w8 & 1;      // value quarter; block and half of it
     {
         const size_t base = (size_t)b * Tlen * C + (size_t)h * HEAD;
         r += base; k += base; v += base;
@@ -159,69 +170,65 @@ __global__ __launch_bounds__(NT) void forward_f32(int bh0, int Tlen, int C, int 
         for (int i = 0; i < 16; i++) S[i >> 2][i & 3] = X[i];
     }
 
-    // preparing wavefronts: block q, channel `lane`
+    // preparing wavefronts: tokens tok0 .. tok0+7 of the step, channel `lane`
+    const int tok0 = 16 * q + 8 * hf;
     const float uf = u[h * HEAD + lane];
     const float l_const = PER_TOKEN_W ? 0.f : log2_decay(to_float(wraw[h * HEAD + lane]), floor_decay);
-    T tr[16], tk[16], tv[16];
-    W tw[16];
+    T tr[8], tk[8], tv[8];
+    W tw[8];
     auto fetch = [&](int sb) __attribute__((always_inline)) {          // (tokens past the end are read from the last one and replaced)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int t = min(sb * SB + 16 * q + i, Tlen - 1);
+        for (int i = 0; i < 8; i++) {
+            const int t = min(sb * SB + tok0 + i, Tlen - 1);
             tr[i] = *row_at(r, t, C, lane); tk[i] = *row_at(k, t, C, lane); tv[i] = *row_at(v, t, C, lane);
             if (PER_TOKEN_W) tw[i] = *row_at(wraw, t, C, lane);
         }
     };
     auto prepare = [&](int sb, FwdTiles &sm) __attribute__((always_inline)) {
-        float em, eb;
+        float lw[8], x[8], p[8];
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
-            float lw[8], x[8], p[8];
+        for (int i = 0; i < 8; i++)
+            lw[i] = sb * SB + tok0 + i >= Tlen ? 0.f : PER_TOKEN_W ? log2_decay(to_float(tw[i]), floor_decay) : l_const;
+        const float total = hf ? half_exponents<8, true>(lw, x) : half_exponents<8, false>(lw, x);
+        (hf ? sm.eb : sm.em)[q][lane] = exp2_fast(total);
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const bool in = sb * SB + 16 * q + 8 * hf + i < Tlen;
-                lw[i] = !in ? 0.f : PER_TOKEN_W ? log2_decay(to_float(tw[8 * hf + i]), floor_decay) : l_const;
-            }
-            const float total = hf ? half_exponents<8, true>(lw, x) : half_exponents<8, false>(lw, x);
-            (hf ? eb : em) = exp2_fast(total);
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const bool in = sb * SB + 16 * q + 8 * hf + i < Tlen;
-                const float rf = in ? to_float(tr[8 * hf + i]) : 0.f, kf = in ? to_float(tk[8 * hf + i]) : 0.f;
-                const int o = (16 * q + 8 * hf + i) * LD + lane;
-                sm.rm[o] = rf * exp2_fast(x[i]);
-                sm.km[o] = kf * exp2_fast(-(x[i] + lw[i]));
-                sm.v[o] = in ? to_float(tv[8 * hf + i]) : 0.f;
-                p[i] = rf * uf * kf;
-            }
-            store_row_sums(p, &sm.rho[16 * q + 8 * hf], lane);
+        for (int i = 0; i < 8; i++) {
+            const bool in = sb * SB + tok0 + i < Tlen;
+            const float rf = in ? to_float(tr[i]) : 0.f, kf = in ? to_float(tk[i]) : 0.f;
+            const int o = (tok0 + i) * LD + lane;
+            sm.rm[o] = rf * exp2_fast(x[i]);
+            sm.km[o] = kf * exp2_fast(-(x[i] + lw[i]));
+            sm.v[o] = in ? to_float(tv[i]) : 0.f;
+            p[i] = rf * uf * kf;
         }
-        sm.em[q][lane] = em;
-        sm.eb[q][lane] = eb;
-        wave_sync();
-        f4 at = zero4(), a2 = zero4();
-#pragma unroll
-        for (int kk = 0; kk < 4; kk += 2) {
-            at = mma(along(sm.km, 16 * q + n, 16 * kk + 4 * g), along(sm.rm, 16 * q + n, 16 * kk + 4 * g), at);
-            a2 = mma(along(sm.km, 16 * q + n, 16 * kk + 16 + 4 * g), along(sm.rm, 16 * q + n, 16 * kk + 16 + 4 * g), a2);
-        }
-        const float4 rho = *reinterpret_cast<const float4 *>(sm.rho[16 * q + n]);
-        at += a2;
-#pragma unroll
-        for (int e = 0; e < 4; e++) at[e] = 4 * g + e < n ? at[e] : 4 * g + e == n ? (rho.x + rho.y) + (rho.z + rho.w) : 0.f;
-        sm.at[q][lane] = at;
+        store_row_sums(p, sm.rho[2 * q + hf], lane);
     };
-
     // (the two roles have loops of their own: in a common one the compiler waits, in either, for what the other may have
     // outstanding)
     if (!chain) {
         fetch(sb0);
-        prepare(sb0, buf[0]);
+        prepare(sb0, sh.step[0]);
         fetch(min(sb0 + 1, sb1 - 1));
         lds_barrier();
         for (int sb = sb0; sb < sb1; sb++) {
+            const int par = (sb - sb0) & 1;
+            if (hf == 0 && y) {      // the masked matrix of block q
+                const FwdTiles &sm = sh.step[par];
+                const int row = 16 * q + n;
+                f4 at = zero4(), a2 = zero4();
+#pragma unroll
+                for (int kk = 0; kk < 4; kk += 2) {
+                    at = mma(along(sm.km, row, 16 * kk + 4 * g), along(sm.rm, row, 16 * kk + 4 * g), at);
+                    a2 = mma(along(sm.km, row, 16 * kk + 16 + 4 * g), along(sm.rm, row, 16 * kk + 16 + 4 * g), a2);
+                }
+                const float rho = row_sum(sm.rho, row);
+                at += a2;
+#pragma unroll
+                for (int e = 0; e < 4; e++) at[e] = 4 * g + e < n ? at[e] : 4 * g + e == n ? rho : 0.f;
+                sh.at[par][q][lane] = at;
+            }
             if (sb + 1 < sb1) {
-                prepare(sb + 1, buf[(sb + 1 - sb0) & 1]);
+                prepare(sb + 1, sh.step[par ^ 1]);
                 fetch(min(sb + 2, sb1 - 1));
             }
             lds_barrier();
@@ -232,26 +239,33 @@ __global__ __launch_bounds__(NT) void forward_f32(int bh0, int Tlen, int C, int 
     const uint32_t y_lane = (uint32_t)n * C + 16 * q + 4 * g;
     lds_barrier();
     for (int sb = sb0; sb < sb1; sb++) {
-        const FwdTiles &sm = buf[(sb - sb0) & 1];
+        const int par = (sb - sb0) & 1;
+        const FwdTiles &sm = sh.step[par];
         if (ckpt) {       // the state at the start of this step, 16 bytes per lane and tile
             f4 *cp = reinterpret_cast<f4 *>(ckpt + ((size_t)bh * (nsb + 1) + sb) * HEAD * HEAD) + q * 256 + lane;
 #pragma unroll
             for (int kk = 0; kk < 4; kk++) cp[64 * kk] = S[kk];
         }
+        f4 vv[4], yy[4];
 #pragma unroll
         for (int blk = 0; blk < 4; blk++) {
-            const f4 vv = across(sm.v, 16 * blk + 4 * g, 16 * q + n);
-            f4 ya = mma(vv, sm.at[blk][lane], zero4()), yb = zero4();
+            vv[blk] = across(sm.v, 16 * blk + 4 * g, 16 * q + n);
+            f4 ya = zero4(), yb = zero4();
 #pragma unroll
             for (int kk = 0; kk < 4; kk++) {
                 S[kk] *= *reinterpret_cast<const f4 *>(&sm.em[blk][16 * kk + 4 * g]);
                 (kk & 1 ? yb : ya) = mma(S[kk], along(sm.rm, 16 * blk + n, 16 * kk + 4 * g), kk & 1 ? yb : ya);
-                S[kk] = mma(across(sm.km, 16 * blk + 4 * g, 16 * kk + n), vv, S[kk]);
+                S[kk] = mma(across(sm.km, 16 * blk + 4 * g, 16 * kk + n), vv[blk], S[kk]);
                 S[kk] *= *reinterpret_cast<const f4 *>(&sm.eb[blk][16 * kk + 4 * g]);
             }
-            if (y) put4<T>(yo, sb * SB + 16 * blk, C, y_lane, ya + yb);      // y^T: values 16q+4g .. +3 of token n
+            yy[blk] = ya + yb;
         }
         lds_barrier();
+        if (y) {
+#pragma unroll
+            for (int blk = 0; blk < 4; blk++)      // y^T: values 16q+4g .. +3 of token n
+                put4<T>(yo, sb * SB + 16 * blk, C, y_lane, mma(vv[blk], sh.at[par][blk][lane], yy[blk]));
+        }
     }
     if (seg == nseg - 1) {
         if (ckpt) {       // the final state takes the slot after the last step
@@ -363,18 +377,23 @@ __global__ __launch_bounds__(256) void summary_f32(int bh0, int Tlen, int C, int
 }
 
 // ----------------------------------------------------------------------------------------------------------- backward --
-// Eight wavefronts; the 64-token steps of a segment from the last to the first.
+// Eight wavefronts; the 64-token steps of a segment from the last to the first, in four parts between barriers:
 //   prepare   wavefront (block q, half): eight tokens of one channel per lane
-//   first     wavefronts 0-3 (keys 16 w .. +15): the state forward from the step's checkpoint, leaving  gy S1^T  of each
-//             block in registers; wavefronts 4-7: the masked matrices of one block each
-//   second    wavefronts 0-3: the state gradient (value-major) backward, gr, gk and the decay gradient of their keys;
-//             wavefronts 4-7: the key-major copy backward, gv of the values 16 w .. +15
-// Bound by the matrix pipe: 480 instructions of 32 clocks per SIMD and step.
+//   walk      wavefronts 0-3 (keys 16 w .. +15): the state forward from the step's checkpoint,  gy S1^T  of each block, then
+//             the state gradient (value-major) backward,  v G1^T;  wavefronts 4-7: the masked matrices of one block each,
+//             then the key-major gradient backward,  km G1  of the values 16 w .. +15
+//   join      the masked matrices' products are added: d(rm), d(km) go to LDS, gv leaves
+//   finish    wavefront (block q, half) again: gr, gk and the decay gradient of eight tokens of one channel per lane, in
+//             whole rows
+// Bound by the matrix pipe: 480 instructions of 32 clocks per SIMD and step, 432 of them in the walk, where a SIMD has one
+// wavefront of either kind.  (With the matrices' products inside the walk, a barrier between the state's walk and the
+// gradient's, and the key wavefronts finishing their own results: 28 k clocks a step against 15 k of matrix work.)
 struct BwdTiles {
     float rm[SB * LD], km[SB * LD], v[SB * LD], gy[SB * LD], x[SB * LD], lw[SB * LD];
     float em[4][HEAD], eb[4][HEAD];
     f4 pm[4][64], pt[4][64], at[4][64];      // P (t > s): rows t, columns s;  P^T (s < t): rows s, columns t;  rm km^T (t >= s): rows t, columns s
-    float rho[SB][4], pdiag[SB];
+    float dr[SB * LD], dk[SB * LD];          // d(rm), d(km)
+    float rho[8][4][8], pdiag[SB], sums[8][HEAD];      // sums: of rm d(rm) - km d(km) over half a block
 };
 
 template <class T, class W, bool PER_TOKEN_W>
@@ -401,7 +420,7 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
 
     // keys: G[kk][e] = G[key own][value 16kk+4g+e];  values: G[kk][e] = G[key 16kk+4g+e][value own]
     f4 G[4] = {zero4(), zero4(), zero4(), zero4()};
-    float A = 0.f;                           // running sum of the decay gradient, key own (the same in the four lane groups)
+    float A = 0.f;                           // running sum of the decay gradient at the end of a step, key `lane`
     {
         float X[16];
         int ki[16], vi[16];
@@ -423,12 +442,12 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
 #pragma unroll
             for (int i = 0; i < 16; i++) A = fmaf(X[i], cp[(i >> 2) * 1024 + (i & 3) * 4], A);
             A = chunked::group_sum4(A);
+            if (g == 0) sm.sums[0][own] = A;
         }
 #pragma unroll
         for (int i = 0; i < 16; i++) G[i >> 2][i & 3] = X[i];
     }
-    const float u_own = u[h * HEAD + own];
-    float gu_acc = 0.f, gw_acc = 0.f;
+    float gu_acc = 0.f, gw_acc = 0.f;        // of the lane's tokens, key `lane`
 
     // preparing: block q, half hf, channel `lane`
     const int hf = w8 >> 2, tok0 = 16 * q + 8 * hf;
@@ -464,7 +483,42 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
             sm.lw[o] = lw[i];
             p[i] = rf * uf * kf;
         }
-        store_row_sums(p, &sm.rho[tok0], lane);
+        store_row_sums(p, sm.rho[2 * q + hf], lane);
+    };
+    const size_t left = (size_t)Tlen * C - h * HEAD;
+    const Out gro = out_of(gr, left), gko = out_of(gk, left), gwo = out_of(PER_TOKEN_W ? gw_tok : nullptr, PER_TOKEN_W ? left : 0);
+    // dL/dlog w_t = A_t - km_t d(km)_t, A_t the running sum after token t
+    auto finish = [&](int sb, int lane) __attribute__((always_inline)) {
+        float rm[8], km[8], dr[8], dk[8], z[8], c[8], sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int o = (tok0 + i) * LD + lane;
+            rm[i] = sm.rm[o]; km[i] = sm.km[o]; dr[i] = sm.dr[o]; dk[i] = sm.dk[o];
+            z[i] = km[i] * dk[i];
+            c[i] = fmaf(rm[i], dr[i], -z[i]);
+            sum += c[i];
+        }
+        sm.sums[2 * q + hf][lane] = sum;
+        lds_barrier();
+        float run = A;
+#pragma unroll
+        for (int j = 7; j >= 0; j--) {
+            const float x = sm.sums[j][lane];
+            A += x;
+            run += j > 2 * q + hf ? x : 0.f;
+        }
+#pragma unroll
+        for (int i = 7; i >= 0; i--) {
+            const int o = (tok0 + i) * LD + lane;
+            const float x = sm.x[o], lw = sm.lw[o], bonus = exp2_fast(lw) * sm.pdiag[tok0 + i], D = run - z[i];
+            run += c[i];
+            gu_acc = fmaf(rm[i] * km[i], bonus, gu_acc);
+            const int t = sb * SB + tok0 + i;
+            put<T>(gro, t, C, lane, exp2_fast(x) * fmaf(uf * km[i], bonus, dr[i]));
+            put<T>(gko, t, C, lane, exp2_fast(-(x + lw)) * fmaf(uf * rm[i], bonus, dk[i]));
+            if (PER_TOKEN_W) put<W>(gwo, t, C, lane, (floor_decay && lw <= LOG2_W_FLOOR) ? 0.f : D * (lw * LN2));
+            else gw_acc += t < Tlen ? D : 0.f;
+        }
     };
     // In the loops below a lane's indices come from an opaque copy of its number: addresses hoisted out of the loop would
     // live, and spill, across all of it.
@@ -473,7 +527,9 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
     asm volatile("" : "+v"(lane));                                                        \
     const int g = lane >> 4, n = lane & 15, own = 16 * q + n;
     const int lane0 = lane;
-    const size_t left = (size_t)Tlen * C - h * HEAD;
+    lds_barrier();
+    A = sm.sums[0][lane];
+    lds_barrier();                                   // (before a step's sums go there)
     if (!keys) {
         const Out gvo = out_of(gv, left);
         fetch(sb1 - 1, lane);
@@ -491,129 +547,127 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
                     pT = mma(c, a, pT);
                     at = mma(along(sm.rm, row, 16 * kk + 4 * g), along(sm.km, row, 16 * kk + 4 * g), at);
                 }
-                const float4 rho = *reinterpret_cast<const float4 *>(sm.rho[row]);
+                const float rho = row_sum(sm.rho, row);
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int x = 4 * g + e;
                     if (x == n) sm.pdiag[row] = p[e];
                     p[e] = x > n ? p[e] : 0.f;
                     pT[e] = x < n ? pT[e] : 0.f;
-                    at[e] = x > n ? at[e] : x == n ? (rho.x + rho.y) + (rho.z + rho.w) : 0.f;
+                    at[e] = x > n ? at[e] : x == n ? rho : 0.f;
                 }
                 sm.pm[q][lane] = p; sm.pt[q][lane] = pT; sm.at[q][lane] = at;
             }
             fetch(max(sb - 1, sb0), lane);          // before this step's stores, see Out
-            lds_barrier();
+            f4 gf[4], gvv[4];
 #pragma unroll
             for (int blk = 3; blk >= 0; blk--) {
-                const f4 gf = across(sm.gy, 16 * blk + 4 * g, own);
-                f4 a = mma(gf, sm.at[blk][lane], zero4()), c = zero4();
+                gf[blk] = across(sm.gy, 16 * blk + 4 * g, own);
+                f4 a = zero4(), c = zero4();
 #pragma unroll
                 for (int kk = 0; kk < 4; kk++) {
                     G[kk] *= *reinterpret_cast<const f4 *>(&sm.eb[blk][16 * kk + 4 * g]);
                     (kk & 1 ? c : a) = mma(G[kk], along(sm.km, 16 * blk + n, 16 * kk + 4 * g), kk & 1 ? c : a);
-                    G[kk] = mma(across(sm.rm, 16 * blk + 4 * g, 16 * kk + n), gf, G[kk]);
+                    G[kk] = mma(across(sm.rm, 16 * blk + 4 * g, 16 * kk + n), gf[blk], G[kk]);
                     G[kk] *= *reinterpret_cast<const f4 *>(&sm.em[blk][16 * kk + 4 * g]);
                 }
-                put4<T>(gvo, sb * SB + 16 * blk, C, (uint32_t)n * C + 16 * q + 4 * g, a + c);      // gv^T: values 16q+4g .. +3 of token n
+                gvv[blk] = a + c;
             }
             lds_barrier();
+#pragma unroll
+            for (int blk = 0; blk < 4; blk++)        // gv^T: values 16q+4g .. +3 of token n
+                put4<T>(gvo, sb * SB + 16 * blk, C, (uint32_t)n * C + 16 * q + 4 * g, mma(gf[blk], sm.at[blk][lane], gvv[blk]));
+            lds_barrier();
+            finish(sb, lane);
+            lds_barrier();
         }
-        return;
-    }
-    const Out gro = out_of(gr, left), gko = out_of(gk, left), gwo = out_of(PER_TOKEN_W ? gw_tok : nullptr, PER_TOKEN_W ? left : 0);
-    f4 S[4];                                         // [key own][value 16kk+4g+e], from the step's checkpoint
-    auto fetch_state = [&](int sb, int lane) __attribute__((always_inline)) {
-        const int g = lane >> 4, n = lane & 15;
-        const float *cp = ckpt + ((size_t)bh * (nsb + 1) + sb) * HEAD * HEAD + ((size_t)q * 64 + 16 * (n >> 2) + 4 * g) * 4 + (n & 3);
+    } else {
+        f4 S[4];                                     // [key own][value 16kk+4g+e], from the step's checkpoint
+        auto fetch_state = [&](int sb, int lane) __attribute__((always_inline)) {
+            const int g = lane >> 4, n = lane & 15;
+            const float *cp = ckpt + ((size_t)bh * (nsb + 1) + sb) * HEAD * HEAD + ((size_t)q * 64 + 16 * (n >> 2) + 4 * g) * 4 + (n & 3);
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++)
+            for (int kk = 0; kk < 4; kk++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) S[kk][e] = cp[kk * 1024 + e * 4];
-    };
-    fetch(sb1 - 1, lane);
-    fetch_state(sb1 - 1, lane);
-    for (int sb = sb1 - 1; sb >= sb0; sb--) {
-        WKV_F32_LANE
-        prepare(sb, lane);
-        lds_barrier();
-        f4 q1[4];
+                for (int e = 0; e < 4; e++) S[kk][e] = cp[kk * 1024 + e * 4];
+        };
+        fetch(sb1 - 1, lane);
+        fetch_state(sb1 - 1, lane);
+        for (int sb = sb1 - 1; sb >= sb0; sb--) {
+            WKV_F32_LANE
+            prepare(sb, lane);
+            lds_barrier();
+            f4 q1[4], q4[4];                         // rows: tokens of the block, column key own
 #pragma unroll
-        for (int blk = 0; blk < 4; blk++) {
-            const float em = sm.em[blk][own];
-            f4 a = zero4(), c = zero4();
+            for (int blk = 0; blk < 4; blk++) {
+                const float em = sm.em[blk][own];
+                f4 a = zero4(), c = zero4();
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                S[kk] *= em;
-                (kk & 1 ? c : a) = mma(along(sm.gy, 16 * blk + n, 16 * kk + 4 * g), S[kk], kk & 1 ? c : a);
+                for (int kk = 0; kk < 4; kk++) {
+                    S[kk] *= em;
+                    (kk & 1 ? c : a) = mma(along(sm.gy, 16 * blk + n, 16 * kk + 4 * g), S[kk], kk & 1 ? c : a);
+                }
+                q1[blk] = a + c;
+                if (blk < 3) {
+                    const float eb = sm.eb[blk][own];
+                    const f4 kf = across(sm.km, 16 * blk + 4 * g, own);
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk++) S[kk] = mma(across(sm.v, 16 * blk + 4 * g, 16 * kk + n), kf, S[kk]) * eb;
+                }
             }
-            q1[blk] = a + c;                         // rows t, column key own
-            if (blk < 3) {
-                const float eb = sm.eb[blk][own];
-                const f4 kf = across(sm.km, 16 * blk + 4 * g, own);
+            fetch(max(sb - 1, sb0), lane);           // before this step's stores, see Out
+            fetch_state(max(sb - 1, sb0), lane);
 #pragma unroll
-                for (int kk = 0; kk < 4; kk++) S[kk] = mma(across(sm.v, 16 * blk + 4 * g, 16 * kk + n), kf, S[kk]) * eb;
+            for (int blk = 3; blk >= 0; blk--) {
+                const float em = sm.em[blk][own], eb = sm.eb[blk][own];
+                const f4 rf = across(sm.rm, 16 * blk + 4 * g, own);
+                f4 a = zero4(), c = zero4();
+#pragma unroll
+                for (int kk = 0; kk < 4; kk++) {
+                    G[kk] *= eb;
+                    (kk & 1 ? c : a) = mma(along(sm.v, 16 * blk + n, 16 * kk + 4 * g), G[kk], kk & 1 ? c : a);
+                    G[kk] = mma(across(sm.gy, 16 * blk + 4 * g, 16 * kk + n), rf, G[kk]) * em;
+                }
+                q4[blk] = a + c;
             }
+            lds_barrier();
+#pragma unroll
+            for (int blk = 0; blk < 4; blk++) {
+                const f4 dr = mma(sm.pt[blk][lane], across(sm.km, 16 * blk + 4 * g, own), q1[blk]);
+                const f4 dk = mma(sm.pm[blk][lane], across(sm.rm, 16 * blk + 4 * g, own), q4[blk]);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int o = (16 * blk + 4 * g + e) * LD + own;
+                    sm.dr[o] = dr[e];
+                    sm.dk[o] = dk[e];
+                }
+            }
+            lds_barrier();
+            finish(sb, lane);
+            lds_barrier();
         }
-        fetch(max(sb - 1, sb0), lane);               // before this step's stores, see Out
-        fetch_state(max(sb - 1, sb0), lane);
-        lds_barrier();
-        const uint32_t g_lane = (uint32_t)(4 * g) * C + own;
+        if (gs_in && seg == 0) {
+            float *gp = gs_in + (size_t)bh * HEAD * HEAD + own * HEAD;
 #pragma unroll
-        for (int blk = 3; blk >= 0; blk--) {
-            const float em = sm.em[blk][own], eb = sm.eb[blk][own];
-            const f4 rf = across(sm.rm, 16 * blk + 4 * g, own), kf = across(sm.km, 16 * blk + 4 * g, own);
-            f4 dk = mma(sm.pm[blk][lane], rf, zero4()), dk2 = zero4();
-            const f4 dr = mma(sm.pt[blk][lane], kf, q1[blk]);
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                G[kk] *= eb;
-                (kk & 1 ? dk2 : dk) = mma(along(sm.v, 16 * blk + n, 16 * kk + 4 * g), G[kk], kk & 1 ? dk2 : dk);
-                G[kk] = mma(across(sm.gy, 16 * blk + 4 * g, 16 * kk + n), rf, G[kk]) * em;
-            }
-            dk += dk2;
-            // tokens 16 blk + 4g + e, key own
-            const f4 xx = across(sm.x, 16 * blk + 4 * g, own), ll = across(sm.lw, 16 * blk + 4 * g, own);
-            const f4 pd = *reinterpret_cast<const f4 *>(&sm.pdiag[16 * blk + 4 * g]);
-            f4 c, z;
-            float sum = 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; e++) { z[e] = kf[e] * dk[e]; c[e] = rf[e] * dr[e] - z[e]; sum += c[e]; }
-            // A after this lane's last token: the sums of the later lane groups of the block
-            const float s1 = __shfl(sum, n + 16), s2 = __shfl(sum, n + 32), s3 = __shfl(sum, n + 48), s0 = __shfl(sum, n);
-            float run = A + (g < 1 ? s1 : 0.f) + (g < 2 ? s2 : 0.f) + (g < 3 ? s3 : 0.f);
-            A += (s0 + s1) + (s2 + s3);
-            const int t0 = sb * SB + 16 * blk + 4 * g;
-#pragma unroll
-            for (int e = 3; e >= 0; e--) {
-                const float D = run - z[e], wd = exp2_fast(ll[e]), er = exp2_fast(xx[e]), ek = exp2_fast(-(xx[e] + ll[e]));
-                run += c[e];
-                const float bonus = wd * pd[e];
-                gu_acc = fmaf(rf[e] * kf[e], bonus, gu_acc);
-                const int row = sb * SB + 16 * blk + e;
-                put<T>(gro, row, C, g_lane, er * fmaf(u_own * kf[e], bonus, dr[e]));
-                put<T>(gko, row, C, g_lane, ek * fmaf(u_own * rf[e], bonus, dk[e]));
-                if (PER_TOKEN_W) put<W>(gwo, row, C, g_lane, (floor_decay && ll[e] <= LOG2_W_FLOOR) ? 0.f : D * (ll[e] * LN2));
-                else gw_acc += t0 + e < Tlen ? D : 0.f;
-            }
+            for (int kk = 0; kk < 4; kk++) *reinterpret_cast<f4 *>(gp + 16 * kk + 4 * g) = G[kk];
         }
-        lds_barrier();
     }
 #undef WKV_F32_LANE
-    if (gs_in && seg == 0) {
-        float *gp = gs_in + (size_t)bh * HEAD * HEAD + own * HEAD;
+    // sums over the segment's tokens: the eight wavefronts' shares in a fixed order
+    float *red = sm.dr;
+    red[w8 * HEAD + lane] = gu_acc;
+    red[(8 + w8) * HEAD + lane] = gw_acc;
+    lds_barrier();
+    if (w8 == 0) {
+        float su = 0.f, sw = 0.f;
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) *reinterpret_cast<f4 *>(gp + 16 * kk + 4 * g) = G[kk];
-    }
-    gu_acc = chunked::group_sum4(gu_acc);
-    gw_acc = chunked::group_sum4(gw_acc);
-    if (g == 0) {
-        const size_t po = ((size_t)(b * nseg + seg) * H + h) * HEAD + own;
-        gu_part[po] = gu_acc;
+        for (int i = 0; i < 8; i++) { su += red[i * HEAD + lane]; sw += red[(8 + i) * HEAD + lane]; }
+        const size_t po = ((size_t)(b * nseg + seg) * H + h) * HEAD + lane;
+        gu_part[po] = su;
         if (!PER_TOKEN_W) {
             bool fl;
-            const float l = log_decay(to_float(wraw[h * HEAD + own]), floor_decay, &fl);
-            gw_part[po] = fl ? 0.f : gw_acc * l;
+            const float l = log_decay(to_float(wraw[h * HEAD + lane]), floor_decay, &fl);
+            gw_part[po] = fl ? 0.f : sw * l;
         }
     }
 }
@@ -623,7 +677,7 @@ template <class T, class W, bool PT> struct Kernels {
     static constexpr auto *fwd = &forward_f32<T, W, PT>;
     static constexpr auto *bwd = &backward_f32<T, W, PT>;
     static hipError_t init() {
-        hipError_t e = hipFuncSetAttribute((const void *)fwd, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * sizeof(FwdTiles));
+        hipError_t e = hipFuncSetAttribute((const void *)fwd, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(FwdShared));
         if (e == hipSuccess) e = hipFuncSetAttribute((const void *)bwd, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BwdTiles));
         return e;
     }
@@ -640,7 +694,7 @@ template <class T, class W, bool PT> struct Kernels {
                                pl.sps, pl.m, pl.pps, (const T *)k, (const T *)v, (const W *)w, part, floor_decay);
         auto launch = [&](int bh0, int n, const chunked::SegPlan &x) {
             if (n > 0)
-                hipLaunchKernelGGL((forward_f32<T, W, PT>), dim3(n * x.nseg), dim3(NT), 2 * sizeof(FwdTiles), s, bh0, Tlen, C, H, x.nseg, x.sps,
+                hipLaunchKernelGGL((forward_f32<T, W, PT>), dim3(n * x.nseg), dim3(NT_FWD), sizeof(FwdShared), s, bh0, Tlen, C, H, x.nseg, x.sps,
                                    x.m, (const T *)r, (const T *)k, (const T *)v, (const W *)w, u, s_in, (T *)y, s_out, ckpt, part, floor_decay);
         };
         prof_begin(KID_CHUNK_FORWARD, s);
