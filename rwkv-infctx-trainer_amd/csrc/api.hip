@@ -33,6 +33,7 @@ int check_dims56(int B, int T, int C, int H, int dtype) {
 // wkv56_chunked.hip, fp32 and fp16 streams of two tokens or more those of wkv56_f32.hip (ALGO_F32, not a selector of the
 // ABI); everything else goes token by token.
 constexpr int ALGO_F32 = 3;
+const chunked::Costs &costs_of(int a) { return a == ALGO_F32 ? chunked::F32_COSTS : chunked::BF16_COSTS; }
 int pick_algo56(int algo, int T, int C, int dtype, unsigned flags) {
     // (the fp32 kernels' stores count on offsets of the last step's missing tokens not wrapping)
     const bool can_f32 = T > 1 && (flags & WKV_FLOOR_DECAY) && (long long)(T + 64) * C < (1ll << 30);
@@ -80,7 +81,7 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
         const bool keep = !(flags & WKV_NO_CHECKPOINTS);
         if (workspace) {
             if (!aligned16(workspace)) return WKV_ERR_ALIGN;
-            if (workspace_bytes < (keep ? chunked::forward_workspace(B, T, H) : chunked::forward_scratch(B, T, H))) return WKV_ERR_WORKSPACE;
+            if (workspace_bytes < (keep ? chunked::forward_workspace(B, T, H, costs_of(a)) : chunked::forward_scratch(B, T, H, costs_of(a)))) return WKV_ERR_WORKSPACE;
         }
         hipError_t e = a == WKV_ALGO_CHUNKED
                            ? chunked::forward_launch((hipStream_t)stream, per_token, w16, B, T, C, H, r, k, v, w, u, state_in, y, state_out,
@@ -99,14 +100,14 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
 size_t forward56_workspace(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
     const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
-    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_workspace(B, T, H) : 0;
+    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_workspace(B, T, H, costs_of(a)) : 0;
 }
 
 size_t backward56_workspace(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
     const size_t rec = recurrent_backward_workspace(B, T, C);
     const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
-    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? std::max(rec, chunked::backward_workspace(B, T, C, H)) : rec;
+    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? std::max(rec, chunked::backward_workspace(B, T, C, H, costs_of(a))) : rec;
 }
 
 int backward56(bool per_token, void *stream, int B, int T, int C, int H, int dtype, unsigned flags, int algo,
@@ -126,7 +127,7 @@ int backward56(bool per_token, void *stream, int B, int T, int C, int H, int dty
     const bool w16 = (flags & (WKV_W_BF16 | WKV_W_F16)) != 0;
     if (!workspace) return WKV_ERR_NULL;
     if (workspace_bytes < (a == WKV_ALGO_RECURRENT ? recurrent_backward_workspace(B, T, C)
-                                                   : chunked::backward_workspace(B, T, C, H)))
+                                                   : chunked::backward_workspace(B, T, C, H, costs_of(a))))
         return WKV_ERR_WORKSPACE;
     if (gstate_in && gstate_out) {      // several workgroups share a head's state gradient: some read gstate_out after
                                         // others have written gstate_in, so the two are never the same memory
@@ -233,7 +234,7 @@ size_t wkv6_forward_workspace(int B, int T, int C, int H, int dtype, int algo) {
 size_t wkv56_forward_scratch(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
     const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
-    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_scratch(B, T, H) : 0;
+    return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_scratch(B, T, H, costs_of(a)) : 0;
 }
 size_t wkv5_forward_workspace(int B, int T, int C, int H, int dtype, int algo) {
     return forward56_workspace(B, T, C, H, dtype, algo);

@@ -39,6 +39,7 @@
 // (S_out = decay o S_in + delta), a small kernel chains the summaries into the state
 // at the start of every segment.  Backward does the same with the state gradient.
 #include "common.h"
+#include <cstddef>
 #include <type_traits>
 
 namespace wkv {
@@ -484,52 +485,58 @@ __global__ __launch_bounds__(NT_F) void summary_pass(int bh0, int Tlen, int C, i
     if (wv == 0) pp[HEAD * HEAD + lane] = stopped ? 0.f : exp2_fast(R);
 }
 
-// Chaining the piece summaries, done by the main kernels for the state elements a lane holds.  A lane's
-// elements are X[i] = X[key ki[i]][value vi[i]], i < N.
-//   chain_state:    the state at the start of segment `seg` = the summaries of the pieces before it applied in
-//                   order to the state handed in.  Walked from the nearest piece backwards,
+// Chaining the piece summaries, done by the main kernels in their prologues.
+//   the state at the start of segment `seg` = the summaries of the pieces before it applied in order to the state handed
+//   in; walked from the nearest piece backwards (dir = -1),
 //                       S = D_p + d_p o (D_{p-1} + d_{p-1} o ( ... + d_0 o S_in)),
-//                   i.e. S = sum_q (prod_{q < q' <= p} d_q') o D_q, so that the walk ends as soon as the running product
-//                   of the decays is 0 for all of the lane's keys (a piece that forgot everything reports exactly 0).
-//   chain_gradient: the state gradient at the end of segment `seg`, from the pieces after it and the gradient handed in,
-//                   walked forward in the same way.
-// The summaries are read two pieces at a time, deltas and decays together, so that the common cases (the nearest piece
-// forgot everything; two pieces per segment) take one round trip to memory.  ONE_KEY: all N elements share the key ki[0].
-template <int N, bool ONE_KEY>
-__device__ __forceinline__ void chain_summaries(float (&X)[N], const int (&ki)[N], const int (&vi)[N], const float *__restrict__ pieces,
-                                                int first, int count, int dir, const float *__restrict__ ends) {
-    constexpr int NK = ONE_KEY ? 1 : N;
-    float run[NK];
+//   i.e. S = sum_q (prod_{q < q' <= p} d_q') o D_q, so that the walk ends as soon as the running product of the decays is
+//   0 for all of a wavefront's keys (a piece that forgot everything reports exactly 0);
+//   the state gradient at the end of segment `seg`, from the pieces after it and the gradient handed in, in the same way
+//   forward (dir = 1).
+// The first 1024 / PER lanes of the workgroup take PER times four consecutive values of a key each, so that a summary is read
+// in whole kilobytes, and leave the result in a table [key][CHAIN_LD] in LDS for everybody.  (Read by the wavefronts that
+// own the state, in their layout of 64-byte pieces, a summary cost some 0.4 us of the prologue and twice that in the
+// kernels with fewer wavefronts.)  Two pieces in one round trip to memory, then four at a time: with a decay that forgets
+// within a piece the walk is over after the first, with one that does not it has up to 63 to go.
+constexpr int CHAIN_LD = 68;
+template <int PER>
+__device__ __forceinline__ void chain_summaries(float *table, const float *__restrict__ pieces, int first, int count, int dir,
+                                                const float *ends, int tid) {
+    if (tid >= 1024 / PER) return;
+    f4 X[PER];
+    float run[PER];
+    int key[PER];
 #pragma unroll
-    for (int i = 0; i < N; i++) X[i] = 0.f;
+    for (int i = 0; i < PER; i++) { X[i] = f4{0.f, 0.f, 0.f, 0.f}; run[i] = 1.f; key[i] = (tid + i * (1024 / PER)) >> 4; }
+    const int v4 = 4 * (tid & 15);
+    bool alive = true;          // (the same for the lanes of a wavefront)
+    auto group = [&](int x, auto size) __attribute__((always_inline)) {
+        constexpr int GROUP = decltype(size)::value;
+        f4 d[GROUP][PER];
+        float dc[GROUP][PER];
 #pragma unroll
-    for (int k = 0; k < NK; k++) run[k] = 1.f;
-    bool alive = true;
-    for (int x = 0; x < count && alive; x += 2) {
-        float d[2][N], dc[2][NK];
-#pragma unroll
-        for (int bb = 0; bb < 2; bb++) {
+        for (int bb = 0; bb < GROUP; bb++) {
             const float *q = pieces + (size_t)(first + dir * min(x + bb, count - 1)) * PART;
 #pragma unroll
-            for (int i = 0; i < N; i++) d[bb][i] = q[ki[i] * HEAD + vi[i]];
-#pragma unroll
-            for (int k = 0; k < NK; k++) dc[bb][k] = q[HEAD * HEAD + ki[k]];
+            for (int i = 0; i < PER; i++) { d[bb][i] = *reinterpret_cast<const f4 *>(q + key[i] * HEAD + v4); dc[bb][i] = q[HEAD * HEAD + key[i]]; }
         }
 #pragma unroll
-        for (int bb = 0; bb < 2; bb++) {
-            if (x + bb < count && alive) {
-                bool any = false;
+        for (int bb = 0; bb < GROUP; bb++)
+            if (x + bb < count) {
 #pragma unroll
-                for (int i = 0; i < N; i++) X[i] = fmaf(run[ONE_KEY ? 0 : i], d[bb][i], X[i]);
-#pragma unroll
-                for (int k = 0; k < NK; k++) { run[k] *= dc[bb][k]; any |= run[k] != 0.f; }
-                alive = any;
+                for (int i = 0; i < PER; i++) { X[i] += run[i] * d[bb][i]; run[i] *= dc[bb][i]; }
             }
-        }
-    }
-    if (alive && ends) {
+        bool any = false;
 #pragma unroll
-        for (int i = 0; i < N; i++) X[i] = fmaf(run[ONE_KEY ? 0 : i], ends[ki[i] * HEAD + vi[i]], X[i]);
+        for (int i = 0; i < PER; i++) any |= run[i] != 0.f;
+        alive = __builtin_amdgcn_ballot_w64(any) != 0;
+    };
+    if (count > 0) group(0, std::integral_constant<int, 2>());
+    for (int x = 2; x < count && alive; x += 4) group(x, std::integral_constant<int, 4>());
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        if (alive && ends) X[i] += run[i] * *reinterpret_cast<const f4 *>(ends + key[i] * HEAD + v4);
+        *reinterpret_cast<f4 *>(table + key[i] * CHAIN_LD + v4) = X[i];
     }
 }
 
@@ -559,22 +566,24 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
 
     // chain wavefronts: S[j][e] = S[key 32hk+16j+4g+e][value 16wv+n]
     f4 S[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
-    if (chain) {
-        if (seg == 0) {
+    if (seg == 0) {
+        if (chain) {
             const float *sp = s_in + (size_t)bh * HEAD * HEAD;
 #pragma unroll
             for (int j = 0; j < 2; j++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) S[j][e] = sp[(32 * hk + 16 * j + 4 * g + e) * HEAD + 16 * wv + n];
-        } else {      // the summaries of the pieces before this segment, chained onto the state handed in
-            float X[8];
-            int ki[8], vi[8];
+        }
+    } else {      // the summaries of the pieces before this segment, chained onto the state handed in
+        float *table = reinterpret_cast<float *>(sm.yi);
+        static_assert(sizeof(sm.yi) >= HEAD * CHAIN_LD * sizeof(float), "the table fits");
+        chain_summaries<1>(table, part + (size_t)bh * nseg * m * PART, seg * m - 1, seg * m, -1, s_in + (size_t)bh * HEAD * HEAD, tid);
+        lds_barrier();
+        if (chain) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) { ki[i] = 32 * hk + 16 * (i >> 2) + 4 * g + (i & 3); vi[i] = 16 * wv + n; }
-            chain_summaries<8, false>(X, ki, vi, part + (size_t)bh * nseg * m * PART, seg * m - 1, seg * m, -1,
-                               s_in + (size_t)bh * HEAD * HEAD);
+            for (int j = 0; j < 2; j++)
 #pragma unroll
-            for (int i = 0; i < 8; i++) S[i >> 2][i & 3] = X[i];
+                for (int e = 0; e < 4; e++) S[j][e] = table[(32 * hk + 16 * j + 4 * g + e) * CHAIN_LD + 16 * wv + n];
         }
     }
     // preparing role: token tok of the step (block q), channels c4..c4+3
@@ -910,38 +919,30 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     {
         // the last segment starts from gs_out, an earlier one from the summaries of the pieces after it chained onto gs_out
         float X[16];
-        bool have = false;
-        if (role < 3) {
-            if (seg == nseg - 1) {
-                have = gs_out != nullptr;
-                if (have) {
-                    const float *gp = gs_out + (size_t)bh * HEAD * HEAD;
-#pragma unroll
-                    for (int i = 0; i < 16; i++) {
-                        const int x = 16 * (i >> 2) + 4 * g + (i & 3);
-                        X[i] = role == 2 ? gp[x * HEAD + own] : gp[own * HEAD + x];
-                    }
-                }
-            } else if (role == 1) {      // the summaries are read and chained once, by the value-major wavefronts
-                int ki[16], vi[16];
-#pragma unroll
-                for (int i = 0; i < 16; i++) { ki[i] = own; vi[i] = 16 * (i >> 2) + 4 * g + (i & 3); }
-                const float *pcs = gpart + (size_t)bh * nseg * m * PART, *ends = gs_out ? gs_out + (size_t)bh * HEAD * HEAD : nullptr;
-                chain_summaries<16, true>(X, ki, vi, pcs, (seg + 1) * m, (nseg - 1 - seg) * m, 1, ends);
-#pragma unroll
-                for (int i = 0; i < 16; i++) sm.q1[swz(own, vi[i])] = X[i];      // (the table is not in use yet)
-            }
-        }
-        if (seg != nseg - 1) {           // ... and handed to the other two roles through LDS, each in its own layout
-            lds_barrier();
-            if (role == 0 || role == 2) {
+        bool have = role < 3;
+        if (seg == nseg - 1) {
+            have = have && gs_out != nullptr;
+            if (have) {
+                const float *gp = gs_out + (size_t)bh * HEAD * HEAD;
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int x = 16 * (i >> 2) + 4 * g + (i & 3);
-                    X[i] = role == 2 ? sm.q1[swz(x, own)] : sm.q1[swz(own, x)];
+                    X[i] = role == 2 ? gp[x * HEAD + own] : gp[own * HEAD + x];
                 }
             }
-            have = role < 3;
+        } else {
+            float *table = sm.q1;            // (not in use yet; the table's rows reach into q4)
+            static_assert(offsetof(Bwd16Tiles, q4) == offsetof(Bwd16Tiles, q1) + sizeof(sm.q1), "q1 and q4 are one region");
+            chain_summaries<1>(table, gpart + (size_t)bh * nseg * m * PART, (seg + 1) * m, (nseg - 1 - seg) * m, 1,
+                               gs_out ? gs_out + (size_t)bh * HEAD * HEAD : nullptr, tid);
+            lds_barrier();
+            if (have) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int x = 16 * (i >> 2) + 4 * g + (i & 3);
+                    X[i] = role == 2 ? table[x * CHAIN_LD + own] : table[own * CHAIN_LD + x];
+                }
+            }
         }
         if (have && (role == 1 || role == 2)) {
 #pragma unroll
@@ -1470,13 +1471,17 @@ size_t checkpoint_bytes(int B, int Tlen, int H) {
     return (size_t)B * H * ((Tlen + SB - 1) / SB + 1) * HEAD * HEAD * sizeof(float);     // one slot per step + the final state
 }
 
-// How many time segments run in parallel for one (batch, head).  More segments mean
-// more workgroups (B*H*nseg) to spread over the compute units but also one more light pass
-// over (part of) the inputs; the estimate below counts CU rounds times steps
-// per segment and prefers fewer segments on ties.  wkv_tune(WKV_TUNE_SEGMENTS) /
-// RWKV_WKV_NSEG override it.
+// How many time segments run in parallel for one (batch, head), and in how many pieces each is summarised.  More segments
+// mean more workgroups (B*H*nseg, one per compute unit at a time) with fewer steps each, for one more pass over the inputs
+// and a longer walk over the summaries; shorter pieces a shorter pass and a longer walk.  The plan is the cheapest by the
+// times below, in us, forward and backward together, fitted to B*H = 4 .. 160, T = 128 .. 4096 with decays that forget
+// nothing (with decays that do, passes and walks end early and the optimum is flat); they reproduce those measurements
+// within some 10 %.  E.g. B*H = 12, bf16, T 512: 2 segments of 4 steps 63 us, 8 of one step 40 us; T 4096: 16 of 4 steps
+// 101 us, 16 of 2 pieces each.  wkv_tune / RWKV_WKV_NSEG / RWKV_WKV_PPS override.
 constexpr int MAX_SEG = 64;
 struct SegPlan { int nseg, sps, m, pps; };     // segments, steps per segment, pieces per segment, steps per piece
+struct Costs { double round, step, pass, pass_step, piece; };
+constexpr Costs BF16_COSTS{12.7, 9.2, 7.0, 4.3, 0.42}, F32_COSTS{14.0, 15.6, 8.0, 6.2, 0.54};      // (F32: wkv56_f32.hip)
 inline int &forced_segments() {          // 0 = choose automatically
     static int v = [] { const char *e = getenv("RWKV_WKV_NSEG"); return e ? std::min(std::max(atoi(e), 0), MAX_SEG) : 0; }();
     return v;
@@ -1485,53 +1490,59 @@ inline int &forced_piece_steps() {       // 0 = choose automatically
     static int v = [] { const char *e = getenv("RWKV_WKV_PPS"); return e ? std::max(atoi(e), 0) : 0; }();
     return v;
 }
-// what the summary pass adds to a run in n segments, as a factor on the main kernels' time
-// (at worst the pass reads (n-1)/n of the tokens at about 40 % of the main kernels' cost per token)
-static double segment_overhead(int n) { return 1.0 + 0.4 * (n - 1) / n; }
-static SegPlan plan_segments(int BH, int Tlen, int ncu) {
-    const int nsb = (Tlen + SB - 1) / SB;
-    const int forced = forced_segments();
-    int want = 1;
-    if (forced > 0) {
-        want = std::min(forced, nsb);
-    } else {
-        double best = 1e30;
-        for (int cand = 1; cand <= 16 && cand * 4 <= std::max(4, nsb); cand++) {
-            const int sps = (nsb + cand - 1) / cand;
-            const double rounds = (double)((BH * cand + ncu - 1) / ncu);
-            const double cost = rounds * (sps + 1) * segment_overhead(cand);
-            if (cost < best * 0.97) { best = cost; want = cand; }
+static double plan_cost(int BH, const SegPlan &x, int ncu, const Costs &c) {
+    const double main = (double)((BH * (long)x.nseg + ncu - 1) / ncu) * (c.round + c.step * x.sps);
+    if (x.nseg == 1) return main;
+    const double crowd = std::max(1.0, (double)BH * (x.nseg - 1) * x.m / (1.5 * ncu));        // one and a half workgroups of the pass per compute unit
+    return main + c.pass + c.pass_step * x.pps * crowd + c.piece * (x.nseg * x.m - 1);
+}
+// max_slots: room for summaries, per (batch, head)
+static SegPlan plan_segments(int BH, int Tlen, int ncu, const Costs &c, int max_slots = MAX_SEG) {
+    const int nsb = (Tlen + SB - 1) / SB, forced = forced_segments();
+    SegPlan best{1, nsb, 1, nsb};
+    double best_cost = forced > 0 ? 1e300 : plan_cost(BH, best, ncu, c);
+    const int lo = forced > 0 ? std::min(forced, nsb) : 2, hi = forced > 0 ? lo : std::min(nsb, MAX_SEG);
+    for (int want = lo; want <= hi; want++) {
+        const int sps = (nsb + want - 1) / want, nseg = (nsb + sps - 1) / sps;
+        if (forced <= 0 && nseg != want) continue;                                   // (the same plan as for fewer)
+        for (int pps = forced_piece_steps() > 0 ? std::min(sps, forced_piece_steps()) : sps; ; pps = (pps + 1) / 2) {
+            int m = (sps + pps - 1) / pps, p = pps;
+            if (nseg * m > MAX_SEG && forced_piece_steps() > 0) { m = std::max(1, MAX_SEG / nseg); p = (sps + m - 1) / m; m = (sps + p - 1) / p; }
+            if (nseg * m > MAX_SEG && pps == sps) { m = 1; p = sps; }
+            const SegPlan x{nseg, sps, nseg == 1 ? 1 : m, nseg == 1 ? sps : p};
+            if (nseg * m <= MAX_SEG && (nseg == 1 || nseg * m <= max_slots || forced > 0)) {
+                const double cost = plan_cost(BH, x, ncu, c);
+                if (cost < 0.97 * best_cost) { best = x; best_cost = cost; }         // (on near ties the fewest: every piece walks two steps or more)
+            }
+            if (pps == 1 || forced_piece_steps() > 0 || nseg == 1) break;
         }
     }
-    const int sps = (nsb + want - 1) / want;
-    const int nseg = (nsb + sps - 1) / sps;
-    // the summary pass: cut each segment into pieces until the pass has about 1.5 workgroups per CU
-    // (every piece costs one 16 KB summary, so no finer than needed and never below 2 steps)
-    int pps = sps;
-    if (nseg == 1) return SegPlan{1, sps, 1, sps};
-    if (forced_piece_steps() > 0) pps = std::min(sps, forced_piece_steps());
-    else
-        while (pps >= 4 && (long)BH * (nseg - 1) * ((sps + pps - 1) / pps) < ncu + ncu / 2) pps = (pps + 1) / 2;
-    int m = (sps + pps - 1) / pps;
-    if (nseg * m > MAX_SEG) { m = std::max(1, MAX_SEG / nseg); pps = (sps + m - 1) / m; m = (sps + pps - 1) / pps; }
-    if (nseg * m > MAX_SEG) { m = 1; pps = sps; }
-    return SegPlan{nseg, sps, m, pps};
+    return best;
 }
 // Two groups of (batch, head) pairs.  When B*H is more than a whole number of CU rounds, the whole rounds run their
 // sequences in one piece (group A: the first nA pairs, no summary pass at all) and only the remainder is cut in time
 // (group B), so that it fills one more, shorter round: 320 pairs = 256 whole + 64 x 4 segments instead of 320 x 4.
 struct GroupPlan { int nA; SegPlan a, b; };
-static GroupPlan plan_groups(int BH, int Tlen) {
-    const int nsb = (Tlen + SB - 1) / SB, ncu = cu_count();
-    GroupPlan p{0, SegPlan{1, nsb, 1, nsb}, plan_segments(BH, Tlen, ncu)};
+static GroupPlan make_plan(int BH, int Tlen, int ncu, const Costs &c, int max_slots) {
+    const int nsb = (Tlen + SB - 1) / SB;
+    GroupPlan p{0, SegPlan{1, nsb, 1, nsb}, plan_segments(BH, Tlen, ncu, c, max_slots)};
     const int whole = BH / ncu * ncu, rest = BH - whole;
     if (forced_segments() > 0 || whole == 0 || rest == 0) return p;
-    const SegPlan r = plan_segments(rest, Tlen, ncu);
-    auto cost = [ncu](int bh, const SegPlan &x) {
-        return (double)((bh * x.nseg + ncu - 1) / ncu) * (x.sps + 1) * segment_overhead(x.nseg);
-    };
-    if (cost(whole, p.a) + cost(rest, r) < 0.97 * cost(BH, p.b)) { p.nA = whole; p.b = r; }
+    const SegPlan r = plan_segments(rest, Tlen, ncu, c, max_slots);
+    if (plan_cost(whole, p.a, ncu, c) + plan_cost(rest, r, ncu, c) < 0.97 * plan_cost(BH, p.b, ncu, c)) { p.nA = whole; p.b = r; }
     return p;
+}
+// (a call asks for its plan several times; the last few shapes of a thread are remembered)
+static GroupPlan plan_groups(int BH, int Tlen, const Costs &c = BF16_COSTS, int max_slots = MAX_SEG) {
+    struct Entry { int BH, Tlen, ncu, nseg, pps, slots; const Costs *c; GroupPlan plan; };
+    static thread_local Entry known[16] = {};
+    const Entry want{BH, Tlen, cu_count(), forced_segments(), forced_piece_steps(), max_slots, &c, {}};
+    Entry &e = known[(BH * 31 + Tlen * 7 + (&c == &F32_COSTS)) & 15];
+    if (e.BH != BH || e.Tlen != Tlen || e.ncu != want.ncu || e.nseg != want.nseg || e.pps != want.pps || e.slots != max_slots || e.c != &c) {
+        e = want;
+        e.plan = make_plan(BH, Tlen, want.ncu, c, max_slots);
+    }
+    return e.plan;
 }
 // the piece summaries of a plan: one slot per (batch, head) and piece (slots are indexed by the pair's number in the
 // whole batch, so the pairs of group A have unused ones)
@@ -1556,9 +1567,9 @@ static Layout layout(int B, int Tlen, int C, int H, const GroupPlan &gp) {
 }
 // true when the plan in force cuts some sequence of this shape into time segments
 bool splits_time(int BH, int Tlen) { return plan_groups(BH, Tlen).b.nseg > 1; }
-size_t forward_workspace(int B, int Tlen, int H) { return layout(B, Tlen, H * HEAD, H, plan_groups(B * H, Tlen)).forward_total; }
-size_t forward_scratch(int B, int Tlen, int H) { return part_bytes(B * H, plan_groups(B * H, Tlen)); }
-size_t backward_workspace(int B, int Tlen, int C, int H) { return layout(B, Tlen, C, H, plan_groups(B * H, Tlen)).total; }
+size_t forward_workspace(int B, int Tlen, int H, const Costs &c) { return layout(B, Tlen, H * HEAD, H, plan_groups(B * H, Tlen, c)).forward_total; }
+size_t forward_scratch(int B, int Tlen, int H, const Costs &c) { return part_bytes(B * H, plan_groups(B * H, Tlen, c)); }
+size_t backward_workspace(int B, int Tlen, int C, int H, const Costs &c) { return layout(B, Tlen, C, H, plan_groups(B * H, Tlen, c)).total; }
 
 // The 16-wavefront kernels use more LDS than a kernel gets by default.  Raising the limit is a property of the loaded
 // code object and is done once per device, from wkv_init() or from the first launch there, whichever comes first.

@@ -40,7 +40,7 @@ using chunked::PART;
 using chunked::SB;
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-constexpr int LD = 68;        // padded rows of a [64][64] table: conflict-free along rows and along columns
+constexpr int LD = chunked::CHAIN_LD;      // padded rows of a [64][64] table: conflict-free along rows and along columns
 constexpr int NT = 512;       // eight wavefronts
 
 __device__ __forceinline__ f4 zero4() { return f4{0.f, 0.f, 0.f, 0.f}; }
@@ -154,20 +154,21 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
 
     // chain wavefronts: S[kk][e] = S[key 16kk+4g+e][value 16q+n]
     f4 S[4] = {zero4(), zero4(), zero4(), zero4()};
-    if (chain) {
-        float X[16];
-        int ki[16], vi[16];
-#pragma unroll
-        for (int i = 0; i < 16; i++) { ki[i] = 16 * (i >> 2) + 4 * g + (i & 3); vi[i] = 16 * q + n; }
+    {
         const float *sp = s_in + (size_t)bh * HEAD * HEAD;
-        if (seg == 0) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) X[i] = sp[ki[i] * HEAD + vi[i]];
-        } else {
-            chunked::chain_summaries<16, false>(X, ki, vi, part + (size_t)bh * nseg * m * PART, seg * m - 1, seg * m, -1, sp);
+        float *table = sh.step[1].rm;            // (not in use yet)
+        if (seg > 0) {
+            chunked::chain_summaries<2>(table, part + (size_t)bh * nseg * m * PART, seg * m - 1, seg * m, -1, sp, threadIdx.x);
+            lds_barrier();
         }
+        if (chain) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) S[i >> 2][i & 3] = X[i];
+            for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    S[kk][e] = seg > 0 ? table[(16 * kk + 4 * g + e) * LD + 16 * q + n] : sp[(16 * kk + 4 * g + e) * HEAD + 16 * q + n];
+        }
+        if (seg > 0) lds_barrier();              // (the table's place is written before the loop's first barrier)
     }
 
     // preparing wavefronts: tokens tok0 .. tok0+7 of the step, channel `lane`
@@ -423,19 +424,16 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
     float A = 0.f;                           // running sum of the decay gradient at the end of a step, key `lane`
     {
         float X[16];
-        int ki[16], vi[16];
+        const float *ends = gs_out ? gs_out + (size_t)bh * HEAD * HEAD : nullptr;
+        float *table = sm.dr;
+        if (seg != nseg - 1) {
+            chunked::chain_summaries<2>(table, gpart + (size_t)bh * nseg * m * PART, (seg + 1) * m, (nseg - 1 - seg) * m, 1, ends, threadIdx.x);
+            lds_barrier();
+        }
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            const int x = 16 * (i >> 2) + 4 * g + (i & 3);
-            ki[i] = keys ? own : x; vi[i] = keys ? x : own;
-            X[i] = 0.f;
-        }
-        const float *ends = gs_out ? gs_out + (size_t)bh * HEAD * HEAD : nullptr;
-        if (seg != nseg - 1)
-            chunked::chain_summaries<16, false>(X, ki, vi, gpart + (size_t)bh * nseg * m * PART, (seg + 1) * m, (nseg - 1 - seg) * m, 1, ends);
-        else if (ends) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) X[i] = ends[ki[i] * HEAD + vi[i]];
+            const int x = 16 * (i >> 2) + 4 * g + (i & 3), key = keys ? own : x, value = keys ? x : own;
+            X[i] = seg != nseg - 1 ? table[key * LD + value] : ends ? ends[key * HEAD + value] : 0.f;
         }
         if (keys) {       // anchored at the segment's end: sum_j G o S
             const float *cp = ck_lane + (size_t)sb1 * HEAD * HEAD;
@@ -707,7 +705,7 @@ template <class T, class W, bool PT> struct Kernels {
                                const float *u, const float *s_in, const void *gy, const float *gs_out, void *gr, void *gk, void *gv, void *gw,
                                float *gu, float *gs_in, void *workspace, bool have_ckpt, int floor_decay) {
         const int BH = B * H;
-        const chunked::GroupPlan gp = chunked::plan_groups(BH, Tlen);
+        const chunked::GroupPlan gp = chunked::plan_groups(BH, Tlen, chunked::F32_COSTS);
         const chunked::Layout L = chunked::layout(B, Tlen, C, H, gp);
         const chunked::SegPlan &pl = gp.b;
         char *ws = (char *)workspace;
@@ -763,7 +761,7 @@ static hipError_t forward_launch(hipStream_t s, int dtype, bool per_token, bool 
                                  bool keep, int floor_decay) {
     hipError_t e = init_kernels();
     if (e != hipSuccess) return e;
-    const chunked::GroupPlan gp = chunked::plan_groups(B * H, Tlen);
+    const chunked::GroupPlan gp = chunked::plan_groups(B * H, Tlen, chunked::F32_COSTS);
     const chunked::Layout L = chunked::layout(B, Tlen, C, H, gp);
     char *ws = (char *)workspace;
     float *part = ws && gp.b.nseg > 1 && s_in != s_out ? (float *)(ws + (keep ? L.part : 0)) : nullptr;

@@ -38,7 +38,8 @@ hipError_t init_static_scratch() {
 hipError_t forward_static_launch(hipStream_t s, bool per_token, bool w16, int B, int Tlen, int C, int H, const void *r, const void *k,
                                  const void *v, const void *w, const float *u, const float *s_in, void *y, float *s_out,
                                  int floor_decay) {
-    const GroupPlan gp = plan_groups(B * H, Tlen);
+    // (as many segments and pieces as the array has room for)
+    const GroupPlan gp = plan_groups(B * H, Tlen, BF16_COSTS, (int)(STATIC_SCRATCH_BYTES / (PART * sizeof(float)) / ((size_t)B * H)));
     if (part_bytes(B * H, gp) > STATIC_SCRATCH_BYTES) return hipErrorOutOfMemory;
     void *ptr = nullptr;
     if (gp.b.nseg > 1) {
