@@ -296,6 +296,10 @@ int wkv_sigmoid_mul_forward(void *stream, size_t n, int dtype, const void *r, co
 int wkv_sigmoid_mul_backward(void *stream, size_t n, int dtype, const void *r, const void *kv, const void *gout,
                              void *gr, void *gkv);
 
+/* in: HOST array of up to 16 device pointers to bf16 parameters of C elements; out (count, C) fp32: their values, the form
+ * in which the functions above take coefficients, weights and biases. */
+int wkv_widen_rows(void *stream, int count, int C, const void *const *in, float *out);
+
 /* ---- A layer for one token per sequence (a serving loop), bf16, at most 64 rows (sequences) at a time.
  *
  * Products of the rows with up to 8 weight matrices in one launch:  out = f(x' W),

@@ -488,6 +488,18 @@ int wkv_ln_gate_backward(void *stream, int rows, int C, int dtype, float scale, 
     return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
 }
 
+int wkv_widen_rows(void *stream, int count, int C, const void *const *in, float *out) {
+    if (count <= 0 || count > edges::MAX_WIDEN || C <= 0) return WKV_ERR_DIMS;
+    if (!in || !out) return WKV_ERR_NULL;
+    edges::ConstPtrs<edges::MAX_WIDEN> p{};
+    for (int i = 0; i < count; i++) {
+        if (!in[i]) return WKV_ERR_NULL;
+        p.p[i] = in[i];
+    }
+    hipLaunchKernelGGL(edges::widen_rows, dim3((C + 255) / 256, count), dim3(256), 0, (hipStream_t)stream, C, p, out);
+    return hipGetLastError() == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
+}
+
 int wkv_rows_products(void *stream, int row_count, int k, int count, const wkv_rows_product *products) {
     if (row_count <= 0 || row_count > rows::MAX_ROWS || k <= 0 || k % 64 != 0 || count <= 0 || count > rows::MAX_JOBS) return WKV_ERR_DIMS;
     if (!products) return WKV_ERR_NULL;

@@ -55,6 +55,13 @@ __device__ __forceinline__ void stream8(f16 *p, const float (&o)[8]) {
 template <int N> struct Ptrs { void *p[N]; };
 template <int N> struct ConstPtrs { const void *p[N]; };
 
+// Several bf16 parameters of C elements as rows of one fp32 table (one launch in place of one per parameter).
+constexpr int MAX_WIDEN = 16;
+__global__ __launch_bounds__(256) void widen_rows(int C, ConstPtrs<MAX_WIDEN> in, float *__restrict__ out) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c < C) out[(size_t)blockIdx.y * C + c] = to_float(static_cast<const bf16 *>(in.p[blockIdx.y])[c]);
+}
+
 // out_j[t] = x[t] + (x[t-1] - x[t]) * d_j[t],  x[-1] = shift.
 // lerp != 0: coef_j is the reference's time_mix_j (weight of x itself), d_j = 1 - coef_j;
 // lerp == 0: coef_j is time_maa_j (weight of the difference), d_j = coef_j (+ dyn_j[t] for the data-dependent mix).

@@ -27,7 +27,11 @@ namespace {
 #define WKV_ABI(X)                                                                                                          \
     X(wkv_strerror) X(wkv5_forward) X(wkv6_forward) X(wkv5_forward_workspace) X(wkv6_forward_workspace) X(wkv5_backward)      \
     X(wkv6_backward) X(wkv5_backward_workspace) X(wkv6_backward_workspace) X(wkv56_forward_scratch) X(wkv6_decode) X(wkv4_forward) X(wkv4_backward)    \
-    X(wkv4_checkpoint_bytes) X(wkv4_backward_workspace) X(wkv_rows_products) X(wkv_lora_mix_rows) X(wkv_timemix_head)
+    X(wkv4_checkpoint_bytes) X(wkv4_backward_workspace) X(wkv_rows_products) X(wkv_lora_mix_rows) X(wkv_timemix_head)         \
+    X(wkv_widen_rows) X(wkv_shift_mix_forward) X(wkv_shift_mix_backward) X(wkv_shift_mix_backward_workspace)                  \
+    X(wkv_lora_mix_forward) X(wkv_lora_mix_backward) X(wkv_lora_mix_backward_workspace) X(wkv_ln_gate_forward)                \
+    X(wkv_ln_gate_backward) X(wkv_ln_gate_backward_workspace) X(wkv_relu_square_forward) X(wkv_relu_square_backward)          \
+    X(wkv_sigmoid_mul_forward) X(wkv_sigmoid_mul_backward)
 struct {
 #define X(name) decltype(&::name) name = nullptr;
     WKV_ABI(X)
@@ -129,11 +133,12 @@ Forward56 forward56(int version, const Dims &d, int algo, const Tensor &r, const
 
 struct Backward56 { Tensor gr, gk, gv, gw, gu, gs; };
 Backward56 backward56(int version, const Dims &d, int algo, const Tensor &r, const Tensor &k, const Tensor &v, const Tensor &w,
-                      const Tensor &u, const Tensor &s, const Tensor &gy, const Tensor &gstate, Tensor ws, bool want_gs) {
+                      const Tensor &u, const Tensor &s, const Tensor &gy, const Tensor &gstate, Tensor ws, bool want_gs,
+                      const Tensor &gu = Tensor()) {
     const int dt = dtype_code(r);
     OnDevice dev(r);
-    Backward56 g{at::empty_like(r), at::empty_like(k), at::empty_like(v), at::empty_like(w), at::empty_like(u),
-                 want_gs ? at::empty_like(s) : Tensor()};
+    Backward56 g{at::empty_like(r), at::empty_like(k), at::empty_like(v), at::empty_like(w),
+                 gu.defined() ? gu : at::empty_like(u), want_gs ? at::empty_like(s) : Tensor()};
     unsigned flags = flags_of(d, w);               // (a bf16 w has its gradient in bf16 too)
     const size_t need = backward_bytes(version, d, dt, algo);
     if (ws.defined() && (size_t)ws.numel() >= need) flags |= WKV_CHECKPOINTS_VALID;
@@ -365,158 +370,17 @@ PyObject *py_wkv4(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// ---- layers, one token per sequence (csrc/layer_decode.hip)
-// A module's parameters and submodules are read from its dictionaries: nn.Module's attribute lookup costs more than a
-// kernel's launch.  Whatever is not plain (hooks, biases, subclasses of Linear, other types or sizes, autograd or
-// autocast switched on) gets no answer here, and the caller takes its general way.
-PyObject *linear_type = nullptr, *group_norm_type = nullptr;
-PyObject *dict_of(PyObject *o) {          // borrowed
-    PyObject **d = _PyObject_GetDictPtr(o);
-    return d ? *d : nullptr;
-}
-PyObject *item(PyObject *dict, const char *name) {          // borrowed, or NULL
-    return dict && PyDict_Check(dict) ? PyDict_GetItemString(dict, name) : nullptr;
-}
-struct Plain {          // collects the tensors of one call; `ok` falls if one of them is not what the kernels take
-    const Tensor &x;
-    bool ok = true;
-    explicit Plain(const Tensor &x_) : x(x_) {}
-    const void *check(const Tensor &t, int64_t numel, at::ScalarType type = at::kBFloat16) {
-        ok = ok && t.defined() && t.device() == x.device() && t.scalar_type() == type && t.numel() == numel && t.is_contiguous() &&
-             !t.key_set().has(c10::DispatchKey::Python) && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
-        return ok ? t.data_ptr() : nullptr;
-    }
-    const void *parameter(PyObject *params, const char *name, int64_t numel) {
-        PyObject *o = item(params, name);
-        if (!o || !THPVariable_Check(o)) { ok = false; return nullptr; }
-        return ok ? check(THPVariable_Unpack(o), numel) : nullptr;
-    }
-    const void *linear(PyObject *modules, const char *name, int64_t n, int64_t k) {          // weight (n, k), no bias
-        PyObject *o = item(modules, name), *d = nullptr, *p;
-        ok = ok && o && (PyObject *)Py_TYPE(o) == linear_type && (d = dict_of(o)) && !item(d, "forward") && (p = item(d, "_parameters")) &&
-             item(p, "bias") == Py_None && unhooked(d);
-        return ok ? parameter(item(d, "_parameters"), "weight", n * k) : nullptr;
-    }
-    static bool unhooked(PyObject *d) {
-        for (const char *name : {"_forward_hooks", "_forward_pre_hooks"}) {
-            PyObject *h = item(d, name);
-            if (!h || PyObject_Length(h) != 0) return false;
-        }
-        return true;
-    }
-};
-// x (B, 1, C) bf16 on the GPU with nothing recording
-bool single_tokens(const Tensor &x) {
-    return x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 3 && x.size(1) == 1 && x.size(0) >= 1 && x.size(0) <= 64 &&
-           x.size(2) % 64 == 0 && !at::GradMode::is_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA);
-}
+#include "host_layers.h"
 
-// timemix_decode(version, module, x, (shift, state)) -> (out, (x[:, -1], new state)), or None: not a call for these kernels
-PyObject *py_timemix_decode(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    HANDLE_TH_ERRORS
-    arity(n, 4);
-    const int version = integer(a[0]);
-    PyObject *d = dict_of(a[1]), *prm = item(d, "_parameters"), *mod = item(d, "_modules"), *heads = item(d, "n_head");
-    if (!prm || !mod || !heads || !THPVariable_Check(a[2]) || !PyTuple_Check(a[3]) || PyTuple_GET_SIZE(a[3]) != 2) Py_RETURN_NONE;
-    const Tensor &x = tensor(a[2]);
-    if (!single_tokens(x)) Py_RETURN_NONE;
-    const int64_t B = x.size(0), C = x.size(2), H = PyLong_AsLong(heads);
-    if (H * 64 != C) { PyErr_Clear(); Py_RETURN_NONE; }
-    const Tensor &shift = tensor(PyTuple_GET_ITEM(a[3], 0)), &state = tensor(PyTuple_GET_ITEM(a[3], 1));
-    Plain p(x);
-    const void *px = p.check(x, B * C), *ps = p.check(shift, B * C);
-    const float *s_in = static_cast<const float *>(p.check(state, B * H * 64 * 64, at::kFloat));
-    const void *wr = p.linear(mod, "receptance", C, C), *wk = p.linear(mod, "key", C, C), *wvv = p.linear(mod, "value", C, C),
-               *wg = p.linear(mod, "gate", C, C), *wo = p.linear(mod, "output", C, C);
-    const void *td = p.parameter(prm, "time_decay", C), *u = p.parameter(prm, "time_faaaa", C);
-    PyObject *ln = item(mod, "ln_x"), *lnd = nullptr, *eps = nullptr;
-    p.ok = p.ok && ln && (PyObject *)Py_TYPE(ln) == group_norm_type && (lnd = dict_of(ln)) && (eps = item(lnd, "eps")) && PyFloat_Check(eps);
-    if (!p.ok) Py_RETURN_NONE;
-    const void *lnw = p.parameter(item(lnd, "_parameters"), "weight", C), *lnb = p.parameter(item(lnd, "_parameters"), "bias", C);
-    const void *maa[5] = {}, *maa_x = nullptr, *w1 = nullptr, *w2 = nullptr, *dw1 = nullptr, *dw2 = nullptr;
-    if (version == 6) {
-        const char *names[5] = {"time_maa_w", "time_maa_k", "time_maa_v", "time_maa_r", "time_maa_g"};
-        for (int j = 0; j < 5; j++) maa[j] = p.parameter(prm, names[j], C);
-        maa_x = p.parameter(prm, "time_maa_x", C);
-        w1 = p.parameter(prm, "time_maa_w1", C * 160); w2 = p.parameter(prm, "time_maa_w2", C * 160);
-        dw1 = p.parameter(prm, "time_decay_w1", C * 64); dw2 = p.parameter(prm, "time_decay_w2", C * 64);
-    } else {
-        const char *names[4] = {"time_mix_k", "time_mix_v", "time_mix_r", "time_mix_g"};
-        for (int j = 0; j < 4; j++) maa[j] = p.parameter(prm, names[j], C);
-    }
-    if (!p.ok) Py_RETURN_NONE;
-
-    at::AutoDispatchBelowADInplaceOrView below;
-    OnDevice dev(x);
-    void *stream = dev.stream();
-    // scratch: r, k, v, gate, the head results; v6 also the five mixes and the two LoRAs' activations
-    const int64_t rows = B * C;
-    constexpr int64_t parts = 2 * WKV_LORA_PARTS;          // (fp32 counted in bf16)
-    Tensor scratch = at::empty({(version == 6 ? 10 : 5) * rows + (version == 6 ? parts * B * 224 : 0)}, x.options());
-    at::BFloat16 *q = scratch.data_ptr<at::BFloat16>();
-    at::BFloat16 *r = q, *k = r + rows, *v = k + rows, *g = v + rows, *z = g + rows, *mixes = z + rows, *act = mixes + 5 * rows, *lora = act + parts * B * 160;
-    Tensor out = at::empty_like(x), new_state = at::empty_like(state);
-    if (version == 6) {
-        const wkv_rows_product first{w1, px, ps, maa_x, nullptr, act, 160, 1, 0, 0};
-        check(abi.wkv_rows_products(stream, B, C, 1, &first), "wkv_rows_products");
-        check(abi.wkv_lora_mix_rows(stream, B, C, px, ps, maa, act, w2, mixes), "wkv_lora_mix_rows");
-        const wkv_rows_product proj[5] = {{dw1, mixes, nullptr, nullptr, nullptr, lora, 64, 1, 0, 0},
-                                          {wk, mixes + rows, nullptr, nullptr, nullptr, k, (int)C, 0, 0, 0},
-                                          {wvv, mixes + 2 * rows, nullptr, nullptr, nullptr, v, (int)C, 0, 0, 0},
-                                          {wr, mixes + 3 * rows, nullptr, nullptr, nullptr, r, (int)C, 0, 0, 0},
-                                          {wg, mixes + 4 * rows, nullptr, nullptr, nullptr, g, (int)C, 0, 0, 0}};
-        check(abi.wkv_rows_products(stream, B, C, 5, proj), "wkv_rows_products");
-    } else {
-        const wkv_rows_product proj[4] = {{wk, px, ps, maa[0], nullptr, k, (int)C, 0, 1, 0}, {wvv, px, ps, maa[1], nullptr, v, (int)C, 0, 1, 0},
-                                          {wr, px, ps, maa[2], nullptr, r, (int)C, 0, 1, 0}, {wg, px, ps, maa[3], nullptr, g, (int)C, 0, 1, 0}};
-        check(abi.wkv_rows_products(stream, B, C, 4, proj), "wkv_rows_products");
-    }
-    check(abi.wkv_timemix_head(stream, B, C, H, r, k, v, g, td, version == 6 ? lora : nullptr, dw2, u, lnw, lnb, version == 6 ? 1.f : 0.125f,
-                               (float)PyFloat_AS_DOUBLE(eps), s_in, fptr(new_state), z), "wkv_timemix_head");
-    const wkv_rows_product last{wo, z, nullptr, nullptr, nullptr, ptr(out), (int)C, 0, 0, 0};
-    check(abi.wkv_rows_products(stream, B, C, 1, &last), "wkv_rows_products");
-    PyObject *states = tuple(x.select(1, 0), new_state);
-    return Py_BuildValue("(NN)", wrapped(out), states);
-    END_HANDLE_TH_ERRORS
-}
-
-// channelmix_decode(version, module, x, shift) -> (out, x[:, -1]), or None
-PyObject *py_channelmix_decode(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    HANDLE_TH_ERRORS
-    arity(n, 4);
-    const bool lerp = integer(a[0]) == 5;
-    PyObject *d = dict_of(a[1]), *prm = item(d, "_parameters"), *mod = item(d, "_modules"), *key = item(mod, "key"), *kp;
-    if (!prm || !key || !THPVariable_Check(a[2]) || !THPVariable_Check(a[3])) Py_RETURN_NONE;
-    const Tensor &x = tensor(a[2]), &shift = tensor(a[3]);
-    if (!single_tokens(x) || !(kp = item(item(dict_of(key), "_parameters"), "weight")) || !THPVariable_Check(kp)) Py_RETURN_NONE;
-    const int64_t B = x.size(0), C = x.size(2), F = THPVariable_Unpack(kp).numel() / C;
-    if (F < 64 || F % 64 != 0 || F > INT_MAX / C) Py_RETURN_NONE;
-    Plain p(x);
-    const void *px = p.check(x, B * C), *ps = p.check(shift, B * C);
-    const void *wk = p.linear(mod, "key", F, C), *wr = p.linear(mod, "receptance", C, C), *wvv = p.linear(mod, "value", C, F);
-    const void *mk = p.parameter(prm, lerp ? "time_mix_k" : "time_maa_k", C), *mr = p.parameter(prm, lerp ? "time_mix_r" : "time_maa_r", C);
-    if (!p.ok) Py_RETURN_NONE;
-
-    at::AutoDispatchBelowADInplaceOrView below;
-    OnDevice dev(x);
-    Tensor scratch = at::empty({B * (F + C)}, x.options()), out = at::empty_like(x);
-    at::BFloat16 *k = scratch.data_ptr<at::BFloat16>(), *r = k + B * F;
-    const wkv_rows_product proj[2] = {{wk, px, ps, mk, nullptr, k, (int)F, 0, lerp, 1}, {wr, px, ps, mr, nullptr, r, (int)C, 0, lerp, 0}};
-    check(abi.wkv_rows_products(dev.stream(), B, C, 2, proj), "wkv_rows_products");
-    const wkv_rows_product last{wvv, k, nullptr, nullptr, r, ptr(out), (int)C, 0, 0, 2};
-    check(abi.wkv_rows_products(dev.stream(), B, F, 1, &last), "wkv_rows_products");
-    return tuple(out, x.select(1, 0));
-    END_HANDLE_TH_ERRORS
-}
-
-// bind(path of the kernel library, WKVError, torch.nn.Linear, torch.nn.GroupNorm)
+// bind(path of the kernel library, WKVError, torch.nn.Linear, torch.nn.GroupNorm, (the dictionaries of hooks on all modules))
 PyObject *py_bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    arity(n, 4);
+    arity(n, 5);
+    REQUIRE(PyTuple_Check(a[4]));
     const char *path = PyUnicode_AsUTF8(a[0]);
     if (!path) throw python_error();
-    for (int i = 1; i < 4; i++) Py_INCREF(a[i]);
-    wkv_error = a[1]; linear_type = a[2]; group_norm_type = a[3];
+    for (int i = 1; i < 5; i++) Py_INCREF(a[i]);
+    wkv_error = a[1]; linear_type = a[2]; group_norm_type = a[3]; global_hooks = a[4];
     void *lib = dlopen(path, RTLD_NOW | RTLD_LOCAL);
     if (!lib) raise(wkv_error, dlerror());
 #define X(name)                                                                   \
@@ -529,8 +393,8 @@ PyObject *py_bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_##name)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {METHOD(bind), METHOD(wkv56), METHOD(forward56), METHOD(backward56), METHOD(decay_operand), METHOD(wkv4), METHOD(timemix_decode),
-                         METHOD(channelmix_decode),
+PyMethodDef methods[] = {METHOD(bind), METHOD(wkv56), METHOD(forward56), METHOD(backward56), METHOD(decay_operand), METHOD(wkv4), METHOD(timemix),
+                         METHOD(channelmix),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "native host side of rwkv_wkv_hip", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -61,6 +61,7 @@ SIGNATURES = {
     "wkv_relu_square_backward": (_I, [_P, c_size_t, _I, _P, _P, _P]),
     "wkv_sigmoid_mul_forward": (_I, [_P, c_size_t, _I, _P, _P, _P]),
     "wkv_sigmoid_mul_backward": (_I, [_P, c_size_t, _I] + [_P] * 5),
+    "wkv_widen_rows": (_I, [_P, _I, _I, _P, _P]),
     "wkv_rows_products": (_I, [_P, _I, _I, _I, _P]),
     "wkv_lora_mix_rows": (_I, [_P, _I, _I] + [_P] * 6),
     "wkv_timemix_head": (_I, [_P, _I, _I, _I] + [_P] * 10 + [c_float, c_float] + [_P] * 3),
@@ -110,7 +111,9 @@ def host():
         except ImportError as e:
             raise WKVError(f"the native host side is missing: build it first (make -C rwkv-infctx-trainer_amd/csrc): {e}") from e
         import torch
-        module.bind(LIB_PATH, WKVError, torch.nn.Linear, torch.nn.GroupNorm)
+        m = torch.nn.modules.module
+        hooks = (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks, m._global_backward_pre_hooks)
+        module.bind(LIB_PATH, WKVError, torch.nn.Linear, torch.nn.GroupNorm, hooks)
         _host = module
     return _host
 

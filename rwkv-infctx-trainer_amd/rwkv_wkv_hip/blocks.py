@@ -23,6 +23,7 @@ import ctypes
 import torch
 
 from . import _lib
+from . import ops as _ops
 from ._lib import check
 from .ops import _DT, _on_gpu, _ptr, _stream, _workspace, WKV_5, WKV_6
 
@@ -273,12 +274,22 @@ class L2Wrap(torch.autograd.Function):
 
 
 # ---- block forwards on these kernels -------------------------------------------------------------------------------
-# One token per sequence without autograd (a serving loop) takes kernels of its own, csrc/layer_decode.hip, where module
-# and inputs are plain bf16; host().*_decode answers None for every other call.
+# A plain bf16 module is run by the native host side (csrc/host_layers.h: each half of a layer one autograd node, single
+# tokens without autograd on kernels of their own); it answers None for every other call, and the code below does the same
+# step by step.
+def _native_timemix(version, self, x, last_state):
+    if _ops._cache is not None or not _lora_mix_on:       # (the recompute cache sees the operator's calls)
+        return None
+    out = _lib.host().timemix(version, _ops._algo, self, x, last_state)
+    if out is not None:
+        _ops.stats["forward_launches"] += 1
+    return out
+
+
 def timemix5_forward(self, x, last_state):
     """RWKV_TimeMix._forward_cuda of v5 (RWKV-v5/src/module/TimeMix.py:286-323): returns
     (out (B,T,C), (shift_state_out (B,C), wkv_state_out (B,H,64,64)))."""
-    out = _lib.host().timemix_decode(5, self, x, last_state)
+    out = _native_timemix(5, self, x, last_state)
     if out is not None:
         return out
     B, T, C = x.shape
@@ -293,7 +304,7 @@ def timemix5_forward(self, x, last_state):
 
 def timemix6_forward(self, x, last_state):
     """RWKV_TimeMix6_0._forward_cuda (RWKV-v6/src/module/TimeMix.py:253-302)."""
-    out = _lib.host().timemix_decode(6, self, x, last_state)
+    out = _native_timemix(6, self, x, last_state)
     if out is not None:
         return out
     B, T, C = x.shape
@@ -318,7 +329,7 @@ def timemix6_forward(self, x, last_state):
 
 def channelmix5_forward(self, x, last_state):
     """RWKV_ChannelMix.forward of v5 (RWKV-v5/src/module/ChannelMix.py:35-49)."""
-    out = _lib.host().channelmix_decode(5, self, x, last_state)
+    out = _lib.host().channelmix(5, self, x, last_state)
     if out is not None:
         return out
     xk, xr = token_shift_mix(x, last_state, (self.time_mix_k, self.time_mix_r), lerp=True)
@@ -328,7 +339,7 @@ def channelmix5_forward(self, x, last_state):
 
 def channelmix6_forward(self, x, last_state):
     """RWKV_ChannelMix6_0.forward (RWKV-v6/src/module/ChannelMix.py:30-37)."""
-    out = _lib.host().channelmix_decode(6, self, x, last_state)
+    out = _lib.host().channelmix(6, self, x, last_state)
     if out is not None:
         return out
     xk, xr = token_shift_mix(x, last_state, (self.time_maa_k, self.time_maa_r))

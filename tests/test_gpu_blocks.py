@@ -313,6 +313,49 @@ def test_layer_of_single_tokens(version, B, H, ffn):
 
 
 @pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("T,frozen", [(1, ()), (2, ("key",)), (65, ()), (130, ("ln_x", "output", "value", "time"))])
+def test_layer_native_matches_the_steps(version, T, frozen):
+    """A layer's halves as the native host side runs them against the same kernels step by step (which a hook on one of the
+    submodules asks for), with and without autograd and with some parameters frozen.  The two do the same operations in the
+    same order; a matrix product may still be given another library kernel, whose sums round differently: one bf16 rounding
+    (2^-8) per element of each result, in norm, carried through at most six products in a row."""
+    from rwkv_wkv_hip import blocks as K
+    B, C, H = 2, 128, 2
+    g = _g(17)
+    x, gy = torch.randn(B, T, C, generator=g), torch.randn(B, T, C, generator=g)
+    tm, cm = (TimeMix5 if version == 5 else TimeMix6)(C, H, seed=8), (ChannelMix5 if version == 5 else ChannelMix6)(C, 4 * C, seed=9)
+    for m in (tm, cm):
+        for n, p in m.named_parameters():
+            p.requires_grad_(not n.startswith(frozen))
+    timemix, channelmix = (K.timemix5_forward, K.channelmix5_forward) if version == 5 else (K.timemix6_forward, K.channelmix6_forward)
+
+    def layer(hooked, grad):
+        mods = [copy.deepcopy(m).cuda().bfloat16() for m in (tm, cm)]
+        if hooked:
+            for m in mods:
+                m.key.register_forward_hook(lambda *a: None)
+        rows = [t.cuda().bfloat16().requires_grad_(grad) for t in (x, x[:, 0] * 0.5, x[:, 0] * 0.25)]
+        wkv = torch.randn(B, H, 64, 64, generator=_g(18)).cuda().requires_grad_(grad)
+        with torch.set_grad_enabled(grad):
+            a, (sh, s) = timemix(mods[0], rows[0], (rows[1], wkv))
+            y, sh2 = channelmix(mods[1], a, rows[2])
+        assert torch.equal(sh, rows[0][:, -1]) and torch.equal(sh2, a[:, -1])
+        if not grad:
+            return {"a": a, "s": s, "y": y}
+        torch.autograd.backward([y, s, sh2], [gy.cuda().bfloat16(), torch.ones_like(s) * 0.1, torch.ones_like(sh2) * 0.1])
+        named = {f"{i}.{n}": p.grad for i, m in enumerate(mods) for n, p in m.named_parameters()}
+        return {"a": a, "s": s, "y": y, "gwkv": wkv.grad, **{f"grow{i}": t.grad for i, t in enumerate(rows)}, **named}
+
+    for grad in (True, False):
+        got, ref = layer(False, grad), layer(True, grad)
+        for n in ref:
+            assert (got[n] is None) == (ref[n] is None), n
+            if ref[n] is not None:
+                assert got[n].dtype == ref[n].dtype and got[n].shape == ref[n].shape, n
+                assert (got[n] - ref[n]).float().norm() <= 6 * 2 ** -8 * ref[n].float().norm(), n
+
+
+@pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_channelmix_forward_on_the_kernels(version, dtype):
     from rwkv_wkv_hip import blocks as K
