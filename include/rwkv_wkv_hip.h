@@ -122,7 +122,8 @@ int wkv_profile_end(float *ms, int capacity);
  * WKV_CHECKPOINTS_VALID saves backward one sweep over k, v, w. */
 /* state_out == state_in (the state updated in place) is accepted for fp32 and fp16 streams, and by the chunked algorithm
  * whenever the plan cuts no sequence of the shape into time segments (B*H at least the number of compute units, or
- * WKV_TUNE_SEGMENTS 1); where it does (short batches, e.g. the 7B shape with B = 1), and for buffers that overlap
+ * WKV_TUNE_SEGMENTS 1, or at most 448 tokens with no segment count set: such calls run in one piece where the state is
+ * updated in place); where it does (short batches, e.g. the 7B shape with B = 1), and for buffers that overlap
  * without being the same, the call returns WKV_ERR_ALIAS and the caller keeps two state buffers and alternates.
  * The same holds for wkv5_forward and wkv6_forward_noalloc. */
 size_t wkv6_forward_workspace(int B, int T, int C, int H, int dtype, int algo);

@@ -71,7 +71,7 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
         if (!aligned16(p)) return WKV_ERR_ALIGN;
     const int a = pick_algo56(algo, T, C, dtype, flags);
     if (a < 0) return a;
-    st = check_state_alias(state_in, state_out, B, H, a == WKV_ALGO_CHUNKED && chunked::splits_time(B * H, T));
+    st = check_state_alias(state_in, state_out, B, H, a == WKV_ALGO_CHUNKED && chunked::needs_two_states(B * H, T));
     if (st) return st;
     if (!decay_type_fits(a, dtype, per_token, flags)) return WKV_ERR_ALGO;
     const bool w16 = (flags & (WKV_W_BF16 | WKV_W_F16)) != 0;
@@ -277,7 +277,7 @@ int wkv6_forward_noalloc(void *stream, int B, int T, int C, int H, int dtype, un
                           (const void *)state_out})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
     if (pick_algo56(WKV_ALGO_CHUNKED, T, C, dtype, flags) != WKV_ALGO_CHUNKED) return WKV_ERR_ALGO;
-    st = check_state_alias(state_in, state_out, B, H, chunked::splits_time(B * H, T));
+    st = check_state_alias(state_in, state_out, B, H, chunked::needs_two_states(B * H, T));
     if (st) return st;
     hipError_t e = chunked::forward_static_launch((hipStream_t)stream, true, (flags & WKV_W_BF16) != 0, B, T, C, H, r, k, v, w,
                                                   u, state_in, y, state_out, (flags & WKV_FLOOR_DECAY) ? 1 : 0);

@@ -1565,8 +1565,11 @@ static Layout layout(int B, int Tlen, int C, int H, const GroupPlan &gp) {
     L.total = L.sums + round256(2 * (size_t)B * (gp.b.nseg + 1) * C * sizeof(float));
     return L;
 }
-// true when the plan in force cuts some sequence of this shape into time segments
-bool splits_time(int BH, int Tlen) { return plan_groups(BH, Tlen).b.nseg > 1; }
+// Whether a call of this shape needs two state buffers: the plan in force cuts some sequence into time segments.  Sequences
+// of fewer than eight steps, which only the automatic plan cuts, run in one piece where the state is updated in place.
+bool needs_two_states(int BH, int Tlen) {
+    return plan_groups(BH, Tlen).b.nseg > 1 && (forced_segments() > 0 || (Tlen + SB - 1) / SB >= 8);
+}
 size_t forward_workspace(int B, int Tlen, int H, const Costs &c) { return layout(B, Tlen, H * HEAD, H, plan_groups(B * H, Tlen, c)).forward_total; }
 size_t forward_scratch(int B, int Tlen, int H, const Costs &c) { return part_bytes(B * H, plan_groups(B * H, Tlen, c)); }
 size_t backward_workspace(int B, int Tlen, int C, int H, const Costs &c) { return layout(B, Tlen, C, H, plan_groups(B * H, Tlen, c)).total; }
@@ -1600,7 +1603,7 @@ hipError_t forward_launch(hipStream_t s, bool per_token, bool w16, int B, int Tl
     if (e0 != hipSuccess) return e0;
     const int mode = per_token ? (w16 ? 2 : 1) : 0;
     const int nsb = (Tlen + SB - 1) / SB, BH = B * H;
-    const GroupPlan gp = part ? plan : GroupPlan{0, SegPlan{1, nsb, 1, nsb}, SegPlan{1, nsb, 1, nsb}};
+    const GroupPlan gp = part && s_in != s_out ? plan : GroupPlan{0, SegPlan{1, nsb, 1, nsb}, SegPlan{1, nsb, 1, nsb}};
     const bf16 *rr = (const bf16 *)r, *kk = (const bf16 *)k, *vv = (const bf16 *)v;
     const SegPlan &pl = gp.b;
     const int nB = BH - gp.nA;

@@ -112,6 +112,39 @@ def test_state_in_place_where_no_sequence_is_cut():
     assert fwd(_lib.ALGO_RECURRENT, big[:g["state"].numel()], big[64:64 + g["state"].numel()], 1)[0] == -8      # partial overlap
 
 
+@pytest.mark.parametrize("T", [65, 128, 448])
+def test_short_sequences_keep_their_state_in_place(T):
+    """Sequences of fewer than eight 64-token steps: the automatic plan cuts them in time where the state has two buffers,
+    and in place they run in one piece, with the bits of one segment."""
+    from rwkv_wkv_hip import _lib, configs
+    L = _lib.lib()
+    B, H = 1, 2
+    C = H * 64
+    wl = configs.make(3, seed=17, B=B, T=T, C=C, H=H, dtype=torch.bfloat16)
+    g = {n: x.cuda().contiguous() for n, x in wl.tensors.items()}
+    p = lambda t: t.data_ptr()
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(L.wkv6_forward_workspace(B, T, C, H, _lib.WKV_BF16, _lib.ALGO_CHUNKED), dtype=torch.uint8, device="cuda")
+
+    def fwd(s_in, s_out, how):
+        y = torch.empty_like(g["r"])
+        head = (stream, B, T, C, H, _lib.WKV_BF16, _lib.FLOOR_DECAY)
+        args = [p(g[n]) for n in "rkvwu"] + [p(s_in), p(y), p(s_out)]
+        if how == "noalloc":
+            st = L.wkv6_forward_noalloc(*head, *args)
+        else:
+            st = L.wkv6_forward(*head, _lib.ALGO_CHUNKED, *args, *((p(ws), ws.numel()) if how == "workspace" else (None, 0)))
+        torch.cuda.synchronize()
+        assert st == 0, L.wkv_strerror(st)
+        return y
+    want_s = torch.empty_like(g["state"])
+    want_y = fwd(g["state"], want_s, "none")
+    for how in ("none", "workspace", "noalloc"):
+        one = g["state"].clone()
+        y = fwd(one, one, how)
+        assert torch.equal(y, want_y) and torch.equal(one, want_s), how
+
+
 def test_noalloc_forward_under_graph_capture():
     """What the entry point is for: recorded into a HIP graph (after wkv_init, nothing is left to set up inside the
     capture) and replayed, with plain launches in between; every replay gives the bits of the plain call."""
