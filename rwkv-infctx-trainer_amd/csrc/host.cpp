@@ -69,6 +69,13 @@ void on_gpu(const Tensor &t) {
 
 void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 float *fptr(const Tensor &t) { return static_cast<float *>(ptr(t)); }
+// whether an autograd node has to see this call: a gradient is recorded, or an input carries a forward-mode tangent (which
+// no node here supports: torch's own error for that comes from the node, and a call passed by it would drop the tangent)
+bool seen_by_autograd(std::initializer_list<const Tensor *> inputs) {
+    for (const Tensor *t : inputs)
+        if (t->defined() && ((at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined())) return true;
+    return false;
+}
 // the caller's tensor: the current device is its device and the stream is that device's current one
 struct OnDevice {
     c10::hip::HIPGuard guard;
@@ -187,8 +194,7 @@ struct Call56 {
         REQUIRE(u.numel() == d.C);
     }
     bool records() const {
-        return at::GradMode::is_enabled() && (r.requires_grad() || k.requires_grad() || v.requires_grad() || w.requires_grad() ||
-                                              u.requires_grad() || (!in_place && s.requires_grad()));
+        return seen_by_autograd({&r, &k, &v, &w, &u}) || (!in_place && seen_by_autograd({&s}));
     }
 };
 
@@ -360,7 +366,7 @@ PyObject *py_wkv4(PyObject *, PyObject *const *a, Py_ssize_t n) {
     REQUIRE(td.dim() == 1 && td.size(0) == C && tf.dim() == 1 && tf.size(0) == C && st.sizes().equals(at::IntArrayRef(state, 3)));
     dtype_code(k);
     for (const Tensor *t : {&td, &tf, &k, &v, &st}) on_gpu(*t);
-    if (at::GradMode::is_enabled() && (td.requires_grad() || tf.requires_grad() || k.requires_grad() || v.requires_grad() || st.requires_grad())) {
+    if (seen_by_autograd({&td, &tf, &k, &v, &st})) {
         const variable_list o = Wkv4::apply(td, tf, k, v, st);
         return tuple(o[0], o[1]);
     }

@@ -29,7 +29,7 @@ struct Plain {
     explicit Plain(const Tensor &x_) : x(x_) {}
     bool takes(const Tensor &t, int64_t numel, at::ScalarType type = at::kBFloat16) {
         return ok = ok && t.defined() && t.device() == x.device() && t.scalar_type() == type && t.numel() == numel && t.is_contiguous() &&
-                    !t.key_set().has(c10::DispatchKey::Python) && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+                    !t.key_set().has(c10::DispatchKey::Python) && !t._fw_grad(0).defined() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
     }
     const Tensor *parameter(PyObject *params, const char *name, int64_t numel) {
         PyObject *o = item(params, name);

@@ -709,3 +709,22 @@ def _with(wl, **tensors):
     other = copy.copy(wl)
     other.tensors = dict(wl.tensors, **tensors)
     return other
+
+
+@pytest.mark.parametrize("op", ["wkv5", "wkv6", "wkv4"])
+def test_forward_mode_is_refused(op):
+    """No node supports forward-mode differentiation: a tangent is refused, not dropped, also where nothing is recorded."""
+    import rwkv_wkv_hip as W
+    import torch.autograd.forward_ad as fwAD
+    B, T, H = 1, 4, 2
+    C = 64 * H
+    a, state, u = torch.randn(B, T, C, device=dev()), torch.zeros(B, H, 64, 64, device=dev()), torch.randn(H, 64, device=dev())
+    with fwAD.dual_level(), torch.no_grad():
+        d = fwAD.make_dual(a, torch.ones_like(a))
+        with pytest.raises(RuntimeError, match="jvp"):
+            if op == "wkv6":
+                W.WKV_6.apply(B, T, C, H, d, a, a, a, u, state)
+            elif op == "wkv5":
+                W.WKV_5.apply(B, T, C, H, state, d, a, a, u, u)
+            else:
+                W.wkv_op(torch.zeros(C, device=dev()), torch.zeros(C, device=dev()), d, a, torch.zeros(B, C, 3, device=dev()))
