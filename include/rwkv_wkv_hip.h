@@ -199,6 +199,13 @@ size_t wkv4_checkpoint_bytes(int B, int T, int C);
 int wkv4_forward(void *stream, int B, int T, int C, int dtype,
                  const float *time_decay, const float *time_first, const void *k, const void *v,
                  const float *state_in, void *y, float *state_out, void *checkpoints);
+/* The same with scratch memory of wkv4_forward_scratch() bytes (which may be 0: then none is needed), 4-byte aligned: few
+ * and long sequences are cut into segments of time that run side by side.  Without it, and where state_out overlaps
+ * state_in, every sequence runs in one piece. */
+size_t wkv4_forward_scratch(int B, int T, int C, int dtype);
+int wkv4_forward_with(void *stream, int B, int T, int C, int dtype,
+                      const float *time_decay, const float *time_first, const void *k, const void *v,
+                      const float *state_in, void *y, float *state_out, void *checkpoints, void *scratch, size_t scratch_bytes);
 size_t wkv4_backward_workspace(int B, int T, int C, int dtype);
 int wkv4_backward(void *stream, int B, int T, int C, int dtype,
                   const float *time_decay, const float *time_first, const void *k, const void *v,

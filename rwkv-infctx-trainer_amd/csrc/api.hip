@@ -314,14 +314,26 @@ size_t wkv4_backward_workspace(int B, int T, int C, int dtype) {
     return check_dims4(B, T, C, dtype) ? 0 : v4_backward_workspace(B, T, C);
 }
 
-int wkv4_forward(void *stream, int B, int T, int C, int dtype, const float *time_decay, const float *time_first,
-                 const void *k, const void *v, const float *state_in, void *y, float *state_out, void *checkpoints) {
+size_t wkv4_forward_scratch(int B, int T, int C, int dtype) {
+    return check_dims4(B, T, C, dtype) ? 0 : v4_forward_scratch(B, T, C);
+}
+
+int wkv4_forward_with(void *stream, int B, int T, int C, int dtype, const float *time_decay, const float *time_first,
+                      const void *k, const void *v, const float *state_in, void *y, float *state_out, void *checkpoints, void *scratch,
+                      size_t scratch_bytes) {
     int st = check_dims4(B, T, C, dtype);
     if (st) return st;
     if (!time_decay || !time_first || !k || !v || !y) return WKV_ERR_NULL;
+    if (scratch && scratch_bytes < v4_forward_scratch(B, T, C)) return WKV_ERR_WORKSPACE;
+    // (a segment's workgroups read the state that the last one's write)
+    const bool cut = scratch && v4_forward_scratch(B, T, C) > 0 && !overlap(state_in, state_out, (size_t)B * C * 3 * sizeof(float));
     hipError_t e = v4_forward_dispatch((hipStream_t)stream, dtype, B, T, C, time_decay, time_first, k, v, state_in, y,
-                                       state_out, (float *)checkpoints);
+                                       state_out, (float *)checkpoints, cut ? (float *)scratch : nullptr);
     return e == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
+}
+int wkv4_forward(void *stream, int B, int T, int C, int dtype, const float *time_decay, const float *time_first,
+                 const void *k, const void *v, const float *state_in, void *y, float *state_out, void *checkpoints) {
+    return wkv4_forward_with(stream, B, T, C, dtype, time_decay, time_first, k, v, state_in, y, state_out, checkpoints, nullptr, 0);
 }
 
 int wkv4_backward(void *stream, int B, int T, int C, int dtype, const float *time_decay, const float *time_first,

@@ -26,7 +26,7 @@ namespace {
 
 #define WKV_ABI(X)                                                                                                          \
     X(wkv_strerror) X(wkv5_forward) X(wkv6_forward) X(wkv5_forward_workspace) X(wkv6_forward_workspace) X(wkv5_backward)      \
-    X(wkv6_backward) X(wkv5_backward_workspace) X(wkv6_backward_workspace) X(wkv56_forward_scratch) X(wkv6_decode) X(wkv4_forward) X(wkv4_backward)    \
+    X(wkv6_backward) X(wkv5_backward_workspace) X(wkv6_backward_workspace) X(wkv56_forward_scratch) X(wkv6_decode) X(wkv4_forward_with) X(wkv4_forward_scratch) X(wkv4_backward) \
     X(wkv4_checkpoint_bytes) X(wkv4_backward_workspace) X(wkv_rows_products) X(wkv_lora_mix_rows) X(wkv_timemix_head)         \
     X(wkv_widen_rows) X(wkv_shift_mix_forward) X(wkv_shift_mix_backward) X(wkv_shift_mix_backward_workspace)                  \
     X(wkv_lora_mix_forward) X(wkv_lora_mix_backward) X(wkv_lora_mix_backward_workspace) X(wkv_ln_gate_forward)                \
@@ -257,8 +257,10 @@ public:
         Tensor ckpt = ctx ? bytes(abi.wkv4_checkpoint_bytes(B, T, C), k) : Tensor();
         Tensor y = at::empty_like(k), out = at::empty_like(st);
         OnDevice dev(k);
-        check(abi.wkv4_forward(dev.stream(), B, T, C, dtype_code(k), fptr(td), fptr(tf), ptr(k), ptr(v), fptr(st), ptr(y), fptr(out),
-                               ptr(ckpt)), "wkv4_forward");
+        const size_t n = abi.wkv4_forward_scratch(B, T, C, dtype_code(k));
+        const Tensor scratch = n > 0 ? bytes(n, k) : Tensor();
+        check(abi.wkv4_forward_with(dev.stream(), B, T, C, dtype_code(k), fptr(td), fptr(tf), ptr(k), ptr(v), fptr(st), ptr(y), fptr(out),
+                                    ptr(ckpt), ptr(scratch), n), "wkv4_forward");
         if (ctx) {
             ctx->set_materialize_grads(false);
             ctx->saved_data["types"] = std::vector<int64_t>{(int64_t)time_decay.scalar_type(), (int64_t)time_first.scalar_type(), (int64_t)state.scalar_type()};
@@ -276,8 +278,8 @@ public:
         // a state gradient of zeros: its exponent is zero too, as the reference's backward is handed when autograd has none
         const Tensor gstate = grads[1].defined() ? as_float(grads[1]).contiguous() : at::zeros_like(st);
         Tensor gtd = at::empty_like(td), gtf = at::empty_like(tf), gk = at::empty_like(k), gv = at::empty_like(v), gst = at::empty_like(st);
+        OnDevice dev(k);          // (before the query: the plan is the device's)
         Tensor ws = bytes(abi.wkv4_backward_workspace(B, T, C, dt), k);
-        OnDevice dev(k);
         check(abi.wkv4_backward(dev.stream(), B, T, C, dt, fptr(td), fptr(tf), ptr(k), ptr(v), fptr(st), ptr(gy), fptr(gstate), fptr(gtd),
                                 fptr(gtf), ptr(gk), ptr(gv), fptr(gst), ptr(ckpt), ptr(ws), ws.numel()), "wkv4_backward");
         return {as_type(gtd, (at::ScalarType)types[0]), as_type(gtf, (at::ScalarType)types[1]), gk, gv, as_type(gst, (at::ScalarType)types[2])};

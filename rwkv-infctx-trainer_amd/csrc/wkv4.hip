@@ -96,7 +96,7 @@ __device__ __forceinline__ void v4_advance(Chain &s, float w, float kk, float vv
 template <class T, bool WIDE> struct V4In;
 template <class T> struct V4In<T, false> {
     T val[CK];
-    __device__ __forceinline__ void fetch(const T *p, int /*chain0*/, int idx, int /*BC*/, int C, int Tlen, int t0, int /*lane*/) {
+    __device__ __forceinline__ void fetch(const T *p, int /*chain0*/, int idx, int /*BC*/, int C, int Tlen, int /*Tend*/, int t0, int /*lane*/) {
         const int b = idx / C, c = idx % C;
         const T *q = p + ((size_t)b * Tlen + t0) * C + c;
         if (t0 + CK <= Tlen) {          // whole block inside the sequence: no per-token checks
@@ -116,13 +116,13 @@ template <class T> struct V4In<T, true> {
     static constexpr int W = 16 / sizeof(T), LPR = 64 / W, ROWS = 64 / LPR, NLD = CK / ROWS;
     typedef unsigned int piece_t __attribute__((ext_vector_type(4)));
     piece_t piece[NLD];
-    // chain0: the wavefront's first chain (a multiple of 64); tokens past the end repeat the last one (never used)
-    __device__ __forceinline__ void fetch(const T *p, int chain0, int /*idx*/, int BC, int C, int Tlen, int t0, int lane) {
+    // chain0: the wavefront's first chain (a multiple of 64); tokens from Tend on repeat the one before (never used)
+    __device__ __forceinline__ void fetch(const T *p, int chain0, int /*idx*/, int BC, int C, int Tlen, int Tend, int t0, int lane) {
         const int q = min(chain0 + (lane % LPR) * W, BC - W);
         const T *row = p + (size_t)(q / C) * Tlen * C + q % C;
 #pragma unroll
         for (int i = 0; i < NLD; i++)
-            piece[i] = *reinterpret_cast<const piece_t *>(row + (size_t)min(t0 + i * ROWS + lane / LPR, Tlen - 1) * C);
+            piece[i] = *reinterpret_cast<const piece_t *>(row + (size_t)min(t0 + i * ROWS + lane / LPR, Tend - 1) * C);
     }
     __device__ __forceinline__ void spread(T *stage, int lane, T (&out)[CK]) const {
 #pragma unroll
@@ -131,6 +131,128 @@ template <class T> struct V4In<T, true> {
         for (int i = 0; i < CK; i++) out[i] = stage[i * 64 + lane];
     }
 };
+
+// ---- Sequences cut in time.  A GPU full of chains has B*C / 64 wavefronts walking; with fewer the walk over T tokens is
+// all there is to the time (some 50 ns a token forward, 125 backward, however few the chains).  Both recurrences are linear in
+// their state, so a sequence may be cut into segments of whole blocks that run side by side (grid row = segment): a pass
+// over all segments but one leaves what each adds to an empty state (its summary), and every segment starts by putting
+// together the summaries before it (backward: after it).
+struct Segment {
+    int blk0, blk1;          // its blocks
+    bool last;
+    __device__ __forceinline__ Segment(int Tlen, int bps) {
+        const int all = (Tlen + CK - 1) / CK;
+        blk0 = blockIdx.y * bps;
+        blk1 = min(blk0 + bps, all);
+        last = blk1 == all;
+    }
+};
+// a state after another L tokens whose summary is x: (p, q, o, dp, dq) of those tokens alone.  L steps without input take
+// dp to e^{Lw} (dp + L p): every step adds p to dp before it decays both.
+__device__ __forceinline__ void v4_append(Chain &s, float L, float w, const float (&x)[5]) {
+    const float wo = fmaf(L, w, s.o);
+    const ExpPair d = exp_pair(wo, x[2]);
+    s.dp = fmaf(d.first, fmaf(L, s.p, s.dp), d.second * x[3]);
+    s.dq = fmaf(d.first, fmaf(L, s.q, s.dq), d.second * x[4]);
+    s.p = fmaf(d.first, s.p, d.second * x[0]);
+    s.q = fmaf(d.first, s.q, d.second * x[1]);
+    s.o = d.first_is_max ? wo : x[2];
+}
+// f(j, summary j) for n summaries from `first` in steps of `step`; four are in flight at a time.  part: [segment][N][B*C]
+template <int N, class F>
+__device__ __forceinline__ void for_summaries(const float *part, int BC, int idx, int first, int n, int step, F f) {
+    for (int i = 0; i < n; i += 4) {
+        float x[4][N];
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int e = 0; e < N; e++) x[a][e] = part[((size_t)(first + step * min(i + a, n - 1)) * N + e) * BC + idx];
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+            if (i + a < n) f(first + step * (i + a), x[a]);
+    }
+}
+// The two summary passes: one wavefront per 64 chains and segment, SW segments per workgroup, the inputs of SD blocks in
+// registers.  Forward: (p, q, o, dp, dq) of segments 0 .. nseg - 2.
+constexpr int SW = 4, SD = 2;
+template <class T>
+__global__ __launch_bounds__(64 * SW) void v4_summary_forward(int BC, int Tlen, int C, const float *__restrict__ time_decay,
+        const T *__restrict__ k, const T *__restrict__ v, float *__restrict__ part, int nseg, int bps)
+{
+    const int lane = threadIdx.x & 63, seg = __builtin_amdgcn_readfirstlane(blockIdx.y * SW + (threadIdx.x >> 6));
+    const int idx = blockIdx.x * 64 + lane;
+    if (seg >= nseg - 1 || idx >= BC) return;
+    const float w = -__expf(time_decay[idx % C]);
+    V4In<T, false> ik[SD], iv[SD];          // (every block of these segments is a whole one)
+    const int blk0 = seg * bps, blk1 = blk0 + bps;
+    auto fetch = [&](int blk, V4In<T, false> &a, V4In<T, false> &b) __attribute__((always_inline)) {
+        const int t0 = min(blk, blk1 - 1) * CK;          // (past the end the last block again, unused)
+        a.fetch(k, 0, idx, BC, C, Tlen, Tlen, t0, lane);
+        b.fetch(v, 0, idx, BC, C, Tlen, Tlen, t0, lane);
+    };
+#pragma unroll
+    for (int d = 0; d < SD; d++) fetch(blk0 + d, ik[d], iv[d]);
+    Chain s{0.f, 0.f, NEG_HUGE, 0.f, 0.f};
+    for (int blk = blk0; blk < blk1; blk += SD)
+#pragma unroll
+        for (int d = 0; d < SD; d++) {
+            if (blk + d >= blk1) break;
+#pragma unroll
+            for (int i = 0; i < CK; i++) v4_advance(s, w, to_float(ik[d].val[i]), to_float(iv[d].val[i]));
+            if (blk + d + SD < blk1) fetch(blk + d + SD, ik[d], iv[d]);
+        }
+    float *o = part + (size_t)seg * 5 * BC + idx;
+    o[0] = s.p; o[BC] = s.q; o[2 * (size_t)BC] = s.o; o[3 * (size_t)BC] = s.dp; o[4 * (size_t)BC] = s.dq;
+}
+// Backward: what the state gradient at the start of segments 1 .. nseg - 1 holds of their own tokens.  A token's share
+// decays over the tokens before it, so with the exponent counted from the segment's start the sum can be taken in the order of
+// the replay, and no second walk is needed.
+template <class T>
+__global__ __launch_bounds__(64 * SW) void v4_summary_backward(int BC, int Tlen, int C, const float *__restrict__ time_decay,
+        const float *__restrict__ time_first, const T *__restrict__ k, const T *__restrict__ v, const T *__restrict__ gy,
+        const float *__restrict__ ckpt, float *__restrict__ part, int nseg, int bps)
+{
+    const int lane = threadIdx.x & 63, seg = __builtin_amdgcn_readfirstlane(1 + blockIdx.y * SW + (threadIdx.x >> 6));
+    const int idx = blockIdx.x * 64 + lane;
+    if (seg >= nseg || idx >= BC) return;
+    const float w = -__expf(time_decay[idx % C]), u = time_first[idx % C];
+    V4In<T, false> ik[SD], iv[SD], ig[SD];
+    const int blk0 = seg * bps, blk1 = min(blk0 + bps, (Tlen + CK - 1) / CK);
+    auto fetch = [&](int blk, int d) __attribute__((always_inline)) {
+        const int t0 = min(blk, blk1 - 1) * CK;
+        ik[d].fetch(k, 0, idx, BC, C, Tlen, Tlen, t0, lane);
+        iv[d].fetch(v, 0, idx, BC, C, Tlen, Tlen, t0, lane);
+        ig[d].fetch(gy, 0, idx, BC, C, Tlen, Tlen, t0, lane);
+    };
+#pragma unroll
+    for (int d = 0; d < SD; d++) fetch(blk0 + d, d);
+    const float *cp = ckpt + (size_t)blk0 * 5 * BC + idx;
+    Chain s{cp[0], cp[BC], cp[2 * (size_t)BC], 0.f, 0.f};
+    float gp = 0.f, gq = 0.f, go = NEG_HUGE;
+    for (int blk = blk0; blk < blk1; blk += SD)
+#pragma unroll
+        for (int d = 0; d < SD; d++) {
+            if (blk + d >= blk1) break;
+            const int cnt = min(CK, Tlen - (blk + d) * CK);
+            const float before = (float)((blk + d - blk0) * CK);
+#pragma unroll
+            for (int i = 0; i < CK; i++) {
+                if (i < cnt) {
+                    float iden, ec, hw, nm;
+                    const float ys = v4_step(s, w, u, to_float(ik[d].val[i]), to_float(iv[d].val[i]), iden, ec, hw, nm);
+                    const float at = fmaf(before + i, w, nm);
+                    const ExpPair e = exp_pair(go, at);
+                    const float add = to_float(ig[d].val[i]) * iden * e.second;
+                    gp = fmaf(e.first, gp, add);
+                    gq = fmaf(e.first, gq, -add * ys);
+                    go = e.first_is_max ? go : at;
+                }
+            }
+            if (blk + d + SD < blk1) fetch(blk + d + SD, d);
+        }
+    float *o = part + (size_t)seg * 3 * BC + idx;
+    o[0] = gp; o[BC] = gq; o[2 * (size_t)BC] = go;
+}
 
 // Forward.  y == nullptr: only checkpoints / final state are produced.
 // ckpt layout: [block][5][B*C].
@@ -144,7 +266,8 @@ constexpr int V4_YW = 3, V4_GROUPS = 2;
 template <class T, bool WIDE>
 __global__ __launch_bounds__(64 * (1 + V4_YW) * V4_GROUPS) void v4_forward(int BC, int Tlen, int C, const float *__restrict__ time_decay,
         const float *__restrict__ time_first, const T *__restrict__ k, const T *__restrict__ v,
-        const float *__restrict__ s_in, T *__restrict__ y, float *__restrict__ s_out, float *__restrict__ ckpt)
+        const float *__restrict__ s_in, T *__restrict__ y, float *__restrict__ s_out, float *__restrict__ ckpt,
+        const float *__restrict__ part, int bps)
 {
     __shared__ float start_all[V4_GROUPS][2 * V4_YW][5][64];      // the state at a block's start: p, q, o (and dp, dq for the checkpoint)
     // k and v of the blocks of two laps, [token][chain]: left there by the walking wavefront on its way (it is also
@@ -166,7 +289,9 @@ __global__ __launch_bounds__(64 * (1 + V4_YW) * V4_GROUPS) void v4_forward(int B
     const int b = idx / C, c = idx % C;
     const float w = -__expf(time_decay[c]), u = time_first[c];
     const size_t base = (size_t)b * Tlen * C + c;
-    const int nblk = (Tlen + CK - 1) / CK, nlap = (nblk + V4_YW - 1) / V4_YW;
+    const Segment sg(Tlen, bps);
+    const int blk0 = sg.blk0, nblk = sg.blk1, nlap = (nblk - blk0 + V4_YW - 1) / V4_YW;          // (nblk: the segment's end)
+    const int Tend = min(Tlen, nblk * CK);
     typedef V4In<T, WIDE> In;
 
     if (role == 0) {
@@ -181,9 +306,13 @@ __global__ __launch_bounds__(64 * (1 + V4_YW) * V4_GROUPS) void v4_forward(int B
         // whose laps in flight are twice the bytes, 316 -> 331 us, so it keeps the conditional fetches.)
         constexpr bool AHEAD = WIDE && sizeof(T) == 2;
         auto first = [&](int d, In &ik, In &iv) __attribute__((always_inline)) {
-            if (AHEAD || d < nblk) { ik.fetch(k, chain0, idx, BC, C, Tlen, d * CK, lane); iv.fetch(v, chain0, idx, BC, C, Tlen, d * CK, lane); }
+            const int t0 = (blk0 + d) * CK;
+            if (AHEAD || blk0 + d < nblk) { ik.fetch(k, chain0, idx, BC, C, Tlen, Tend, t0, lane); iv.fetch(v, chain0, idx, BC, C, Tlen, Tend, t0, lane); }
         };
         first(0, k0, v0); first(1, k1, v1); first(2, k2, v2); first(3, k3, v3); first(4, k4, v4); first(5, k5, v5);
+        for_summaries<5>(part, BC, idx, 0, blk0 / bps, 1, [&](int, const float (&x)[5]) __attribute__((always_inline)) {
+            v4_append(s, (float)(bps * CK), w, x);
+        });
         auto block = [&](int blk, int slot, In &ik, In &iv) __attribute__((always_inline)) {
             if (!AHEAD && blk >= nblk) return;
             const bool on = blk < nblk;          // scalar
@@ -198,7 +327,7 @@ __global__ __launch_bounds__(64 * (1 + V4_YW) * V4_GROUPS) void v4_forward(int B
             iv.spread(kv_all[grp][slot][1], lane, vv);
             }
             const int nb = blk + 2 * V4_YW;
-            if (AHEAD || nb < nblk) { ik.fetch(k, chain0, idx, BC, C, Tlen, nb * CK, lane); iv.fetch(v, chain0, idx, BC, C, Tlen, nb * CK, lane); }
+            if (AHEAD || nb < nblk) { ik.fetch(k, chain0, idx, BC, C, Tlen, Tend, nb * CK, lane); iv.fetch(v, chain0, idx, BC, C, Tlen, Tend, nb * CK, lane); }
             if (!on) return;
             const int t0 = blk * CK, cnt = min(CK, Tlen - t0);
             if (cnt == CK) {
@@ -211,17 +340,18 @@ __global__ __launch_bounds__(64 * (1 + V4_YW) * V4_GROUPS) void v4_forward(int B
             }
         };
         for (int rd = 0; rd <= nlap; rd += 2) {
-            block(rd * V4_YW, 0, k0, v0); block(rd * V4_YW + 1, 1, k1, v1); block(rd * V4_YW + 2, 2, k2, v2);
+            const int b0 = blk0 + rd * V4_YW;
+            block(b0, 0, k0, v0); block(b0 + 1, 1, k1, v1); block(b0 + 2, 2, k2, v2);
             lds_barrier();
-            block((rd + 1) * V4_YW, 3, k3, v3); block((rd + 1) * V4_YW + 1, 4, k4, v4); block((rd + 1) * V4_YW + 2, 5, k5, v5);
+            block(b0 + 3, 3, k3, v3); block(b0 + 4, 4, k4, v4); block(b0 + 5, 5, k5, v5);
             lds_barrier();                       // (both halves always: blocks past the end do nothing)
         }
-        if (s_out && live) { s_out[idx * 3] = s.p; s_out[idx * 3 + 1] = s.q; s_out[idx * 3 + 2] = s.o; }
+        if (s_out && live && sg.last) { s_out[idx * 3] = s.p; s_out[idx * 3 + 1] = s.q; s_out[idx * 3 + 2] = s.o; }
     } else {
         const int r = role - 1;
         // the outputs of this wavefront's block of lap pr (whose starting state and inputs wait in slot `slot`)
         auto outputs = [&](int pr, int slot) __attribute__((always_inline)) {
-            const int blk = pr * V4_YW + r;
+            const int blk = blk0 + pr * V4_YW + r;
             if (pr < 0 || blk >= nblk) return;
             if (ckpt && live) {
                 float *cp = ckpt + (size_t)blk * 5 * BC + idx;
@@ -276,7 +406,7 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
         const float *__restrict__ time_first, const T *__restrict__ k, const T *__restrict__ v,
         const T *__restrict__ gy, const float *__restrict__ gs_out, const float *__restrict__ ckpt,
         float *__restrict__ gw_part, float *__restrict__ gu_part, T *__restrict__ gk, T *__restrict__ gv,
-        float *__restrict__ gs_in)
+        float *__restrict__ gs_in, const float *__restrict__ part, int bps)
 {
     __shared__ V4Replay sh[RB];
     const int lane = threadIdx.x & 63, role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -285,7 +415,8 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
     const int b = idx / C, c = idx % C;
     const float w = -__expf(time_decay[c]), u = time_first[c];
     const size_t base = (size_t)b * Tlen * C + c;
-    const int nblk = (Tlen + CK - 1) / CK;
+    const Segment sg(Tlen, bps);
+    const int blk0 = sg.blk0, end = sg.blk1, nblk = end - blk0;          // nblk: the segment's
 
     // RB blocks of k, v, gy per lane: one being consumed, the others in flight
     T bk[RB][CK], bv[RB][CK], bg[RB][CK];        // (as they came; converted where they are used)
@@ -312,12 +443,12 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
     };
 
     if (role == 0) {
-        // ---------------- replay: step j handles block nblk-1-j, register set and LDS buffer j % RB
+        // ---------------- replay: step j handles block end-1-j, register set and LDS buffer j % RB
         float acc_w = 0.f, acc_u = 0.f;
         Chain bs[RB];
 #pragma unroll
         for (int d = 0; d < RB; d++)
-            if (nblk - 1 - d >= 0) { fetch(nblk - 1 - d, bk[d], bv[d], bg[d]); bs[d] = load_ckpt(nblk - 1 - d); }
+            if (nblk - 1 - d >= 0) { fetch(end - 1 - d, bk[d], bv[d], bg[d]); bs[d] = load_ckpt(end - 1 - d); }
         auto replay = [&](auto full_tag, int blk, T (&kk)[CK], T (&vv)[CK], T (&gg)[CK], Chain s, V4Replay &out) {
             constexpr bool FULL = decltype(full_tag)::value;
             const int cnt = FULL ? CK : Tlen - blk * CK;
@@ -333,18 +464,18 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
                     out.ys[i][lane] = yy; out.iden[i][lane] = iden; out.ec[i][lane] = ec; out.neg_m[i][lane] = nm;
                 }
             }
-            if (blk == nblk - 1 && gs_out) {       // gradient arriving through the state handed out
+            if (sg.last && blk == end - 1 && gs_out) {       // gradient arriving through the state handed out
                 const float gp = gs_out[idx * 3], gq = gs_out[idx * 3 + 1];
                 const float go = (gp == 0.f && gq == 0.f) ? NEG_HUGE : gs_out[idx * 3 + 2];
                 acc_w += (gp * s.dp + gq * s.dq) * __expf(s.o + go);
             }
         };
         auto step = [&](int j, T (&kk)[CK], T (&vv)[CK], T (&gg)[CK], Chain &cs, V4Replay &out) {
-            const int blk = nblk - 1 - j;
-            if (blk >= 0) {
+            const int blk = end - 1 - j;
+            if (blk >= blk0) {
                 if ((blk + 1) * CK <= Tlen) replay(std::true_type{}, blk, kk, vv, gg, cs, out);
                 else replay(std::false_type{}, blk, kk, vv, gg, cs, out);
-                if (blk - RB >= 0) { fetch(blk - RB, kk, vv, gg); cs = load_ckpt(blk - RB); }
+                if (blk - RB >= blk0) { fetch(blk - RB, kk, vv, gg); cs = load_ckpt(blk - RB); }
             }
             lds_barrier();
         };
@@ -353,10 +484,10 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
             for (int d = 0; d < RB; d++)
                 if (j + d <= nblk) step(j + d, bk[d], bv[d], bg[d], bs[d], sh[d]);
         }
-        gw_part[idx] = acc_w * w;
-        gu_part[idx] = acc_u;
+        gw_part[(size_t)blockIdx.y * BC + idx] = acc_w * w;
+        gu_part[(size_t)blockIdx.y * BC + idx] = acc_u;
     } else {
-        // ---------------- reverse walk: step j handles block nblk-j (none at j = 0), register set and buffer (j-1) % RB
+        // ---------------- reverse walk: step j handles block end-j (none at j = 0), register set and buffer (j-1) % RB
         float gp = 0.f, gq = 0.f, go = NEG_HUGE;
         if (gs_out) {
             gp = gs_out[idx * 3]; gq = gs_out[idx * 3 + 1]; go = gs_out[idx * 3 + 2];
@@ -364,7 +495,17 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
         }
 #pragma unroll
         for (int d = 0; d < RB; d++)
-            if (nblk - 1 - d >= 0) fetch(nblk - 1 - d, bk[d], bv[d], bg[d]);
+            if (nblk - 1 - d >= 0) fetch(end - 1 - d, bk[d], bv[d], bg[d]);
+        if (!sg.last) {          // the segments after this one, from the last
+            const int nseg = gridDim.y, seg = blockIdx.y, tail = Tlen - (nseg - 1) * bps * CK;          // tokens of the last
+            for_summaries<3>(part, BC, idx, nseg - 1, nseg - 1 - seg, -1, [&](int j, const float (&x)[3]) __attribute__((always_inline)) {
+                const float wg = fmaf((float)(j == nseg - 1 ? tail : bps * CK), w, go);
+                const ExpPair e = exp_pair(wg, x[2]);
+                gp = fmaf(e.first, gp, e.second * x[0]);
+                gq = fmaf(e.first, gq, e.second * x[1]);
+                go = e.first_is_max ? wg : x[2];
+            });
+        }
         auto walk = [&](auto full_tag, int blk, T (&kk)[CK], T (&vv)[CK], T (&gg)[CK], const V4Replay &in) {
             constexpr bool FULL = decltype(full_tag)::value;
             const int t0 = blk * CK, cnt = FULL ? CK : Tlen - t0;
@@ -389,11 +530,11 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
             }
         };
         auto step = [&](int j, T (&kk)[CK], T (&vv)[CK], T (&gg)[CK], const V4Replay &in) {
-            const int blk = nblk - j;
+            const int blk = end - j;
             if (j >= 1) {
                 if ((blk + 1) * CK <= Tlen) walk(std::true_type{}, blk, kk, vv, gg, in);
                 else walk(std::false_type{}, blk, kk, vv, gg, in);
-                if (blk - RB >= 0) fetch(blk - RB, kk, vv, gg);
+                if (blk - RB >= blk0) fetch(blk - RB, kk, vv, gg);
             }
             lds_barrier();
         };
@@ -405,15 +546,60 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
                 if (j + d <= nblk) step(j + d, bk[e], bv[e], bg[e], sh[e]);
             }
         }
-        if (gs_in) { gs_in[idx * 3] = gp; gs_in[idx * 3 + 1] = gq; gs_in[idx * 3 + 2] = go; }
+        if (gs_in && blk0 == 0) { gs_in[idx * 3] = gp; gs_in[idx * 3 + 1] = gq; gs_in[idx * 3 + 2] = go; }
     }
 }
 
+// g_time_decay and g_time_first: the rows of the partial sums, one per batch row and segment, in a fixed order: 32 columns x 8
+// row groups per workgroup, grid row 0 the first, 1 the second
+__global__ __launch_bounds__(256) void v4_sum(int rows, int C, const float *__restrict__ gw_part, const float *__restrict__ gu_part,
+                                              float *__restrict__ gtd, float *__restrict__ gtf) {
+    __shared__ float red[8][32];
+    const float *in = blockIdx.y ? gu_part : gw_part;
+    const int lane = threadIdx.x & 31, rg = threadIdx.x >> 5, c = blockIdx.x * 32 + lane;
+    float s = 0.f;
+    if (c < C) {
+#pragma unroll 4
+        for (int r = rg; r < rows; r += 8) s += in[(size_t)r * C + c];
+    }
+    red[rg][lane] = s;
+    __syncthreads();
+    if (rg != 0 || c >= C) return;
+#pragma unroll
+    for (int g = 1; g < 8; g++) s += red[g][lane];
+    (blockIdx.y ? gtf : gtd)[c] = s;
+}
+
+static bool overlap(const float *a, const float *b, size_t bytes) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return a && b && x < y + bytes && y < x + bytes;
+}
+
+// Segments and blocks per segment.  As many segments as give every compute unit two wavefronts to walk with, or four where
+// that leaves fewer than eight; at least two blocks each.  The passes over the summaries read the inputs once more, so a
+// sequence is cut only where its chains take less than two thirds of the compute units (six segments or more) and where it has 16 blocks.
+// Measured, fp32 forward+backward of whole calls in us, one piece against the rule's: 12 wavefronts of chains (B1 C768), T 4096
+// 731 -> 80, T 1000 188 -> 52, T 256 58 -> 56 (T 128 48 -> 55: not cut); 40 (B1 C2560), T 4096 733 -> 173; 128 (B2 C4096) 802 ->
+// 424; 160 (B4 C2560), T 1024 200 -> 152; 256 (B8 C2048), T 512 111 -> 121 with four segments: not cut.  bf16 a little more so.
+constexpr int V4_MAX_SEG = 64;
+struct V4Plan { int nseg, bps; };
+static V4Plan v4_plan(int B, int Tlen, int C) {
+    const int nblk = (Tlen + CK - 1) / CK, groups = (B * C + 63) / 64, ncu = cu_count();
+    const int want = std::min({V4_MAX_SEG, std::max(2 * ncu / groups, std::min(8, 4 * ncu / groups)), nblk / 2});
+    if (want < 6 || nblk < 16) return V4Plan{1, nblk};
+    const int bps = (nblk + want - 1) / want;
+    return V4Plan{(nblk + bps - 1) / bps, bps};
+}
 size_t v4_checkpoint_bytes(int B, int Tlen, int C) {
     return (size_t)((Tlen + CK - 1) / CK) * 5 * (size_t)B * C * sizeof(float);
 }
-size_t v4_backward_workspace(int B, int Tlen, int C) {       // gw, gu partials + room for checkpoints
-    return 2 * (size_t)B * C * sizeof(float) + v4_checkpoint_bytes(B, Tlen, C);
+size_t v4_forward_scratch(int B, int Tlen, int C) {          // the summaries; none where nothing is cut
+    const V4Plan pl = v4_plan(B, Tlen, C);
+    return pl.nseg > 1 ? (size_t)pl.nseg * 5 * B * C * sizeof(float) : 0;
+}
+// gw, gu partials of every segment, the summaries, room for checkpoints
+size_t v4_backward_workspace(int B, int Tlen, int C) {
+    return 2 * (size_t)v4_plan(B, Tlen, C).nseg * B * C * sizeof(float) + v4_forward_scratch(B, Tlen, C) + v4_checkpoint_bytes(B, Tlen, C);
 }
 
 // whether the 16-byte fetches apply: a piece of 16 / sizeof(T) chains must not straddle two batch rows, and the
@@ -429,8 +615,9 @@ template <class T> constexpr size_t v4_forward_lds() { return (size_t)V4_GROUPS 
 
 template <class T>
 static hipError_t fwd(hipStream_t s, int B, int Tlen, int C, const float *td, const float *tf, const void *k,
-                      const void *v, const float *s_in, void *y, float *s_out, float *ckpt) {
+                      const void *v, const float *s_in, void *y, float *s_out, float *ckpt, float *part) {
     const int BC = B * C;
+    const V4Plan pl = part ? v4_plan(B, Tlen, C) : V4Plan{1, (Tlen + CK - 1) / CK};
     static PerDevice lds_limit;
     const hipError_t lds_ok = lds_limit.once([] {           // (more than the 64 KB a kernel gets by default, for fp32)
         hipError_t e = hipFuncSetAttribute((const void *)v4_forward<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)v4_forward_lds<T>());
@@ -438,14 +625,17 @@ static hipError_t fwd(hipStream_t s, int B, int Tlen, int C, const float *td, co
         return e;
     });
     if (lds_ok != hipSuccess) return lds_ok;
+    if (pl.nseg > 1)
+        hipLaunchKernelGGL((v4_summary_forward<T>), dim3((BC + 63) / 64, (pl.nseg - 1 + SW - 1) / SW), dim3(64 * SW), 0, s, BC, Tlen, C, td,
+                           (const T *)k, (const T *)v, part, pl.nseg, pl.bps);
     prof_begin(KID_V4_FORWARD, s);
-    const dim3 grid(((BC + 63) / 64 + V4_GROUPS - 1) / V4_GROUPS), block(64 * (1 + V4_YW) * V4_GROUPS);
+    const dim3 grid(((BC + 63) / 64 + V4_GROUPS - 1) / V4_GROUPS, pl.nseg), block(64 * (1 + V4_YW) * V4_GROUPS);
     if (v4_wide<T>(C, {k, v, y}))
         hipLaunchKernelGGL((v4_forward<T, true>), grid, block, v4_forward_lds<T>(), s, BC, Tlen, C, td, tf, (const T *)k,
-                           (const T *)v, s_in, (T *)y, s_out, ckpt);
+                           (const T *)v, s_in, (T *)y, s_out, ckpt, part, pl.bps);
     else
         hipLaunchKernelGGL((v4_forward<T, false>), grid, block, v4_forward_lds<T>(), s, BC, Tlen, C, td, tf, (const T *)k,
-                           (const T *)v, s_in, (T *)y, s_out, ckpt);
+                           (const T *)v, s_in, (T *)y, s_out, ckpt, part, pl.bps);
     prof_end(KID_V4_FORWARD, s);
     return hipGetLastError();
 }
@@ -455,29 +645,35 @@ static hipError_t bwd(hipStream_t s, int B, int Tlen, int C, const float *td, co
                       const void *v, const float *s_in, const void *gy, const float *gs_out, float *gtd, float *gtf,
                       void *gk, void *gv, float *gs_in, const float *ckpt, float *ws) {
     const int BC = B * C;
-    float *gw_part = ws, *gu_part = ws + BC, *own_ckpt = ws + 2 * (size_t)BC;
+    // (in place, the first segment's workgroups would write the state gradient that the others read)
+    const bool cut = !overlap(gs_in, gs_out, (size_t)BC * 3 * sizeof(float));
+    const V4Plan pl = cut ? v4_plan(B, Tlen, C) : V4Plan{1, (Tlen + CK - 1) / CK};
+    float *gw_part = ws, *gu_part = gw_part + (size_t)pl.nseg * BC, *part = gu_part + (size_t)pl.nseg * BC;
     if (!ckpt) {           // no checkpoints from the forward call: make them now
-        hipError_t e = fwd<T>(s, B, Tlen, C, td, tf, k, v, s_in, nullptr, nullptr, own_ckpt);
+        float *own = part + (pl.nseg > 1 ? (size_t)pl.nseg * 5 * BC : 0);
+        hipError_t e = fwd<T>(s, B, Tlen, C, td, tf, k, v, s_in, nullptr, nullptr, own, pl.nseg > 1 ? part : nullptr);
         if (e != hipSuccess) return e;
-        ckpt = own_ckpt;
+        ckpt = own;
     }
+    if (pl.nseg > 1)
+        hipLaunchKernelGGL((v4_summary_backward<T>), dim3((BC + 63) / 64, (pl.nseg - 1 + SW - 1) / SW), dim3(64 * SW), 0, s, BC, Tlen, C, td, tf,
+                           (const T *)k, (const T *)v, (const T *)gy, ckpt, part, pl.nseg, pl.bps);
     prof_begin(KID_V4_BACKWARD, s);
-    hipLaunchKernelGGL((v4_backward<T>), dim3((BC + 63) / 64), dim3(128), 0, s, BC, Tlen, C, td, tf, (const T *)k,
-                       (const T *)v, (const T *)gy, gs_out, ckpt, gw_part, gu_part, (T *)gk, (T *)gv, gs_in);
+    hipLaunchKernelGGL((v4_backward<T>), dim3((BC + 63) / 64, pl.nseg), dim3(128), 0, s, BC, Tlen, C, td, tf, (const T *)k,
+                       (const T *)v, (const T *)gy, gs_out, ckpt, gw_part, gu_part, (T *)gk, (T *)gv, gs_in, part, pl.bps);
     prof_end(KID_V4_BACKWARD, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sum_over_batch, dim3((C + 255) / 256), dim3(256), 0, s, B, C, gw_part, gtd);
-    hipLaunchKernelGGL(sum_over_batch, dim3((C + 255) / 256), dim3(256), 0, s, B, C, gu_part, gtf);
+    hipLaunchKernelGGL(v4_sum, dim3((C + 31) / 32, 2), dim3(256), 0, s, B * pl.nseg, C, gw_part, gu_part, gtd, gtf);
     return hipGetLastError();
 }
 
 hipError_t v4_forward_dispatch(hipStream_t s, int dtype, int B, int Tlen, int C, const float *td, const float *tf,
-                               const void *k, const void *v, const float *s_in, void *y, float *s_out, float *ckpt) {
+                               const void *k, const void *v, const float *s_in, void *y, float *s_out, float *ckpt, float *part) {
     switch (dtype) {
-        case 0: return fwd<float>(s, B, Tlen, C, td, tf, k, v, s_in, y, s_out, ckpt);
-        case 1: return fwd<bf16>(s, B, Tlen, C, td, tf, k, v, s_in, y, s_out, ckpt);
-        default: return fwd<f16>(s, B, Tlen, C, td, tf, k, v, s_in, y, s_out, ckpt);
+        case 0: return fwd<float>(s, B, Tlen, C, td, tf, k, v, s_in, y, s_out, ckpt, part);
+        case 1: return fwd<bf16>(s, B, Tlen, C, td, tf, k, v, s_in, y, s_out, ckpt, part);
+        default: return fwd<f16>(s, B, Tlen, C, td, tf, k, v, s_in, y, s_out, ckpt, part);
     }
 }
 

@@ -44,6 +44,8 @@ SIGNATURES = {
     "wkv5_backward": (_I, [_P, _I, _I, _I, _I, _I, c_uint, _I] + [_P] * 14 + [_P, c_size_t]),
     "wkv4_checkpoint_bytes": (c_size_t, [_I] * 3),
     "wkv4_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 8),
+    "wkv4_forward_scratch": (c_size_t, [_I] * 4),
+    "wkv4_forward_with": (_I, [_P, _I, _I, _I, _I] + [_P] * 9 + [c_size_t]),
     "wkv4_backward_workspace": (c_size_t, [_I] * 4),
     "wkv4_backward": (_I, [_P, _I, _I, _I, _I] + [_P] * 13 + [_P, c_size_t]),
     "wkv_cumsum_decay": (_I, [_P, _I, _I, _I, _I, _I] + [_P] * 6),

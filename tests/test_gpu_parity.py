@@ -260,6 +260,59 @@ def test_v4_shapes(dtype, B, T, C):
     assert_close(und(L["state"].grad), und(ref[4]), rt, "v4 gstate (undivided)")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,C", [(1, 241, 64), (2, 256, 100), (1, 1003, 130), (3, 777, 256), (1, 2049, 72), (1, 300, 4096)])
+def test_v4_cut_in_time(dtype, B, T, C):
+    """Few and long sequences run in segments of whole blocks: lengths just past the shortest that is cut, ending inside a
+    block and with a last segment of one token, widths with and without the 16-byte fetches, with and without the forward's
+    checkpoints, and where the buffers of the state or of its gradient are one (then in one piece, the same results)."""
+    import rwkv_wkv_hip as W
+    from rwkv_wkv_hip import _lib
+    L = _lib.lib()
+    dt = {torch.float32: _lib.WKV_F32, torch.bfloat16: _lib.WKV_BF16}[dtype]
+    assert L.wkv4_forward_scratch(B, T, C, dt) > 0
+    t = v4_case(B, T, C, dtype, seed=B + T + C, with_state=True).tensors
+    f32 = lambda x: x.float()
+    y_ref, s_ref = O4.forward(t["time_decay"], f32(t["time_first"]), f32(t["k"]), f32(t["v"]), t["state"])
+    ref = O4.backward(t["time_decay"], f32(t["time_first"]), f32(t["k"]), f32(t["v"]), t["state"], f32(t["dy"]), t["dstate"])
+    g = {n: x.to(dev()).contiguous() for n, x in t.items()}
+    und = lambda st: st[..., :2].float().cpu() * torch.exp(st[..., 2:3].float().cpu())
+    rt = RTOL[dtype]
+
+    def compare(y, s, gtd, gtf, gk, gv, gst, what):
+        assert_close(y, y_ref, rt, what + " y")
+        assert_close(und(s), und(s_ref), 1e-3, what + " state (undivided sums)")
+        assert_close(gtd, ref[0], rt, what + " g_time_decay")
+        assert_close(gtf, ref[1], rt, what + " g_time_first")
+        assert_close(gk, ref[2], rt, what + " gk")
+        assert_close(gv, ref[3], rt, what + " gv")
+        assert_close(und(gst), und(ref[4]), rt, what + " gstate (undivided)")
+    leaves = [g[n].clone().requires_grad_(True) for n in ("time_decay", "time_first", "k", "v", "state")]
+    y, s = W.wkv_op(*leaves)
+    compare(y, s, *torch.autograd.grad([y, s], leaves, [g["dy"], g["dstate"]]), "cut")
+    with torch.no_grad():
+        y, s = W.wkv_op(*[x.detach() for x in leaves])
+    assert_close(y, y_ref, rt, "prefill y")
+    # the C entry points: no checkpoints handed in; one buffer for the state, one for its gradient
+    p, stream = (lambda x: x.data_ptr()), torch.cuda.current_stream().cuda_stream
+    td, tf = g["time_decay"].float(), g["time_first"].float()
+    scratch = torch.empty(L.wkv4_forward_scratch(B, T, C, dt), dtype=torch.uint8, device=dev())
+    ws = torch.empty(L.wkv4_backward_workspace(B, T, C, dt), dtype=torch.uint8, device=dev())
+    for in_place in (False, True):
+        y, gk, gv = (torch.empty_like(g["k"]) for _ in range(3))
+        s_in, gs_out = g["state"].clone(), g["dstate"].float().clone()
+        s_out, gst = (s_in, gs_out) if in_place else (torch.empty_like(s_in), torch.empty_like(gs_out))
+        gtd, gtf = torch.empty_like(td), torch.empty_like(tf)
+        assert L.wkv4_forward_with(stream, B, T, C, dt, p(td), p(tf), p(g["k"]), p(g["v"]), p(s_in), p(y), p(s_out), None, p(scratch),
+                                   scratch.numel()) == 0
+        assert L.wkv4_backward(stream, B, T, C, dt, p(td), p(tf), p(g["k"]), p(g["v"]), p(g["state"]), p(g["dy"]), p(gs_out), p(gtd),
+                               p(gtf), p(gk), p(gv), p(gst), None, p(ws), ws.numel()) == 0
+        torch.cuda.synchronize()
+        compare(y, s_out, gtd, gtf, gk, gv, gst, "in place" if in_place else "no checkpoints")
+    assert L.wkv4_forward_with(stream, B, T, C, dt, p(td), p(tf), p(g["k"]), p(g["v"]), p(s_in), p(y), p(s_out), None, p(scratch),
+                               scratch.numel() - 1) == -5
+
+
 def test_v4_backward_without_forward_checkpoints():
     """The C entry point rebuilds its checkpoints when none are passed."""
     import ctypes
