@@ -60,11 +60,10 @@ __device__ __forceinline__ s8 mixed(s8 x, s8 xx, s8 c, int lerp) {
 // that way into registers (two such segments in flight, used in turn) and turns them in LDS that belongs to it alone;
 // the same for the rows of x, of which only those that exist are read, and mixed on the way.
 //
-// TN columns (16, or 8 where 16 would leave compute units without a workgroup) and XL fetches of x, each fetch 512
-// consecutive elements: two rows of a segment of 256 k, or one row of 512.
+// TN columns and XL fetches of x, each fetch 512 elements: two rows of a segment of 256 k, one of 512, or four of 128.
 template <int TN, int XL> struct Shape {
     static constexpr int SEG = 4096 / TN, LD = SEG + 8, PER = TN / 8;     // k of a segment, padded row in LDS, rows per fetch
-    static constexpr int XROWS = PER * XL, MT = (XROWS + 15) / 16;
+    static constexpr int XROWS = PER * XL, MT = (XROWS + 15) / 16, NT = (TN + 15) / 16;      // MFMA tiles of rows, of columns
     static __device__ int row(int lane) { return lane / (SEG / 8); }
     static __device__ int k(int lane) { return 8 * (lane % (SEG / 8)); }
 };
@@ -100,7 +99,7 @@ __device__ __forceinline__ void turn(const Segment<XL, MIX> &s, Turn<TN, XL> &t,
 // (lanes whose row of x does not exist repeat the last one, and those beyond 8 weight rows repeat them: rows and columns
 // of the result that nobody reads)
 template <int TN, int XL>
-__device__ __forceinline__ void multiply(const Turn<TN, XL> &t, int steps, int live, int lane, f4 (&acc)[Shape<TN, XL>::MT]) {
+__device__ __forceinline__ void multiply(const Turn<TN, XL> &t, int steps, int live, int lane, f4 (&acc)[Shape<TN, XL>::NT][Shape<TN, XL>::MT]) {
     typedef Shape<TN, XL> Sh;
     const int n = lane & 15, k = 8 * (lane >> 4);
     int xo[Sh::MT];
@@ -109,9 +108,15 @@ __device__ __forceinline__ void multiply(const Turn<TN, XL> &t, int steps, int l
 #pragma unroll
     for (int i = 0; i < Sh::SEG / 32; i++)
         if (i < steps) {
-            const s8 a = *reinterpret_cast<const s8 *>(&t.w[(n % TN) * Sh::LD + k + 32 * i]);
+            s8 a[Sh::NT];
 #pragma unroll
-            for (int mt = 0; mt < Sh::MT; mt++) acc[mt] = mma(a, *reinterpret_cast<const s8 *>(&t.x[xo[mt] + 32 * i]), acc[mt]);
+            for (int nt = 0; nt < Sh::NT; nt++) a[nt] = *reinterpret_cast<const s8 *>(&t.w[(16 * nt + n % TN) * Sh::LD + k + 32 * i]);
+#pragma unroll
+            for (int mt = 0; mt < Sh::MT; mt++) {
+                const s8 x = *reinterpret_cast<const s8 *>(&t.x[xo[mt] + 32 * i]);
+#pragma unroll
+                for (int nt = 0; nt < Sh::NT; nt++) acc[nt][mt] = mma(a[nt], x, acc[nt][mt]);
+            }
         }
 }
 // the lanes of a wavefront exchange data through LDS: program order is enough for the hardware, the compiler is told
@@ -121,7 +126,7 @@ __device__ __forceinline__ void wave_sync() {
 }
 template <int TN, int XL, int WAVES, bool MIX>
 __device__ __forceinline__ void accumulate(const Job &job, Turn<TN, XL> &t, int tile, int row0, int rows, int K, int wv, int lane,
-                                           f4 (&acc)[Shape<TN, XL>::MT]) {
+                                           f4 (&acc)[Shape<TN, XL>::NT][Shape<TN, XL>::MT]) {
     typedef Shape<TN, XL> Sh;
     constexpr bool TWO = XL <= 8;                            // two segments in flight where the registers allow it
     const bf16 *w = job.w + (size_t)(TN * tile + Sh::row(lane)) * K;
@@ -169,52 +174,58 @@ template <int TN> __host__ __device__ inline int workgroups(const Job &job) { re
 
 template <int TN, int XL, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, XL <= 2 ? 4 : 2) void rows_products(int rows, int K, Jobs jobs) {
-    constexpr int MT = Shape<TN, XL>::MT;
+    constexpr int MT = Shape<TN, XL>::MT, NT = Shape<TN, XL>::NT;
     __shared__ __align__(16) Turn<TN, XL> turned[WAVES];
-    f4 (*part)[MT][64] = reinterpret_cast<f4 (*)[MT][64]>(turned);       // (used after the contraction)
-    static_assert(sizeof(turned[0]) >= MT * 64 * sizeof(f4), "the sums fit where the weights were turned");
+    f4 (*part)[NT][MT][64] = reinterpret_cast<f4 (*)[NT][MT][64]>(turned);       // (used after the contraction)
+    static_assert(sizeof(turned[0]) >= NT * MT * 64 * sizeof(f4), "the sums fit where the weights were turned");
     int wg = blockIdx.x, ji = 0;
     const int row0 = Shape<TN, XL>::XROWS * blockIdx.y;
     while (wg >= workgroups<TN>(jobs.j[ji])) wg -= workgroups<TN>(jobs.j[ji++]);     // (the grid is the sum over all jobs)
     const Job job = jobs.j[ji];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, n = lane & 15;
-    f4 acc[MT];
+    f4 acc[NT][MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[mt] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[nt][mt] = f4{0.f, 0.f, 0.f, 0.f};
     if (job.k_major) {
-        if (job.mix) accumulate_k_major<MT, WAVES, true>(job, wg / SPLIT, wg % SPLIT, row0, rows, K, wv, lane, acc);
-        else accumulate_k_major<MT, WAVES, false>(job, wg / SPLIT, wg % SPLIT, row0, rows, K, wv, lane, acc);
+        if (job.mix) accumulate_k_major<MT, WAVES, true>(job, wg / SPLIT, wg % SPLIT, row0, rows, K, wv, lane, acc[0]);
+        else accumulate_k_major<MT, WAVES, false>(job, wg / SPLIT, wg % SPLIT, row0, rows, K, wv, lane, acc[0]);
     } else {
         if (job.mix) accumulate<TN, XL, WAVES, true>(job, turned[wv], wg, row0, rows, K, wv, lane, acc);
         else accumulate<TN, XL, WAVES, false>(job, turned[wv], wg, row0, rows, K, wv, lane, acc);
     }
     __syncthreads();
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) part[wv][mt][lane] = acc[mt];
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) part[wv][nt][mt][lane] = acc[nt][mt];
     __syncthreads();
-    if (wv >= MT) return;
-    f4 s = part[0][wv][lane];
+    for (int tile = wv; tile < (job.k_major ? 1 : NT) * MT; tile += WAVES) {
+        const int nt = tile / MT, mt = tile % MT;
+        f4 s = part[0][nt][mt][lane];
 #pragma unroll
-    for (int i = 1; i < WAVES; i++) s += part[i][wv][lane];
-    const int m = row0 + 16 * wv + n;                   // the lane holds four consecutive columns of row m
-    if (m >= rows) return;
-    float y[4] = {s[0], s[1], s[2], s[3]};
-    if (job.k_major) {
-        store4((float *)job.out + ((size_t)(wg % SPLIT) * rows + m) * job.n + 16 * (wg / SPLIT) + 4 * kg, y);
-        return;
+        for (int i = 1; i < WAVES; i++) s += part[i][nt][mt][lane];
+        const int m = row0 + 16 * mt + n;                   // the lane holds four consecutive columns of row m
+        if (m >= rows) continue;
+        float y[4] = {s[0], s[1], s[2], s[3]};
+        if (job.k_major) {
+            store4((float *)job.out + ((size_t)(wg % SPLIT) * rows + m) * job.n + 16 * (wg / SPLIT) + 4 * kg, y);
+            continue;
+        }
+        if (TN == 8 && kg >= 2) continue;
+        const size_t o = (size_t)m * job.n + TN * wg + 16 * nt + 4 * kg;
+        if (job.act == ACT_RELU_SQUARE) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) { const float p = fmaxf(round_bf16(y[e]), 0.f); y[e] = p * p; }
+        } else if (job.act == ACT_SIGMOID_MUL) {
+            float q[4];
+            load4(job.mul + o, q);
+#pragma unroll
+            for (int e = 0; e < 4; e++) y[e] = sigmoid(q[e]) * round_bf16(y[e]);
+        }
+        store4((bf16 *)job.out + o, y);
     }
-    if (TN == 8 && kg >= 2) return;
-    const size_t o = (size_t)m * job.n + TN * wg + 4 * kg;
-    if (job.act == ACT_RELU_SQUARE) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) { const float p = fmaxf(round_bf16(y[e]), 0.f); y[e] = p * p; }
-    } else if (job.act == ACT_SIGMOID_MUL) {
-        float q[4];
-        load4(job.mul + o, q);
-#pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = sigmoid(q[e]) * round_bf16(y[e]);
-    }
-    store4((bf16 *)job.out + o, y);
 }
 
 // out[j] = x + (shift - x) (maa_j + act_j w2_j): a wavefront per mix and 16 channels, whose 32-deep product is one MFMA
@@ -329,19 +340,37 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
     out[base + tid] = from_float<bf16>(z * g * sigmoid(g));
 }
 
-// Eight wavefronts per workgroup where the workgroups do not fill the compute units twice over, four (of which several
-// share a compute unit) otherwise.  One or two rows: 8 columns per workgroup where 16 would leave compute units idle.
+// Which shape.  Every workgroup reads all the rows of x for its columns, so from three rows on that traffic, and the mixing,
+// is of the weights' size with 16 columns; 32 columns halve it for half as many workgroups.  v6 layer, 16 -> 32 columns in
+// us: 20 rows H40 97.6 -> 80.7, 64 rows H40 203 -> 158, 64 rows H64 389 -> 289, 16 rows H28 50.7 -> 45.3.  Up to 16 rows they pay
+// where the workgroups still reach most compute units and not yet all of them twice (H64, 544 workgroups: 140 us with 16
+// columns, 154 with 32; its output projection, 128: 256 of 16 columns are 5 % faster); from 33 rows on, where 16 columns
+// read the weights twice, once half the compute units have one (H12: 56 against 61 us); between, down to 32 workgroups.
+// One or two rows: 8 columns where 16 would leave compute units idle.  Eight wavefronts where the workgroups do not fill
+// the compute units twice over, four (of which several workgroups share a compute unit) otherwise.
 static hipError_t rows_products_launch(hipStream_t s, int rows, int K, const Jobs &jobs) {
-    int wgs16 = 0, wgs8 = 0;
-    for (int i = 0; i < jobs.count; i++) { wgs16 += workgroups<16>(jobs.j[i]); wgs8 += workgroups<8>(jobs.j[i]); }
-    const bool wide = wgs16 < 2 * cu_count();
+    int wgs32 = 0, wgs16 = 0, wgs8 = 0;
+    bool by32 = true;
+    for (int i = 0; i < jobs.count; i++) {
+        wgs32 += workgroups<32>(jobs.j[i]); wgs16 += workgroups<16>(jobs.j[i]); wgs8 += workgroups<8>(jobs.j[i]);
+        by32 = by32 && (jobs.j[i].k_major || jobs.j[i].n % 32 == 0);
+    }
 #define WKV_ROWS(TN, XL, WAVES)                                                                                        \
-    hipLaunchKernelGGL((rows_products<TN, XL, WAVES>), dim3(TN == 16 ? wgs16 : wgs8, (rows + TN * XL / 8 - 1) / (TN * XL / 8)), \
+    hipLaunchKernelGGL((rows_products<TN, XL, WAVES>), dim3(TN == 32 ? wgs32 : TN == 16 ? wgs16 : wgs8, (rows + TN * XL / 8 - 1) / (TN * XL / 8)), \
                        dim3(64 * WAVES), 0, s, rows, K, jobs)
-    if (rows > 16) WKV_ROWS(16, 16, 4);    // (the LDS of more wavefronts does not fit; 33..64 rows: two workgroups read a tile's weights together)
-    else if (rows > 2) { if (wide) WKV_ROWS(16, 8, 8); else WKV_ROWS(16, 8, 4); }
-    else if (wgs16 < cu_count()) WKV_ROWS(8, 2, 8);
-    else if (wide) WKV_ROWS(16, 1, 8);
+    const int ncu = cu_count();
+    if (rows > 32) { if (by32 && wgs32 > ncu / 2) WKV_ROWS(32, 16, 4); else WKV_ROWS(16, 16, 4); }
+    else if (rows > 16) {
+        if (!by32 || wgs32 < ncu / 8) WKV_ROWS(16, 16, 4);
+        else if (wgs32 < 2 * ncu) WKV_ROWS(32, 8, 8);
+        else WKV_ROWS(32, 8, 4);
+    } else if (rows > 2) {
+        if (by32 && wgs32 > ncu / 2 && wgs32 < 2 * ncu) { if (wgs32 < ncu) WKV_ROWS(32, 4, 8); else WKV_ROWS(32, 4, 4); }
+        else if (wgs16 < 2 * ncu) WKV_ROWS(16, 8, 8);
+        else WKV_ROWS(16, 8, 4);
+    }
+    else if (wgs16 < ncu) WKV_ROWS(8, 2, 8);
+    else if (wgs16 < 2 * ncu) WKV_ROWS(16, 1, 8);
     else WKV_ROWS(16, 1, 4);
 #undef WKV_ROWS
     return hipGetLastError();

@@ -273,6 +273,33 @@ def test_timemix_forward_on_the_kernels_bf16_module(version):
     assert_close(s_got, s_ref, 6e-2, f"timemix bf16 v{version} state")
 
 
+@pytest.mark.parametrize("rows", [3, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,K", [(256, 64), (1024, 192), (4128, 192), (8224, 2112), (16416, 64)])
+def test_products_of_a_few_rows(rows, n, K):
+    """Each shape of the kernel: 16 and 32 columns, four and eight wavefronts, one to four tiles of rows, contractions that
+    end inside a segment; two products in one launch, one mixed and squared, one (n + 32 columns) as it is.  Against 64 bits:
+    the mixed row and the result round to bf16 (2^-9 each, the square doubles it), the sums to 32 bits."""
+    import ctypes
+    from rwkv_wkv_hip import _lib
+
+    class Product(ctypes.Structure):
+        _fields_ = [(f, ctypes.c_void_p) for f in ("w", "x", "shift", "mix", "mul", "out")] + [(f, ctypes.c_int) for f in ("n", "k_major", "lerp", "act")]
+    g = torch.Generator().manual_seed(rows + n)
+    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
+    x, shift, mix, w1, w2 = r(rows, K), r(rows, K), torch.rand(K, generator=g).bfloat16().cuda(), r(n, K), r(n + 32, K)
+    o1, o2 = torch.full((rows, n), 9.0, dtype=torch.bfloat16, device="cuda"), torch.full((rows, n + 32), 9.0, dtype=torch.bfloat16, device="cuda")
+    p = lambda t: t.data_ptr()
+    jobs = (Product * 2)(Product(p(w1), p(x), p(shift), p(mix), None, p(o1), n, 0, 0, 1), Product(p(w2), p(x), None, None, None, p(o2), n + 32, 0, 0, 0))
+    assert _lib.lib().wkv_rows_products(torch.cuda.current_stream().cuda_stream, rows, K, 2, jobs) == 0
+    torch.cuda.synchronize()
+    d = lambda t: t.double()
+    mixed = (d(x) + (d(shift) - d(x)) * d(mix)).bfloat16()
+    e1, e2 = torch.relu(d(mixed) @ d(w1).t()) ** 2, d(x) @ d(w2).t()
+    for got, want, tol in ((o1, e1, 3 * 2 ** -8), (o2, e2, 2 ** -8)):
+        err = (d(got) - want).abs()
+        assert bool((err <= tol * want.abs() + 2 ** -9 * want.pow(2).mean().sqrt()).all()), err.max().item()
+
+
 @pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("B,H,ffn", [(1, 1, 64), (3, 2, 448), (16, 1, 192), (17, 3, 640), (33, 2, 256), (64, 9, 2016), (65, 1, 128)])
 def test_layer_of_single_tokens(version, B, H, ffn):
