@@ -308,12 +308,6 @@ int wkv_sigmoid_mul_backward(void *stream, size_t n, int dtype, const void *r, c
  * in which the functions above take coefficients, weights and biases. */
 int wkv_widen_rows(void *stream, int count, int C, const void *const *in, float *out);
 
-/* The LoRAs' contractions over the channels (RWKV-v6/src/module/TimeMix.py:264,280-281), bf16:
- *   out[row][p n + j] = f(sum over k of x[p][row][k] w[p](k, j)),  p < planes;  x (planes, rows, k)
- * act NULL: f = tanh; else act (rows, planes n) holds that tanh's values t and f multiplies by 1 - t^2, its backward.
- * k_major: w (planes, k, n) with n 160 or 64, else w (planes, n, k) with n 64 or 32.  k a multiple of 32. */
-int wkv_lora_down(void *stream, int rows, int k, int n, int planes, int k_major, const void *x, const void *w, const void *act, void *out);
-
 /* ---- A layer for one token per sequence (a serving loop), bf16, at most 64 rows (sequences) at a time.
  *
  * Products of the rows with up to 8 weight matrices in one launch:  out = f(x' W),

@@ -13,7 +13,6 @@
 #include "block_edges.hip"
 #include "lora_mix.hip"
 #include "layer_decode.hip"
-#include "lora_down.hip"
 
 using namespace wkv;
 
@@ -511,14 +510,6 @@ int wkv_widen_rows(void *stream, int count, int C, const void *const *in, float 
     }
     hipLaunchKernelGGL(edges::widen_rows, dim3((C + 255) / 256, count), dim3(256), 0, (hipStream_t)stream, C, p, out);
     return hipGetLastError() == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
-}
-
-int wkv_lora_down(void *stream, int row_count, int k, int n, int planes, int k_major, const void *x, const void *w, const void *act, void *out) {
-    if (row_count <= 0 || k <= 0 || k % 32 != 0 || planes <= 0 || planes > 65535 || !lora::lora_down_takes(n, k_major != 0)) return WKV_ERR_DIMS;
-    if (!x || !w || !out) return WKV_ERR_NULL;
-    for (const void *p : {x, w, act, (const void *)out})
-        if (!aligned16(p)) return WKV_ERR_ALIGN;
-    return lora::lora_down_launch((hipStream_t)stream, row_count, k, n, planes, k_major != 0, x, w, act, out) == hipSuccess ? WKV_OK : WKV_ERR_LAUNCH;
 }
 
 int wkv_rows_products(void *stream, int row_count, int k, int count, const wkv_rows_product *products) {

@@ -31,7 +31,7 @@ namespace {
     X(wkv_widen_rows) X(wkv_shift_mix_forward) X(wkv_shift_mix_backward) X(wkv_shift_mix_backward_workspace)                  \
     X(wkv_lora_mix_forward) X(wkv_lora_mix_backward) X(wkv_lora_mix_backward_workspace) X(wkv_ln_gate_forward)                \
     X(wkv_ln_gate_backward) X(wkv_ln_gate_backward_workspace) X(wkv_relu_square_forward) X(wkv_relu_square_backward)          \
-    X(wkv_sigmoid_mul_forward) X(wkv_sigmoid_mul_backward) X(wkv_lora_down)
+    X(wkv_sigmoid_mul_forward) X(wkv_sigmoid_mul_backward)
 struct {
 #define X(name) decltype(&::name) name = nullptr;
     WKV_ABI(X)

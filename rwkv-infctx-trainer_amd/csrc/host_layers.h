@@ -148,14 +148,6 @@ MixGrads shift_mix_backward(void *stream, const Dims &d, int n, bool lerp, const
 Tensor plane(const Tensor &t, int64_t j) { return t.select(0, j); }
 Tensor times_t(const Tensor &x, const Tensor &w) { return at::mm(x, w.t()); }          // x W^T, the projection
 
-// The LoRAs' contractions over the channels with the tanh that follows, or its backward from `act`: one launch (csrc/lora_down.hip)
-Tensor lora_down(void *stream, const Tensor &x, const Tensor &w, int64_t n, bool k_major, const Tensor &act = Tensor()) {
-    const int64_t planes = x.dim() == 3 ? x.size(0) : 1, rows = x.size(-2);
-    Tensor out = at::empty({rows, planes * n}, x.options());
-    check(abi.wkv_lora_down(stream, (int)rows, (int)x.size(-1), (int)n, (int)planes, k_major, ptr(x), ptr(w), ptr(act), ptr(out)), "wkv_lora_down");
-    return out;
-}
-
 // What the backward needs of the forward, in the order in which it is saved after the operands
 enum { COEF, XXX, ACT, W2T, MIXES, RR, KK, VV, GG, LORA, WW, YY, ZZ, WS, SAVED };
 struct TimeMixOut { Tensor out, state, saved[SAVED]; };
@@ -174,7 +166,7 @@ TimeMixOut timemix_forward(const TimeMixCall &c) {
     int r, k, v, g;
     if (c.version == 6) {
         o.saved[XXX] = shift_mix(stream, d, 1, false, *t[X], *t[SHIFT], mix).view({M, C});
-        o.saved[ACT] = lora_down(stream, o.saved[XXX], *t[W1], 160, true);
+        o.saved[ACT] = at::mm(o.saved[XXX], *t[W1]).tanh_();
         o.saved[W2T] = t[W2]->transpose(1, 2).contiguous();
         o.saved[MIXES] = at::empty({5, M, C}, t[X]->options());
         check(abi.wkv_lora_mix_forward(stream, d.B, d.T, d.C, ptr(*t[X]), ptr(*t[SHIFT]), mix + C, ptr(o.saved[ACT]), ptr(o.saved[W2T]),
@@ -192,7 +184,7 @@ TimeMixOut timemix_forward(const TimeMixCall &c) {
     const int64_t streams[3] = {d.B, d.T, d.C};
     auto seq = [&](const Tensor &x) { return x.view(at::IntArrayRef(streams, 3)); };
     if (c.version == 6) {
-        o.saved[LORA] = t[DW1]->size(1) == 64 ? lora_down(stream, plane(m, 0), *t[DW1], 64, true) : at::mm(plane(m, 0), *t[DW1]).tanh_();
+        o.saved[LORA] = at::mm(plane(m, 0), *t[DW1]).tanh_();
         // the broadcast addition of time_decay rides on the product as its bias
         const Tensor w = at::addmm(t[DECAY]->view({C}), o.saved[LORA], *t[DW2]);
         o.saved[WW] = decay_operand(6, d, c.algo, seq(o.saved[RR]), seq(w), c.keep);
@@ -280,7 +272,7 @@ public:
             const Tensor gw = as_type(b.gw, at::kBFloat16).view({M, C});
             if (wants(DECAY)) out(DECAY) = gw.sum(0).view(t[DECAY].sizes());
             if (wants(DW2)) out(DW2) = at::mm(s[LORA].t(), gw);
-            const Tensor gl = s[LORA].size(1) == 64 ? lora_down(stream, gw, t[DW2], 64, false, s[LORA]) : at::tanh_backward(at::mm(gw, t[DW2].t()), s[LORA]);
+            const Tensor gl = at::tanh_backward(at::mm(gw, t[DW2].t()), s[LORA]);
             if (wants(DW1)) out(DW1) = at::mm(plane(s[MIXES], 0).t(), gl);
             Tensor into = plane(gm, 0);
             at::mm_out(into, gl, t[DW1].t());
@@ -292,8 +284,10 @@ public:
                       "wkv_lora_mix_backward");
             }
             // the two reductions of the second LoRA product's backward, and the first product
-            const Tensor gpre = lora_down(stream, gdyn, t[W2], 32, false, s[ACT]);
+            Tensor ga = at::empty({M, 5, 32}, t[X].options());
+            ga.copy_(at::bmm(gdyn, s[W2T]).transpose(0, 1));
             if (wants(W2)) out(W2) = at::bmm(s[ACT].view({M, 5, 32}).permute({1, 2, 0}), gdyn);
+            const Tensor gpre = at::tanh_backward(ga.view({M, 160}), s[ACT]);
             if (wants(W1)) out(W1) = at::mm(s[XXX].t(), gpre);
             const MixGrads first = shift_mix_backward(stream, d, 1, false, t[X], t[SHIFT], mix, at::mm(gpre, t[W1].t()), gmix);
             out(X) = gx.add_(first.gx);

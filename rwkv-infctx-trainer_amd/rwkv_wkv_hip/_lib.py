@@ -64,7 +64,6 @@ SIGNATURES = {
     "wkv_sigmoid_mul_forward": (_I, [_P, c_size_t, _I, _P, _P, _P]),
     "wkv_sigmoid_mul_backward": (_I, [_P, c_size_t, _I] + [_P] * 5),
     "wkv_widen_rows": (_I, [_P, _I, _I, _P, _P]),
-    "wkv_lora_down": (_I, [_P, _I, _I, _I, _I, _I] + [_P] * 4),
     "wkv_rows_products": (_I, [_P, _I, _I, _I, _P]),
     "wkv_lora_mix_rows": (_I, [_P, _I, _I] + [_P] * 6),
     "wkv_timemix_head": (_I, [_P, _I, _I, _I] + [_P] * 10 + [c_float, c_float] + [_P] * 3),

@@ -273,27 +273,6 @@ def test_timemix_forward_on_the_kernels_bf16_module(version):
     assert_close(s_got, s_ref, 6e-2, f"timemix bf16 v{version} state")
 
 
-@pytest.mark.parametrize("backward", [False, True])
-@pytest.mark.parametrize("n,planes,k_major", [(160, 1, 1), (64, 1, 1), (64, 1, 0), (32, 5, 0), (64, 2, 1)])
-@pytest.mark.parametrize("rows,K", [(1, 64), (17, 192), (300, 1792), (4095, 320), (2049, 256)])
-def test_lora_down(rows, K, n, planes, k_major, backward):
-    """The LoRAs' contractions with tanh or its backward: rows that end inside a tile, 16 and 32 rows a workgroup, contractions
-    of fewer steps than wavefronts and of odd counts.  Against 64 bits: one rounding to bf16 (2^-9) over sums in 32 bits."""
-    from rwkv_wkv_hip import _lib
-    g = torch.Generator().manual_seed(rows + n)
-    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
-    x, w = r(planes, rows, K), r(planes, *((K, n) if k_major else (n, K))) * K ** -0.5
-    act = torch.tanh(r(rows, planes * n)) if backward else None
-    out = torch.full((rows, planes * n), 9.0, dtype=torch.bfloat16, device="cuda")
-    p = lambda t: None if t is None else t.data_ptr()
-    assert _lib.lib().wkv_lora_down(torch.cuda.current_stream().cuda_stream, rows, K, n, planes, k_major, p(x), p(w), p(act), p(out)) == 0
-    torch.cuda.synchronize()
-    want = (x.double() @ (w.double() if k_major else w.double().transpose(1, 2).contiguous())).transpose(0, 1).reshape(rows, planes * n)
-    want = want * (1 - act.double() ** 2) if backward else torch.tanh(want)
-    err = (out.double() - want).abs()
-    assert bool((err <= 2 ** -8 * want.abs() + 2e-5).all()), err.max().item()
-
-
 @pytest.mark.parametrize("rows", [3, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("n,K", [(256, 64), (1024, 192), (4128, 192), (8224, 2112), (16416, 64)])
 def test_products_of_a_few_rows(rows, n, K):
