@@ -340,6 +340,28 @@ def test_layer_of_single_tokens(version, B, H, ffn):
 
 
 @pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("B,H", [(1, 2), (3, 5), (17, 12), (64, 4)])
+def test_single_token_layer_rounds_where_the_steps_round(version, B, H):
+    """The TimeMix of one token per sequence without autograd (kernels of its own) against the same call with autograd on
+    (the steps, with a bf16 tensor between any two).  Both round at the same places, so they differ only where sums in another order
+    land on the other side of a rounding: of the state's two factors and decay some percent of the elements by 2^-8,
+    1e-3 in norm; of the output, behind four roundings, 2.5e-3.  (Kept in fp32 in between they differ by 1.2e-3 to 1.6e-3 and by 4e-3.)"""
+    from rwkv_wkv_hip import blocks as K
+    C = 64 * H
+    g = _g(B + H)
+    m = (TimeMix5 if version == 5 else TimeMix6)(C, H, seed=8).cuda().bfloat16()
+    x, shift = torch.randn(B, 1, C, generator=g).cuda().bfloat16(), torch.randn(B, C, generator=g).cuda().bfloat16()
+    state = (torch.randn(B, H, 64, 64, generator=g) * 0.1).cuda()
+    timemix = K.timemix5_forward if version == 5 else K.timemix6_forward
+    ref, (_, s_ref) = timemix(m, x, (shift, state))
+    assert ref.requires_grad
+    with torch.no_grad():
+        got, (_, s) = timemix(m, x, (shift, state))
+    rel = lambda a, b: ((a - b).double().norm() / b.double().norm()).item()
+    assert rel(s, s_ref) < 1e-3 and rel(got, ref) < 2.5e-3, (rel(s, s_ref), rel(got, ref))
+
+
+@pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("T,frozen", [(1, ()), (2, ("key",)), (65, ()), (130, ("ln_x", "output", "value", "time"))])
 def test_layer_native_matches_the_steps(version, T, frozen):
     """A layer's halves as the native host side runs them against the same kernels step by step (which a hook on one of the
