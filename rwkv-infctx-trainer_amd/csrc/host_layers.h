@@ -31,6 +31,10 @@ struct Plain {
         return ok = ok && t.defined() && t.device() == x.device() && t.scalar_type() == type && t.numel() == numel && t.is_contiguous() &&
                     !t.key_set().has(c10::DispatchKey::Python) && !t._fw_grad(0).defined() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
     }
+    // an input: its shape too (the parameters' C elements may come in any)
+    bool takes(const Tensor &t, at::IntArrayRef shape, at::ScalarType type = at::kBFloat16) {
+        return ok = ok && t.defined() && t.sizes().equals(shape) && takes(t, t.numel(), type);
+    }
     const Tensor *parameter(PyObject *params, const char *name, int64_t numel) {
         PyObject *o = item(params, name);
         if (!o || !THPVariable_Check(o)) ok = false;
@@ -79,8 +83,8 @@ bool collect(TimeMixCall &c, PyObject *module, PyObject *px, PyObject *states) {
     c.d = {(int)B, (int)T, (int)C, (int)H};
     Plain p(x);
     p.takes(x, B * T * C);
-    p.takes(THPVariable_Unpack(sh), B * C);
-    p.takes(THPVariable_Unpack(st), B * H * 64 * 64, at::kFloat);
+    p.takes(THPVariable_Unpack(sh), {B, C});
+    p.takes(THPVariable_Unpack(st), {B, H, 64, 64}, at::kFloat);
     PyObject *ln = item(mod, "ln_x"), *lnd = nullptr, *eps = nullptr;
     p.ok = p.ok && ln && (PyObject *)Py_TYPE(ln) == group_norm_type && (lnd = dict_of(ln)) && (eps = item(lnd, "eps")) && PyFloat_Check(eps);
     if (!p.ok) return false;
@@ -329,7 +333,7 @@ bool collect(ChannelMixCall &c, PyObject *module, PyObject *px, PyObject *sh) {
     c.d = {(int)B, (int)T, (int)C, (int)(C / 64)};
     Plain p(x);
     p.takes(x, B * T * C);
-    p.takes(THPVariable_Unpack(sh), B * C);
+    p.takes(THPVariable_Unpack(sh), {B, C});
     c.t[CM_X] = &x; c.t[CM_SHIFT] = &THPVariable_Unpack(sh);
     c.t[CM_MIX_K] = p.parameter(prm, c.lerp ? "time_mix_k" : "time_maa_k", C);
     c.t[CM_MIX_R] = p.parameter(prm, c.lerp ? "time_mix_r" : "time_maa_r", C);

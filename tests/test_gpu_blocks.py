@@ -362,6 +362,30 @@ def test_single_token_layer_rounds_where_the_steps_round(version, B, H):
 
 
 @pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("T,grad", [(1, False), (1, True), (5, False), (5, True)])
+def test_layer_refuses_states_of_another_shape(version, T, grad):
+    """A shift state that is not (B, C) and a WKV state that is not (B, H, 64, 64) are refused, also where they have as many
+    elements as the right ones."""
+    from rwkv_wkv_hip import blocks as K
+    B, H = 3, 2
+    C = 64 * H
+    tm, cm = ((TimeMix5 if version == 5 else TimeMix6)(C, H, seed=8).cuda().bfloat16(),
+              (ChannelMix5 if version == 5 else ChannelMix6)(C, 4 * C, seed=9).cuda().bfloat16())
+    timemix, channelmix = (K.timemix5_forward, K.channelmix5_forward) if version == 5 else (K.timemix6_forward, K.channelmix6_forward)
+    x, shift, state = torch.randn(B, T, C).cuda().bfloat16(), torch.randn(B, C).cuda().bfloat16(), torch.randn(B, H, 64, 64).cuda()
+    with torch.set_grad_enabled(grad):
+        timemix(tm, x, (shift, state)), channelmix(cm, x, shift)
+        for wrong in (shift.view(C, B), shift.view(B, 1, C), shift.view(-1)):
+            with pytest.raises(Exception):
+                timemix(tm, x, (wrong, state))
+            with pytest.raises(Exception):
+                channelmix(cm, x, wrong)
+        for wrong in (state.view(H, B, 64, 64), state.view(B, H, 4096), state.view(B * H, 64, 64)):
+            with pytest.raises(Exception):
+                timemix(tm, x, (shift, wrong))
+
+
+@pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("T,frozen", [(1, ()), (2, ("key",)), (65, ()), (130, ("ln_x", "output", "value", "time"))])
 def test_layer_native_matches_the_steps(version, T, frozen):
     """A layer's halves as the native host side runs them against the same kernels step by step (which a hook on one of the
