@@ -121,10 +121,10 @@ int wkv_profile_end(float *ms, int capacity);
  * wkv6_backward_workspace() (>= the forward size), to backward together with
  * WKV_CHECKPOINTS_VALID saves backward one sweep over k, v, w. */
 /* state_out == state_in (the state updated in place) is accepted for fp32 and fp16 streams, and by the chunked algorithm
- * whenever the plan cuts no sequence of the shape into time segments (B*H at least the number of compute units, or
- * WKV_TUNE_SEGMENTS 1, or at most 448 tokens with no segment count set: such calls run in one piece where the state is
- * updated in place); where it does (short batches, e.g. the 7B shape with B = 1), and for buffers that overlap
- * without being the same, the call returns WKV_ERR_ALIAS and the caller keeps two state buffers and alternates.
+ * for sequences of at most 448 tokens, with WKV_TUNE_SEGMENTS 1, and for longer ones wherever B*H fills the compute units so
+ * well that a cut in time would not save a round of workgroups; such calls run every sequence in one piece.  Otherwise
+ * (short batches, e.g. the 7B shape with B = 1; a segment count set), and for buffers that overlap without being the
+ * same, the call returns WKV_ERR_ALIAS and the caller keeps two state buffers and alternates.
  * The same holds for wkv5_forward and wkv6_forward_noalloc. */
 size_t wkv6_forward_workspace(int B, int T, int C, int H, int dtype, int algo);
 size_t wkv56_forward_scratch(int B, int T, int C, int H, int dtype, int algo);      /* see WKV_NO_CHECKPOINTS; may be 0 */

@@ -1565,10 +1565,29 @@ static Layout layout(int B, int Tlen, int C, int H, const GroupPlan &gp) {
     L.total = L.sums + round256(2 * (size_t)B * (gp.b.nseg + 1) * C * sizeof(float));
     return L;
 }
-// Whether a call of this shape needs two state buffers: the plan in force cuts some sequence into time segments.  Sequences
-// of fewer than eight steps, which only the automatic plan cuts, run in one piece where the state is updated in place.
+// Whether a call of this shape is refused where the state is updated in place (it runs in one piece where it is not: the
+// workgroups of a sequence's later segments would read what the last one's has overwritten).  The answer belongs to the
+// interface and must not move with the fitted costs above, or a new fit would refuse calls that ran (129 to 142 pairs of 17
+// steps, for instance).  So the rule has its own estimate: rounds of workgroups times steps per segment, a cut adding up
+// to 40 % for the summary pass, segments of at least four steps and at most 16 of them.
 bool needs_two_states(int BH, int Tlen) {
-    return plan_groups(BH, Tlen).b.nseg > 1 && (forced_segments() > 0 || (Tlen + SB - 1) / SB >= 8);
+    const int nsb = (Tlen + SB - 1) / SB, ncu = cu_count();
+    if (forced_segments() > 0) return std::min(forced_segments(), nsb) > 1;
+    auto cost = [ncu, nsb](int bh, int n) {
+        return (double)((bh * (long)n + ncu - 1) / ncu) * ((nsb + n - 1) / n + 1) * (1.0 + 0.4 * (n - 1) / n);
+    };
+    auto segments = [&](int bh) {
+        int want = 1;
+        double best = 1e30;
+        for (int n = 1; n <= 16 && n * 4 <= std::max(4, nsb); n++)
+            if (cost(bh, n) < best * 0.97) { best = cost(bh, n); want = n; }
+        const int sps = (nsb + want - 1) / want;
+        return (nsb + sps - 1) / sps;
+    };
+    const int whole = BH / ncu * ncu, rest = BH - whole, all = segments(BH);
+    if (whole == 0 || rest == 0) return all > 1;
+    const int last = segments(rest);          // whole rounds in one piece, only the remainder cut
+    return (cost(whole, 1) + cost(rest, last) < 0.97 * cost(BH, all) ? last : all) > 1;
 }
 size_t forward_workspace(int B, int Tlen, int H, const Costs &c) { return layout(B, Tlen, H * HEAD, H, plan_groups(B * H, Tlen, c)).forward_total; }
 size_t forward_scratch(int B, int Tlen, int H, const Costs &c) { return part_bytes(B * H, plan_groups(B * H, Tlen, c)); }

@@ -5,6 +5,7 @@ import os
 import re
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "rwkv_wkv_hip.h")
@@ -39,6 +40,21 @@ def test_version_and_messages(L):
     assert L.wkv_strerror(0) == b"ok"
     for code in range(-8, 0):
         assert L.wkv_strerror(code) not in (b"ok", b"unknown status")
+
+
+@pytest.mark.parametrize("BH,steps", [(129, 17), (142, 17), (641, 18), (400, 20), (1, 7), (256, 64)])
+@pytest.mark.parametrize("entry", ["wkv6_forward", "wkv5_forward", "wkv6_forward_noalloc"])
+def test_state_in_place_is_not_refused_by_a_cost_estimate(L, entry, BH, steps):
+    """Shapes whose state may be updated in place whatever the planner makes of them with two buffers (256 compute units):
+    the call gets as far as the launch, which fails without a GPU.  Other shapes stay refused."""
+    if torch.cuda.is_available():
+        pytest.skip("the pointers are not memory")
+    p = ctypes.c_void_p(1 << 40)
+    tail = () if entry == "wkv6_forward_noalloc" else (None, 0)
+    algo = () if entry == "wkv6_forward_noalloc" else (2,)
+    call = lambda BH, T: getattr(L, entry)(None, BH, T, 64, 1, 1, 1, *algo, *([p] * 8), *tail)
+    assert call(BH, 64 * steps) == -6
+    assert call(64, 4096) == -8 and call(320, 4096) == -8 and call(1, 512) == -8
 
 
 def test_argument_checks_return_before_any_launch(L):

@@ -145,6 +145,31 @@ def test_short_sequences_keep_their_state_in_place(T):
         assert torch.equal(y, want_y) and torch.equal(one, want_s), how
 
 
+def test_state_in_place_where_the_planner_would_cut():
+    """129 pairs of 17 steps: cut in time where the state has two buffers, in one piece in place, with the bits of one segment."""
+    from rwkv_wkv_hip import _lib, configs
+    L = _lib.lib()
+    B, T, H, C = 129, 1088, 1, 64
+    g = {n: x.cuda().contiguous() for n, x in configs.make(3, seed=18, B=B, T=T, C=C, H=H, dtype=torch.bfloat16).tensors.items()}
+    assert L.wkv56_forward_scratch(B, T, C, H, _lib.WKV_BF16, _lib.ALGO_CHUNKED) > 0
+    ws = torch.empty(L.wkv6_forward_workspace(B, T, C, H, _lib.WKV_BF16, _lib.ALGO_CHUNKED), dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def fwd(s_in, s_out, *w):
+        y = torch.empty_like(g["r"])
+        st = L.wkv6_forward(stream, B, T, C, H, _lib.WKV_BF16, _lib.FLOOR_DECAY, _lib.ALGO_CHUNKED, *(g[n].data_ptr() for n in "rkvwu"),
+                            s_in.data_ptr(), y.data_ptr(), s_out.data_ptr(), *(w or (None, 0)))
+        torch.cuda.synchronize()
+        assert st == 0, L.wkv_strerror(st)
+        return y
+    want_s = torch.empty_like(g["state"])
+    want_y = fwd(g["state"], want_s)          # (no workspace: one piece)
+    for w in ((), (ws.data_ptr(), ws.numel())):
+        one = g["state"].clone()
+        y = fwd(one, one, *w)
+        assert torch.equal(y, want_y) and torch.equal(one, want_s)
+
+
 def test_noalloc_forward_under_graph_capture():
     """What the entry point is for: recorded into a HIP graph (after wkv_init, nothing is left to set up inside the
     capture) and replayed, with plain launches in between; every replay gives the bits of the plain call."""
