@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256) void cumsum_decay_kernel(int Bw, int Tlen, int
 // The same for the reference's chunk length (RWKV-v5/src/module/rwkv_inner.py:12), with or without the exponentiated
 // tables.  Bound by the bytes written: 4 read and 16 written per element, 4 and 40 with every table in fp64.  Four
 // wavefronts share a chunk, 32 tokens each, and a lane owns V neighbouring channels of them: w is read once (32
-// independent loads per lane in flight), the wavefronts' sums meet in LDS, and every table is then written row by row
+// independent loads per lane in flight), the running sum goes from one to the next through LDS, and every table is then written row by row
 // in pieces of 64 V elements.  (One lane per channel walking all 128 tokens, w read twice, left ten wavefronts per
 // compute unit: B2 T4096 C2560 with every fp64 table 304 us = 3.05 TB/s; now 200 us = 4.6 TB/s.)  V = 2 wherever the rows allow 8-byte accesses.
 constexpr int DT_CHUNK = 128, DT_WAVES = 4, DT_TOK = DT_CHUNK / DT_WAVES;
@@ -77,27 +77,39 @@ __global__ __launch_bounds__(64 * DT_WAVES) void decay_tables_128(int Tlen, int 
             }
         }
     }
-    float sum[V], run[V], total[V], mid[V];
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        sum[i] = run[i] = total[i] = mid[i] = 0.f;
         const float fixed = per_token ? 0.f : log_decay(w[(in ? c : 0) + i], true);
 #pragma unroll
-        for (int t = 0; t < DT_TOK; t++) {
-            l[t][i] = per_token ? log_decay(l[t][i], true) : fixed;
-            sum[i] += l[t][i];
-        }
-        part[wv][lane * V + i] = sum[i];
+        for (int t = 0; t < DT_TOK; t++) l[t][i] = per_token ? log_decay(l[t][i], true) : fixed;
     }
-    __syncthreads();
+    // The running sum goes through the wavefronts in turn, each adding its tokens to where the one before it ended: one sum from
+    // the chunk's first token to its last, so that the total is exactly the last token's running sum (inter there exactly
+    // 0) and no running sum rises.  The three waits are hidden by the other workgroups.
+    float run[V], total[V], mid[V];
 #pragma unroll
-    for (int q = 0; q < DT_WAVES; q++)
+    for (int i = 0; i < V; i++) run[i] = 0.f;
 #pragma unroll
-        for (int i = 0; i < V; i++) {
-            if (q == wv) run[i] = total[i];
-            if (q == DT_WAVES / 2) mid[i] = total[i];         // exclusive running sum at token 64
-            total[i] += part[q][lane * V + i];
+    for (int q = 0; q < DT_WAVES; q++) {
+        if (q == wv) {
+            if (q > 0)
+#pragma unroll
+                for (int i = 0; i < V; i++) run[i] = part[q - 1][lane * V + i];
+#pragma unroll
+            for (int i = 0; i < V; i++) {
+                float s = run[i];
+#pragma unroll
+                for (int t = 0; t < DT_TOK; t++) s += l[t][i];
+                part[q][lane * V + i] = s;
+            }
         }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+        mid[i] = part[DT_WAVES / 2 - 1][lane * V + i];          // exclusive running sum at token 64
+        total[i] = part[DT_WAVES - 1][lane * V + i];
+    }
     if (!in) return;
     if (wv == 0) {
         const size_t o = ((size_t)b * nchunk + n) * C + c;

@@ -417,6 +417,26 @@ def run_gpu56_forward(version, wl, algo):
     return y, s
 
 
+@pytest.mark.parametrize("C", [64, 130, 77])
+@pytest.mark.parametrize("factors", [False, True])
+def test_decay_tables_are_one_running_sum(C, factors):
+    """A chunk's running sum is taken token by token in 32 bits, to the bit: so it never rises, its last value is the chunk's sum,
+    and from there to the chunk's end nothing is left (inter 0, its exponential 1)."""
+    import rwkv_wkv_hip as W
+    raw = (torch.randn(2, 256, C, generator=torch.Generator().manual_seed(4)) * 2.5).cuda()
+    out = W.cumsum_decay(raw, 128, factors=factors)
+    lw, incl, inter = (out[n].view(2, 2, 128, C) for n in ("log_w", "incl", "inter"))
+    run = torch.zeros_like(lw[:, :, 0])
+    for t in range(128):
+        run = run + lw[:, :, t]
+        assert torch.equal(incl[:, :, t], run), t
+    assert torch.equal(out["chunk_sum"], run)
+    assert bool((inter[:, :, -1] == 0).all()) and inter.max() == 0 and bool((incl.diff(dim=2) <= 0).all())
+    if factors:
+        e = out["inter_exp"].view(2, 2, 128, C)
+        assert bool((e[:, :, -1] == 1).all()) and e.max() == 1
+
+
 @pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("T", [16, 50, 64, 128, 200, 512])
 def test_chunked_forward_matches_oracle(version, T):
