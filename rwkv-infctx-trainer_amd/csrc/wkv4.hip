@@ -233,7 +233,8 @@ __global__ __launch_bounds__(64 * SW) void v4_summary_backward(int BC, int Tlen,
     const int lane = threadIdx.x & 63, seg = __builtin_amdgcn_readfirstlane(1 + blockIdx.y * SW + (threadIdx.x >> 6));
     const int idx = blockIdx.x * 64 + lane;
     if (seg >= nseg || idx >= BC) return;
-    const float w = -__expf(time_decay[idx % C]), u = time_first[idx % C];
+    // (bounded: from time_decay = 89 on the decay is e^-inf, and no token before the segment's first, 0 times that, is not a number)
+    const float w = fmaxf(-__expf(time_decay[idx % C]), -1e30f), u = time_first[idx % C];
     V4In<T, false> ik[SD], iv[SD], ig[SD];
     const int blk0 = seg * bps, blk1 = min(blk0 + bps, (Tlen + CK - 1) / CK);
     auto fetch = [&](int blk, int d) __attribute__((always_inline)) {

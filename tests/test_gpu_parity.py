@@ -313,6 +313,23 @@ def test_v4_cut_in_time(dtype, B, T, C):
                                scratch.numel() - 1) == -5
 
 
+@pytest.mark.parametrize("T", [40, 300, 1000])
+def test_v4_decay_that_forgets_everything(T):
+    """time_decay beyond 88.7, whose decay exponent is -inf in 32 bits, gives what one gives that forgets as completely with a
+    finite exponent, whether the sequence is cut in time or not; its own gradient (0 times infinity) is left out."""
+    import rwkv_wkv_hip as W
+    t = v4_case(1, T, 64, torch.float32, seed=T, with_state=True).tensors
+
+    def run(td):
+        leaves = [x.cuda().requires_grad_(True) for x in (torch.where(torch.arange(64) % 3 == 0, torch.tensor(td), t["time_decay"]),
+                                                          t["time_first"], t["k"], t["v"], t["state"])]
+        y, s = W.wkv_op(*leaves)
+        gtd, *rest = torch.autograd.grad([y, s], leaves, [t["dy"].cuda(), t["dstate"].cuda()])
+        return [y, s, gtd[torch.arange(64) % 3 != 0], *(r[..., :2] if r.dim() == 3 and r.shape[2] == 3 else r for r in rest)]
+    for n, a, b in zip(("y", "state", "g_time_decay", "g_time_first", "gk", "gv", "gstate"), run(100.0), run(80.0)):
+        assert bool(torch.isfinite(b).all()) and torch.equal(a, b), n
+
+
 def test_v4_backward_without_forward_checkpoints():
     """The C entry point rebuilds its checkpoints when none are passed."""
     import ctypes
