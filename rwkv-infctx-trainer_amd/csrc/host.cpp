@@ -8,6 +8,7 @@
 // The kernel library stays free of torch: its entry points are looked up by name in the file that `bind` is given.
 #include <Python.h>
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <ATen/autocast_mode.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -76,6 +77,10 @@ bool seen_by_autograd(std::initializer_list<const Tensor *> inputs) {
         if (t->defined() && ((at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined())) return true;
     return false;
 }
+// torch.jit.trace is recording.  It sees what goes through torch's dispatcher or a Python autograd Function, not the calls
+// made here: a graph recorded through them would hold the uninitialised results.  The entry points answer None, and the
+// Python front end makes the call one node of the graph (a layer is recorded step by step).
+bool traced() { return at::tracer::impl::is_dispatch_enabled(); }
 // the caller's tensor: the current device is its device and the stream is that device's current one
 struct OnDevice {
     c10::hip::HIPGuard guard;
@@ -313,10 +318,11 @@ void arity(Py_ssize_t n, Py_ssize_t want) {
     if (n != want) raise(PyExc_TypeError, "wrong number of arguments");
 }
 
-// wkv56(version, algo, in_place, B, T, C, H, r, k, v, w, u, s) -> (y, new_state), or y with the new state in s
+// wkv56(version, algo, in_place, B, T, C, H, r, k, v, w, u, s) -> (y, new_state), or y with the new state in s; None: traced
 PyObject *py_wkv56(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arity(n, 13);
+    if (traced()) Py_RETURN_NONE;
     const Call56 c{integer(a[0]), integer(a[1]), {integer(a[3]), integer(a[4]), integer(a[5]), integer(a[6])}, a[2] == Py_True,
                    tensor(a[7]), tensor(a[8]), tensor(a[9]), tensor(a[10]), tensor(a[11]), tensor(a[12])};
     const auto [y, state] = call56(c);
@@ -358,10 +364,11 @@ PyObject *py_decay_operand(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// wkv4(time_decay, time_first, k, v, state) -> (y, new_state)
+// wkv4(time_decay, time_first, k, v, state) -> (y, new_state); None: traced
 PyObject *py_wkv4(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arity(n, 5);
+    if (traced()) Py_RETURN_NONE;
     const Tensor &td = tensor(a[0]), &tf = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &st = tensor(a[4]);
     REQUIRE(k.dim() == 3 && v.sizes().equals(k.sizes()) && k.scalar_type() == v.scalar_type());
     const int64_t B = k.size(0), C = k.size(2), state[3] = {B, C, 3};

@@ -77,7 +77,7 @@ bool collect(TimeMixCall &c, PyObject *module, PyObject *px, PyObject *states) {
     PyObject *sh = PyTuple_GET_ITEM(states, 0), *st = PyTuple_GET_ITEM(states, 1);
     if (!THPVariable_Check(sh) || !THPVariable_Check(st)) return false;
     const Tensor &x = THPVariable_Unpack(px);
-    if (!x.is_cuda() || x.dim() != 3 || globally_hooked() || at::autocast::is_autocast_enabled(at::kCUDA)) return false;
+    if (!x.is_cuda() || x.dim() != 3 || traced() || globally_hooked() || at::autocast::is_autocast_enabled(at::kCUDA)) return false;
     const int64_t B = x.size(0), T = x.size(1), C = x.size(2), H = PyLong_AsLong(heads);
     if (H <= 0 || H * 64 != C || B <= 0 || T <= 0 || B > 65535 || T > (1 << 20) || B * T > INT_MAX) return false;
     c.d = {(int)B, (int)T, (int)C, (int)H};
@@ -325,7 +325,7 @@ bool collect(ChannelMixCall &c, PyObject *module, PyObject *px, PyObject *sh) {
         !THPVariable_Check(kp))
         return false;
     const Tensor &x = THPVariable_Unpack(px);
-    if (!x.is_cuda() || x.dim() != 3 || globally_hooked() || at::autocast::is_autocast_enabled(at::kCUDA)) return false;
+    if (!x.is_cuda() || x.dim() != 3 || traced() || globally_hooked() || at::autocast::is_autocast_enabled(at::kCUDA)) return false;
     const int64_t B = x.size(0), T = x.size(1), C = x.size(2);
     if (C <= 0 || C % 64 != 0 || B <= 0 || T <= 0 || B > 65535 || T > (1 << 20) || B * T > INT_MAX) return false;
     c.F = THPVariable_Unpack(kp).numel() / C;

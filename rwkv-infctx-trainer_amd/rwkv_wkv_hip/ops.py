@@ -18,6 +18,7 @@ native: csrc/host.cpp.
 """
 from __future__ import annotations
 
+import contextlib
 import os
 
 import torch
@@ -243,10 +244,56 @@ class _Cached56(torch.autograd.Function):
         return (None,) * 7 + (gr, gk, gv, gw.to(wdtype), gu.to(udtype), None if in_place else gs.to(sdtype))
 
 
+@contextlib.contextmanager
+def _untraced():
+    recording = torch._C._get_tracing_state()
+    torch._C._set_tracing_state(None)
+    try:
+        yield recording
+    finally:
+        torch._C._set_tracing_state(recording)
+
+
+class _Traced(torch.autograd.Function):
+    """An operator's call while ``torch.jit.trace`` records: one node of the graph, which makes the call again on the inputs
+    the graph is run with.  (The tracer does not see the native front end, csrc/host.cpp.)  ``written``: the tensor the call
+    writes its new state into."""
+
+    @staticmethod
+    def forward(ctx, call, written, *args):
+        ctx.call, ctx.args = call, [None if torch.is_tensor(a) else a for a in args]
+        ctx.save_for_backward(*[a.detach().clone() if a is written else a for a in args if torch.is_tensor(a)])
+        ctx.set_materialize_grads(False)
+        with _untraced() as recording:
+            outs = call(*args)
+        if recording is None:
+            return outs
+        outs, many = outs if isinstance(outs, tuple) else (outs,), isinstance(outs, tuple)
+        known = [torch.empty(o.shape, dtype=o.dtype, device=o.device) for o in outs]      # seen by the tracer, as results that
+        with _untraced():                                                                 # require a gradient have to be
+            for a, o in zip(known, outs):
+                a.copy_(o)
+        return tuple(known) if many else known[0]
+
+    @staticmethod
+    def backward(ctx, *gouts):
+        saved = iter(ctx.saved_tensors)
+        args = [next(saved).detach().requires_grad_(need) if a is None else a for a, need in zip(ctx.args, ctx.needs_input_grad[2:])]
+        with torch.enable_grad():
+            outs = ctx.call(*args)
+        outs = outs if isinstance(outs, tuple) else (outs,)
+        leaves = [a for a, need in zip(args, ctx.needs_input_grad[2:]) if need]
+        pairs = [(o, g) for o, g in zip(outs, gouts) if g is not None]
+        grads = iter(torch.autograd.grad([o for o, _ in pairs], leaves, [g for _, g in pairs], allow_unused=True))
+        return (None, None, *(next(grads) if need else None for need in ctx.needs_input_grad[2:]))
+
+
 def _op56(version, in_place, B, T, C, H, r, k, v, w, u, s):
     if _cache is not None:
         return _Cached56.apply(version, in_place, torch.is_grad_enabled(), B, T, C, H, r, k, v, w, u, s)
     out = _lib.host().wkv56(version, _algo, in_place, B, T, C, H, r, k, v, w, u, s)
+    if out is None:
+        return _Traced.apply(_op56, s if in_place else None, version, in_place, B, T, C, H, r, k, v, w, u, s)
     stats["forward_launches"] += 1
     return out
 
@@ -304,7 +351,8 @@ def wkv_op(time_decay, time_first, k, v, wkv_state):
     """RWKV-v4 WKV with the signature of torch.ops.rwkv.wkv
     (RWKV-v4neo/src/model.py:130-132): time_decay, time_first (C); k, v (B,T,C);
     wkv_state (B,C,3) = (aa, bb, pp).  Returns (y, new_state)."""
-    return _lib.host().wkv4(time_decay, time_first, k, v, wkv_state)
+    out = _lib.host().wkv4(time_decay, time_first, k, v, wkv_state)
+    return _Traced.apply(wkv_op, None, time_decay, time_first, k, v, wkv_state) if out is None else out
 
 
 def cumsum_decay(w, chunk_len=128, per_token=True, factors=False, precision=64):
