@@ -16,6 +16,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
 
 #include "../../include/rwkv_wkv_hip.h"
 
@@ -292,6 +293,9 @@ public:
 };
 
 // ---- Python arguments
+// The interpreter lock is given up once the arguments are in hand (the tensors' own handles are held, nothing borrowed from Python
+// objects): allocations, launches and library products may wait for the GPU, and other threads run meanwhile.
+typedef pybind11::gil_scoped_release NoLock;
 const Tensor &tensor(PyObject *o) {
     if (!THPVariable_Check(o)) raise(PyExc_TypeError, std::string("expected a torch.Tensor, got ") + Py_TYPE(o)->tp_name);
     return THPVariable_Unpack(o);
@@ -325,7 +329,11 @@ PyObject *py_wkv56(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (traced()) Py_RETURN_NONE;
     const Call56 c{integer(a[0]), integer(a[1]), {integer(a[3]), integer(a[4]), integer(a[5]), integer(a[6])}, a[2] == Py_True,
                    tensor(a[7]), tensor(a[8]), tensor(a[9]), tensor(a[10]), tensor(a[11]), tensor(a[12])};
-    const auto [y, state] = call56(c);
+    Tensor y, state;
+    {
+        NoLock no_lock;
+        std::tie(y, state) = call56(c);
+    }
     return c.in_place ? wrapped(y) : tuple(y, state);
     END_HANDLE_TH_ERRORS
 }
@@ -335,10 +343,15 @@ PyObject *py_wkv56(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *py_forward56(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arity(n, 13);
-    at::AutoDispatchBelowADInplaceOrView below;
+    const int version = integer(a[0]), algo = integer(a[1]);
     const Dims d{integer(a[2]), integer(a[3]), integer(a[4]), integer(a[5])};
-    const Forward56 o = forward56(integer(a[0]), d, integer(a[1]), tensor(a[6]), tensor(a[7]), tensor(a[8]), tensor(a[9]), tensor(a[10]),
-                                  tensor(a[11]), maybe_tensor(a[12]), true);
+    const Tensor r = tensor(a[6]), k = tensor(a[7]), v = tensor(a[8]), w = tensor(a[9]), u = tensor(a[10]), st = tensor(a[11]), out = maybe_tensor(a[12]);
+    Forward56 o;
+    {
+        NoLock no_lock;
+        at::AutoDispatchBelowADInplaceOrView below;
+        o = forward56(version, d, algo, r, k, v, w, u, st, out, true);
+    }
     return tuple(o.y, o.state, o.ws);
     END_HANDLE_TH_ERRORS
 }
@@ -347,10 +360,16 @@ PyObject *py_forward56(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *py_backward56(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arity(n, 15);
-    at::AutoDispatchBelowADInplaceOrView below;
+    const int version = integer(a[0]), algo = integer(a[1]);
     const Dims d{integer(a[2]), integer(a[3]), integer(a[4]), integer(a[5])};
-    const Backward56 g = backward56(integer(a[0]), d, integer(a[1]), tensor(a[6]), tensor(a[7]), tensor(a[8]), tensor(a[9]), tensor(a[10]),
-                                    tensor(a[11]), tensor(a[12]), maybe_tensor(a[13]), maybe_tensor(a[14]), true);
+    const Tensor r = tensor(a[6]), k = tensor(a[7]), v = tensor(a[8]), w = tensor(a[9]), u = tensor(a[10]), st = tensor(a[11]), gy = tensor(a[12]);
+    const Tensor gstate = maybe_tensor(a[13]), ws = maybe_tensor(a[14]);
+    Backward56 g;
+    {
+        NoLock no_lock;
+        at::AutoDispatchBelowADInplaceOrView below;
+        g = backward56(version, d, algo, r, k, v, w, u, st, gy, gstate, ws, true);
+    }
     return tuple(g.gr, g.gk, g.gv, g.gw, g.gu, g.gs);
     END_HANDLE_TH_ERRORS
 }
@@ -360,7 +379,14 @@ PyObject *py_decay_operand(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arity(n, 7);
     const Dims d{integer(a[1]), integer(a[2]), integer(a[3]), integer(a[4])};
-    return wrapped(decay_operand(6, d, integer(a[0]), tensor(a[5]), tensor(a[6]), true));
+    const int algo = integer(a[0]);
+    const Tensor r = tensor(a[5]), w = tensor(a[6]);
+    Tensor o;
+    {
+        NoLock no_lock;
+        o = decay_operand(6, d, algo, r, w, true);
+    }
+    return wrapped(o);
     END_HANDLE_TH_ERRORS
 }
 
@@ -369,18 +395,22 @@ PyObject *py_wkv4(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     arity(n, 5);
     if (traced()) Py_RETURN_NONE;
-    const Tensor &td = tensor(a[0]), &tf = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &st = tensor(a[4]);
-    REQUIRE(k.dim() == 3 && v.sizes().equals(k.sizes()) && k.scalar_type() == v.scalar_type());
-    const int64_t B = k.size(0), C = k.size(2), state[3] = {B, C, 3};
-    REQUIRE(td.dim() == 1 && td.size(0) == C && tf.dim() == 1 && tf.size(0) == C && st.sizes().equals(at::IntArrayRef(state, 3)));
-    dtype_code(k);
-    for (const Tensor *t : {&td, &tf, &k, &v, &st}) on_gpu(*t);
-    if (seen_by_autograd({&td, &tf, &k, &v, &st})) {
-        const variable_list o = Wkv4::apply(td, tf, k, v, st);
-        return tuple(o[0], o[1]);
+    const Tensor td = tensor(a[0]), tf = tensor(a[1]), k = tensor(a[2]), v = tensor(a[3]), st = tensor(a[4]);
+    variable_list o;
+    {
+        NoLock no_lock;
+        REQUIRE(k.dim() == 3 && v.sizes().equals(k.sizes()) && k.scalar_type() == v.scalar_type());
+        const int64_t B = k.size(0), C = k.size(2), state[3] = {B, C, 3};
+        REQUIRE(td.dim() == 1 && td.size(0) == C && tf.dim() == 1 && tf.size(0) == C && st.sizes().equals(at::IntArrayRef(state, 3)));
+        dtype_code(k);
+        for (const Tensor *t : {&td, &tf, &k, &v, &st}) on_gpu(*t);
+        if (seen_by_autograd({&td, &tf, &k, &v, &st})) {
+            o = Wkv4::apply(td, tf, k, v, st);
+        } else {
+            at::AutoDispatchBelowADInplaceOrView below;
+            o = Wkv4::forward(nullptr, td, tf, k, v, st);
+        }
     }
-    at::AutoDispatchBelowADInplaceOrView below;
-    const variable_list o = Wkv4::forward(nullptr, td, tf, k, v, st);
     return tuple(o[0], o[1]);
     END_HANDLE_TH_ERRORS
 }

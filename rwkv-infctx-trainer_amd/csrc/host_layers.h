@@ -35,21 +35,21 @@ struct Plain {
     bool takes(const Tensor &t, at::IntArrayRef shape, at::ScalarType type = at::kBFloat16) {
         return ok = ok && t.defined() && t.sizes().equals(shape) && takes(t, t.numel(), type);
     }
-    const Tensor *parameter(PyObject *params, const char *name, int64_t numel) {
+    Tensor parameter(PyObject *params, const char *name, int64_t numel) {          // (undefined where `ok` fell)
         PyObject *o = item(params, name);
         if (!o || !THPVariable_Check(o)) ok = false;
-        return ok && takes(THPVariable_Unpack(o), numel) ? &THPVariable_Unpack(o) : nullptr;
+        return ok && takes(THPVariable_Unpack(o), numel) ? THPVariable_Unpack(o) : Tensor();
     }
-    const Tensor *matrix(PyObject *params, const char *name, int64_t rows, int64_t cols) {
-        const Tensor *t = parameter(params, name, rows * cols);
-        ok = ok && t->dim() == 2 && t->size(0) == rows;
-        return ok ? t : nullptr;
+    Tensor matrix(PyObject *params, const char *name, int64_t rows, int64_t cols) {
+        Tensor t = parameter(params, name, rows * cols);
+        ok = ok && t.dim() == 2 && t.size(0) == rows;
+        return t;
     }
-    const Tensor *linear(PyObject *modules, const char *name, int64_t n, int64_t k) {          // weight (n, k), no bias
+    Tensor linear(PyObject *modules, const char *name, int64_t n, int64_t k) {          // weight (n, k), no bias
         PyObject *o = item(modules, name), *d = nullptr, *p;
         ok = ok && o && (PyObject *)Py_TYPE(o) == linear_type && (d = dict_of(o)) && !item(d, "forward") && (p = item(d, "_parameters")) &&
              item(p, "bias") == Py_None && unhooked(d);
-        return ok ? matrix(item(d, "_parameters"), "weight", n, k) : nullptr;
+        return ok ? matrix(item(d, "_parameters"), "weight", n, k) : Tensor();
     }
     static bool unhooked(PyObject *d) {
         for (const char *name : {"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"}) {
@@ -68,7 +68,7 @@ struct TimeMixCall {
     int version, algo;
     Dims d;
     float eps;
-    const Tensor *t[N6];
+    Tensor t[N6];          // (handles of their own: the interpreter lock is given up after collecting them)
     bool keep;          // a backward will follow
 };
 bool collect(TimeMixCall &c, PyObject *module, PyObject *px, PyObject *states) {
@@ -89,7 +89,7 @@ bool collect(TimeMixCall &c, PyObject *module, PyObject *px, PyObject *states) {
     p.ok = p.ok && ln && (PyObject *)Py_TYPE(ln) == group_norm_type && (lnd = dict_of(ln)) && (eps = item(lnd, "eps")) && PyFloat_Check(eps);
     if (!p.ok) return false;
     c.eps = (float)PyFloat_AS_DOUBLE(eps);
-    c.t[X] = &x; c.t[SHIFT] = &THPVariable_Unpack(sh); c.t[STATE] = &THPVariable_Unpack(st);
+    c.t[X] = x; c.t[SHIFT] = THPVariable_Unpack(sh); c.t[STATE] = THPVariable_Unpack(st);
     c.t[DECAY] = p.parameter(prm, "time_decay", C);
     c.t[U] = p.parameter(prm, "time_faaaa", C);
     c.t[LN_W] = p.parameter(item(lnd, "_parameters"), "weight", C);
@@ -101,7 +101,7 @@ bool collect(TimeMixCall &c, PyObject *module, PyObject *px, PyObject *states) {
         for (int j = 0; j < 6; j++) c.t[MAA_X + j] = p.parameter(prm, maa[j], C);
         c.t[W1] = p.matrix(prm, "time_maa_w1", C, 160);
         c.t[W2] = p.parameter(prm, "time_maa_w2", C * 160);
-        p.ok = p.ok && c.t[W2]->dim() == 3 && c.t[W2]->size(0) == 5 && c.t[W2]->size(1) == 32;
+        p.ok = p.ok && c.t[W2].dim() == 3 && c.t[W2].size(0) == 5 && c.t[W2].size(1) == 32;
         PyObject *o = item(prm, "time_decay_w1");
         const int64_t D = o && THPVariable_Check(o) ? THPVariable_Unpack(o).numel() / C : 0;
         c.t[DW1] = p.matrix(prm, "time_decay_w1", C, D);
@@ -112,18 +112,16 @@ bool collect(TimeMixCall &c, PyObject *module, PyObject *px, PyObject *states) {
     }
     return p.ok;
 }
-bool any_requires_grad(const Tensor *const *t, int n) {
+bool any_requires_grad(const Tensor *t, int n) {
     for (int i = 0; i < n; i++)
-        if (t[i]->requires_grad()) return true;
+        if (t[i].requires_grad()) return true;
     return false;
 }
 
 // ---- the steps, on tensors of one device whose stream is handed in
-Tensor widen_rows(void *stream, const Tensor *const *rows, int count, int64_t C) {      // bf16 parameters of C elements -> (count, C) fp32
-    Tensor out = at::empty({count, C}, rows[0]->options().dtype(at::kFloat));
-    const void *p[16];
-    for (int i = 0; i < count; i++) p[i] = rows[i]->data_ptr();
-    check(abi.wkv_widen_rows(stream, count, C, p, fptr(out)), "wkv_widen_rows");
+Tensor widen_rows(void *stream, const Tensor &like, const void *const *rows, int count, int64_t C) {      // bf16 parameters of C elements -> (count, C) fp32
+    Tensor out = at::empty({count, C}, like.options().dtype(at::kFloat));
+    check(abi.wkv_widen_rows(stream, count, C, rows, fptr(out)), "wkv_widen_rows");
     return out;
 }
 template <int N> struct Planes {          // the N planes of a tensor (N, ...)
@@ -157,53 +155,53 @@ enum { COEF, XXX, ACT, W2T, MIXES, RR, KK, VV, GG, LORA, WW, YY, ZZ, WS, SAVED }
 struct TimeMixOut { Tensor out, state, saved[SAVED]; };
 TimeMixOut timemix_forward(const TimeMixCall &c) {
     const Dims &d = c.d;
-    const Tensor *const *t = c.t;
+    const Tensor *t = c.t;
     const int64_t M = d.B * (int64_t)d.T, C = d.C;
-    OnDevice dev(*t[X]);
+    OnDevice dev(t[X]);
     void *stream = dev.stream();
     TimeMixOut o;
-    const Tensor *rows[9] = {t[U], t[LN_W], t[LN_B]};
+    const void *rows[9] = {ptr(t[U]), ptr(t[LN_W]), ptr(t[LN_B])};
     const int mixes = c.version == 6 ? 6 : 4;
-    for (int j = 0; j < mixes; j++) rows[3 + j] = t[MIX0 + j];
-    const Tensor coef = o.saved[COEF] = widen_rows(stream, rows, 3 + mixes, C);
+    for (int j = 0; j < mixes; j++) rows[3 + j] = ptr(t[MIX0 + j]);
+    const Tensor coef = o.saved[COEF] = widen_rows(stream, t[X], rows, 3 + mixes, C);
     const float *mix = fptr(coef) + 3 * C;
     int r, k, v, g;
     if (c.version == 6) {
-        o.saved[XXX] = shift_mix(stream, d, 1, false, *t[X], *t[SHIFT], mix).view({M, C});
-        o.saved[ACT] = at::mm(o.saved[XXX], *t[W1]).tanh_();
-        o.saved[W2T] = t[W2]->transpose(1, 2).contiguous();
-        o.saved[MIXES] = at::empty({5, M, C}, t[X]->options());
-        check(abi.wkv_lora_mix_forward(stream, d.B, d.T, d.C, ptr(*t[X]), ptr(*t[SHIFT]), mix + C, ptr(o.saved[ACT]), ptr(o.saved[W2T]),
+        o.saved[XXX] = shift_mix(stream, d, 1, false, t[X], t[SHIFT], mix).view({M, C});
+        o.saved[ACT] = at::mm(o.saved[XXX], t[W1]).tanh_();
+        o.saved[W2T] = t[W2].transpose(1, 2).contiguous();
+        o.saved[MIXES] = at::empty({5, M, C}, t[X].options());
+        check(abi.wkv_lora_mix_forward(stream, d.B, d.T, d.C, ptr(t[X]), ptr(t[SHIFT]), mix + C, ptr(o.saved[ACT]), ptr(o.saved[W2T]),
                                        Planes<5>(o.saved[MIXES]).p), "wkv_lora_mix_forward");
         r = 3; k = 1; v = 2; g = 4;
     } else {
-        o.saved[MIXES] = shift_mix(stream, d, 4, true, *t[X], *t[SHIFT], mix);
+        o.saved[MIXES] = shift_mix(stream, d, 4, true, t[X], t[SHIFT], mix);
         r = 2; k = 0; v = 1; g = 3;
     }
     const Tensor &m = o.saved[MIXES];
-    o.saved[RR] = times_t(plane(m, r), *t[WR]);
-    o.saved[KK] = times_t(plane(m, k), *t[WK]);
-    o.saved[VV] = times_t(plane(m, v), *t[WV]);
-    o.saved[GG] = times_t(plane(m, g), *t[WG]);
+    o.saved[RR] = times_t(plane(m, r), t[WR]);
+    o.saved[KK] = times_t(plane(m, k), t[WK]);
+    o.saved[VV] = times_t(plane(m, v), t[WV]);
+    o.saved[GG] = times_t(plane(m, g), t[WG]);
     const int64_t streams[3] = {d.B, d.T, d.C};
     auto seq = [&](const Tensor &x) { return x.view(at::IntArrayRef(streams, 3)); };
     if (c.version == 6) {
-        o.saved[LORA] = at::mm(plane(m, 0), *t[DW1]).tanh_();
+        o.saved[LORA] = at::mm(plane(m, 0), t[DW1]).tanh_();
         // the broadcast addition of time_decay rides on the product as its bias
-        const Tensor w = at::addmm(t[DECAY]->view({C}), o.saved[LORA], *t[DW2]);
+        const Tensor w = at::addmm(t[DECAY].view({C}), o.saved[LORA], t[DW2]);
         o.saved[WW] = decay_operand(6, d, c.algo, seq(o.saved[RR]), seq(w), c.keep);
     } else {
-        o.saved[WW] = t[DECAY]->to(at::kFloat);
+        o.saved[WW] = t[DECAY].to(at::kFloat);
     }
-    Forward56 f = forward56(c.version, d, c.algo, seq(o.saved[RR]), seq(o.saved[KK]), seq(o.saved[VV]), o.saved[WW], coef.select(0, 0), *t[STATE],
+    Forward56 f = forward56(c.version, d, c.algo, seq(o.saved[RR]), seq(o.saved[KK]), seq(o.saved[VV]), o.saved[WW], coef.select(0, 0), t[STATE],
                             Tensor(), c.keep);
     o.saved[YY] = f.y;
     o.saved[WS] = f.ws;
     o.state = f.state;
-    o.saved[ZZ] = at::empty({M, C}, t[X]->options());
+    o.saved[ZZ] = at::empty({M, C}, t[X].options());
     check(abi.wkv_ln_gate_forward(stream, M, C, WKV_BF16, c.version == 6 ? 1.f : 0.125f, c.eps, ptr(f.y), ptr(o.saved[GG]), fptr(coef) + C,
                                   fptr(coef) + 2 * C, ptr(o.saved[ZZ])), "wkv_ln_gate_forward");
-    o.out = seq(times_t(o.saved[ZZ], *t[WO]));
+    o.out = seq(times_t(o.saved[ZZ], t[WO]));
     return o;
 }
 
@@ -309,7 +307,7 @@ public:
         return g;
     }
 };
-template <class F, size_t... I> variable_list apply_node(const TimeMixCall &c, std::index_sequence<I...>) { return F::apply(&c, *c.t[I]...); }
+template <class F, size_t... I> variable_list apply_node(const TimeMixCall &c, std::index_sequence<I...>) { return F::apply(&c, c.t[I]...); }
 
 // ---- channel mix
 enum { CM_X, CM_SHIFT, CM_MIX_K, CM_MIX_R, CM_WK, CM_WR, CM_WV, CM_N };
@@ -317,7 +315,7 @@ struct ChannelMixCall {
     bool lerp;
     Dims d;
     int64_t F;
-    const Tensor *t[CM_N];
+    Tensor t[CM_N];
 };
 bool collect(ChannelMixCall &c, PyObject *module, PyObject *px, PyObject *sh) {
     PyObject *dict = dict_of(module), *prm = item(dict, "_parameters"), *mod = item(dict, "_modules"), *key = item(mod, "key"), *kp;
@@ -334,7 +332,7 @@ bool collect(ChannelMixCall &c, PyObject *module, PyObject *px, PyObject *sh) {
     Plain p(x);
     p.takes(x, B * T * C);
     p.takes(THPVariable_Unpack(sh), {B, C});
-    c.t[CM_X] = &x; c.t[CM_SHIFT] = &THPVariable_Unpack(sh);
+    c.t[CM_X] = x; c.t[CM_SHIFT] = THPVariable_Unpack(sh);
     c.t[CM_MIX_K] = p.parameter(prm, c.lerp ? "time_mix_k" : "time_maa_k", C);
     c.t[CM_MIX_R] = p.parameter(prm, c.lerp ? "time_mix_r" : "time_maa_r", C);
     c.t[CM_WK] = p.linear(mod, "key", c.F, C);
@@ -346,18 +344,19 @@ enum { CM_COEF, CM_MIXES, CM_K, CM_K2, CM_KV, CM_R, CM_SAVED };
 struct ChannelMixOut { Tensor out, saved[CM_SAVED]; };
 ChannelMixOut channelmix_forward(const ChannelMixCall &c) {
     const Dims &d = c.d;
-    const Tensor *const *t = c.t;
-    OnDevice dev(*t[CM_X]);
+    const Tensor *t = c.t;
+    OnDevice dev(t[CM_X]);
     void *stream = dev.stream();
     ChannelMixOut o;
-    o.saved[CM_COEF] = widen_rows(stream, t + CM_MIX_K, 2, d.C);
-    o.saved[CM_MIXES] = shift_mix(stream, d, 2, c.lerp, *t[CM_X], *t[CM_SHIFT], fptr(o.saved[CM_COEF]));
-    const Tensor k = o.saved[CM_K] = times_t(plane(o.saved[CM_MIXES], 0), *t[CM_WK]);
+    const void *rows[2] = {ptr(t[CM_MIX_K]), ptr(t[CM_MIX_R])};
+    o.saved[CM_COEF] = widen_rows(stream, t[CM_X], rows, 2, d.C);
+    o.saved[CM_MIXES] = shift_mix(stream, d, 2, c.lerp, t[CM_X], t[CM_SHIFT], fptr(o.saved[CM_COEF]));
+    const Tensor k = o.saved[CM_K] = times_t(plane(o.saved[CM_MIXES], 0), t[CM_WK]);
     o.saved[CM_K2] = at::empty_like(k);
     check(abi.wkv_relu_square_forward(stream, k.numel(), WKV_BF16, ptr(k), ptr(o.saved[CM_K2])), "wkv_relu_square_forward");
-    o.saved[CM_KV] = times_t(o.saved[CM_K2], *t[CM_WV]);
-    const Tensor r = o.saved[CM_R] = times_t(plane(o.saved[CM_MIXES], 1), *t[CM_WR]);
-    o.out = at::empty_like(*t[CM_X]);
+    o.saved[CM_KV] = times_t(o.saved[CM_K2], t[CM_WV]);
+    const Tensor r = o.saved[CM_R] = times_t(plane(o.saved[CM_MIXES], 1), t[CM_WR]);
+    o.out = at::empty_like(t[CM_X]);
     check(abi.wkv_sigmoid_mul_forward(stream, r.numel(), WKV_BF16, ptr(r), ptr(o.saved[CM_KV]), ptr(o.out)), "wkv_sigmoid_mul_forward");
     return o;
 }
@@ -415,9 +414,9 @@ public:
 // ---- one token per sequence, nothing recorded (csrc/layer_decode.hip)
 bool single_tokens(const Dims &d) { return d.T == 1 && d.B <= 64; }
 std::pair<Tensor, Tensor> timemix_decode(const TimeMixCall &c) {
-    const Tensor *const *t = c.t;
+    const Tensor *t = c.t;
     const int64_t B = c.d.B, C = c.d.C, rows = B * C;
-    const Tensor &x = *t[X];
+    const Tensor &x = t[X];
     const bool v6 = c.version == 6;
     OnDevice dev(x);
     void *stream = dev.stream();
@@ -426,44 +425,44 @@ std::pair<Tensor, Tensor> timemix_decode(const TimeMixCall &c) {
     Tensor scratch = at::empty({(v6 ? 10 : 5) * rows + (v6 ? parts * B * 224 : 0)}, x.options());
     at::BFloat16 *q = scratch.data_ptr<at::BFloat16>();
     at::BFloat16 *r = q, *k = r + rows, *v = k + rows, *g = v + rows, *z = g + rows, *mixes = z + rows, *act = mixes + 5 * rows, *lora = act + parts * B * 160;
-    Tensor out = at::empty_like(x), state = at::empty_like(*t[STATE]);
-    const void *px = ptr(x), *ps = ptr(*t[SHIFT]), *wr = ptr(*t[WR]), *wk = ptr(*t[WK]), *wv = ptr(*t[WV]), *wg = ptr(*t[WG]);
+    Tensor out = at::empty_like(x), state = at::empty_like(t[STATE]);
+    const void *px = ptr(x), *ps = ptr(t[SHIFT]), *wr = ptr(t[WR]), *wk = ptr(t[WK]), *wv = ptr(t[WV]), *wg = ptr(t[WG]);
     const int n = (int)C;
     if (v6) {
         const void *maa[5];
-        for (int j = 0; j < 5; j++) maa[j] = ptr(*t[MAA_W + j]);
-        const wkv_rows_product first{ptr(*t[W1]), px, ps, ptr(*t[MAA_X]), nullptr, act, 160, 1, 0, 0};
+        for (int j = 0; j < 5; j++) maa[j] = ptr(t[MAA_W + j]);
+        const wkv_rows_product first{ptr(t[W1]), px, ps, ptr(t[MAA_X]), nullptr, act, 160, 1, 0, 0};
         check(abi.wkv_rows_products(stream, B, C, 1, &first), "wkv_rows_products");
-        check(abi.wkv_lora_mix_rows(stream, B, C, px, ps, maa, act, ptr(*t[W2]), mixes), "wkv_lora_mix_rows");
-        const wkv_rows_product proj[5] = {{ptr(*t[DW1]), mixes, nullptr, nullptr, nullptr, lora, 64, 1, 0, 0},
+        check(abi.wkv_lora_mix_rows(stream, B, C, px, ps, maa, act, ptr(t[W2]), mixes), "wkv_lora_mix_rows");
+        const wkv_rows_product proj[5] = {{ptr(t[DW1]), mixes, nullptr, nullptr, nullptr, lora, 64, 1, 0, 0},
                                           {wk, mixes + rows, nullptr, nullptr, nullptr, k, n, 0, 0, 0},
                                           {wv, mixes + 2 * rows, nullptr, nullptr, nullptr, v, n, 0, 0, 0},
                                           {wr, mixes + 3 * rows, nullptr, nullptr, nullptr, r, n, 0, 0, 0},
                                           {wg, mixes + 4 * rows, nullptr, nullptr, nullptr, g, n, 0, 0, 0}};
         check(abi.wkv_rows_products(stream, B, C, 5, proj), "wkv_rows_products");
     } else {
-        const wkv_rows_product proj[4] = {{wk, px, ps, ptr(*t[MIX0]), nullptr, k, n, 0, 1, 0}, {wv, px, ps, ptr(*t[MIX0 + 1]), nullptr, v, n, 0, 1, 0},
-                                          {wr, px, ps, ptr(*t[MIX0 + 2]), nullptr, r, n, 0, 1, 0}, {wg, px, ps, ptr(*t[MIX0 + 3]), nullptr, g, n, 0, 1, 0}};
+        const wkv_rows_product proj[4] = {{wk, px, ps, ptr(t[MIX0]), nullptr, k, n, 0, 1, 0}, {wv, px, ps, ptr(t[MIX0 + 1]), nullptr, v, n, 0, 1, 0},
+                                          {wr, px, ps, ptr(t[MIX0 + 2]), nullptr, r, n, 0, 1, 0}, {wg, px, ps, ptr(t[MIX0 + 3]), nullptr, g, n, 0, 1, 0}};
         check(abi.wkv_rows_products(stream, B, C, 4, proj), "wkv_rows_products");
     }
-    check(abi.wkv_timemix_head(stream, B, C, c.d.H, r, k, v, g, ptr(*t[DECAY]), v6 ? lora : nullptr, v6 ? ptr(*t[DW2]) : nullptr, ptr(*t[U]), ptr(*t[LN_W]),
-                               ptr(*t[LN_B]), v6 ? 1.f : 0.125f, c.eps, fptr(*t[STATE]), fptr(state), z), "wkv_timemix_head");
-    const wkv_rows_product last{ptr(*t[WO]), z, nullptr, nullptr, nullptr, ptr(out), n, 0, 0, 0};
+    check(abi.wkv_timemix_head(stream, B, C, c.d.H, r, k, v, g, ptr(t[DECAY]), v6 ? lora : nullptr, v6 ? ptr(t[DW2]) : nullptr, ptr(t[U]), ptr(t[LN_W]),
+                               ptr(t[LN_B]), v6 ? 1.f : 0.125f, c.eps, fptr(t[STATE]), fptr(state), z), "wkv_timemix_head");
+    const wkv_rows_product last{ptr(t[WO]), z, nullptr, nullptr, nullptr, ptr(out), n, 0, 0, 0};
     check(abi.wkv_rows_products(stream, B, C, 1, &last), "wkv_rows_products");
     return {out, state};
 }
 Tensor channelmix_decode(const ChannelMixCall &c) {
-    const Tensor *const *t = c.t;
+    const Tensor *t = c.t;
     const int64_t B = c.d.B, C = c.d.C, F = c.F;
-    const Tensor &x = *t[CM_X];
+    const Tensor &x = t[CM_X];
     OnDevice dev(x);
     Tensor scratch = at::empty({B * (F + C)}, x.options()), out = at::empty_like(x);
     at::BFloat16 *k = scratch.data_ptr<at::BFloat16>(), *r = k + B * F;
-    const void *px = ptr(x), *ps = ptr(*t[CM_SHIFT]);
-    const wkv_rows_product proj[2] = {{ptr(*t[CM_WK]), px, ps, ptr(*t[CM_MIX_K]), nullptr, k, (int)F, 0, c.lerp, 1},
-                                      {ptr(*t[CM_WR]), px, ps, ptr(*t[CM_MIX_R]), nullptr, r, (int)C, 0, c.lerp, 0}};
+    const void *px = ptr(x), *ps = ptr(t[CM_SHIFT]);
+    const wkv_rows_product proj[2] = {{ptr(t[CM_WK]), px, ps, ptr(t[CM_MIX_K]), nullptr, k, (int)F, 0, c.lerp, 1},
+                                      {ptr(t[CM_WR]), px, ps, ptr(t[CM_MIX_R]), nullptr, r, (int)C, 0, c.lerp, 0}};
     check(abi.wkv_rows_products(dev.stream(), B, C, 2, proj), "wkv_rows_products");
-    const wkv_rows_product last{ptr(*t[CM_WV]), k, nullptr, nullptr, r, ptr(out), (int)C, 0, 0, 2};
+    const wkv_rows_product last{ptr(t[CM_WV]), k, nullptr, nullptr, r, ptr(out), (int)C, 0, 0, 2};
     check(abi.wkv_rows_products(dev.stream(), B, F, 1, &last), "wkv_rows_products");
     return out;
 }
@@ -476,21 +475,25 @@ PyObject *py_timemix(PyObject *, PyObject *const *a, Py_ssize_t n) {
     c.version = integer(a[0]);
     c.algo = integer(a[1]);
     if (!collect(c, a[2], a[3], a[4])) Py_RETURN_NONE;
-    c.keep = at::GradMode::is_enabled() && any_requires_grad(c.t, c.version == 6 ? (int)N6 : (int)N5);
-    Tensor out, state;
-    if (c.keep) {
-        const variable_list o = c.version == 6 ? apply_node<TimeMix<6>>(c, std::make_index_sequence<N6>()) : apply_node<TimeMix<5>>(c, std::make_index_sequence<N5>());
-        out = o[0]; state = o[1];
-    } else {
-        at::AutoDispatchBelowADInplaceOrView below;
-        if (single_tokens(c.d) && (c.version == 5 || c.t[DW1]->size(1) == 64)) {
-            std::tie(out, state) = timemix_decode(c);
+    Tensor out, state, last;
+    {
+        NoLock no_lock;
+        c.keep = at::GradMode::is_enabled() && any_requires_grad(c.t, c.version == 6 ? (int)N6 : (int)N5);
+        if (c.keep) {
+            const variable_list o = c.version == 6 ? apply_node<TimeMix<6>>(c, std::make_index_sequence<N6>()) : apply_node<TimeMix<5>>(c, std::make_index_sequence<N5>());
+            out = o[0]; state = o[1];
         } else {
-            TimeMixOut o = timemix_forward(c);
-            out = o.out; state = o.state;
+            at::AutoDispatchBelowADInplaceOrView below;
+            if (single_tokens(c.d) && (c.version == 5 || c.t[DW1].size(1) == 64)) {
+                std::tie(out, state) = timemix_decode(c);
+            } else {
+                TimeMixOut o = timemix_forward(c);
+                out = o.out; state = o.state;
+            }
         }
+        last = c.t[X].select(1, c.d.T - 1);
     }
-    PyObject *states = tuple(c.t[X]->select(1, c.d.T - 1), state);
+    PyObject *states = tuple(last, state);
     return Py_BuildValue("(NN)", wrapped(out), states);
     END_HANDLE_TH_ERRORS
 }
@@ -502,13 +505,17 @@ PyObject *py_channelmix(PyObject *, PyObject *const *a, Py_ssize_t n) {
     ChannelMixCall c{};
     c.lerp = integer(a[0]) == 5;
     if (!collect(c, a[1], a[2], a[3])) Py_RETURN_NONE;
-    Tensor out;
-    if (at::GradMode::is_enabled() && any_requires_grad(c.t, CM_N)) {
-        out = ChannelMix::apply(&c, *c.t[0], *c.t[1], *c.t[2], *c.t[3], *c.t[4], *c.t[5], *c.t[6])[0];
-    } else {
-        at::AutoDispatchBelowADInplaceOrView below;
-        out = single_tokens(c.d) && c.F % 64 == 0 ? channelmix_decode(c) : channelmix_forward(c).out;
+    Tensor out, last;
+    {
+        NoLock no_lock;
+        if (at::GradMode::is_enabled() && any_requires_grad(c.t, CM_N)) {
+            out = ChannelMix::apply(&c, c.t[0], c.t[1], c.t[2], c.t[3], c.t[4], c.t[5], c.t[6])[0];
+        } else {
+            at::AutoDispatchBelowADInplaceOrView below;
+            out = single_tokens(c.d) && c.F % 64 == 0 ? channelmix_decode(c) : channelmix_forward(c).out;
+        }
+        last = c.t[CM_X].select(1, c.d.T - 1);
     }
-    return tuple(out, c.t[CM_X]->select(1, c.d.T - 1));
+    return tuple(out, last);
     END_HANDLE_TH_ERRORS
 }
