@@ -386,6 +386,40 @@ def test_layer_refuses_states_of_another_shape(version, T, grad):
 
 
 @pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("grad", [True, False])
+def test_layer_native_holds_no_more_memory_than_the_steps(version, grad):
+    """The most memory a layer's pass (with its backward) holds at once, against the same layer as a node per step, which lets go of every
+    saved tensor on the way: within a tenth."""
+    from rwkv_wkv_hip import blocks as K
+    B, T, H = 1, 2048, 32
+    C = 64 * H
+    timemix, channelmix = (K.timemix5_forward, K.channelmix5_forward) if version == 5 else (K.timemix6_forward, K.channelmix6_forward)
+    x, gy = torch.randn(B, T, C).cuda().bfloat16(), torch.randn(B, T, C).cuda().bfloat16()
+    shift, state = torch.randn(B, C).cuda().bfloat16(), torch.randn(B, H, 64, 64).cuda()
+
+    def peak(hooked):
+        tm, cm = ((TimeMix5 if version == 5 else TimeMix6)(C, H, seed=8).cuda().bfloat16(),
+                  (ChannelMix5 if version == 5 else ChannelMix6)(C, C * 7 // 2, seed=9).cuda().bfloat16())
+        if hooked:
+            tm.key.register_forward_hook(lambda *a: None)
+            cm.key.register_forward_hook(lambda *a: None)
+        leaves = [x.clone().requires_grad_(grad), *tm.parameters(), *cm.parameters()]
+
+        def run():
+            with torch.set_grad_enabled(grad):
+                y, _ = channelmix(cm, timemix(tm, leaves[0], (shift, state))[0], shift)
+            return torch.autograd.grad(y, leaves, gy) if grad else y
+        run()
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        run()
+        return torch.cuda.max_memory_allocated() - before
+    native, steps = peak(False), peak(True)
+    assert native <= 1.1 * steps, (native / 2**20, steps / 2**20)
+
+
+@pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("T,frozen", [(1, ()), (2, ("key",)), (65, ()), (130, ("ln_x", "output", "value", "time"))])
 def test_layer_native_matches_the_steps(version, T, frozen):
     """A layer's halves as the native host side runs them against the same kernels step by step (which a hook on one of the
