@@ -61,11 +61,12 @@ typedef enum { WKV_F32 = 0, WKV_BF16 = 1, WKV_F16 = 2 } wkv_dtype;
                                  wkv56_forward_scratch() bytes that holds the summaries of the time split alone.
                                  (Without any workspace a forward call runs every sequence in one piece.) */
 
-#define WKV_W_F16 16u         /* as WKV_W_BF16, for fp16 streams and WKV_ALGO_AUTO with two tokens or more */
+#define WKV_W_F16 16u         /* as WKV_W_BF16, for fp16 streams and WKV_ALGO_AUTO with two tokens or more (such calls are worked in
+                                 64-token steps whatever their length) */
 
 /* algorithm selector */
 #define WKV_ALGO_AUTO      0  /* blocked where it applies (with WKV_FLOOR_DECAY: bf16 streams as WKV_ALGO_CHUNKED, fp32
-                                 and fp16 streams with fp32 products), else recurrent */
+                                 and fp16 streams with fp32 products from some 30 to 50 tokens on, by B*H), else recurrent */
 #define WKV_ALGO_RECURRENT 1  /* per-token fp32 recurrence, any T, any dtype */
 #define WKV_ALGO_CHUNKED   2  /* 64-token chunks on the matrix cores, bf16 operands */
 

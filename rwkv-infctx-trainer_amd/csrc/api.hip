@@ -30,15 +30,33 @@ int check_dims56(int B, int T, int C, int H, int dtype) {
 }
 
 // The blocked kernels rely on the decay floor (whose range analysis they need).  With it bf16 streams take those of
-// wkv56_chunked.hip, fp32 and fp16 streams of two tokens or more those of wkv56_f32.hip (ALGO_F32, not a selector of the
-// ABI); everything else goes token by token.
+// wkv56_chunked.hip, fp32 and fp16 streams those of wkv56_f32.hip (ALGO_F32, not a selector of the ABI) where the sequences
+// are long enough for them; everything else goes token by token.
 constexpr int ALGO_F32 = 3;
 const chunked::Costs &costs_of(int a) { return a == ALGO_F32 ? chunked::F32_COSTS : chunked::BF16_COSTS; }
-int pick_algo56(int algo, int T, int C, int dtype, unsigned flags) {
+// Short fp32 and fp16 sequences: the kernels of wkv56_f32.hip work whole 64-token steps, one workgroup per compute unit, so a few
+// tokens cost them what 64 do, once per round of B*H over the compute units; the per-token kernels share a compute unit and
+// pay by the token.  Both costs in us, fitted to B*H 12 .. 4096 (r = B*H in rounds of 256), for a forward alone and for one
+// with its backward; on either side of the line, e.g. (token by token / in steps), fp32 forward and backward: B*H 12 T 16 19 / 27,
+// T 40 35 / 27; 512, T 32 52 / 61, T 48 68 / 65; 1024, T 16 60 / 108, T 40 109 / 118, T 56 142 / 124; forward: 256, T 16 6.6 / 8.5,
+// T 40 11.4 / 8.8; 1024, T 80 45 / 54, T 112 59 / 56.  The line lies where the two agree within some 10 %; from 129 tokens
+// on steps always pay.  (A segment count set asks for steps.)
+bool steps_pay(int BH, int T, bool backward) {
+    if (T > 2 * chunked::SB || chunked::forced_segments() > 0) return true;
+    const int ncu = cu_count(), steps = (T + chunked::SB - 1) / chunked::SB;
+    const double r = (BH + ncu - 1) / ncu;
+    return backward ? r * (14.0 + 15.6 * steps) < 7.0 + 4.7 * r + (0.12 + 0.475 * r) * T : r * (3.7 + 4.8 * steps) < 2.0 + 1.5 * r + (0.07 + 0.1 * r) * T;
+}
+// backward: the call is one of a forward and its backward (they have to agree: the checkpoints between the two)
+int pick_algo56(int algo, int BH, int T, int C, int dtype, unsigned flags, bool backward) {
     // (the fp32 kernels' stores count on offsets of the last step's missing tokens not wrapping)
     const bool can_f32 = T > 1 && (flags & WKV_FLOOR_DECAY) && (long long)(T + 64) * C < (1ll << 30);
     const bool can_chunk = dtype == WKV_BF16 && (flags & WKV_FLOOR_DECAY);
-    if (algo == WKV_ALGO_AUTO) return can_chunk ? WKV_ALGO_CHUNKED : can_f32 ? ALGO_F32 : WKV_ALGO_RECURRENT;
+    if (algo == WKV_ALGO_AUTO) {
+        if (can_chunk) return WKV_ALGO_CHUNKED;
+        // (an fp16 decay is read by those kernels alone)
+        return can_f32 && ((flags & WKV_W_F16) || steps_pay(BH, T, backward)) ? ALGO_F32 : WKV_ALGO_RECURRENT;
+    }
     if (algo == WKV_ALGO_RECURRENT) return algo;
     if (algo == WKV_ALGO_CHUNKED) return can_chunk ? algo : WKV_ERR_ALGO;
     return WKV_ERR_ALGO;
@@ -69,7 +87,8 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
     for (const void *p : {r, k, v, (const void *)w, (const void *)u, (const void *)state_in, (const void *)y,
                           (const void *)state_out})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
-    const int a = pick_algo56(algo, T, C, dtype, flags);
+    const bool keep = workspace && !(flags & WKV_NO_CHECKPOINTS);          // state checkpoints, for a backward
+    const int a = pick_algo56(algo, B * H, T, C, dtype, flags, keep);
     if (a < 0) return a;
     st = check_state_alias(state_in, state_out, B, H, a == WKV_ALGO_CHUNKED && chunked::needs_two_states(B * H, T));
     if (st) return st;
@@ -78,7 +97,6 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
     const int floor_decay = (flags & WKV_FLOOR_DECAY) ? 1 : 0;
     if (a != WKV_ALGO_RECURRENT) {
         // with a workspace the state at the start of every 64-token step is left there for backward
-        const bool keep = !(flags & WKV_NO_CHECKPOINTS);
         if (workspace) {
             if (!aligned16(workspace)) return WKV_ERR_ALIGN;
             if (workspace_bytes < (keep ? chunked::forward_workspace(B, T, H, costs_of(a)) : chunked::forward_scratch(B, T, H, costs_of(a)))) return WKV_ERR_WORKSPACE;
@@ -99,14 +117,14 @@ int forward56(bool per_token, void *stream, int B, int T, int C, int H, int dtyp
 // (sizes are for the larger of the two algorithms a call with these arguments can take)
 size_t forward56_workspace(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
-    const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
+    const int a = pick_algo56(algo, B * H, T, C, dtype, WKV_FLOOR_DECAY, true);
     return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_workspace(B, T, H, costs_of(a)) : 0;
 }
 
 size_t backward56_workspace(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
     const size_t rec = recurrent_backward_workspace(B, T, C);
-    const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
+    const int a = pick_algo56(algo, B * H, T, C, dtype, WKV_FLOOR_DECAY | (dtype == WKV_F16 ? WKV_W_F16 : 0u), true);
     return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? std::max(rec, chunked::backward_workspace(B, T, C, H, costs_of(a))) : rec;
 }
 
@@ -121,7 +139,7 @@ int backward56(bool per_token, void *stream, int B, int T, int C, int H, int dty
                           (const void *)gstate_out, (const void *)gr, (const void *)gk, (const void *)gv,
                           (const void *)gw, (const void *)gu, (const void *)gstate_in, (const void *)workspace})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
-    const int a = pick_algo56(algo, T, C, dtype, flags);
+    const int a = pick_algo56(algo, B * H, T, C, dtype, flags, true);
     if (a < 0) return a;
     if (!decay_type_fits(a, dtype, per_token, flags)) return WKV_ERR_ALGO;
     const bool w16 = (flags & (WKV_W_BF16 | WKV_W_F16)) != 0;
@@ -233,7 +251,7 @@ size_t wkv6_forward_workspace(int B, int T, int C, int H, int dtype, int algo) {
 }
 size_t wkv56_forward_scratch(int B, int T, int C, int H, int dtype, int algo) {
     if (check_dims56(B, T, C, H, dtype)) return 0;
-    const int a = pick_algo56(algo, T, C, dtype, WKV_FLOOR_DECAY);
+    const int a = pick_algo56(algo, B * H, T, C, dtype, WKV_FLOOR_DECAY, false);
     return a == WKV_ALGO_CHUNKED || a == ALGO_F32 ? chunked::forward_scratch(B, T, H, costs_of(a)) : 0;
 }
 size_t wkv5_forward_workspace(int B, int T, int C, int H, int dtype, int algo) {
@@ -276,7 +294,7 @@ int wkv6_forward_noalloc(void *stream, int B, int T, int C, int H, int dtype, un
     for (const void *p : {r, k, v, (const void *)w, (const void *)u, (const void *)state_in, (const void *)y,
                           (const void *)state_out})
         if (!aligned16(p)) return WKV_ERR_ALIGN;
-    if (pick_algo56(WKV_ALGO_CHUNKED, T, C, dtype, flags) != WKV_ALGO_CHUNKED) return WKV_ERR_ALGO;
+    if (pick_algo56(WKV_ALGO_CHUNKED, B * H, T, C, dtype, flags, false) != WKV_ALGO_CHUNKED) return WKV_ERR_ALGO;
     st = check_state_alias(state_in, state_out, B, H, chunked::needs_two_states(B * H, T));
     if (st) return st;
     hipError_t e = chunked::forward_static_launch((hipStream_t)stream, true, (flags & WKV_W_BF16) != 0, B, T, C, H, r, k, v, w,

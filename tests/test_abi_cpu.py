@@ -42,6 +42,29 @@ def test_version_and_messages(L):
         assert L.wkv_strerror(code) not in (b"ok", b"unknown status")
 
 
+@pytest.mark.parametrize("dtype", [0, 2])
+@pytest.mark.parametrize("BH,short,long", [(12, 16, 40), (256, 16, 40), (320, 32, 56), (1024, 40, 64), (2048, 48, 64), (4096, 96, 129)])
+def test_short_sequences_go_token_by_token(L, dtype, BH, short, long):
+    """fp32 and fp16 streams on 256 compute units: lengths a little below and above the measured line, by the workspaces the
+    calls ask for (token by token a forward leaves no checkpoints); a segment count set asks for 64-token steps at any
+    length; an fp16 decay is worked in steps at any length, so a backward's workspace always has room for that."""
+    if torch.cuda.is_available():
+        pytest.skip("the line depends on the device")
+    keep = lambda T, fn=L.wkv6_forward_workspace: fn(1, T, 64 * BH, BH, dtype, 0)
+    back = lambda T: keep(T, L.wkv6_backward_workspace)
+    if BH < 4096:
+        assert keep(short) == 0 and keep(2) == 0
+    assert keep(long) > 0 and keep(129) > 0 and L.wkv6_forward_workspace(1, 2, 64 * BH, BH, 1, 0) > 0
+    assert keep(long, L.wkv5_forward_workspace) == keep(long)
+    assert L.wkv_tune(1, 1) == 0
+    try:
+        assert keep(short) > 0 and back(short) > keep(short)
+        steps = back(short)
+    finally:
+        assert L.wkv_tune(1, 0) == 0
+    assert back(short) == steps if dtype == 2 else back(short) <= steps
+
+
 @pytest.mark.parametrize("BH,steps", [(129, 17), (142, 17), (641, 18), (400, 20), (1, 7), (256, 64)])
 @pytest.mark.parametrize("entry", ["wkv6_forward", "wkv5_forward", "wkv6_forward_noalloc"])
 def test_state_in_place_is_not_refused_by_a_cost_estimate(L, entry, BH, steps):

@@ -768,6 +768,51 @@ def test_f32_blocked(version, dtype, B, H, T, nseg, pps, regime):
         assert (got["gw"].cpu()[hit] == 0).all(), "no gradient where the floor holds"
 
 
+@pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("B,H,T", [(1, 1, 2), (2, 3, 15), (1, 2, 17), (1, 3, 33), (5, 64, 24)])
+def test_f32_short_sequences(version, dtype, B, H, T):
+    """Sequences too short for 64-token steps to pay go token by token, to the bit, in every form of the call; with a segment count
+    set, or an fp16 decay, they are worked in steps."""
+    import rwkv_wkv_hip as W
+    from rwkv_wkv_hip import _lib, configs
+    L = _lib.lib()
+    wl = configs.make(1 if version == 5 else 3, B=B, T=T, C=64 * H, H=H, dtype=dtype, seed=6100 + T)
+    ref = run_oracle56(version, wl)
+    tokens = run_gpu56(version, wl, algo="recurrent")
+    if T <= 24:
+        got = run_gpu56(version, wl)
+        assert all(torch.equal(got[n], tokens[n]) for n in NAMES)
+        g = {n: x.to(dev()) for n, x in wl.tensors.items()}
+        with torch.no_grad():
+            args = [g[n] for n in (("state", "r", "k", "v", "w", "u") if version == 5 else ("r", "k", "v", "w", "u", "state"))]
+            y, s = (W.WKV_5 if version == 5 else W.WKV_6).apply(B, T, 64 * H, H, *args)
+            y2 = (W.RUN_WKV5_CUDA if version == 5 else W.RUN_WKV6STATE_CUDA)(B, T, 64 * H, H, *args)
+        assert torch.equal(y, tokens["y"]) and torch.equal(y2, y) and torch.equal(s, tokens["state"]) and torch.equal(g["state"], s)
+    assert L.wkv_tune(_lib.TUNE_SEGMENTS, 1) == 0
+    try:
+        steps = run_gpu56(version, wl)
+    finally:
+        assert L.wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0
+    compare(steps, ref, 1e-3 if dtype == torch.float32 else 2e-2, "in steps")
+    if version == 6 and dtype == torch.float16:
+        half = _with(wl, w=wl.tensors["w"].half())
+        compare(run_gpu56(6, half), run_oracle56(6, _with(wl, w=half.tensors["w"].float())), 2e-2, "fp16 decay")
+        # the C entry points with an fp16 decay
+        p, B, C = (lambda t: t.data_ptr()), wl.B, 64 * H
+        g = {n: x.to(dev()) for n, x in half.tensors.items()}
+        o = {n: torch.empty_like(g[n]) for n in ("r", "k", "v", "w", "u", "state")}
+        y, s, stream = torch.empty_like(g["r"]), torch.empty_like(g["state"]), torch.cuda.current_stream().cuda_stream
+        ws = torch.empty(L.wkv6_backward_workspace(B, T, C, H, _lib.WKV_F16, 0), dtype=torch.uint8, device=dev())
+        flags, ins = _lib.FLOOR_DECAY | 16, [p(g[n]) for n in ("r", "k", "v", "w", "u", "state")]
+        assert L.wkv6_forward(stream, B, T, C, H, _lib.WKV_F16, flags, 0, *ins, p(y), p(s), p(ws), ws.numel()) == 0
+        assert L.wkv6_backward(stream, B, T, C, H, _lib.WKV_F16, flags | _lib.CHECKPOINTS_VALID, 0, *ins, p(g["dy"]), p(g["dstate"]),
+                               *(p(o[n]) for n in ("r", "k", "v", "w", "u", "state")), p(ws), ws.numel()) == 0
+        torch.cuda.synchronize()
+        compare(dict(y=y, state=s, gr=o["r"], gk=o["k"], gv=o["v"], gw=o["w"], gu=o["u"], gstate=o["state"]),
+                run_oracle56(6, _with(wl, w=half.tensors["w"].float())), 2e-2, "fp16 decay, C entry points")
+
+
 @pytest.mark.parametrize("T,nseg", [(50, 0), (520, 3)])
 def test_f32_blocked_fp16_decay_and_scratch(T, nseg):
     """fp16 raw decay read as it is (its gradient comes back in fp16), and a forward call that keeps no checkpoints: the
