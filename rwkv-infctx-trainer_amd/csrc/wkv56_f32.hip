@@ -27,6 +27,15 @@
 // dL/dlog w_t = A_t - km_t d(km)_t.  The bonus terms come from the scaled copies too: u k_t P = e^{x_t} (u w_t km_t P),
 // u r_t P = e^{-(x_t + log w_t)} (u w_t rm_t P).
 //
+// Non-finite and very large values.  The masked products multiply zeros with what a later (backward: an earlier) token of the
+// block holds, which an infinity or a NaN turns into NaN, and the scaled copies and their products reach 2^61 times the values:
+// a token's past would not stay clean of it, and some results would overflow that fit.  So a step that holds a NaN, an
+// infinity or anything beyond 2^18 (found where it is prepared) is walked token by token by the wavefronts that own the
+// states, in the recurrence's own terms.  Up to that bound no product of the blocked form overflows: 16 tokens x 64 values x
+// 2^(18+18) x 2^(61.2+18) < 2^126.  The check costs 0 to 2 % of a forward; B8 T2048 H40 fp32, forward and backward, without it
+// 722 us (WKV5) and 800 us (WKV6), with it 749 and 774.  What the state holds, an infinity too, is carried from step to step as the
+// recurrence carries it; between time segments it is forgotten once its decay has left 2^-PASS_CUT of it, like anything else.
+//
 // Operand layouts (lane = 16 g + n): A[m = n][k = 4 g' .. ] and B[k][n], where the k of a 16-deep product may be dealt out
 // in any order; taken as k = 4 g + e for the e-th of four instructions, the operand read along its rows is one 16-byte LDS
 // read, the one read along its columns four 4-byte ones, and a result tile (rows 4 g + e, column n) is at once the
@@ -115,6 +124,25 @@ __device__ __forceinline__ float row_sum(const float (*part)[4][8], int tok) {  
     return (p[0][tok & 7] + p[1][tok & 7]) + (p[2][tok & 7] + p[3][tok & 7]);
 }
 
+// the largest absolute value, NaN if there is one (one v_maximum3_f32)
+__device__ __forceinline__ float largest(float m, float a, float b) {
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(a)), fabsf(b));
+}
+constexpr float PLAIN_LIMIT = 262144.f;      // 2^18
+__device__ __forceinline__ void store_plain(int *plain, float m, int lane) {          // m: of the wavefront's eight tokens, per channel
+    const bool any = __builtin_amdgcn_ballot_w64(!(m <= PLAIN_LIMIT)) != 0;
+    if (lane == 0) *plain = any;
+}
+__device__ __forceinline__ int any_plain(const int (&plain)[8]) {
+    const int4 a = *reinterpret_cast<const int4 *>(&plain[0]), b = *reinterpret_cast<const int4 *>(&plain[4]);
+    return (a.x | a.y) | (a.z | a.w) | (b.x | b.y) | (b.z | b.w);
+}
+__device__ __forceinline__ bool rarely(int x) { return __builtin_expect(__builtin_amdgcn_readfirstlane(x) != 0, 0); }      // the same in all lanes
+__device__ __forceinline__ float over_groups(float x) {          // over the four lane groups, in every lane
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+}
+
 // ------------------------------------------------------------------------------------------------------------ forward --
 // Twelve wavefronts, one barrier per 64-token step.  Wavefronts 0-3 walk the state (values 16 w .. +15, all keys) over
 // the step's four blocks.  Wavefronts 4-11 meanwhile build the masked matrices of the step and prepare half a block each
@@ -126,6 +154,7 @@ struct FwdTiles {
     float rm[SB * LD], km[SB * LD], v[SB * LD];
     float em[4][HEAD], eb[4][HEAD];      // e^{m}, e^{b-m} per block and key
     float rho[8][4][8];                  // r . (u o k) per token, in parts
+    alignas(16) int plain[8];            // half a block each: the step is walked token by token
 };
 struct FwdShared {
     FwdTiles step[2];
@@ -186,7 +215,7 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
         }
     };
     auto prepare = [&](int sb, FwdTiles &sm) __attribute__((always_inline)) {
-        float lw[8], x[8], p[8];
+        float lw[8], x[8], p[8], m = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++)
             lw[i] = sb * SB + tok0 + i >= Tlen ? 0.f : PER_TOKEN_W ? log2_decay(to_float(tw[i]), floor_decay) : l_const;
@@ -195,14 +224,17 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const bool in = sb * SB + tok0 + i < Tlen;
-            const float rf = in ? to_float(tr[i]) : 0.f, kf = in ? to_float(tk[i]) : 0.f;
+            const float rf = in ? to_float(tr[i]) : 0.f, kf = in ? to_float(tk[i]) : 0.f, vf = in ? to_float(tv[i]) : 0.f;
             const int o = (tok0 + i) * LD + lane;
             sm.rm[o] = rf * exp2_fast(x[i]);
             sm.km[o] = kf * exp2_fast(-(x[i] + lw[i]));
-            sm.v[o] = in ? to_float(tv[i]) : 0.f;
+            sm.v[o] = vf;
             p[i] = rf * uf * kf;
+            m = largest(m, rf, kf);
+            m = largest(m, vf, PER_TOKEN_W ? lw[i] : vf);
         }
         store_row_sums(p, sm.rho[2 * q + hf], lane);
+        store_plain(&sm.plain[2 * q + hf], m, lane);
     };
     // (the two roles have loops of their own: in a common one the compiler waits, in either, for what the other may have
     // outstanding)
@@ -238,7 +270,33 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
     }
     const Out yo = out_of(y, (size_t)Tlen * C - h * HEAD);
     const uint32_t y_lane = (uint32_t)n * C + 16 * q + 4 * g;
+    // a step token by token, from memory: the lane's sixteen keys of its value, added over the lane groups
+    auto walk_tokens = [&](int sb) {
+        const int t1 = min((sb + 1) * SB, Tlen);
+#pragma unroll 1
+        for (int t = sb * SB; t < t1; t++) {
+            const size_t row = (size_t)t * C;
+            const float vt = to_float(v[row + 16 * q + n]);
+            float acc = 0.f, rho = 0.f;
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                float r4[4], k4[4], w4[4], u4[4];
+                const int key = 16 * kk + 4 * g;
+                load4(r + row + key, r4); load4(k + row + key, k4); load4(wraw + (PER_TOKEN_W ? row : (size_t)h * HEAD) + key, w4); load4(u + h * HEAD + key, u4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    rho = fmaf(r4[e] * u4[e], k4[e], rho);
+                    acc = fmaf(r4[e], S[kk][e], acc);
+                    S[kk][e] = fmaf(k4[e], vt, exp2_fast(log2_decay(w4[e], floor_decay)) * S[kk][e]);
+                }
+            }
+            acc = over_groups(acc);
+            rho = over_groups(rho);
+            if (y && g == 0) put<T>(yo, t, C, 16 * q + n, fmaf(vt, rho, acc));
+        }
+    };
     lds_barrier();
+    int plain = any_plain(sh.step[0].plain);
     for (int sb = sb0; sb < sb1; sb++) {
         const int par = (sb - sb0) & 1;
         const FwdTiles &sm = sh.step[par];
@@ -246,6 +304,12 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
             f4 *cp = reinterpret_cast<f4 *>(ckpt + ((size_t)bh * (nsb + 1) + sb) * HEAD * HEAD) + q * 256 + lane;
 #pragma unroll
             for (int kk = 0; kk < 4; kk++) cp[64 * kk] = S[kk];
+        }
+        if (rarely(plain)) {
+            walk_tokens(sb);
+            lds_barrier();
+            plain = any_plain(sh.step[par ^ 1].plain);
+            continue;
         }
         f4 vv[4], yy[4];
 #pragma unroll
@@ -262,6 +326,7 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
             yy[blk] = ya + yb;
         }
         lds_barrier();
+        plain = any_plain(sh.step[par ^ 1].plain);          // the next step's (read here, it costs the walk no wait)
         if (y) {
 #pragma unroll
             for (int blk = 0; blk < 4; blk++)      // y^T: values 16q+4g .. +3 of token n
@@ -395,6 +460,7 @@ struct BwdTiles {
     f4 pm[4][64], pt[4][64], at[4][64];      // P (t > s): rows t, columns s;  P^T (s < t): rows s, columns t;  rm km^T (t >= s): rows t, columns s
     float dr[SB * LD], dk[SB * LD];          // d(rm), d(km)
     float rho[8][4][8], pdiag[SB], sums[8][HEAD];      // sums: of rm d(rm) - km d(km) over half a block
+    alignas(16) int plain[8];                // half a block each: the step is walked token by token
 };
 
 template <class T, class W, bool PER_TOKEN_W>
@@ -462,7 +528,7 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
         }
     };
     auto prepare = [&](int sb, int lane) __attribute__((always_inline)) {
-        float lw[8], x[8], p[8];
+        float lw[8], x[8], p[8], m = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++)
             lw[i] = sb * SB + tok0 + i >= Tlen ? 0.f : PER_TOKEN_W ? log2_decay(to_float(tw[i]), floor_decay) : l_const;
@@ -472,21 +538,43 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
         for (int i = 0; i < 8; i++) {
             const bool in = sb * SB + tok0 + i < Tlen;
             const float rf = in ? to_float(tr[i]) : 0.f, kf = in ? to_float(tk[i]) : 0.f;
+            const float vf = in ? to_float(tv[i]) : 0.f, gf = in ? to_float(tg[i]) : 0.f;
             const int o = (tok0 + i) * LD + lane;
             sm.rm[o] = rf * exp2_fast(x[i]);
             sm.km[o] = kf * exp2_fast(-(x[i] + lw[i]));
-            sm.v[o] = in ? to_float(tv[i]) : 0.f;
-            sm.gy[o] = in ? to_float(tg[i]) : 0.f;
+            sm.v[o] = vf;
+            sm.gy[o] = gf;
             sm.x[o] = x[i];
             sm.lw[o] = lw[i];
             p[i] = rf * uf * kf;
+            m = largest(m, rf, kf);
+            m = largest(m, vf, gf);
+            if (PER_TOKEN_W && (i & 1)) m = largest(m, lw[i - 1], lw[i]);          // (at most 8; for its NaN)
         }
         store_row_sums(p, sm.rho[2 * q + hf], lane);
+        store_plain(&sm.plain[2 * q + hf], m, lane);
+    };
+    // For the walk token by token: r, k as they are, no exponents.  (Both kinds of wavefronts come here after work on the step
+    // that is then done again, so that the flags are there by the time they are looked at; what others still read of
+    // the tables meanwhile is of no use to them.)
+    auto prepare_plain = [&](int sb, int lane) {
+        fetch(sb, lane);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const bool in = sb * SB + tok0 + i < Tlen;
+            const int o = (tok0 + i) * LD + lane;
+            sm.rm[o] = in ? to_float(tr[i]) : 0.f;
+            sm.km[o] = in ? to_float(tk[i]) : 0.f;
+            sm.x[o] = 0.f;
+        }
+        fetch(max(sb - 1, sb0), lane);
+        lds_barrier();
     };
     const size_t left = (size_t)Tlen * C - h * HEAD;
     const Out gro = out_of(gr, left), gko = out_of(gk, left), gwo = out_of(PER_TOKEN_W ? gw_tok : nullptr, PER_TOKEN_W ? left : 0);
-    // dL/dlog w_t = A_t - km_t d(km)_t, A_t the running sum after token t
-    auto finish = [&](int sb, int lane) __attribute__((always_inline)) {
+    // dL/dlog w_t = A_t - km_t d(km)_t, A_t the running sum after token t.  plain: after a walk token by token, whose r, k, d(rm)
+    // and d(km) carry no factor
+    auto finish = [&](int sb, int lane, bool plain) __attribute__((always_inline)) {
         float rm[8], km[8], dr[8], dk[8], z[8], c[8], sum = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
@@ -508,12 +596,12 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
 #pragma unroll
         for (int i = 7; i >= 0; i--) {
             const int o = (tok0 + i) * LD + lane;
-            const float x = sm.x[o], lw = sm.lw[o], bonus = exp2_fast(lw) * sm.pdiag[tok0 + i], D = run - z[i];
+            const float x = sm.x[o], lw = sm.lw[o], ls = plain ? 0.f : lw, bonus = exp2_fast(ls) * sm.pdiag[tok0 + i], D = run - z[i];
             run += c[i];
             gu_acc = fmaf(rm[i] * km[i], bonus, gu_acc);
             const int t = sb * SB + tok0 + i;
             put<T>(gro, t, C, lane, exp2_fast(x) * fmaf(uf * km[i], bonus, dr[i]));
-            put<T>(gko, t, C, lane, exp2_fast(-(x + lw)) * fmaf(uf * rm[i], bonus, dk[i]));
+            put<T>(gko, t, C, lane, exp2_fast(-(x + ls)) * fmaf(uf * rm[i], bonus, dk[i]));
             if (PER_TOKEN_W) put<W>(gwo, t, C, lane, (floor_decay && lw <= LOG2_W_FLOOR) ? 0.f : D * (lw * LN2));
             else gw_acc += t < Tlen ? D : 0.f;
         }
@@ -535,6 +623,7 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
             WKV_F32_LANE
             prepare(sb, lane);
             lds_barrier();
+            const int plain = any_plain(sm.plain);
             {       // the masked matrices of block q
                 const int row = 16 * q + n;
                 f4 p = zero4(), pT = zero4(), at = zero4();
@@ -557,6 +646,30 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
                 sm.pm[q][lane] = p; sm.pt[q][lane] = pT; sm.at[q][lane] = at;
             }
             fetch(max(sb - 1, sb0), lane);          // before this step's stores, see Out
+            if (rarely(plain)) {
+                prepare_plain(sb, lane);
+#pragma unroll 1
+                for (int i = SB - 1; i >= 0; i--) {
+                    const float gt = sm.gy[i * LD + own];
+                    float a = 0.f;
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk++) {
+                        const f4 k4 = along(sm.km, i, 16 * kk + 4 * g), r4 = along(sm.rm, i, 16 * kk + 4 * g), l4 = along(sm.lw, i, 16 * kk + 4 * g);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            a = fmaf(k4[e], G[kk][e], a);
+                            G[kk][e] = fmaf(r4[e], gt, exp2_fast(l4[e]) * G[kk][e]);
+                        }
+                    }
+                    a = over_groups(a);
+                    if (g == 0) put<T>(gvo, sb * SB + i, C, own, fmaf(row_sum(sm.rho, i), gt, a));
+                }
+                lds_barrier();
+                lds_barrier();
+                finish(sb, lane, true);
+                lds_barrier();
+                continue;
+            }
             f4 gf[4], gvv[4];
 #pragma unroll
             for (int blk = 3; blk >= 0; blk--) {
@@ -576,7 +689,7 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
             for (int blk = 0; blk < 4; blk++)        // gv^T: values 16q+4g .. +3 of token n
                 put4<T>(gvo, sb * SB + 16 * blk, C, (uint32_t)n * C + 16 * q + 4 * g, mma(gf[blk], sm.at[blk][lane], gvv[blk]));
             lds_barrier();
-            finish(sb, lane);
+            finish(sb, lane, false);
             lds_barrier();
         }
     } else {
@@ -595,6 +708,7 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
             WKV_F32_LANE
             prepare(sb, lane);
             lds_barrier();
+            const int plain = any_plain(sm.plain);
             f4 q1[4], q4[4];                         // rows: tokens of the block, column key own
 #pragma unroll
             for (int blk = 0; blk < 4; blk++) {
@@ -612,6 +726,48 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
 #pragma unroll
                     for (int kk = 0; kk < 4; kk++) S[kk] = mma(across(sm.v, 16 * blk + 4 * g, 16 * kk + n), kf, S[kk]) * eb;
                 }
+            }
+            if (rarely(plain)) {
+                fetch_state(sb, lane);
+                prepare_plain(sb, lane);
+#pragma unroll 1
+                for (int i = 0; i < SB; i++) {
+                    const float kt = sm.km[i * LD + own], wt = exp2_fast(sm.lw[i * LD + own]);
+                    float a = 0.f;
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk++) {
+                        const f4 g4 = along(sm.gy, i, 16 * kk + 4 * g), v4 = along(sm.v, i, 16 * kk + 4 * g);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            a = fmaf(S[kk][e], g4[e], a);
+                            S[kk][e] = fmaf(kt, v4[e], wt * S[kk][e]);
+                        }
+                    }
+                    a = over_groups(a);
+                    if (g == 0) sm.dr[i * LD + own] = a;
+                }
+                fetch_state(max(sb - 1, sb0), lane);
+#pragma unroll 1
+                for (int i = SB - 1; i >= 0; i--) {
+                    const float rt = sm.rm[i * LD + own], wt = exp2_fast(sm.lw[i * LD + own]);
+                    float a = 0.f;
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk++) {
+                        const f4 g4 = along(sm.gy, i, 16 * kk + 4 * g), v4 = along(sm.v, i, 16 * kk + 4 * g);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            a = fmaf(G[kk][e], v4[e], a);
+                            G[kk][e] = fmaf(rt, g4[e], wt * G[kk][e]);
+                        }
+                    }
+                    a = over_groups(a);
+                    if (g == 0) sm.dk[i * LD + own] = a;
+                }
+                lds_barrier();
+                lds_barrier();
+                finish(sb, lane, true);
+                lds_barrier();
+                continue;
             }
             fetch(max(sb - 1, sb0), lane);           // before this step's stores, see Out
             fetch_state(max(sb - 1, sb0), lane);
@@ -641,7 +797,7 @@ __global__ __launch_bounds__(NT) void backward_f32(int bh0, int Tlen, int C, int
                 }
             }
             lds_barrier();
-            finish(sb, lane);
+            finish(sb, lane, false);
             lds_barrier();
         }
         if (gs_in && seg == 0) {

@@ -770,6 +770,62 @@ def test_f32_blocked(version, dtype, B, H, T, nseg, pps, regime):
 
 @pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("name", ["r", "k", "v", "w", "dy"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_f32_blocked_non_finite_values_stay_where_they_belong(version, dtype, name, value):
+    """An infinity or a NaN in one token: every element of every result is finite where the token-by-token kernels leave it
+    finite (a token's outputs do not depend on later ones, nor a token's gk, gv on earlier ones), and is what they give there:
+    within the tolerances of the tests without such values."""
+    from rwkv_wkv_hip import _lib, configs
+    if name == "w" and version == 5:
+        pytest.skip("one decay for all tokens")
+    L = _lib.lib()
+    B, T, H = 2, 200, 2
+    wl = configs.make(1 if version == 5 else 3, B=B, T=T, C=64 * H, H=H, dtype=dtype, seed=6200)
+    for b, t, c in ((0, 75, 70), (0, 150, 3), (1, 8, 100)):          # the end, the middle and the half of a block of 16
+        wl.tensors[name][b, t, c] = value
+    assert L.wkv_tune(_lib.TUNE_SEGMENTS, 1) == 0
+    try:
+        got = run_gpu56(version, wl)
+    finally:
+        assert L.wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0
+    want = run_gpu56(version, wl, algo="recurrent")
+    rt = 1e-3 if dtype == torch.float32 else 2e-2
+    for n in NAMES:
+        fine = torch.isfinite(want[n])
+        assert torch.equal(torch.isfinite(got[n]), fine), n
+        assert_close(torch.where(fine, got[n], 0), torch.where(fine, want[n], 0), rt, n)
+    if name in "rkv":
+        assert not torch.isfinite(want["y"]).all() and torch.isfinite(want["y"][0, :75]).all()
+
+
+@pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("name,size", [("r", 1e30), ("k", 1e25), ("v", 1e30), ("dy", 1e30), ("k", 3e5)])
+def test_f32_blocked_very_large_values(version, name, size):
+    """fp32 values whose scaled copies, or products with them, do not fit 32 bits under decays at the floor: the results that fit are
+    those of the token-by-token kernels, per token and head within 1e-4 (sums of 64 and of at most 200 terms in another order; the
+    decay gradient is a difference of much larger sums and left out)."""
+    from rwkv_wkv_hip import _lib, configs
+    L = _lib.lib()
+    B, T, H = 1, 200, 2
+    wl = configs.make(1 if version == 5 else 3, B=B, T=T, C=64 * H, H=H, dtype=torch.float32, seed=6300)
+    wl.tensors["w"][..., ::3] = 2.5
+    wl.tensors[name][0, 70:74] *= size
+    wl.tensors[name][0, 120] *= size
+    assert L.wkv_tune(_lib.TUNE_SEGMENTS, 1) == 0
+    try:
+        got = run_gpu56(version, wl)
+    finally:
+        assert L.wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0
+    want = run_gpu56(version, wl, algo="recurrent")
+    for n in ("y", "gr", "gk", "gv"):
+        a, b = (x[n].double().view(T, H, 64) for x in (got, want))
+        assert bool(torch.isfinite(b).all()) and bool(torch.isfinite(a).all()), n
+        assert bool(((a - b).norm(dim=2) <= 1e-4 * b.norm(dim=2)).all()), n
+
+
+@pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("B,H,T", [(1, 1, 2), (2, 3, 15), (1, 2, 17), (1, 3, 33), (5, 64, 24)])
 def test_f32_short_sequences(version, dtype, B, H, T):
     """Sequences too short for 64-token steps to pay go token by token, to the bit, in every form of the call; with a segment count
