@@ -273,10 +273,10 @@ def test_timemix_forward_on_the_kernels_bf16_module(version):
     assert_close(s_got, s_ref, 6e-2, f"timemix bf16 v{version} state")
 
 
-@pytest.mark.parametrize("rows", [3, 16, 17, 32, 33, 64])
-@pytest.mark.parametrize("n,K", [(256, 64), (1024, 192), (4128, 192), (8224, 2112), (16416, 64)])
+@pytest.mark.parametrize("rows", [1, 2, 3, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,K", [(256, 64), (1024, 192), (2080, 320), (4128, 192), (8224, 2112), (16416, 64)])
 def test_products_of_a_few_rows(rows, n, K):
-    """Each shape of the kernel: 16 and 32 columns, four and eight wavefronts, one to four tiles of rows, contractions that
+    """Each shape of the kernel: 8, 16 and 32 columns, four and eight wavefronts, one to four tiles of rows, contractions that
     end inside a segment; two products in one launch, one mixed and squared, one (n + 32 columns) as it is.  Against 64 bits:
     the mixed row and the result round to bf16 (2^-9 each, the square doubles it), the sums to 32 bits."""
     import ctypes
@@ -300,11 +300,49 @@ def test_products_of_a_few_rows(rows, n, K):
         assert bool((err <= tol * want.abs() + 2 ** -9 * want.pow(2).mean().sqrt()).all()), err.max().item()
 
 
+@pytest.mark.parametrize("rows", [1, 2, 3, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,K", [(1024, 192), (4096, 2048), (8192, 64)])
+def test_products_of_a_few_rows_of_every_kind(rows, n, K):
+    """Every kind of job in one launch, in the shapes that each number of workgroups gives it: weights kept [k][n] (mixed and
+    not; the sum of their parts), a mix with 1 - mix, and a product behind its gate.  Against 64 bits: an fp32 sum of K terms is
+    off by at most K 2^-24 of the sum of their sizes, one element of the mixed row may round to the neighbouring bf16 (2^-7), the result
+    rounds to bf16 before and after the gate (eight significant bits: 2^-8 each; the gate's own error, 2^-20, is lost in them)."""
+    import ctypes
+    from rwkv_wkv_hip import _lib
+
+    class Product(ctypes.Structure):
+        _fields_ = [(f, ctypes.c_void_p) for f in ("w", "x", "shift", "mix", "mul", "out")] + [(f, ctypes.c_int) for f in ("n", "k_major", "lerp", "act")]
+    g = torch.Generator().manual_seed(rows + n)
+    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
+    x, shift, mix, mul = r(rows, K), r(rows, K), torch.rand(K, generator=g).bfloat16().cuda(), r(rows, n)
+    wa, wb, wc, wd = r(K, 160), r(K, 64), r(n, K), r(n, K)
+    oa, ob = (torch.full((8, rows, m), 9.0, device="cuda") for m in (160, 64))
+    oc, od = (torch.full((rows, n), 9.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    p = lambda t: t.data_ptr()
+    jobs = (Product * 4)(Product(p(wa), p(x), p(shift), p(mix), None, p(oa), 160, 1, 0, 0), Product(p(wb), p(x), None, None, None, p(ob), 64, 1, 0, 0),
+                         Product(p(wc), p(x), p(shift), p(mix), None, p(oc), n, 0, 1, 0), Product(p(wd), p(x), None, None, p(mul), p(od), n, 0, 0, 2))
+    assert _lib.lib().wkv_rows_products(torch.cuda.current_stream().cuda_stream, rows, K, 4, jobs) == 0
+    torch.cuda.synchronize()
+    d = lambda t: t.double()
+    mixed = (d(x) + (d(shift) - d(x)) * d(mix)).bfloat16()
+    lerped = (d(x) + (d(shift) - d(x)) * (1 - d(mix))).bfloat16()
+    for name, got, a, w, rounding in (("k major, mixed", d(oa).sum(0), mixed, wa, 0), ("k major", d(ob).sum(0), x, wb, 0), ("lerp", d(oc), lerped, wc.t(), 2 ** -8),
+                                      ("gated", d(od), x, wd.t(), 2 * 2 ** -8)):
+        want, sizes = d(a) @ d(w), d(a).abs() @ d(w).abs()
+        bound = K * 2 ** -24 * sizes + (2 ** -7 * d(a).abs().amax(1, keepdim=True) * d(w).abs().amax(0) if a is not x else 0)
+        if name == "gated":
+            want, bound = torch.sigmoid(d(mul)) * want, torch.sigmoid(d(mul)) * bound
+        err = (got - want).abs() - bound - 1.01 * rounding * want.abs()
+        assert bool((err <= 0).all()), (name, err.max().item())
+
+
 @pytest.mark.parametrize("version", [5, 6])
-@pytest.mark.parametrize("B,H,ffn", [(1, 1, 64), (3, 2, 448), (16, 1, 192), (17, 3, 640), (33, 2, 256), (64, 9, 2016), (65, 1, 128)])
+@pytest.mark.parametrize("B,H,ffn", [(1, 1, 64), (3, 2, 448), (16, 1, 192), (17, 3, 640), (33, 2, 256), (64, 9, 2016), (65, 1, 128),
+                                     (1, 32, 7168), (20, 40, 8960)])
 def test_layer_of_single_tokens(version, B, H, ffn):
     """A serving loop's layer (one token per sequence, no autograd, bf16): row counts at the edges of the 16-row tiles, widths
-    of fewer and of more 64-deep chunks than a workgroup has wavefronts; 65 rows and ffn = 2016 take the general way.
+    of fewer and of more 64-deep chunks than a workgroup has wavefronts, and the widths of models in use, whose products take other
+    shapes; 65 rows and ffn = 2016 take the general way.
     Against the fp32 modules on the same rounded parameters.  Six bf16 roundings (2^-9 each, added in squares: 4.8e-3) lie
     between input and output: 1e-2 in norm over all rows.  In one row the operator's sum over 64 keys and ln_x's mean can
     cancel, which divides by what is left: among 64 rows some lose a digit, 4.8e-2 (the general way's worst row: 2.1e-2)."""
@@ -460,6 +498,104 @@ def test_layer_native_matches_the_steps(version, T, frozen):
             if ref[n] is not None:
                 assert got[n].dtype == ref[n].dtype and got[n].shape == ref[n].shape, n
                 assert (got[n] - ref[n]).float().norm() <= 6 * 2 ** -8 * ref[n].float().norm(), n
+
+
+def _layer(version, C, H):
+    from rwkv_wkv_hip import blocks as K
+    tm, cm = ((TimeMix5 if version == 5 else TimeMix6)(C, H, seed=8).cuda().bfloat16(),
+              (ChannelMix5 if version == 5 else ChannelMix6)(C, 4 * C, seed=9).cuda().bfloat16())
+    return tm, cm, *((K.timemix5_forward, K.channelmix5_forward) if version == 5 else (K.timemix6_forward, K.channelmix6_forward))
+
+
+@pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("T", [1, 5])
+@pytest.mark.parametrize("grad", [False, True])
+def test_which_calls_the_native_layer_answers(version, T, grad):
+    """A plain bf16 module is answered by the native host side; whatever is not plain gets None from it (and so goes the
+    general way)."""
+    from rwkv_wkv_hip import _lib, ops
+    B, H = 2, 2
+    C = 64 * H
+    x, shift, state = torch.randn(B, T, C).cuda().bfloat16(), torch.randn(B, C).cuda().bfloat16(), torch.randn(B, H, 64, 64).cuda()
+
+    def answered(change=lambda tm, cm: None, x=x, shift=shift, state=state):
+        tm, cm, _, _ = _layer(version, C, H)
+        undo = change(tm, cm)
+        with torch.set_grad_enabled(grad):
+            got = _lib.host().timemix(version, ops._algo, tm, x, (shift, state)), _lib.host().channelmix(version, cm, x, shift)
+        if undo is not None:
+            undo.remove()
+        assert (got[0] is None) == (got[1] is None)
+        return got[0] is not None
+
+    def replace(make):
+        def change(tm, cm):
+            for m in (tm, cm):
+                new = make(m.key)
+                new.weight = m.key.weight
+                m.key = new.cuda().bfloat16()
+        return change
+
+    class Own(torch.nn.Linear):
+        pass
+    hook = lambda *a: None
+    assert answered()
+    assert not answered(lambda tm, cm: [m.key.register_forward_hook(hook) for m in (tm, cm)] and None)
+    assert not answered(lambda tm, cm: [m.value.register_forward_pre_hook(hook) for m in (tm, cm)] and None)
+    assert not answered(lambda tm, cm: [m.receptance.register_full_backward_hook(hook) for m in (tm, cm)] and None)
+    assert not answered(lambda tm, cm: torch.nn.modules.module.register_module_forward_hook(hook))
+    assert not answered(lambda tm, cm: [setattr(m.key, "forward", hook) for m in (tm, cm)] and None)
+    assert not answered(replace(lambda l: torch.nn.Linear(l.in_features, l.out_features, bias=True)))
+    assert not answered(replace(lambda l: Own(l.in_features, l.out_features, bias=False)))
+    assert not answered(lambda tm, cm: [m.float() for m in (tm, cm)] and None)
+    assert not answered(x=x.float())
+    assert not answered(x=torch.empty(B, C, T, device="cuda", dtype=x.dtype).transpose(1, 2)) or T == 1
+    assert not answered(x=torch.empty(B * T * C + 1, device="cuda", dtype=x.dtype)[1:].view(B, T, C))
+    assert not answered(shift=shift.float())
+    assert not answered(shift=shift.view(1, B, C))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not answered()
+
+
+@pytest.mark.parametrize("version", [5, 6])
+@pytest.mark.parametrize("way", ["saved on the host", "recomputed", "autocast"])
+def test_layer_native_under_hooks_and_autocast(version, way):
+    """What a layer saves for its backward may be taken away in between (packed by saved-tensor hooks, dropped and recomputed by
+    activation checkpointing): the same bits.  Under autocast a layer goes step by step: as the same steps without."""
+    from torch.utils.checkpoint import checkpoint
+    B, T, H = 2, 70, 2
+    C = 64 * H
+    tm, cm, timemix, channelmix = _layer(version, C, H)
+    g = _g(21)
+    n = lambda *shape: torch.randn(*shape, generator=g).cuda()
+    x, shift, shift2, state, gy, gs = n(B, T, C).bfloat16(), n(B, C).bfloat16(), n(B, C).bfloat16(), n(B, H, 64, 64), n(B, T, C).bfloat16(), n(B, H, 64, 64)
+
+    def run(how):
+        leaves = [t.clone().requires_grad_(True) for t in (x, shift, shift2, state)]
+        wrt = [*leaves, *tm.parameters(), *cm.parameters()]
+
+        def layer(x, shift, shift2, state):
+            a, (_, s) = timemix(tm, x, (shift, state))
+            return channelmix(cm, a, shift2)[0], s
+        if how == "recomputed":
+            out = checkpoint(layer, *leaves, use_reentrant=False)
+        elif how == "saved on the host":
+            with torch.autograd.graph.save_on_cpu():
+                out = layer(*leaves)
+        elif how == "autocast":
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                out = layer(*leaves)
+        else:
+            out = layer(*leaves)
+        return [*out, *torch.autograd.grad(out, wrt, [gy, gs])]
+    if way == "autocast":
+        got = run(way)
+        for m in (tm, cm):
+            m.key.register_forward_hook(lambda *a: None)
+    else:
+        got = run(way)
+    for a, b in zip(got, run("plain")):
+        assert a.dtype == b.dtype and torch.equal(a, b)
 
 
 @pytest.mark.parametrize("version", [5, 6])
