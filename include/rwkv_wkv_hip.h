@@ -8,8 +8,8 @@
  *
  * Layouts (all contiguous, row-major):
  *   r, k, v, y, gy, gr, gk, gv   (B, T, C) in `dtype`          C = H * 64
- *   w (WKV6), gw (WKV6)          (B, T, C) fp32 (bf16 with WKV_W_BF16), RAW decay
- *                                parameter: the decay applied is exp(-exp(w))
+ *   w (WKV6), gw (WKV6)          (B, T, C) fp32 (bf16 with WKV_W_BF16, fp16 with WKV_W_F16), RAW
+ *                                decay parameter: the decay applied is exp(-exp(w))
  *   w (WKV5), gw (WKV5), u, gu   (H, 64)   fp32 (gw, gu summed over batch and time)
  *   state                        (B, H, 64, 64) fp32, [key index][value index]
  *   WKV4: time_decay, time_first (C) fp32;  state (B, C, 3) fp32 = (aa, bb, pp)
@@ -89,7 +89,7 @@ int wkv_init(void);
  * on it). */
 #define WKV_TUNE_SEGMENTS 1
 /* WKV_TUNE_PIECE_STEPS: the summary pass of the time split cuts every segment into pieces of this many 64-token
- * steps (one workgroup and one 16 KiB summary per piece); 0 = choose from the shape (default).  Same rules as above. */
+ * steps (one workgroup and one 16.25 KiB summary per piece); 0 = choose from the shape (default).  Same rules as above. */
 #define WKV_TUNE_PIECE_STEPS 2
 int wkv_tune(int key, int value);
 
@@ -145,8 +145,9 @@ int wkv6_decode(void *stream, int B, int C, int H, int dtype, int w_dtype, const
  * arguments and results as wkv6_forward with the chunked algorithm (bf16 r/k/v/y and WKV_FLOOR_DECAY required,
  * else WKV_ERR_ALGO) and no state checkpoints kept; the scratch memory of the time-parallel split (the piece
  * summaries) is a 16 MiB array inside the library, one per GPU, held until the process ends.  The call allocates
- * nothing and frees nothing.  Shapes whose summaries exceed the array (B*H*segments*pieces*16640 bytes > 16 MiB,
- * e.g. B*H above about 120 at T = 4096) are rejected with WKV_ERR_WORKSPACE.  All calls on one GPU share that
+ * nothing and frees nothing.  A sequence is cut into as many segments and pieces as the array has room for summaries
+ * (B*H*segments*pieces*16640 bytes <= 16 MiB; from B*H about 500 on none is cut); a segment count set by
+ * WKV_TUNE_SEGMENTS whose summaries exceed it is rejected with WKV_ERR_WORKSPACE.  All calls on one GPU share that
  * GPU's array: two calls that overlap in time on the same GPU (different streams) race on it. */
 #define WKV_NOALLOC_SCRATCH_BYTES (16u << 20)
 int wkv6_forward_noalloc(void *stream, int B, int T, int C, int H, int dtype, unsigned flags,

@@ -54,16 +54,16 @@ __device__ __forceinline__ s8 mixed(s8 x, s8 xx, s8 c, int lerp) {
     return __builtin_bit_cast(s8, p);
 }
 
-// A workgroup per 16 columns; its wavefronts share the contraction and meet in LDS.  The weights are the A operand of the
-// MFMAs (their columns are the rows there), the rows of x the B operand: lane (kg = lane/16, n = lane%16) supplies
-// weight row n and x row n, eight consecutive k each.
+// A workgroup per TN columns (8, 16 or 32); its wavefronts share the contraction and meet in LDS.  The weights are the A
+// operand of the MFMAs (their columns are the rows there), the rows of x the B operand: lane (kg = lane/16, n = lane%16)
+// supplies weight row n and x row n, eight consecutive k each.
 //
 // Bound by the weights, so by how they are fetched.  Read in the operand's own layout (16 rows x 64 bytes an instruction)
-// they come at 3.4 TB/s; read along the rows, 512 bytes each of two, at 5.  So a wavefront takes 16 rows x 256 k at a time
-// that way into registers (two such segments in flight, used in turn) and turns them in LDS that belongs to it alone;
-// the same for the rows of x, of which only those that exist are read, and mixed on the way.
+// a layer's weights come at 3.4 TB/s; read along the rows, at up to 4.  So a wavefront takes TN rows x SEG = 4096 / TN k
+// at a time that way into registers (two such segments in flight, used in turn, where XL leaves the registers) and turns them in
+// LDS that belongs to it alone; the same for the rows of x, of which only those that exist are read, and mixed on the way.
 //
-// TN columns and XL fetches of x, each fetch 512 elements: two rows of a segment of 256 k, one of 512, or four of 128.
+// XL fetches of x, each 512 elements: one row of a segment of 512 k (TN 8), two of 256 (TN 16) or four of 128 (TN 32).
 template <int TN, int XL> struct Shape {
     static constexpr int SEG = 4096 / TN, LD = SEG + 8, PER = TN / 8;     // k of a segment, padded row in LDS, rows per fetch
     static constexpr int XROWS = PER * XL, MT = (XROWS + 15) / 16, NT = (TN + 15) / 16;      // MFMA tiles of rows, of columns

@@ -36,8 +36,8 @@
 //
 // Time-parallel split: a sequence is cut into segments that run as separate
 // workgroups; a light pass leaves each piece's effect on a state handed in
-// (S_out = decay o S_in + delta), a small kernel chains the summaries into the state
-// at the start of every segment.  Backward does the same with the state gradient.
+// (S_out = decay o S_in + delta), and every segment's workgroup chains the summaries
+// before it into its first state.  Backward does the same with the state gradient.
 #include "common.h"
 #include <cstddef>
 #include <type_traits>

@@ -1,5 +1,6 @@
-// WKV5 / WKV6 in blocked form with fp32 products: fp32 and fp16 streams, sequences of two tokens or more with the decay
-// floor (wkv56_chunked.hip is the same for bf16 streams, whose operands it splits into bf16 parts).
+// WKV5 / WKV6 in blocked form with fp32 products: fp32 and fp16 streams with the decay floor, sequences long enough for
+// 64-token steps to pay (steps_pay in api.hip; wkv56_chunked.hip is the same for bf16 streams, whose operands it splits
+// into bf16 parts).
 //
 // The token-by-token kernels (wkv56_recurrent.hip) walk the tokens one after another at 4096 multiply-adds a head and
 // token forward, four times that backward, on the vector pipe: B8 T4096 H40 fp32 4.05 ms forward and backward, and a

@@ -274,7 +274,7 @@ class L2Wrap(torch.autograd.Function):
 
 
 # ---- block forwards on these kernels -------------------------------------------------------------------------------
-# A plain bf16 module is run by the native host side (csrc/host_layers.h: each half of a layer one autograd node, single
+# A plain bf16 module is run by the native host side (csrc/host_layers.h: each half of a layer two autograd nodes, single
 # tokens without autograd on kernels of their own); it answers None for every other call, and the code below does the same
 # step by step.
 def _native_timemix(version, self, x, last_state):

@@ -310,8 +310,9 @@ class WKV_5:
 
 class WKV_6:
     """WKV6: per-token decay.  ``WKV_6.apply(B, T, C, H, r, k, v, w, u, s) -> (y, new_state)`` with r,k,v (B,T,C);
-    w (B,T,C) raw (any float dtype, used in fp32; a bf16 w is read as it is by the blocked algorithm and its
-    gradient comes back in bf16, as in the reference, RWKV-v6/src/module/TimeMix.py:50,90); u (H,64);
+    w (B,T,C) raw (any float dtype, used in fp32; a bf16 or fp16 w of the streams' type is read as it is by the blocked
+    algorithms and by a single token without a backward; its gradient comes back in its type, as in the reference,
+    RWKV-v6/src/module/TimeMix.py:50,90); u (H,64);
     s (B,H,64,64) [key][value]."""
 
     @staticmethod
