@@ -420,7 +420,10 @@ __global__ __launch_bounds__(64 * (1 + V4_YW) * V4_GROUPS) void v4_forward(int B
 constexpr int RB = 4;
 struct V4Replay { float ys[CK][64], iden[CK][64], ec[CK][64], neg_m[CK][64]; };
 
-template <class T>
+// CUT: for sequences cut in time.  bf16 and fp16 sequences in one piece have a kernel of their own, because with the segment's bounds in
+// registers and the summaries' loop in it the compiler schedules the walk worse: bf16 B8 T4096 C4096 621 us without them, 711 with
+// (fp32 gains nothing: 665 and 661).
+template <class T, bool CUT>
 __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, const float *__restrict__ time_decay,
         const float *__restrict__ time_first, const T *__restrict__ k, const T *__restrict__ v,
         const T *__restrict__ gy, const float *__restrict__ gs_out, const float *__restrict__ ckpt,
@@ -434,8 +437,9 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
     const int b = idx / C, c = idx % C;
     const float w = -__expf(time_decay[c]), u = time_first[c];
     const size_t base = (size_t)b * Tlen * C + c;
-    const Segment sg(Tlen, bps);
-    const int blk0 = sg.blk0, end = sg.blk1, nblk = end - blk0;          // nblk: the segment's
+    const int all = (Tlen + CK - 1) / CK, blk0 = CUT ? blockIdx.y * bps : 0, end = CUT ? min(blk0 + bps, all) : all;
+    const int nblk = CUT ? end - blk0 : all;          // the segment's
+    const bool last = !CUT || end == all;
 
     // RB blocks of k, v, gy per lane: one being consumed, the others in flight
     T bk[RB][CK], bv[RB][CK], bg[RB][CK];        // (as they came; converted where they are used)
@@ -483,7 +487,7 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
                     out.ys[i][lane] = yy; out.iden[i][lane] = iden; out.ec[i][lane] = ec; out.neg_m[i][lane] = nm;
                 }
             }
-            if (sg.last && blk == end - 1 && gs_out) {       // gradient arriving through the state handed out
+            if (last && blk == end - 1 && gs_out) {       // gradient arriving through the state handed out
                 const float gp = gs_out[idx * 3], gq = gs_out[idx * 3 + 1];
                 const float go = (gp == 0.f && gq == 0.f) ? NEG_HUGE : gs_out[idx * 3 + 2];
                 acc_w += (gp * s.dp + gq * s.dq) * __expf(s.o + go);
@@ -503,8 +507,9 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
             for (int d = 0; d < RB; d++)
                 if (j + d <= nblk) step(j + d, bk[d], bv[d], bg[d], bs[d], sh[d]);
         }
-        gw_part[(size_t)blockIdx.y * BC + idx] = acc_w * w;
-        gu_part[(size_t)blockIdx.y * BC + idx] = acc_u;
+        const size_t o = (CUT ? (size_t)blockIdx.y * BC : 0) + idx;
+        gw_part[o] = acc_w * w;
+        gu_part[o] = acc_u;
     } else {
         // ---------------- reverse walk: step j handles block end-j (none at j = 0), register set and buffer (j-1) % RB
         float gp = 0.f, gq = 0.f, go = NEG_HUGE;
@@ -515,7 +520,7 @@ __global__ __launch_bounds__(128) void v4_backward(int BC, int Tlen, int C, cons
 #pragma unroll
         for (int d = 0; d < RB; d++)
             if (nblk - 1 - d >= 0) fetch(end - 1 - d, bk[d], bv[d], bg[d]);
-        if (!sg.last) {          // the segments after this one, from the last
+        if (!last) {          // the segments after this one, from the last
             const int nseg = gridDim.y, seg = blockIdx.y, tail = Tlen - (nseg - 1) * bps * CK;          // tokens of the last
             for_summaries<3>(part, BC, idx, nseg - 1, nseg - 1 - seg, -1, [&](int j, const float (&x)[3]) __attribute__((always_inline)) {
                 const float wg = fmaf((float)(j == nseg - 1 ? tail : bps * CK), w, go);
@@ -684,8 +689,9 @@ static hipError_t bwd(hipStream_t s, int B, int Tlen, int C, const float *td, co
         hipLaunchKernelGGL((v4_summary_backward<T>), dim3((BC + 63) / 64, (pl.nseg - 1 + SW - 1) / SW), dim3(64 * SW), 0, s, BC, Tlen, C, td, tf,
                            (const T *)k, (const T *)v, (const T *)gy, ckpt, part, pl.nseg, pl.bps);
     prof_begin(KID_V4_BACKWARD, s);
-    hipLaunchKernelGGL((v4_backward<T>), dim3((BC + 63) / 64, pl.nseg), dim3(128), 0, s, BC, Tlen, C, td, tf, (const T *)k,
-                       (const T *)v, (const T *)gy, gs_out, ckpt, gw_part, gu_part, (T *)gk, (T *)gv, gs_in, part, pl.bps);
+    auto kernel = pl.nseg > 1 || sizeof(T) == 4 ? v4_backward<T, true> : v4_backward<T, sizeof(T) == 4>;
+    hipLaunchKernelGGL(kernel, dim3((BC + 63) / 64, pl.nseg), dim3(128), 0, s, BC, Tlen, C, td, tf, (const T *)k, (const T *)v,
+                       (const T *)gy, gs_out, ckpt, gw_part, gu_part, (T *)gk, (T *)gv, gs_in, part, pl.bps);
     prof_end(KID_V4_BACKWARD, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
