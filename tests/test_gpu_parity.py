@@ -401,7 +401,7 @@ def test_cumsum_decay_helper(chunk):
 @pytest.mark.parametrize("B,T,C", [(1, 128, 1), (2, 256, 63), (1, 128, 130), (1, 384, 129)])
 @pytest.mark.parametrize("precision", [64, 32])
 def test_decay_tables_of_128_token_chunks_ragged_widths(B, T, C, precision):
-    """Widths that do not fill the last workgroup, odd ones (one channel per lane) and even ones (two), against fp64.
+    """Widths that do not fill the last workgroup, against fp64.
     fp32 sums of up to 128 terms bounded by 5.3: off by at most 128 * 2^-24 * 128 * 5.3 / 2 = 2.6e-3 in the worst case and
     by some 1e-4 in practice, which an exponential turns into a relative error of the same size."""
     import rwkv_wkv_hip as W
@@ -432,6 +432,22 @@ def run_gpu56_forward(version, wl, algo):
     torch.cuda.synchronize()
     W.set_algo("auto")
     return y, s
+
+
+@pytest.mark.parametrize("B,T,C", [(8, 2048, 1057), (16, 16384, 32), (16, 16384, 160)])
+@pytest.mark.parametrize("precision", [None, 32, 64])
+def test_decay_tables_of_many_chunks(B, T, C, precision):
+    """Calls of many chunks take wider workgroups (two or four columns of wavefronts, the last of them partly past the row's
+    end); every chunk comes out as it does from a call of its own, to the bit."""
+    import rwkv_wkv_hip as W
+    raw = torch.randn(B, T, C, generator=torch.Generator().manual_seed(C)).to(dev()) * 0.5 - 1.5
+    tables = lambda w: W.cumsum_decay(w, 128, **(dict(factors=True, precision=precision) if precision else {}))
+    many = tables(raw)
+    for b, n in [(0, 0), (1, 7), (B - 1, T // 128 - 1)]:
+        one = tables(raw[b:b + 1, 128 * n:128 * n + 128].contiguous())
+        for name, x in one.items():
+            got = many[name][b, n] if many[name].shape[1] == T // 128 else many[name][b, 128 * n:128 * n + 128]
+            assert torch.equal(got.flatten(), x.flatten()), (name, b, n)
 
 
 @pytest.mark.parametrize("C", [64, 130, 77])
