@@ -106,22 +106,32 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t 
     hi = bf16_pack2(a, b);
     lo = bf16_pack2(a - bf_lo(hi), b - bf_hi(hi));
 }
-__device__ __forceinline__ void split4(f4 x, s4 &hi, s4 &lo) {
-    uint32_t h0, l0, h1, l1;
-    split2(x[0], x[1], h0, l0);
-    split2(x[2], x[3], h1, l1);
-    hi = as_s4(h0, h1);
-    lo = as_s4(l0, l1);
+// The same for a pair of accumulator tiles (rows 4g+e, column n) that go into one product, with the subtraction on the
+// matrix cores: x - hi = x + (-1) hi, exact as on the vector pipe, bit for bit the same results.  Sixteen vector
+// instructions of twenty-four become two MFMAs: a third of the chains' vector work.  `minus`: minus_one().
+// (A non-finite element makes the remainders of its column of both tiles NaN, all of them terms of the sum its own is a term of.)
+__device__ __forceinline__ s8 pair(s4 a, s4 b) { return s8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
+__device__ __forceinline__ s4 minus_one(int g, int n) {
+    const int at = n - 4 * g;            // the lane's row holds its -1 at element `at` of its four, if that is one of them
+    return s4{at == 0 ? (short)0xbf80 : (short)0, at == 1 ? (short)0xbf80 : (short)0, at == 2 ? (short)0xbf80 : (short)0, at == 3 ? (short)0xbf80 : (short)0};
 }
+__device__ __forceinline__ void split_pair(f4 x0, f4 x1, s4 minus, s8 &hi, s8 &lo) {
+    const s4 h0 = as_s4(bf16_pack2(x0[0], x0[1]), bf16_pack2(x0[2], x0[3])), h1 = as_s4(bf16_pack2(x1[0], x1[1]), bf16_pack2(x1[2], x1[3]));
+    x0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(minus, h0, x0, 0, 0, 0);
+    x1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(minus, h1, x1, 0, 0, 0);
+    hi = pair(h0, h1);
+    lo = pair(as_s4(bf16_pack2(x0[0], x0[1]), bf16_pack2(x0[2], x0[3])), as_s4(bf16_pack2(x1[0], x1[1]), bf16_pack2(x1[2], x1[3])));
+}
+__device__ __forceinline__ f4 mma32(s8 a, s8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0); }
 // The builders' r operand of the masked intra-block matrix: (r e^{excl}) e^{-b} = r e^{excl-b}, from the head/remainder
 // fragments of r e^{excl} (four keys of one token) and e^{-b} of those keys, as head + remainder again.  With
 // k e^{b-incl} as the other operand the product is r k e^{excl_t - incl_s}, at most |r k| where it is used (s < t).
-// A block's first token has no earlier token; its row is zeroed (its exponent -b is the only one beyond 79.5).
-__device__ __forceinline__ void scale_split(s4 hi, s4 lo, float4 f, bool zero, s4 &oh, s4 &ol) {
+// A block's first token has no earlier token: its products are masked, whatever they are (its exponent -b is the only one
+// beyond 79.5).
+__device__ __forceinline__ void scale_split(s4 hi, s4 lo, float4 f, s4 &oh, s4 &ol) {
     const uint2 h = __builtin_bit_cast(uint2, hi), l = __builtin_bit_cast(uint2, lo);
     float x0 = (bf_lo(h.x) + bf_lo(l.x)) * f.x, x1 = (bf_hi(h.x) + bf_hi(l.x)) * f.y;
     float x2 = (bf_lo(h.y) + bf_lo(l.y)) * f.z, x3 = (bf_hi(h.y) + bf_hi(l.y)) * f.w;
-    if (zero) x0 = x1 = x2 = x3 = 0.f;
     uint32_t h0, l0, h1, l1;
     split2(x0, x1, h0, l0);
     split2(x2, x3, h1, l1);
@@ -192,6 +202,19 @@ template <> struct WReg<true> {
 __device__ __forceinline__ void needed_here(uint2 &a) { asm volatile("" : "+v"(a.x), "+v"(a.y)); }
 __device__ __forceinline__ void needed_here(float4 &a) { asm volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z), "+v"(a.w)); }
 
+// Access by buffer instructions: what lies at or beyond the range's end reads as 0 and is not written, so that an access
+// that may have to be left out needs no branch (`nowhere`), and the compiler can count the accesses in flight.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00027000);
+}
+constexpr uint32_t NOWHERE = 0xfffffff0u;
+constexpr int NT_HINT = 2;          // the non-temporal hint of a buffer store
+typedef uint32_t dwords2 __attribute__((ext_vector_type(2)));
+typedef uint32_t dwords4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 buffer_load8(__amdgpu_buffer_rsrc_t b, uint32_t at) {
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(b, (int)at, 0, 0));
+}
+
 // One segment's summary for the time-parallel split: what the segment does to a
 // state handed in, S_out = decay o S_in + delta (forward), or to a state gradient
 // handed back (backward).  [key][value] fp32 plus one decay per key.
@@ -227,6 +250,7 @@ struct Fwd16Tiles {
     uint4 amat[2][4][64];     // masked intra-block matrix of each block, one part per half of the keys, as A-operand fragments (head, remainder)
     float4 yi[2][4][4][64];   // rh S per key half, block, value quarter: accumulator layout, one float4 per lane
     float wtot[16][HEAD];     // per wavefront (four tokens) and channel: sum of log w, for the block-wide running sum
+    float ub[HEAD];
 };
 
 __device__ __forceinline__ float row_prefix_sum(float x) {      // inclusive, over the 16 lanes of a DPP row
@@ -497,7 +521,8 @@ __global__ __launch_bounds__(NT_F) void summary_pass(int bh0, int Tlen, int C, i
 // in whole kilobytes, and leave the result in a table [key][CHAIN_LD] in LDS for everybody.  (Read by the wavefronts that
 // own the state, in their layout of 64-byte pieces, a summary cost some 0.4 us of the prologue and twice that in the
 // kernels with fewer wavefronts.)  Two pieces in one round trip to memory, then four at a time: with a decay that forgets
-// within a piece the walk is over after the first, with one that does not it has up to 63 to go.
+// within a piece the walk is over after the first, with one that does not it has up to 63 to go.  What was handed in
+// comes with the round trip of the last pieces.
 constexpr int CHAIN_LD = 68;
 template <int PER>
 __device__ __forceinline__ void chain_summaries(float *table, const float *__restrict__ pieces, int first, int count, int dir,
@@ -512,7 +537,7 @@ __device__ __forceinline__ void chain_summaries(float *table, const float *__res
     bool alive = true;          // (the same for the lanes of a wavefront)
     auto group = [&](int x, auto size) __attribute__((always_inline)) {
         constexpr int GROUP = decltype(size)::value;
-        f4 d[GROUP][PER];
+        f4 d[GROUP][PER], end[PER];
         float dc[GROUP][PER];
 #pragma unroll
         for (int bb = 0; bb < GROUP; bb++) {
@@ -520,6 +545,9 @@ __device__ __forceinline__ void chain_summaries(float *table, const float *__res
 #pragma unroll
             for (int i = 0; i < PER; i++) { d[bb][i] = *reinterpret_cast<const f4 *>(q + key[i] * HEAD + v4); dc[bb][i] = q[HEAD * HEAD + key[i]]; }
         }
+        const bool last = ends && x + GROUP >= count;
+#pragma unroll
+        for (int i = 0; i < PER; i++) end[i] = last ? *reinterpret_cast<const f4 *>(ends + key[i] * HEAD + v4) : f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int bb = 0; bb < GROUP; bb++)
             if (x + bb < count) {
@@ -530,14 +558,15 @@ __device__ __forceinline__ void chain_summaries(float *table, const float *__res
 #pragma unroll
         for (int i = 0; i < PER; i++) any |= run[i] != 0.f;
         alive = __builtin_amdgcn_ballot_w64(any) != 0;
+        if (alive && last) {
+#pragma unroll
+            for (int i = 0; i < PER; i++) X[i] += run[i] * end[i];
+        }
     };
-    if (count > 0) group(0, std::integral_constant<int, 2>());
+    group(0, std::integral_constant<int, 2>());            // (there is always a piece: the first, or last, segment chains nothing)
     for (int x = 2; x < count && alive; x += 4) group(x, std::integral_constant<int, 4>());
 #pragma unroll
-    for (int i = 0; i < PER; i++) {
-        if (alive && ends) X[i] += run[i] * *reinterpret_cast<const f4 *>(ends + key[i] * HEAD + v4);
-        *reinterpret_cast<f4 *>(table + key[i] * CHAIN_LD + v4) = X[i];
-    }
+    for (int i = 0; i < PER; i++) *reinterpret_cast<f4 *>(table + key[i] * CHAIN_LD + v4) = X[i];
 }
 
 // ALL_WHOLE (time-invariant decay only): the sequence is a whole number of 64-token steps, so the general way of
@@ -558,7 +587,8 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
     const int hk = w16 >> 2;                       // chain wavefronts: key half
     {       // the streams of this (batch, head): from here on every address is a 32-bit offset into its sequence
         const size_t base = (size_t)b * Tlen * C + (size_t)h * HEAD;
-        r += base; k += base; v += base; y += base;
+        r += base; k += base; v += base;
+        if (y) y += base;
         if (PER_TOKEN_W) wraw = W16 ? (const void *)(static_cast<const bf16 *>(wraw) + base) : (const void *)(static_cast<const float *>(wraw) + base);
     }
     const int nsb = (Tlen + SB - 1) / SB;
@@ -595,20 +625,27 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
         l_const = make_float4(log2_decay(w4.x, floor_decay), log2_decay(w4.y, floor_decay), log2_decay(w4.z, floor_decay),
                               log2_decay(w4.w, floor_decay));
     }
-    // the inputs of this lane's token, fetched two steps ahead into two register sets used in turn
-    struct Row { uint2 r, k, v; WReg<W16> w; };
+    // the inputs of this lane's token, fetched two steps ahead into two register sets used in turn.  Every access to memory in
+    // the step loop is there on every path (NOWHERE where there is nothing to do): loads and stores share one counter, and
+    // where the compiler cannot count it waits for all of them, i.e. at every step for the loads of the step after and for
+    // the results just stored, microseconds away.  For the same reason u waits in LDS.
+    struct Row { uint2 r, k, v, w0, w1; };
     Row rowA, rowB;
-    auto fetch = [&](int sb, Row &x) __attribute__((always_inline)) {
-        const int t = sb * SB + tok;
-        if (t < Tlen) {
-            const uint32_t o = (uint32_t)t * C + c4;
-            x.r = *reinterpret_cast<const uint2 *>(seq_at(r, o));
-            x.k = *reinterpret_cast<const uint2 *>(seq_at(k, o));
-            x.v = *reinterpret_cast<const uint2 *>(seq_at(v, o));
-            x.w = PER_TOKEN_W ? WReg<W16>::load(wraw, o) : WReg<W16>::from(l_const);
-        } else {
-            x.r = x.k = x.v = make_uint2(0u, 0u);
-            x.w = WReg<W16>::from(PER_TOKEN_W ? WKV_NEG_INF4 : make_float4(0.f, 0.f, 0.f, 0.f));
+    const uint32_t left = (uint32_t)Tlen * C - h * HEAD;             // elements to the sequence's end
+    const __amdgpu_buffer_rsrc_t r_buf = buffer_of(r, 2 * left), k_buf = buffer_of(k, 2 * left), v_buf = buffer_of(v, 2 * left);
+    const __amdgpu_buffer_rsrc_t w_buf = buffer_of(wraw, PER_TOKEN_W ? (W16 ? 2 : 4) * left : 0), y_buf = buffer_of(y, y ? 2 * left : 0);
+    auto fetch = [&](int sb, Row &x) __attribute__((always_inline)) {          // (tokens past the end: r = k = v = 0)
+        const uint32_t o = ((uint32_t)sb * SB + tok) * C + c4, at = sb < sb1 ? 2 * o : NOWHERE;
+        x.r = buffer_load8(r_buf, at);
+        x.k = buffer_load8(k_buf, at);
+        x.v = buffer_load8(v_buf, at);
+        if (PER_TOKEN_W) {
+            if (W16) x.w0 = buffer_load8(w_buf, at);
+            else {
+                const dwords4 w4 = __builtin_amdgcn_raw_buffer_load_b128(w_buf, (int)(sb < sb1 ? 4 * o : NOWHERE), 0, 0);
+                x.w0 = make_uint2(w4[0], w4[1]);
+                x.w1 = make_uint2(w4[2], w4[3]);
+            }
         }
     };
     const int tro = tr_lane_offset(lane, LD);
@@ -616,16 +653,29 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
     const size_t ck_off = (size_t)bh * (nsb + 1) * HEAD * HEAD;
 
     bool have_y = false;
+    if (tid < HEAD) sm.ub[tid] = u[h * HEAD + tid];
     fetch(sb0, rowA);
-    if (sb0 + 1 < sb1) fetch(sb0 + 1, rowB);
+    {      // (as many as a step leaves in flight, so that the wait for the loop's first step is counted as the others are)
+        __builtin_amdgcn_raw_buffer_store_b64(dwords2{0u, 0u}, y_buf, (int)NOWHERE, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(dwords2{0u, 0u}, y_buf, (int)NOWHERE, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(dwords2{0u, 0u}, y_buf, (int)NOWHERE, 0, 0);
+    }
+    fetch(sb0 + 1, rowB);
     // log w of this lane's token and its running sum inside the wavefront, always one step ahead (see scan_local)
     float lc[4], ic[4];
-    auto scan_ahead = [&](const WReg<W16> &pwr) __attribute__((always_inline)) {
-        const float4 pw = pwr.f4();
-        lc[0] = pw.x; lc[1] = pw.y; lc[2] = pw.z; lc[3] = pw.w;
+    auto scan_ahead = [&](int sb, const Row &x) __attribute__((always_inline)) {
         if (PER_TOKEN_W) {
+            lc[0] = W16 ? bf_lo(x.w0.x) : __uint_as_float(x.w0.x); lc[1] = W16 ? bf_hi(x.w0.x) : __uint_as_float(x.w0.y);
+            lc[2] = W16 ? bf_lo(x.w0.y) : __uint_as_float(x.w1.x); lc[3] = W16 ? bf_hi(x.w0.y) : __uint_as_float(x.w1.y);
 #pragma unroll
             for (int c = 0; c < 4; c++) lc[c] = log2_decay(lc[c], floor_decay);
+        } else {
+            lc[0] = l_const.x; lc[1] = l_const.y; lc[2] = l_const.z; lc[3] = l_const.w;
+        }
+        if ((sb + 1) * SB > Tlen) {      // (scalar) tokens past the end count as w = 1
+            const bool in = sb * SB + tok < Tlen;
+#pragma unroll
+            for (int c = 0; c < 4; c++) lc[c] = in ? lc[c] : 0.f;
         }
         scan_local(lc, ic, sm.wtot, w16, g, n);
     };
@@ -646,7 +696,7 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
     auto whole_step = [&](int sb) { return ALL_WHOLE ? true : !PER_TOKEN_W && (sb + 1) * SB <= Tlen; };       // scalar
 #pragma unroll
     for (int c = 0; c < 4; c++) lc[c] = ic[c] = 0.f;
-    if (!whole_step(sb0)) scan_ahead(rowA.w);
+    if (!whole_step(sb0)) scan_ahead(sb0, rowA);
     lds_barrier();
     PT_DECL
     // one step; `cur` holds its inputs (and takes those of the step after the next), `nxt` those of the next step
@@ -658,11 +708,11 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
             float l[4] = {lc[0], lc[1], lc[2], lc[3]}, inc[4] = {ic[0], ic[1], ic[2], ic[3]}, tot[4];
             const float rf[4] = {bf_lo(pr.x), bf_hi(pr.x), bf_lo(pr.y), bf_hi(pr.y)};
             const float kf[4] = {bf_lo(pk.x), bf_hi(pk.x), bf_lo(pk.y), bf_hi(pk.y)};
-            const float4 u4 = *reinterpret_cast<const float4 *>(u + h * HEAD + c4);
+            const float4 u4 = *reinterpret_cast<const float4 *>(&sm.ub[c4]);
             const float uf[4] = {u4.x, u4.y, u4.z, u4.w};
-            if (have_y) {      // y of the previous step waits in the rh tile: out as full rows, by the lanes that overwrite it next
-                const int t = (sb - 1) * SB + tok;
-                if (t < Tlen) store_row(seq_at(y, (uint32_t)t * C + c4), *reinterpret_cast<const uint2 *>(&sm.rh[tok * LD + c4]));
+            {      // y of the previous step waits in the rh tile: out as full rows, by the lanes that overwrite it next
+                const uint2 yv = *reinterpret_cast<const uint2 *>(&sm.rh[tok * LD + c4]);
+                __builtin_amdgcn_raw_buffer_store_b64(dwords2{yv.x, yv.y}, y_buf, (int)(have_y ? 2 * (((uint32_t)(sb - 1) * SB + tok) * C + c4) : NOWHERE), 0, NT_HINT);
             }
             const bool whole = whole_step(sb);
             float rhv[4], khv[4], p = 0.f;
@@ -700,27 +750,27 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
         PT_MARK(0)
         lds_barrier();
         PT_MARK(1)
-        if (sb + 2 < sb1) fetch(sb + 2, cur);     // these loads have two steps to arrive
+        {       // the state at the start of this step, 16 bytes per lane and tile, from the wavefronts that own it
+            const __amdgpu_buffer_rsrc_t c_buf = buffer_of(ckpt ? ckpt + ck_off + (size_t)sb * HEAD * HEAD : nullptr, ckpt ? HEAD * HEAD * 4 : 0);
+            const uint32_t at = chain ? (uint32_t)((wv * 4 + 2 * hk) * 64 + lane) * 16 : NOWHERE;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dwords4, S[0]), c_buf, (int)at, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dwords4, S[1]), c_buf, (int)(chain ? at + 1024 : NOWHERE), 0, 0);
+        }
+        fetch(sb + 2, cur);     // these loads have two steps to arrive
 
         if (chain) {
-            if (ckpt) {       // state at the start of this step, 16 bytes per lane and tile
-                float4 *cp = reinterpret_cast<float4 *>(ckpt + ck_off + (size_t)sb * HEAD * HEAD) + (wv * 4 + 2 * hk) * 64 + lane;
-                cp[0] = make_float4(S[0][0], S[0][1], S[0][2], S[0][3]);
-                cp[64] = make_float4(S[1][0], S[1][1], S[1][2], S[1][3]);
-            }
             // ---------------- the state over the four blocks; per block this half's share of rh S
+            const s4 minus = minus_one(g, n);
 #pragma unroll
             for (int blk = 0; blk < 4; blk++) {
                 const int row = 16 * blk + n, ca = 32 * hk + 4 * g, cb = ca + 16;
-                s4 s0h, s0l, s1h, s1l;
-                split4(S[0], s0h, s0l);
-                split4(S[1], s1h, s1l);
-                const s4 r0 = frag(sm.rh, row, ca), r1 = frag(sm.rh, row, cb);
-                const s4 r0l = frag(sm.rhl, row, ca), r1l = frag(sm.rhl, row, cb);
+                s8 sh, sl;
+                split_pair(S[0], S[1], minus, sh, sl);
+                const s8 rr = pair(frag(sm.rh, row, ca), frag(sm.rh, row, cb)), rl = pair(frag(sm.rhl, row, ca), frag(sm.rhl, row, cb));
                 f4 y0 = {0.f, 0.f, 0.f, 0.f}, y1 = y0, y2 = y0;
-                y2 = mma2(r0l, r1l, s0h, s1h, y2);
-                y0 = mma2(r0, r1, s0h, s1h, y0);
-                y1 = mma2(r0, r1, s0l, s1l, y1);
+                y2 = mma32(rl, sh, y2);
+                y0 = mma32(rr, sh, y0);
+                y1 = mma32(rr, sl, y1);
                 // S <- e^{b} o S + (k e^{b-incl})^T v
                 const s4 v_op = frag_tr(sm.v, tro + (16 * blk) * LD + 16 * wv);
 #pragma unroll
@@ -748,8 +798,8 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
             __builtin_amdgcn_sched_barrier(0);
             {
                 s4 r0, r1, r0l, r1l;
-                scale_split(ra, ral, ea, n == 0, r0, r0l);
-                scale_split(rb, rbl, eb, n == 0, r1, r1l);
+                scale_split(ra, ral, ea, r0, r0l);
+                scale_split(rb, rbl, eb, r1, r1l);
                 a0 = mma2(k0, k1, r0, r1, a0);
                 a1 = mma2(k0l, k1l, r0, r1, a1);
                 a2 = mma2(k0, k1, r0l, r1l, a2);
@@ -781,16 +831,18 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
 #pragma unroll
             for (int e = 0; e < 4; e++) sm.rh[(16 * q + 4 * g + e) * LD + 16 * wv + n] = bf16_bits(yt[e]);
         }
-        if (sb + 1 < sb1 && !whole_step(sb + 1)) scan_ahead(nxt.w);
+        if (sb + 1 < sb1 && !whole_step(sb + 1)) scan_ahead(sb + 1, nxt);
         PT_MARK(4)
         lds_barrier();
-        have_y = y != nullptr;
+        have_y = true;
     };
-    for (int sb = sb0; sb < sb1; sb += 2) {
+    for (int sb = sb0;;) {          // (left where it ends: a way round the second step would count as a way into the first)
         do_step(sb, rowA, rowB);
-        if (sb + 1 < sb1) do_step(sb + 1, rowB, rowA);
+        if (++sb >= sb1) break;
+        do_step(sb, rowB, rowA);
+        if (++sb >= sb1) break;
     }
-    if (have_y) {
+    if (y) {
         const int t = (sb1 - 1) * SB + tok;
         if (t < Tlen) store_row(seq_at(y, (uint32_t)t * C + c4), *reinterpret_cast<const uint2 *>(&sm.rh[tok * LD + c4]));
     }
@@ -861,19 +913,19 @@ struct Bwd16Tiles {
     float tot[4][HEAD];      // b per block and key
     float dec[4][HEAD];      // e^{b}
     float ent[4][HEAD];      // e^{-b}
-    float rho[SB];           // r . (u o k) per token
+    float rho[SB];           // r . (u o k) per token; from the builders on P[t][t]
     float ub[HEAD];
     float wtot[16][HEAD];    // per wavefront (four tokens) and channel: sum of log w, for the block-wide running sum
     float q1[SB * HEAD];     // gy S^T          [token][key]
     float q4[SB * HEAD];     // v G^T           [token][key]
     uint4 pfr[4][2][64];     // per block: P^T masked to s < t, P masked to t > s, as A-operand fragments (head, remainder)
-    float pdiag[4][16];      // P[t][t]
     uint4 amat[4][64];       // A~ masked to t >= s (diagonal r.(u o k)), A-operand fragments (head, remainder)
     float tots[4][HEAD];     // per block and key: sum over the block's tokens of r gr - k gk
     float arun[2][HEAD];     // the running sum of the decay gradient at the end of a step (two copies, used in turn)
-    float red[4][HEAD];      // gu partial sums of the four block groups
-    float4 kg3[4][64];       // kh G of the step's last block, parked here by wavefronts 8-11 (they are short of registers)
+    float4 kg[2][4][64];     // kh G of blocks 1 and 3, parked here by wavefronts 8-11 (they are short of registers);
+                             // that of block 2 in wtot, which is idle between the preparation and the next step
 };
+static_assert(sizeof(Bwd16Tiles) <= 160 * 1024 && 2 * sizeof(Bwd16Tiles::wtot) == sizeof(Bwd16Tiles::kg), "");
 constexpr int NT_B16 = 1024;
 // Re-derives the lane-dependent indices from an opaque copy of the lane id, so that the
 // address arithmetic of a phase stays inside the phase instead of being hoisted out of the
@@ -1002,15 +1054,17 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     // by the lanes that overwrite those entries next.  The decay gradient is finished on the way out:
     //   dL/dlog w_t = (running sum at the end of the token's block) + (inside-block part, waiting in the incl table),
     // the first being the sum at the step's end (arun[par]) plus the totals of the step's later blocks.
-    auto write_out = [&](int sb, int tok, int c4, int par) {
-        const int t = sb * SB + tok;
+    const uint32_t left = (uint32_t)Tlen * C - h * HEAD;             // elements to the sequence's end
+    const __amdgpu_buffer_rsrc_t gr_buf = buffer_of(gr, 2 * left), gk_buf = buffer_of(gk, 2 * left), gv_buf = buffer_of(gv, 2 * left);
+    const __amdgpu_buffer_rsrc_t gw_buf = buffer_of(gw_tok, PER_TOKEN_W ? (W16 ? 2 : 4) * left : 0);
+    auto write_out = [&](int sb, int tok, int c4, int par, int q) __attribute__((always_inline)) {
+        const uint32_t o = ((uint32_t)sb * SB + tok) * C + c4;       // (past the sequence's end: dropped)
+        auto out = [&](const __amdgpu_buffer_rsrc_t &b, const uint16_t *tile) __attribute__((always_inline)) {
+            const uint2 x = *reinterpret_cast<const uint2 *>(&tile[tok * LD + c4]);
+            __builtin_amdgcn_raw_buffer_store_b64(dwords2{x.x, x.y}, b, (int)(2 * o), 0, NT_HINT);
+        };
         if (!PER_TOKEN_W) {         // nothing per token to finish: gr, gk, gv only
-            if (t < Tlen) {
-                const uint32_t o = (uint32_t)t * C + c4;
-                store_row(seq_at(gr, o), *reinterpret_cast<const uint2 *>(&sm.rh[tok * LD + c4]));
-                store_row(seq_at(gk, o), *reinterpret_cast<const uint2 *>(&sm.kh[tok * LD + c4]));
-                store_row(seq_at(gv, o), *reinterpret_cast<const uint2 *>(&sm.v[tok * LD + c4]));
-            }
+            out(gr_buf, sm.rh); out(gk_buf, sm.kh); out(gv_buf, sm.v);
             return;
         }
         float4 A = *reinterpret_cast<const float4 *>(&sm.arun[par][c4]);
@@ -1029,11 +1083,8 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
         if (q < 1) { A.x += t1.x; A.y += t1.y; A.z += t1.z; A.w += t1.w; }
         const float4 D = *reinterpret_cast<const float4 *>(&sm.incl[swz(tok, c4)]);
         A.x += D.x; A.y += D.y; A.z += D.z; A.w += D.w;
-        if (t < Tlen) {
-            const uint32_t o = (uint32_t)t * C + c4;
-            store_row(seq_at(gr, o), *reinterpret_cast<const uint2 *>(&sm.rh[tok * LD + c4]));
-            store_row(seq_at(gk, o), *reinterpret_cast<const uint2 *>(&sm.kh[tok * LD + c4]));
-            store_row(seq_at(gv, o), *reinterpret_cast<const uint2 *>(&sm.v[tok * LD + c4]));
+        out(gr_buf, sm.rh); out(gk_buf, sm.kh); out(gv_buf, sm.v);
+        {
             {                       // dL/dw_raw = dL/dlog w x log w (natural logarithm); nothing where the floor holds
                 const float4 l4 = *reinterpret_cast<const float4 *>(&sm.lw[swz(tok, c4)]);
                 const float lf[4] = {l4.x, l4.y, l4.z, l4.w};
@@ -1041,8 +1092,11 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
 #pragma unroll
                 for (int c = 0; c < 4; c++) f[c] = (floor_decay && lf[c] <= LOG2_W_FLOOR) ? 0.f : lf[c] * LN2;
                 const float gw4[4] = {A.x * f[0], A.y * f[1], A.z * f[2], A.w * f[3]};
-                if (W16) store_row(seq_at(static_cast<bf16 *>(gw_tok), o), gw4);
-                else store_row(seq_at(static_cast<float *>(gw_tok), o), gw4);
+                if (W16)
+                    __builtin_amdgcn_raw_buffer_store_b64(dwords2{bf16_pack2(gw4[0], gw4[1]), bf16_pack2(gw4[2], gw4[3])}, gw_buf, (int)(2 * o), 0, NT_HINT);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b128(dwords4{__float_as_uint(gw4[0]), __float_as_uint(gw4[1]), __float_as_uint(gw4[2]), __float_as_uint(gw4[3])},
+                                                           gw_buf, (int)(o < left ? 4 * o : NOWHERE), 0, NT_HINT);
             }
         }
     };
@@ -1061,354 +1115,373 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     if (tid < HEAD) sm.ub[tid] = u[h * HEAD + tid];
     lds_barrier();
     PT_DECL
-    for (int sb = sb1 - 1; sb >= sb0; sb--) {
-      PT_MARK(5)
-      const bool whole = whole_step(sb);
-      if (whole && !tables_valid) {
-          const int key = tid & 63, pl = tid >> 6;
-          const float lk = log2_decay(static_cast<const float *>(wraw)[h * HEAD + key], floor_decay);
-          tab_r[swz(pl, key)] = exp2_fast(pl * lk);
-          tab_k[swz(pl, key)] = exp2_fast((15 - pl) * lk);
-          if (pl < 4) {
-              sm.tot[pl][key] = 16.f * lk;
-              sm.dec[pl][key] = exp2_fast(16.f * lk);
-              sm.ent[pl][key] = exp2_fast(-16.f * lk);
+    // A loop for each role: in a common one the registers that take the checkpoint in one role and hold the gradient in two
+    // others count as awaited in all of them, and those two waited in every step for the results of the step before to be
+    // written (one counter covers a wavefront's loads and stores).  With it, the results leaving by buffer stores and two
+    // more blocks of kh G parked in LDS: forward and backward of B8 T4096, WKV6 H40 bf16 decay 983 -> 938 us, WKV5 H32
+    // 549 -> 523 (the forward's part of it some 5 and 12), B1 T4096 H64 fp32 decay 211 -> 203, on one GPU in turn.  Measured and
+    // not kept: the next step's inputs asked for before the chains start in every role (961, 526, 206; left to itself the
+    // compiler asks for them after the chain where that is the long one), the checkpoint asked for where the chain
+    // starts (972, 525, 210), blocks counted from their middle, which spares the builders their factor (943, 531, 205,
+    // but it moves the state gradient's error from 1.6e-6 to 2.3e-6).
+    auto walk = [&](auto its_role) __attribute__((always_inline)) {
+        constexpr int role = decltype(its_role)::value, q = role;
+        for (int sb = sb1 - 1; sb >= sb0; sb--) {
+          PT_MARK(5)
+          const bool whole = whole_step(sb);
+          if (whole && !tables_valid) {
+              const int key = tid & 63, pl = tid >> 6;
+              const float lk = log2_decay(static_cast<const float *>(wraw)[h * HEAD + key], floor_decay);
+              tab_r[swz(pl, key)] = exp2_fast(pl * lk);
+              tab_k[swz(pl, key)] = exp2_fast((15 - pl) * lk);
+              if (pl < 4) {
+                  sm.tot[pl][key] = 16.f * lk;
+                  sm.dec[pl][key] = exp2_fast(16.f * lk);
+                  sm.ent[pl][key] = exp2_fast(-16.f * lk);
+              }
+              tables_valid = true;
+              lds_barrier();
           }
-          tables_valid = true;
-          lds_barrier();
-      }
-      if (!whole) tables_valid = false;
-      {
-        WKV_LOCAL_LANE
-        needed_here(pr); needed_here(pk); needed_here(pv); needed_here(pg);
-        if (PER_TOKEN_W) needed_here(pw.v);
-        // the step's checkpoint: loads issued now are back when the chains start
-        if (role == 0) {
-            const float *ck_lane = ckpt + (size_t)bh * (nsb + 1) * HEAD * HEAD + (wv * 64 + 16 * (n >> 2) + 4 * g) * 4 + (n & 3);
-            const float *cp = ck_lane + (size_t)sb * HEAD * HEAD;
+          if (!whole) tables_valid = false;
+          {
+            WKV_LOCAL_LANE
+            needed_here(pr); needed_here(pk); needed_here(pv); needed_here(pg);
+            if (PER_TOKEN_W) needed_here(pw.v);
+            // the step's checkpoint: loads issued now are back when the chains start
+            if (role == 0) {
+                const float *ck_lane = ckpt + (size_t)bh * (nsb + 1) * HEAD * HEAD + (wv * 64 + 16 * (n >> 2) + 4 * g) * 4 + (n & 3);
+                const float *cp = ck_lane + (size_t)sb * HEAD * HEAD;
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++)
+                for (int kk = 0; kk < 4; kk++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) G[kk][e] = cp[kk * 1024 + e * 4];
-        }
-        // ---------------- prepare the operands of this lane's token
-        {
-            const float4 pf = pw.f4();
-            float l[4] = {pf.x, pf.y, pf.z, pf.w}, inc[4], tot[4];
-            const float rf[4] = {bf_lo(pr.x), bf_hi(pr.x), bf_lo(pr.y), bf_hi(pr.y)};
-            const float kf[4] = {bf_lo(pk.x), bf_hi(pk.x), bf_lo(pk.y), bf_hi(pk.y)};
-            const float4 u4 = *reinterpret_cast<const float4 *>(&sm.ub[c4]);
-            const float uf[4] = {u4.x, u4.y, u4.z, u4.w};
-            if (PER_TOKEN_W) {
-#pragma unroll
-                for (int c = 0; c < 4; c++) l[c] = log2_decay(l[c], floor_decay);
-            } else if (!whole) {       // a step with missing tokens: they count as w = 1
-                const float4 w4 = *reinterpret_cast<const float4 *>(static_cast<const float *>(wraw) + h * HEAD + c4);
-                const bool in = sb * SB + tok < Tlen;
-                l[0] = in ? log2_decay(w4.x, floor_decay) : 0.f; l[1] = in ? log2_decay(w4.y, floor_decay) : 0.f;
-                l[2] = in ? log2_decay(w4.z, floor_decay) : 0.f; l[3] = in ? log2_decay(w4.w, floor_decay) : 0.f;
+                    for (int e = 0; e < 4; e++) G[kk][e] = cp[kk * 1024 + e * 4];
             }
-            PT_MARK(5)
-            if (have_out) { write_out(sb + 1, tok, c4, par); par ^= 1; }
-            PT_MARK(6)
-            float rhv[4], khv[4], p = 0.f;
-            if (whole) {
-                const float4 fr = *reinterpret_cast<const float4 *>(&tab_r[swz(tok & 15, c4)]);
-                const float4 fk = *reinterpret_cast<const float4 *>(&tab_k[swz(tok & 15, c4)]);
-                rhv[0] = rf[0] * fr.x; rhv[1] = rf[1] * fr.y; rhv[2] = rf[2] * fr.z; rhv[3] = rf[3] * fr.w;
-                khv[0] = kf[0] * fk.x; khv[1] = kf[1] * fk.y; khv[2] = kf[2] * fk.z; khv[3] = kf[3] * fk.w;
-            } else {
-                scan_local(l, inc, sm.wtot, w16, g, n);      // (the one-step-ahead form of forward16 costs registers this kernel lacks)
-                lds_barrier();
-                PT_MARK(7)
-                scan_join(inc, tot, sm.wtot, w16, n);
+            // ---------------- prepare the operands of this lane's token
+            {
+                const float4 pf = pw.f4();
+                float l[4] = {pf.x, pf.y, pf.z, pf.w}, inc[4], tot[4];
+                const float rf[4] = {bf_lo(pr.x), bf_hi(pr.x), bf_lo(pr.y), bf_hi(pr.y)};
+                const float kf[4] = {bf_lo(pk.x), bf_hi(pk.x), bf_lo(pk.y), bf_hi(pk.y)};
+                const float4 u4 = *reinterpret_cast<const float4 *>(&sm.ub[c4]);
+                const float uf[4] = {u4.x, u4.y, u4.z, u4.w};
+                if (PER_TOKEN_W) {
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    rhv[c] = rf[c] * exp2_fast(inc[c] - l[c]);
-                    khv[c] = kf[c] * exp2_fast(tot[c] - inc[c]);
+                    for (int c = 0; c < 4; c++) l[c] = log2_decay(l[c], floor_decay);
+                } else if (!whole) {       // a step with missing tokens: they count as w = 1
+                    const float4 w4 = *reinterpret_cast<const float4 *>(static_cast<const float *>(wraw) + h * HEAD + c4);
+                    const bool in = sb * SB + tok < Tlen;
+                    l[0] = in ? log2_decay(w4.x, floor_decay) : 0.f; l[1] = in ? log2_decay(w4.y, floor_decay) : 0.f;
+                    l[2] = in ? log2_decay(w4.z, floor_decay) : 0.f; l[3] = in ? log2_decay(w4.w, floor_decay) : 0.f;
                 }
-            }
+                PT_MARK(5)
+                if (have_out) { write_out(sb + 1, tok, c4, par, q); par ^= 1; }
+                PT_MARK(6)
+                float rhv[4], khv[4], p = 0.f;
+                if (whole) {
+                    const float4 fr = *reinterpret_cast<const float4 *>(&tab_r[swz(tok & 15, c4)]);
+                    const float4 fk = *reinterpret_cast<const float4 *>(&tab_k[swz(tok & 15, c4)]);
+                    rhv[0] = rf[0] * fr.x; rhv[1] = rf[1] * fr.y; rhv[2] = rf[2] * fr.z; rhv[3] = rf[3] * fr.w;
+                    khv[0] = kf[0] * fk.x; khv[1] = kf[1] * fk.y; khv[2] = kf[2] * fk.z; khv[3] = kf[3] * fk.w;
+                } else {
+                    scan_local(l, inc, sm.wtot, w16, g, n);      // (the one-step-ahead form of forward16 costs registers this kernel lacks)
+                    lds_barrier();
+                    PT_MARK(7)
+                    scan_join(inc, tot, sm.wtot, w16, n);
 #pragma unroll
-            for (int c = 0; c < 4; c++) p = fmaf(rf[c] * uf[c], kf[c], p);
-            uint32_t h0, l0, h1, l1;
-            const int o = tok * LD + c4;
-            *reinterpret_cast<uint2 *>(&sm.gy[o]) = pg;
-            *reinterpret_cast<uint2 *>(&sm.v[o]) = pv;
-            split2(rhv[0], rhv[1], h0, l0); split2(rhv[2], rhv[3], h1, l1);
-            *reinterpret_cast<uint2 *>(&sm.rh[o]) = make_uint2(h0, h1);
-            *reinterpret_cast<uint2 *>(&sm.rhl[o]) = make_uint2(l0, l1);
-            split2(khv[0], khv[1], h0, l0); split2(khv[2], khv[3], h1, l1);
-            *reinterpret_cast<uint2 *>(&sm.kh[o]) = make_uint2(h0, h1);
-            *reinterpret_cast<uint2 *>(&sm.khl[o]) = make_uint2(l0, l1);
-            *reinterpret_cast<uint4 *>(&sm.rk[swz(tok, c4)]) =
-                make_uint4((pr.x & 0xffffu) | (pk.x << 16), (pr.x >> 16) | (pk.x & 0xffff0000u),
-                           (pr.y & 0xffffu) | (pk.y << 16), (pr.y >> 16) | (pk.y & 0xffff0000u));
-            if (!whole) {
-                *reinterpret_cast<float4 *>(&sm.incl[swz(tok, c4)]) = make_float4(inc[0], inc[1], inc[2], inc[3]);
-                *reinterpret_cast<float4 *>(&sm.lw[swz(tok, c4)]) = make_float4(l[0], l[1], l[2], l[3]);
-            }
-            if (!whole && (w16 & 3) == 3) {       // wavefront-uniform: only the wavefront with the block's last token
-                if (g == 3) {
-                    *reinterpret_cast<float4 *>(&sm.tot[q][c4]) = make_float4(tot[0], tot[1], tot[2], tot[3]);
-                    *reinterpret_cast<float4 *>(&sm.dec[q][c4]) = make_float4(exp2_fast(tot[0]), exp2_fast(tot[1]), exp2_fast(tot[2]), exp2_fast(tot[3]));
-                    *reinterpret_cast<float4 *>(&sm.ent[q][c4]) = make_float4(exp2_fast(-tot[0]), exp2_fast(-tot[1]), exp2_fast(-tot[2]), exp2_fast(-tot[3]));
-                }
-            }
-            p = row_prefix_sum(p);           // lane 15 of the row ends with the sum over the 64 channels
-            if (n == 15) sm.rho[tok] = p;
-        }
-      }
-        PT_MARK(0)
-        lds_barrier();
-        PT_MARK(1)
-
-        f4 KG[4];                    // wavefronts 8-11: kh G per block, KG[q][e] at [token 4g+e][value own]
-      {
-        WKV_LOCAL_LANE
-        fetch_whole(max(sb - 1, sb0), tok, c4);      // (the segment's first step fetches itself once more: unused)
-        if (role == 0) {
-            // ---------------- state chain, first block to last; Q1[t][key own] = sum_j gy[t][j] S[key own][j]
-#pragma unroll
-            for (int qq = 0; qq < 4; qq++) {
-                f4 qa = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int kk = 0; kk < 4; kk += 2) {
-                    s4 s0h, s0l, s1h, s1l;
-                    split4(G[kk], s0h, s0l);
-                    split4(G[kk + 1], s1h, s1l);
-                    const s4 y0 = frag(sm.gy, 16 * qq + n, 16 * kk + 4 * g), y1 = frag(sm.gy, 16 * qq + n, 16 * kk + 16 + 4 * g);
-                    qa = mma2(s0l, s1l, y0, y1, qa);       // (the state as the A operand: the product comes out as [key][token])
-                    qa = mma2(s0h, s1h, y0, y1, qa);
-                }
-                *reinterpret_cast<float4 *>(&sm.q1[swz(16 * qq + n, 16 * wv + 4 * g)]) = make_float4(qa[0], qa[1], qa[2], qa[3]);
-                if (qq < 3) {
-                    const float dq = sm.dec[qq][own];
-                    const s4 khf = frag_tr(sm.kh, tro + (16 * qq) * LD + 16 * wv), khfl = frag_tr(sm.khl, tro + (16 * qq) * LD + 16 * wv);
-#pragma unroll
-                    for (int kk = 0; kk < 4; kk++) {
-                        G[kk] = G[kk] * dq;
-                        const s4 vf_ = frag_tr(sm.v, tro + (16 * qq) * LD + 16 * kk);
-                        G[kk] = mma2(vf_, vf_, khf, khfl, G[kk]);
+                    for (int c = 0; c < 4; c++) {
+                        rhv[c] = rf[c] * exp2_fast(inc[c] - l[c]);
+                        khv[c] = kf[c] * exp2_fast(tot[c] - inc[c]);
                     }
                 }
-            }
-        } else if (role == 1) {
-            // ---------------- state-gradient chain (value-major), last block to first; Q4[s][key own] = sum_j v[s][j] G[key own][j]
 #pragma unroll
-            for (int qq = 3; qq >= 0; qq--) {
-                f4 q4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int kk = 0; kk < 4; kk += 2) {
-                    s4 g0h, g0l, g1h, g1l;
-                    split4(G[kk], g0h, g0l);
-                    split4(G[kk + 1], g1h, g1l);
-                    const s4 v0 = frag(sm.v, 16 * qq + n, 16 * kk + 4 * g), v1 = frag(sm.v, 16 * qq + n, 16 * kk + 16 + 4 * g);
-                    q4 = mma2(g0l, g1l, v0, v1, q4);
-                    q4 = mma2(g0h, g1h, v0, v1, q4);
+                for (int c = 0; c < 4; c++) p = fmaf(rf[c] * uf[c], kf[c], p);
+                uint32_t h0, l0, h1, l1;
+                const int o = tok * LD + c4;
+                *reinterpret_cast<uint2 *>(&sm.gy[o]) = pg;
+                *reinterpret_cast<uint2 *>(&sm.v[o]) = pv;
+                split2(rhv[0], rhv[1], h0, l0); split2(rhv[2], rhv[3], h1, l1);
+                *reinterpret_cast<uint2 *>(&sm.rh[o]) = make_uint2(h0, h1);
+                *reinterpret_cast<uint2 *>(&sm.rhl[o]) = make_uint2(l0, l1);
+                split2(khv[0], khv[1], h0, l0); split2(khv[2], khv[3], h1, l1);
+                *reinterpret_cast<uint2 *>(&sm.kh[o]) = make_uint2(h0, h1);
+                *reinterpret_cast<uint2 *>(&sm.khl[o]) = make_uint2(l0, l1);
+                *reinterpret_cast<uint4 *>(&sm.rk[swz(tok, c4)]) =
+                    make_uint4((pr.x & 0xffffu) | (pk.x << 16), (pr.x >> 16) | (pk.x & 0xffff0000u),
+                               (pr.y & 0xffffu) | (pk.y << 16), (pr.y >> 16) | (pk.y & 0xffff0000u));
+                if (!whole) {
+                    *reinterpret_cast<float4 *>(&sm.incl[swz(tok, c4)]) = make_float4(inc[0], inc[1], inc[2], inc[3]);
+                    *reinterpret_cast<float4 *>(&sm.lw[swz(tok, c4)]) = make_float4(l[0], l[1], l[2], l[3]);
                 }
-                *reinterpret_cast<float4 *>(&sm.q4[swz(16 * qq + n, 16 * wv + 4 * g)]) = make_float4(q4[0], q4[1], q4[2], q4[3]);
-                const float dq = sm.dec[qq][own];
-                const s4 rhTf = frag_tr(sm.rh, tro + (16 * qq) * LD + 16 * wv), rhTfl = frag_tr(sm.rhl, tro + (16 * qq) * LD + 16 * wv);
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++) {      // G <- e^{b} o G + rh^T gy
-                    G[kk] = G[kk] * dq;
-                    const s4 gT_ = frag_tr(sm.gy, tro + (16 * qq) * LD + 16 * kk);
-                    G[kk] = mma2(gT_, gT_, rhTf, rhTfl, G[kk]);
+                if (!whole && (w16 & 3) == 3) {       // wavefront-uniform: only the wavefront with the block's last token
+                    if (g == 3) {
+                        *reinterpret_cast<float4 *>(&sm.tot[q][c4]) = make_float4(tot[0], tot[1], tot[2], tot[3]);
+                        *reinterpret_cast<float4 *>(&sm.dec[q][c4]) = make_float4(exp2_fast(tot[0]), exp2_fast(tot[1]), exp2_fast(tot[2]), exp2_fast(tot[3]));
+                        *reinterpret_cast<float4 *>(&sm.ent[q][c4]) = make_float4(exp2_fast(-tot[0]), exp2_fast(-tot[1]), exp2_fast(-tot[2]), exp2_fast(-tot[3]));
+                    }
                 }
+                p = row_prefix_sum(p);           // lane 15 of the row ends with the sum over the 64 channels
+                if (n == 15) sm.rho[tok] = p;
             }
-        } else if (role == 2) {
-            // ---------------- state-gradient chain (key-major), last block to first; KG[s][value own] = sum_i kh[s][i] G[i][value own]
+          }
+            PT_MARK(0)
+            lds_barrier();
+            PT_MARK(1)
+
+            f4 KG;                       // wavefronts 8-11: kh G of the first block, KG[e] at [token 4g+e][value own]
+            float4 (*const kg2)[64] = reinterpret_cast<float4 (*)[64]>(sm.wtot);
+          {
+            WKV_LOCAL_LANE
+            fetch_whole(max(sb - 1, sb0), tok, c4);      // (the segment's first step fetches itself once more: unused)
+            if (role == 0) {
+                // ---------------- state chain, first block to last; Q1[t][key own] = sum_j gy[t][j] S[key own][j]
+                const s4 minus = minus_one(g, n);
 #pragma unroll
-            for (int qq = 3; qq >= 0; qq--) {
-                const int row = 16 * qq + n;
-                // The LDS operands of the block's products are fetched before the arithmetic on G starts: this wavefront
-                // is the longest of the phase and walks a dependent sequence, so a fetch issued where it is used costs
-                // the whole step its latency.
-                s4 kh_[4], kl_[4];
+                for (int qq = 0; qq < 4; qq++) {
+                    f4 qa = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk += 2) {
+                        s8 sh, sl;
+                        split_pair(G[kk], G[kk + 1], minus, sh, sl);
+                        const s8 y = pair(frag(sm.gy, 16 * qq + n, 16 * kk + 4 * g), frag(sm.gy, 16 * qq + n, 16 * kk + 16 + 4 * g));
+                        qa = mma32(sl, y, qa);       // (the state as the A operand: the product comes out as [key][token])
+                        qa = mma32(sh, y, qa);
+                    }
+                    *reinterpret_cast<float4 *>(&sm.q1[swz(16 * qq + n, 16 * wv + 4 * g)]) = make_float4(qa[0], qa[1], qa[2], qa[3]);
+                    if (qq < 3) {
+                        const float dq = sm.dec[qq][own];
+                        const s4 khf = frag_tr(sm.kh, tro + (16 * qq) * LD + 16 * wv), khfl = frag_tr(sm.khl, tro + (16 * qq) * LD + 16 * wv);
+#pragma unroll
+                        for (int kk = 0; kk < 4; kk++) {
+                            G[kk] = G[kk] * dq;
+                            const s4 vf_ = frag_tr(sm.v, tro + (16 * qq) * LD + 16 * kk);
+                            G[kk] = mma2(vf_, vf_, khf, khfl, G[kk]);
+                        }
+                    }
+                }
+            } else if (role == 1) {
+                // ---------------- state-gradient chain (value-major), last block to first; Q4[s][key own] = sum_j v[s][j] G[key own][j]
+                const s4 minus = minus_one(g, n);
+#pragma unroll
+                for (int qq = 3; qq >= 0; qq--) {
+                    f4 q4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk += 2) {
+                        s8 gh, gl;
+                        split_pair(G[kk], G[kk + 1], minus, gh, gl);
+                        const s8 vv = pair(frag(sm.v, 16 * qq + n, 16 * kk + 4 * g), frag(sm.v, 16 * qq + n, 16 * kk + 16 + 4 * g));
+                        q4 = mma32(gl, vv, q4);
+                        q4 = mma32(gh, vv, q4);
+                    }
+                    *reinterpret_cast<float4 *>(&sm.q4[swz(16 * qq + n, 16 * wv + 4 * g)]) = make_float4(q4[0], q4[1], q4[2], q4[3]);
+                    const float dq = sm.dec[qq][own];
+                    const s4 rhTf = frag_tr(sm.rh, tro + (16 * qq) * LD + 16 * wv), rhTfl = frag_tr(sm.rhl, tro + (16 * qq) * LD + 16 * wv);
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk++) {      // G <- e^{b} o G + rh^T gy
+                        G[kk] = G[kk] * dq;
+                        const s4 gT_ = frag_tr(sm.gy, tro + (16 * qq) * LD + 16 * kk);
+                        G[kk] = mma2(gT_, gT_, rhTf, rhTfl, G[kk]);
+                    }
+                }
+            } else if (role == 2) {
+                // ---------------- state-gradient chain (key-major), last block to first; KG[s][value own] = sum_i kh[s][i] G[i][value own]
+                const s4 minus = minus_one(g, n);
+#pragma unroll
+                for (int qq = 3; qq >= 0; qq--) {
+                    const int row = 16 * qq + n;
+                    // The LDS operands of the block's products are fetched before the arithmetic on G starts: this wavefront
+                    // is the longest of the phase and walks a dependent sequence, so a fetch issued where it is used costs
+                    // the whole step its latency.
+                    s8 kh_[2], kl_[2];
+#pragma unroll
+                    for (int kk = 0; kk < 2; kk++) {
+                        kh_[kk] = pair(frag(sm.kh, row, 32 * kk + 4 * g), frag(sm.kh, row, 32 * kk + 16 + 4 * g));
+                        kl_[kk] = pair(frag(sm.khl, row, 32 * kk + 4 * g), frag(sm.khl, row, 32 * kk + 16 + 4 * g));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    f4 g0 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int kk = 0; kk < 2; kk++) {
+                        s8 gh, gl;
+                        split_pair(G[2 * kk], G[2 * kk + 1], minus, gh, gl);
+                        g0 = mma32(gl, kh_[kk], g0);       // (the gradient as the A operand: [value][token])
+                        g0 = mma32(gh, kl_[kk], g0);
+                        g0 = mma32(gh, kh_[kk], g0);
+                    }
+                    if (qq > 0) (qq == 2 ? kg2 : sm.kg[qq >> 1])[wv][lane] = make_float4(g0[0], g0[1], g0[2], g0[3]);
+                    else KG = g0;
+                    const s4 gyTf = frag_tr(sm.gy, tro + (16 * qq) * LD + 16 * wv);
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk++) {      // G <- e^{b} o G + rh^T gy
+                        const float4 d4 = *reinterpret_cast<const float4 *>(&sm.dec[qq][16 * kk + 4 * g]);
+                        G[kk][0] *= d4.x; G[kk][1] *= d4.y; G[kk][2] *= d4.z; G[kk][3] *= d4.w;
+                        G[kk] = mma2(frag_tr(sm.rh, tro + (16 * qq) * LD + 16 * kk), frag_tr(sm.rhl, tro + (16 * qq) * LD + 16 * kk),
+                                     gyTf, gyTf, G[kk]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);      // one block at a time: keeps the register need of the chain bounded
+                }
+            } else {
+                // ---------------- the masked matrices of block wv, once for everybody
+                // (the LDS operands of each matrix are fetched together and ahead of their use: the builders are, with the
+                // key-major chain, the longest wavefronts of the phase, and a fetch issued where it is used costs the whole
+                // step its latency)
+                const int row = 16 * wv + n;
+                const float rho_s = sm.rho[row];           // (this wavefront leaves P[t][t] in its place)
+                s4 gyf[4], vf[4], rhf[4], rlf[4], khf[4], klf[4];
+                float4 en[4];
 #pragma unroll
                 for (int kk = 0; kk < 4; kk++) {
-                    kh_[kk] = frag(sm.kh, row, 16 * kk + 4 * g);
-                    kl_[kk] = frag(sm.khl, row, 16 * kk + 4 * g);
+                    gyf[kk] = frag(sm.gy, row, 16 * kk + 4 * g);
+                    vf[kk] = frag(sm.v, row, 16 * kk + 4 * g);
+                }
+                // pt[e] = P[t = 4g+e][s = n],  ptT[e] = P[t = n][s = 4g+e],  P[t][s] = gy_t . v_s
+                f4 pt = {0.f, 0.f, 0.f, 0.f}, ptT = pt;
+                pt = mma2(gyf[0], gyf[1], vf[0], vf[1], pt);
+                ptT = mma2(vf[0], vf[1], gyf[0], gyf[1], ptT);
+                pt = mma2(gyf[2], gyf[3], vf[2], vf[3], pt);
+                ptT = mma2(vf[2], vf[3], gyf[2], gyf[3], ptT);
+                f4 pm, pTm;
+                {
+                    const int e_diag = n & 3;
+                    if ((n >> 2) == g) sm.rho[row] = e_diag == 0 ? pt[0] : e_diag == 1 ? pt[1] : e_diag == 2 ? pt[2] : pt[3];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int x = 4 * g + e;
+                        pm[e] = x > n ? pt[e] : 0.f;        // later tokens t > s
+                        pTm[e] = x < n ? ptT[e] : 0.f;      // earlier tokens s < t
+                    }
+                    uint32_t h0, l0, h1, l1;
+                    split2(pTm[0], pTm[1], h0, l0); split2(pTm[2], pTm[3], h1, l1);
+                    sm.pfr[wv][0][lane] = make_uint4(h0, h1, l0, l1);
+                    split2(pm[0], pm[1], h0, l0); split2(pm[2], pm[3], h1, l1);
+                    sm.pfr[wv][1][lane] = make_uint4(h0, h1, l0, l1);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                f4 g0 = {0.f, 0.f, 0.f, 0.f};
+                // A~[t = 4g+e][s = n] = (r e^{excl-b})_t . (k e^{b-incl})_s; its operands all at once
+#pragma unroll
+                for (int kk = 0; kk < 4; kk++) {
+                    rhf[kk] = frag(sm.rh, row, 16 * kk + 4 * g);
+                    rlf[kk] = frag(sm.rhl, row, 16 * kk + 4 * g);
+                    khf[kk] = frag(sm.kh, row, 16 * kk + 4 * g);
+                    klf[kk] = frag(sm.khl, row, 16 * kk + 4 * g);
+                    en[kk] = *reinterpret_cast<const float4 *>(&sm.ent[wv][16 * kk + 4 * g]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                f4 at = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int kk = 0; kk < 4; kk += 2) {
-                    s4 g0h, g0l, g1h, g1l;
-                    split4(G[kk], g0h, g0l);
-                    split4(G[kk + 1], g1h, g1l);
-                    g0 = mma2(g0l, g1l, kh_[kk], kh_[kk + 1], g0);       // (the gradient as the A operand: [value][token])
-                    g0 = mma2(g0h, g1h, kl_[kk], kl_[kk + 1], g0);
-                    g0 = mma2(g0h, g1h, kh_[kk], kh_[kk + 1], g0);
+                    s4 r0, r1, r0l, r1l;
+                    scale_split(rhf[kk], rlf[kk], en[kk], r0, r0l);
+                    scale_split(rhf[kk + 1], rlf[kk + 1], en[kk + 1], r1, r1l);
+                    at = mma2(r0l, r1l, khf[kk], khf[kk + 1], at);
+                    at = mma2(r0, r1, klf[kk], klf[kk + 1], at);
+                    at = mma2(r0, r1, khf[kk], khf[kk + 1], at);
                 }
-                KG[qq] = g0;
-                if (qq == 3) sm.kg3[wv][lane] = make_float4(KG[3][0], KG[3][1], KG[3][2], KG[3][3]);
-                const s4 gyTf = frag_tr(sm.gy, tro + (16 * qq) * LD + 16 * wv);
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++) {      // G <- e^{b} o G + rh^T gy
-                    const float4 d4 = *reinterpret_cast<const float4 *>(&sm.dec[qq][16 * kk + 4 * g]);
-                    G[kk][0] *= d4.x; G[kk][1] *= d4.y; G[kk][2] *= d4.z; G[kk][3] *= d4.w;
-                    G[kk] = mma2(frag_tr(sm.rh, tro + (16 * qq) * LD + 16 * kk), frag_tr(sm.rhl, tro + (16 * qq) * LD + 16 * kk),
-                                 gyTf, gyTf, G[kk]);
-                }
-                __builtin_amdgcn_sched_barrier(0);      // one block at a time: keeps the register need of the chain bounded
-            }
-        } else {
-            // ---------------- the masked matrices of block wv, once for everybody
-            // (the LDS operands of each matrix are fetched together and ahead of their use: the builders are, with the
-            // key-major chain, the longest wavefronts of the phase, and a fetch issued where it is used costs the whole
-            // step its latency)
-            const int row = 16 * wv + n;
-            s4 gyf[4], vf[4], rhf[4], rlf[4], khf[4], klf[4];
-            float4 en[4];
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                gyf[kk] = frag(sm.gy, row, 16 * kk + 4 * g);
-                vf[kk] = frag(sm.v, row, 16 * kk + 4 * g);
-            }
-            // pt[e] = P[t = 4g+e][s = n],  ptT[e] = P[t = n][s = 4g+e],  P[t][s] = gy_t . v_s
-            f4 pt = {0.f, 0.f, 0.f, 0.f}, ptT = pt;
-            pt = mma2(gyf[0], gyf[1], vf[0], vf[1], pt);
-            ptT = mma2(vf[0], vf[1], gyf[0], gyf[1], ptT);
-            pt = mma2(gyf[2], gyf[3], vf[2], vf[3], pt);
-            ptT = mma2(vf[2], vf[3], gyf[2], gyf[3], ptT);
-            f4 pm, pTm;
-            {
-                const int e_diag = n & 3;
-                if ((n >> 2) == g) sm.pdiag[wv][n] = e_diag == 0 ? pt[0] : e_diag == 1 ? pt[1] : e_diag == 2 ? pt[2] : pt[3];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int x = 4 * g + e;
-                    pm[e] = x > n ? pt[e] : 0.f;        // later tokens t > s
-                    pTm[e] = x < n ? ptT[e] : 0.f;      // earlier tokens s < t
+                    at[e] = x > n ? at[e] : (x == n ? rho_s : 0.f);
                 }
                 uint32_t h0, l0, h1, l1;
-                split2(pTm[0], pTm[1], h0, l0); split2(pTm[2], pTm[3], h1, l1);
-                sm.pfr[wv][0][lane] = make_uint4(h0, h1, l0, l1);
-                split2(pm[0], pm[1], h0, l0); split2(pm[2], pm[3], h1, l1);
-                sm.pfr[wv][1][lane] = make_uint4(h0, h1, l0, l1);
+                split2(at[0], at[1], h0, l0); split2(at[2], at[3], h1, l1);
+                sm.amat[wv][lane] = make_uint4(h0, h1, l0, l1);
             }
-            __builtin_amdgcn_sched_barrier(0);
-            // A~[t = 4g+e][s = n] = (r e^{excl-b})_t . (k e^{b-incl})_s; its operands all at once
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                rhf[kk] = frag(sm.rh, row, 16 * kk + 4 * g);
-                rlf[kk] = frag(sm.rhl, row, 16 * kk + 4 * g);
-                khf[kk] = frag(sm.kh, row, 16 * kk + 4 * g);
-                klf[kk] = frag(sm.khl, row, 16 * kk + 4 * g);
-                en[kk] = *reinterpret_cast<const float4 *>(&sm.ent[wv][16 * kk + 4 * g]);
-            }
-            const float rho_s = sm.rho[row];
-            __builtin_amdgcn_sched_barrier(0);
-            f4 at = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < 4; kk += 2) {
-                s4 r0, r1, r0l, r1l;
-                scale_split(rhf[kk], rlf[kk], en[kk], n == 0, r0, r0l);
-                scale_split(rhf[kk + 1], rlf[kk + 1], en[kk + 1], n == 0, r1, r1l);
-                at = mma2(r0l, r1l, khf[kk], khf[kk + 1], at);
-                at = mma2(r0, r1, klf[kk], klf[kk + 1], at);
-                at = mma2(r0, r1, khf[kk], khf[kk + 1], at);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int x = 4 * g + e;
-                at[e] = x > n ? at[e] : (x == n ? rho_s : 0.f);
-            }
-            uint32_t h0, l0, h1, l1;
-            split2(at[0], at[1], h0, l0); split2(at[2], at[3], h1, l1);
-            sm.amat[wv][lane] = make_uint4(h0, h1, l0, l1);
-        }
-      }
-        PT_MARK(2)
-        lds_barrier();
-        PT_MARK(3)
+          }
+            PT_MARK(2)
+            lds_barrier();
+            PT_MARK(3)
 
-      {
-        WKV_LOCAL_LANE
-        // In this phase the products come out transposed, [channel][token]: a lane holds four consecutive channels
-        // of one token (token 16 blk + n, channels 16 wv + 4 g ..), so every table access is one 16-byte piece, the
-        // results go into their tiles eight bytes at a time, and the sums over a block's tokens run along a DPP row.
-        if (role == 2) {
-            // ---------------- gv[s][value] = kh G + sum_{t>=s} A~[t][s] gy[t], values 16wv..16wv+15
+          {
+            WKV_LOCAL_LANE
+            // In this phase the products come out transposed, [channel][token]: a lane holds four consecutive channels
+            // of one token (token 16 blk + n, channels 16 wv + 4 g ..), so every table access is one 16-byte piece, the
+            // results go into their tiles eight bytes at a time, and the sums over a block's tokens run along a DPP row.
+            if (role == 2) {
+                // ---------------- gv[s][value] = kh G + sum_{t>=s} A~[t][s] gy[t], values 16wv..16wv+15
 #pragma unroll
-            for (int qq = 0; qq < 4; qq++) {
-                const uint4 am = sm.amat[qq][lane];
-                const s4 gyTf = frag_tr(sm.gy, tro + (16 * qq) * LD + 16 * wv);
-                f4 kgq = KG[qq < 3 ? qq : 0];
-                if (qq == 3) { const float4 t4 = sm.kg3[wv][lane]; kgq = f4{t4.x, t4.y, t4.z, t4.w}; }
-                const f4 gvt = mma2(gyTf, gyTf, as_s4(am.x, am.y), as_s4(am.z, am.w), kgq);
-                *reinterpret_cast<uint2 *>(&sm.v[(16 * qq + n) * LD + 16 * wv + 4 * g]) =
-                    make_uint2(bf16_pack2(gvt[0], gvt[1]), bf16_pack2(gvt[2], gvt[3]));      // v is not read any more
+                for (int qq = 0; qq < 4; qq++) {
+                    const uint4 am = sm.amat[qq][lane];
+                    const s4 gyTf = frag_tr(sm.gy, tro + (16 * qq) * LD + 16 * wv);
+                    f4 kgq = KG;
+                    if (qq > 0) { const float4 t4 = (qq == 2 ? kg2 : sm.kg[qq >> 1])[wv][lane]; kgq = f4{t4.x, t4.y, t4.z, t4.w}; }
+                    const f4 gvt = mma2(gyTf, gyTf, as_s4(am.x, am.y), as_s4(am.z, am.w), kgq);
+                    *reinterpret_cast<uint2 *>(&sm.v[(16 * qq + n) * LD + 16 * wv + 4 * g]) =
+                        make_uint2(bf16_pack2(gvt[0], gvt[1]), bf16_pack2(gvt[2], gvt[3]));      // v is not read any more
+                }
             }
-        }
-        // ---------------- block q, token 16q+n, keys 16wv+4g..+3: gr, gk, decay gradient
-        {
-            const uint4 pa = sm.pfr[q][0][lane], pb = sm.pfr[q][1][lane];
-            const s4 pT_h = as_s4(pa.x, pa.y), pT_l = as_s4(pa.z, pa.w), pm_h = as_s4(pb.x, pb.y), pm_l = as_s4(pb.z, pb.w);
-            const s4 khTf = frag_tr(sm.kh, tro + (16 * q) * LD + 16 * wv), khTfl = frag_tr(sm.khl, tro + (16 * q) * LD + 16 * wv);
-            const s4 rhTf = frag_tr(sm.rh, tro + (16 * q) * LD + 16 * wv), rhTfl = frag_tr(sm.rhl, tro + (16 * q) * LD + 16 * wv);
-            f4 q2 = {0.f, 0.f, 0.f, 0.f}, q3 = q2;
-            q2 = mma(khTfl, pT_h, q2);
-            q3 = mma(rhTfl, pm_h, q3);
-            q2 = mma2(khTf, khTf, pT_h, pT_l, q2);      // sum_{s<t} P[t][s] kh_s   at [key][t]
-            q3 = mma2(rhTf, rhTf, pm_h, pm_l, q3);      // sum_{t>s} P[t][s] rh_t   at [key][s]
-            const int tk = 16 * q + n, k4 = 16 * wv + 4 * g, ti = swz(tk, k4);
-            const float4 tot4 = *reinterpret_cast<const float4 *>(&sm.tot[q][k4]), ent4 = *reinterpret_cast<const float4 *>(&sm.ent[q][k4]);
-            const float4 q1v = *reinterpret_cast<const float4 *>(&sm.q1[ti]), q4v = *reinterpret_cast<const float4 *>(&sm.q4[ti]);
-            const uint4 rk4 = *reinterpret_cast<const uint4 *>(&sm.rk[ti]);
-            const float pd = sm.pdiag[q][n];
-            float E1[4], E2[4];
-            if (whole) {
-                const float4 fr = *reinterpret_cast<const float4 *>(&tab_r[swz(n, k4)]), fk = *reinterpret_cast<const float4 *>(&tab_k[swz(n, k4)]);
-                E1[0] = fr.x; E1[1] = fr.y; E1[2] = fr.z; E1[3] = fr.w;
-                E2[0] = fk.x; E2[1] = fk.y; E2[2] = fk.z; E2[3] = fk.w;
-            } else {
-                const float4 in4 = *reinterpret_cast<const float4 *>(&sm.incl[ti]), lw4 = *reinterpret_cast<const float4 *>(&sm.lw[ti]);
-                E1[0] = exp2_fast(in4.x - lw4.x); E1[1] = exp2_fast(in4.y - lw4.y); E1[2] = exp2_fast(in4.z - lw4.z); E1[3] = exp2_fast(in4.w - lw4.w);
-                E2[0] = exp2_fast(tot4.x - in4.x); E2[1] = exp2_fast(tot4.y - in4.y); E2[2] = exp2_fast(tot4.z - in4.z); E2[3] = exp2_fast(tot4.w - in4.w);
-            }
-            const float entf[4] = {ent4.x, ent4.y, ent4.z, ent4.w}, uf[4] = {u4.x, u4.y, u4.z, u4.w};
-            const float q1f[4] = {q1v.x, q1v.y, q1v.z, q1v.w}, q4f[4] = {q4v.x, q4v.y, q4v.z, q4v.w};
-            const uint32_t rkf[4] = {rk4.x, rk4.y, rk4.z, rk4.w};
-            float c[4], z[4], grv[4], gkv[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float rr = bf_lo(rkf[e]), kr = bf_hi(rkf[e]), upd = uf[e] * pd;
-                grv[e] = E1[e] * (q1f[e] + entf[e] * q2[e]) + upd * kr;
-                const float gkn = E2[e] * (entf[e] * q3[e] + q4f[e]);
-                gkv[e] = gkn + upd * rr;
-                c[e] = rr * grv[e] - kr * gkv[e];
-                z[e] = kr * gkn;
-                gu_acc[e] = fmaf(rr * kr, pd, gu_acc[e]);
-            }
-            // this wavefront was the only reader left of its (block, quarter) corner of the rh and kh tiles
-            *reinterpret_cast<uint2 *>(&sm.rh[tk * LD + k4]) = make_uint2(bf16_pack2(grv[0], grv[1]), bf16_pack2(grv[2], grv[3]));
-            *reinterpret_cast<uint2 *>(&sm.kh[tk * LD + k4]) = make_uint2(bf16_pack2(gkv[0], gkv[1]), bf16_pack2(gkv[2], gkv[3]));
-            if (PER_TOKEN_W) {
-                // dL/dlog w_t = A_t - z_t with A_t = A(end of block) + sum over the block's later tokens of c
-                float dpart[4], all[4];
+            // ---------------- block q, token 16q+n, keys 16wv+4g..+3: gr, gk, decay gradient
+            {
+                const uint4 pa = sm.pfr[q][0][lane], pb = sm.pfr[q][1][lane];
+                const s4 pT_h = as_s4(pa.x, pa.y), pT_l = as_s4(pa.z, pa.w), pm_h = as_s4(pb.x, pb.y), pm_l = as_s4(pb.z, pb.w);
+                const s4 khTf = frag_tr(sm.kh, tro + (16 * q) * LD + 16 * wv), khTfl = frag_tr(sm.khl, tro + (16 * q) * LD + 16 * wv);
+                const s4 rhTf = frag_tr(sm.rh, tro + (16 * q) * LD + 16 * wv), rhTfl = frag_tr(sm.rhl, tro + (16 * q) * LD + 16 * wv);
+                f4 q2 = {0.f, 0.f, 0.f, 0.f}, q3 = q2;
+                q2 = mma(khTfl, pT_h, q2);
+                q3 = mma(rhTfl, pm_h, q3);
+                q2 = mma2(khTf, khTf, pT_h, pT_l, q2);      // sum_{s<t} P[t][s] kh_s   at [key][t]
+                q3 = mma2(rhTf, rhTf, pm_h, pm_l, q3);      // sum_{t>s} P[t][s] rh_t   at [key][s]
+                const int tk = 16 * q + n, k4 = 16 * wv + 4 * g, ti = swz(tk, k4);
+                const float4 tot4 = *reinterpret_cast<const float4 *>(&sm.tot[q][k4]), ent4 = *reinterpret_cast<const float4 *>(&sm.ent[q][k4]);
+                const float4 q1v = *reinterpret_cast<const float4 *>(&sm.q1[ti]), q4v = *reinterpret_cast<const float4 *>(&sm.q4[ti]);
+                const uint4 rk4 = *reinterpret_cast<const uint4 *>(&sm.rk[ti]);
+                const float pd = sm.rho[16 * q + n];
+                float E1[4], E2[4];
+                if (whole) {
+                    const float4 fr = *reinterpret_cast<const float4 *>(&tab_r[swz(n, k4)]), fk = *reinterpret_cast<const float4 *>(&tab_k[swz(n, k4)]);
+                    E1[0] = fr.x; E1[1] = fr.y; E1[2] = fr.z; E1[3] = fr.w;
+                    E2[0] = fk.x; E2[1] = fk.y; E2[2] = fk.z; E2[3] = fk.w;
+                } else {
+                    const float4 in4 = *reinterpret_cast<const float4 *>(&sm.incl[ti]), lw4 = *reinterpret_cast<const float4 *>(&sm.lw[ti]);
+                    E1[0] = exp2_fast(in4.x - lw4.x); E1[1] = exp2_fast(in4.y - lw4.y); E1[2] = exp2_fast(in4.z - lw4.z); E1[3] = exp2_fast(in4.w - lw4.w);
+                    E2[0] = exp2_fast(tot4.x - in4.x); E2[1] = exp2_fast(tot4.y - in4.y); E2[2] = exp2_fast(tot4.z - in4.z); E2[3] = exp2_fast(tot4.w - in4.w);
+                }
+                const float entf[4] = {ent4.x, ent4.y, ent4.z, ent4.w}, uf[4] = {u4.x, u4.y, u4.z, u4.w};
+                const float q1f[4] = {q1v.x, q1v.y, q1v.z, q1v.w}, q4f[4] = {q4v.x, q4v.y, q4v.z, q4v.w};
+                const uint32_t rkf[4] = {rk4.x, rk4.y, rk4.z, rk4.w};
+                float c[4], z[4], grv[4], gkv[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const float incl_suf = row_suffix_sum(c[e]);          // c of this token and the later ones
-                    dpart[e] = (incl_suf - c[e]) - z[e];
-                    all[e] = incl_suf;                                    // (lane n = 0: the whole block)
+                    const float rr = bf_lo(rkf[e]), kr = bf_hi(rkf[e]), upd = uf[e] * pd;
+                    grv[e] = E1[e] * (q1f[e] + entf[e] * q2[e]) + upd * kr;
+                    const float gkn = E2[e] * (entf[e] * q3[e] + q4f[e]);
+                    gkv[e] = gkn + upd * rr;
+                    c[e] = rr * grv[e] - kr * gkv[e];
+                    z[e] = kr * gkn;
+                    gu_acc[e] = fmaf(rr * kr, pd, gu_acc[e]);
                 }
-                // (the incl entries of this block and quarter had this wavefront as their only reader)
-                *reinterpret_cast<float4 *>(&sm.incl[ti]) = make_float4(dpart[0], dpart[1], dpart[2], dpart[3]);
-                if (n == 0) *reinterpret_cast<float4 *>(&sm.tots[q][k4]) = make_float4(all[0], all[1], all[2], all[3]);
-            } else {
-                const float before = (float)((sb - sb0) * SB + tk);      // tokens of the segment before this one
+                // this wavefront was the only reader left of its (block, quarter) corner of the rh and kh tiles
+                *reinterpret_cast<uint2 *>(&sm.rh[tk * LD + k4]) = make_uint2(bf16_pack2(grv[0], grv[1]), bf16_pack2(grv[2], grv[3]));
+                *reinterpret_cast<uint2 *>(&sm.kh[tk * LD + k4]) = make_uint2(bf16_pack2(gkv[0], gkv[1]), bf16_pack2(gkv[2], gkv[3]));
+                if (PER_TOKEN_W) {
+                    // dL/dlog w_t = A_t - z_t with A_t = A(end of block) + sum over the block's later tokens of c
+                    float dpart[4], all[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) gw_acc[e] += fmaf(before, c[e], -z[e]);
+                    for (int e = 0; e < 4; e++) {
+                        const float incl_suf = row_suffix_sum(c[e]);          // c of this token and the later ones
+                        dpart[e] = (incl_suf - c[e]) - z[e];
+                        all[e] = incl_suf;                                    // (lane n = 0: the whole block)
+                    }
+                    // (the incl entries of this block and quarter had this wavefront as their only reader)
+                    *reinterpret_cast<float4 *>(&sm.incl[ti]) = make_float4(dpart[0], dpart[1], dpart[2], dpart[3]);
+                    if (n == 0) *reinterpret_cast<float4 *>(&sm.tots[q][k4]) = make_float4(all[0], all[1], all[2], all[3]);
+                } else {
+                    const float before = (float)((sb - sb0) * SB + tk);      // tokens of the segment before this one
+#pragma unroll
+                    for (int e = 0; e < 4; e++) gw_acc[e] += fmaf(before, c[e], -z[e]);
+                }
             }
+          }
+            PT_MARK(4)
+            lds_barrier();
+            have_out = true;
         }
-      }
-        PT_MARK(4)
-        lds_barrier();
-        have_out = true;
+    };
+    switch (role) {
+        case 0: walk(std::integral_constant<int, 0>()); break;
+        case 1: walk(std::integral_constant<int, 1>()); break;
+        case 2: walk(std::integral_constant<int, 2>()); break;
+        default: walk(std::integral_constant<int, 3>());
     }
-    if (have_out) write_out(sb0, tok, c4, par);
+    if (have_out) write_out(sb0, tok, c4, par, q);
 
     PT_PRINT("bwd16")
     if (role == 1 && gs_in && seg == 0) {
@@ -1419,8 +1492,8 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     }
 #pragma unroll
     for (int e = 0; e < 4; e++) gu_acc[e] = row_suffix_sum(gu_acc[e]);       // lane n = 0: the sum over the row's 16 tokens
-    if (n == 0) *reinterpret_cast<float4 *>(&sm.red[q][16 * wv + 4 * g]) = make_float4(gu_acc[0], gu_acc[1], gu_acc[2], gu_acc[3]);
-    float *gw4 = sm.q1;             // [4][HEAD]; the q1 table is dead by now
+    float *red = sm.q4, *gw4 = sm.q1;             // [4][HEAD]: gu (gw) sums of the four block groups; the tables are dead by now
+    if (n == 0) *reinterpret_cast<float4 *>(&red[q * HEAD + 16 * wv + 4 * g]) = make_float4(gu_acc[0], gu_acc[1], gu_acc[2], gu_acc[3]);
     if (!PER_TOKEN_W) {
 #pragma unroll
         for (int e = 0; e < 4; e++) gw_acc[e] = row_suffix_sum(gw_acc[e]);
@@ -1429,7 +1502,7 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     lds_barrier();
     if (q == 0 && g == 0) {      // partial sums per (batch, segment): [(b*nseg + seg)][C]
         const size_t po = ((size_t)(b * nseg + seg) * H + h) * HEAD + own;
-        gu_part[po] = (sm.red[0][own] + sm.red[1][own]) + (sm.red[2][own] + sm.red[3][own]);
+        gu_part[po] = (red[own] + red[HEAD + own]) + (red[2 * HEAD + own] + red[3 * HEAD + own]);
         if (!PER_TOKEN_W) {
             bool fl;
             const float l = log_decay(static_cast<const float *>(wraw)[h * HEAD + own], floor_decay, &fl);
