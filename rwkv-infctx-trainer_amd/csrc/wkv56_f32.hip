@@ -182,25 +182,6 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
     }
     const int nsb = (Tlen + SB - 1) / SB, sb0 = seg * sps, sb1 = min(nsb, (seg + 1) * sps);
 
-    // chain wavefronts: S[kk][e] = S[key 16kk+4g+e][value 16q+n]
-    f4 S[4] = {zero4(), zero4(), zero4(), zero4()};
-    {
-        const float *sp = s_in + (size_t)bh * HEAD * HEAD;
-        float *table = sh.step[1].rm;            // (not in use yet)
-        if (seg > 0) {
-            chunked::chain_summaries<2>(table, part + (size_t)bh * nseg * m * PART, seg * m - 1, seg * m, -1, sp, threadIdx.x);
-            lds_barrier();
-        }
-        if (chain) {
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    S[kk][e] = seg > 0 ? table[(16 * kk + 4 * g + e) * LD + 16 * q + n] : sp[(16 * kk + 4 * g + e) * HEAD + 16 * q + n];
-        }
-        if (seg > 0) lds_barrier();              // (the table's place is written before the loop's first barrier)
-    }
-
     // preparing wavefronts: tokens tok0 .. tok0+7 of the step, channel `lane`
     const int tok0 = 16 * q + 8 * hf;
     const float uf = u[h * HEAD + lane];
@@ -244,6 +225,7 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
         prepare(sb0, sh.step[0]);
         fetch(min(sb0 + 1, sb1 - 1));
         lds_barrier();
+        if (seg > 0) lds_barrier();              // (the chained state has been read from where the next step's tables go)
         for (int sb = sb0; sb < sb1; sb++) {
             const int par = (sb - sb0) & 1;
             if (hf == 0 && y) {      // the masked matrix of block q
@@ -268,6 +250,23 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
             lds_barrier();
         }
         return;
+    }
+    // the state at the segment's start, put together while the other wavefronts prepare the first step:
+    // S[kk][e] = S[key 16kk+4g+e][value 16q+n]
+    f4 S[4];
+    {
+        const float *sp = s_in + (size_t)bh * HEAD * HEAD;
+        float *table = sh.step[1].rm;            // (not in use yet)
+        if (seg > 0) {
+            chunked::chain_summaries<4>(table, part + (size_t)bh * nseg * m * PART, seg * m - 1, seg * m, -1, sp, threadIdx.x);
+            lds_barrier();
+        }
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                S[kk][e] = seg > 0 ? table[(16 * kk + 4 * g + e) * LD + 16 * q + n] : sp[(16 * kk + 4 * g + e) * HEAD + 16 * q + n];
+        lds_barrier();
     }
     const Out yo = out_of(y, (size_t)Tlen * C - h * HEAD);
     const uint32_t y_lane = (uint32_t)n * C + 16 * q + 4 * g;
@@ -296,7 +295,6 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
             if (y && g == 0) put<T>(yo, t, C, 16 * q + n, fmaf(vt, rho, acc));
         }
     };
-    lds_barrier();
     int plain = any_plain(sh.step[0].plain);
     for (int sb = sb0; sb < sb1; sb++) {
         const int par = (sb - sb0) & 1;
