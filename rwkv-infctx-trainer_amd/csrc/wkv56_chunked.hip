@@ -132,6 +132,10 @@ __device__ __forceinline__ void scale_split(s4 hi, s4 lo, float4 f, s4 &oh, s4 &
     const uint2 h = __builtin_bit_cast(uint2, hi), l = __builtin_bit_cast(uint2, lo);
     float x0 = (bf_lo(h.x) + bf_lo(l.x)) * f.x, x1 = (bf_hi(h.x) + bf_hi(l.x)) * f.y;
     float x2 = (bf_lo(h.y) + bf_lo(l.y)) * f.z, x3 = (bf_hi(h.y) + bf_hi(l.y)) * f.w;
+    // The remainder is that of the rounded product: fused into it (the compiler does that unless it cannot see through)
+    // one in ten thousand results of a call comes out at the other neighbour in bf16, which a layer's own roundings then
+    // spread to 1 % of its smallest gradients.
+    asm("" : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3));
     uint32_t h0, l0, h1, l1;
     split2(x0, x1, h0, l0);
     split2(x2, x3, h1, l1);
