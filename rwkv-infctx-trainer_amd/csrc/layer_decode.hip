@@ -1,6 +1,7 @@
 // The layer of a serving loop: one token per sequence, a few rows (sequences) at a time, bf16.  What a row costs is the
 // weights, read once; as library products, element-wise passes and dtype conversions a v6 layer of one row was some 45
-// launches (H32: 560 us, of which the weights need 22 us).  Here it is seven kernels, 47 us:
+// launches (H32: 560 us, of which the weights need 22 us).  Here it is seven kernels, 46 us (47 with a walk over the jobs,
+// the head's inputs and the last factor asked for where they are used, and barriers that wait for the new state to be written):
 //
 //   rows_products   any number of products  out = f(x' W)  of up to 64 rows with weights of their own, in one launch;
 //                   x' may be the token-shift mix of x, formed where it is read (RWKV-v5/src/module/TimeMix.py:295-298,
@@ -32,7 +33,10 @@ struct Job {
     void *out;              // bf16 [rows][N]; k_major: fp32 [SPLIT][rows][N], parts of the sum
     int n, k_major, lerp, act;
 };
-struct Jobs { Job j[MAX_JOBS]; int count; };
+// end[i]: the workgroups of jobs 0 .. i, past the last job INT_MAX.  A workgroup finds its job by one scalar load of all of
+// them; a walk over the jobs is a scalar load and its latency for each.
+struct Jobs { Job j[MAX_JOBS]; int end[MAX_JOBS], count; };
+static_assert(MAX_JOBS == 8, "");
 enum { ACT_NONE = 0, ACT_RELU_SQUARE = 1, ACT_SIGMOID_MUL = 2 };
 
 __device__ __forceinline__ f4 mma(s8 a, s8 b, f4 c) {
@@ -179,13 +183,24 @@ template <int TN, int XL, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, XL <= 2 ? 4 : 2) void rows_products(int rows, int K, Jobs jobs) {
     constexpr int MT = Shape<TN, XL>::MT, NT = Shape<TN, XL>::NT;
     __shared__ __align__(16) Turn<TN, XL> turned[WAVES];
-    f4 (*part)[NT][MT][64] = reinterpret_cast<f4 (*)[NT][MT][64]>(turned);       // (used after the contraction)
+    // a wavefront's sums go where it turned its own weights, so that no other has to be done with them
+    auto part = [&](int wave, int tile) __attribute__((always_inline)) { return reinterpret_cast<f4 *>(&turned[wave]) + tile * 64; };
+    static_assert(sizeof(turned[0]) % sizeof(f4) == 0, "");
     static_assert(sizeof(turned[0]) >= NT * MT * 64 * sizeof(f4), "the sums fit where the weights were turned");
-    int wg = blockIdx.x, ji = 0;
+    int ji = 0, before = 0;
     const int row0 = Shape<TN, XL>::XROWS * blockIdx.y;
-    while (wg >= workgroups<TN>(jobs.j[ji])) wg -= workgroups<TN>(jobs.j[ji++]);     // (the grid is the sum over all jobs)
+#pragma unroll
+    for (int i = 0; i < MAX_JOBS - 1; i++)                   // (the grid is the sum over all jobs)
+        if ((int)blockIdx.x >= jobs.end[i]) { ji = i + 1; before = jobs.end[i]; }
+    const int wg = blockIdx.x - before;
     const Job job = jobs.j[ji];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = lane >> 4, n = lane & 15;
+    // the lane holds four consecutive columns of row m of a tile
+    auto row_of = [&](int tile) { return row0 + 16 * (tile % MT) + n; };
+    auto at = [&](int tile) { return (size_t)row_of(tile) * job.n + TN * wg + 16 * (tile / MT) + 4 * kg; };
+    auto mine = [&](int tile) { return tile < NT * MT && row_of(tile) < rows && (TN > 8 || kg < 2); };
+    uint2 factor = make_uint2(0u, 0u);                       // asked for before the weights, not behind the sums
+    if (job.act == ACT_SIGMOID_MUL && !job.k_major && mine(wv)) factor = *reinterpret_cast<const uint2 *>(job.mul + at(wv));
     f4 acc[NT][MT];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
@@ -198,18 +213,17 @@ __global__ __launch_bounds__(64 * WAVES, XL <= 2 ? 4 : 2) void rows_products(int
         if (job.mix) accumulate<TN, XL, WAVES, true>(job, turned[wv], wg, row0, rows, K, wv, lane, acc);
         else accumulate<TN, XL, WAVES, false>(job, turned[wv], wg, row0, rows, K, wv, lane, acc);
     }
-    __syncthreads();
+    wave_sync();
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) part[wv][nt][mt][lane] = acc[nt][mt];
-    __syncthreads();
+        for (int mt = 0; mt < MT; mt++) part(wv, nt * MT + mt)[lane] = acc[nt][mt];
+    lds_barrier();
     for (int tile = wv; tile < (job.k_major ? 1 : NT) * MT; tile += WAVES) {
-        const int nt = tile / MT, mt = tile % MT;
-        f4 s = part[0][nt][mt][lane];
+        f4 s = part(0, tile)[lane];
 #pragma unroll
-        for (int i = 1; i < WAVES; i++) s += part[i][nt][mt][lane];
-        const int m = row0 + 16 * mt + n;                   // the lane holds four consecutive columns of row m
+        for (int i = 1; i < WAVES; i++) s += part(i, tile)[lane];
+        const int m = row_of(tile);
         if (m >= rows) continue;
         float y[4] = {s[0], s[1], s[2], s[3]};
         if (job.k_major) {
@@ -217,13 +231,13 @@ __global__ __launch_bounds__(64 * WAVES, XL <= 2 ? 4 : 2) void rows_products(int
             continue;
         }
         if (TN == 8 && kg >= 2) continue;
-        const size_t o = (size_t)m * job.n + TN * wg + 16 * nt + 4 * kg;
+        const size_t o = at(tile);
         if (job.act == ACT_RELU_SQUARE) {
 #pragma unroll
             for (int e = 0; e < 4; e++) { const float p = fmaxf(round_bf16(y[e]), 0.f); y[e] = p * p; }
         } else if (job.act == ACT_SIGMOID_MUL) {
-            float q[4];
-            load4(job.mul + o, q);
+            if (tile != wv) factor = *reinterpret_cast<const uint2 *>(job.mul + o);
+            const float q[4] = {bf((uint16_t)factor.x), bf((uint16_t)(factor.x >> 16)), bf((uint16_t)factor.y), bf((uint16_t)(factor.y >> 16))};
 #pragma unroll
             for (int e = 0; e < 4; e++) y[e] = sigmoid(q[e]) * round_bf16(y[e]);
         }
@@ -247,6 +261,10 @@ __global__ __launch_bounds__(320) void lora_mix_rows(int rows, int C, const bf16
     load4(maa.p[j] + c0 + 4 * kg, d);
     for (int m0 = 0; m0 < rows; m0 += 16) {
         const int m = m0 + n, mc = min(m, rows - 1);
+        const size_t o = (size_t)mc * C + c0 + 4 * kg;
+        float xv[4], xx[4], y[4];
+        load4(x + o, xv);
+        load4(shift + o, xx);
         float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int p = 0; p < SPLIT; p++) {
@@ -259,10 +277,6 @@ __global__ __launch_bounds__(320) void lora_mix_rows(int rows, int C, const bf16
         for (int e = 0; e < 8; e++) t[e] = tanhf(round_bf16(t[e]));
         const uint4 bp = make_uint4(bf16_pack2(t[0], t[1]), bf16_pack2(t[2], t[3]), bf16_pack2(t[4], t[5]), bf16_pack2(t[6], t[7]));
         const s8 b = __builtin_bit_cast(s8, bp);
-        const size_t o = (size_t)mc * C + c0 + 4 * kg;
-        float xv[4], xx[4], y[4];
-        load4(x + o, xv);
-        load4(shift + o, xx);
         const f4 dyn = mma(a, b, f4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
         for (int e = 0; e < 4; e++) y[e] = fmaf(xx[e] - xv[e], d[e] + dyn[e], xv[e]);
@@ -280,9 +294,20 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
     __shared__ __align__(16) float part[4][HEAD], dec[HEAD];
     const int row = blockIdx.x / H, h = blockIdx.x % H, C = H * HEAD, tid = threadIdx.x, kq = tid >> 4, c4 = 4 * (tid & 15);
     const size_t base = (size_t)row * C + h * HEAD, so = (size_t)blockIdx.x * HEAD * HEAD;
+    // Latency, one round trip to memory after another: everything is asked for here, and no barrier waits for the state
+    // to be written.
     float4 S[4];
+    bf16 rb[4], kb[4], ub[4];
+    uint2 vb = *reinterpret_cast<const uint2 *>(v + base + c4);
 #pragma unroll
-    for (int i = 0; i < 4; i++) S[i] = *reinterpret_cast<const float4 *>(s_in + so + (kq + 16 * i) * HEAD + c4);
+    for (int i = 0; i < 4; i++) {
+        const int key = kq + 16 * i;
+        rb[i] = r[base + key]; kb[i] = k[base + key]; ub[i] = u[h * HEAD + key];
+        S[i] = *reinterpret_cast<const float4 *>(s_in + so + key * HEAD + c4);
+    }
+    const int own = h * HEAD + (tid & 63);
+    const float decay_own = to_float(time_decay[own]), g = to_float(gate[base + (tid & 63)]);
+    const float lnw = to_float(ln_w[own]), lnb = to_float(ln_b[own]);
     {
         const int ch = tid & 63, q = tid >> 6;
         float a = 0.f, w2v[16];
@@ -295,23 +320,23 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
                 for (int p = 0; p < SPLIT; p++) t += lora[((size_t)p * (gridDim.x / H) + row) * HEAD + tid];
                 dec[tid] = round_bf16(tanhf(round_bf16(t)));
             }
-            __syncthreads();
+            lds_barrier();
 #pragma unroll
             for (int e = 0; e < 16; e++) a = fmaf(dec[16 * q + e], w2v[e], a);
         }
         part[q][ch] = a;
-        __syncthreads();
+        lds_barrier();
         if (tid < HEAD)
-            dec[tid] = __expf(log_decay(round_bf16(to_float(time_decay[h * HEAD + tid]) + ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]))), false));
-        __syncthreads();
+            dec[tid] = __expf(log_decay(round_bf16(decay_own + ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]))), false));
+        lds_barrier();
     }
-    float v4[4], acc[4] = {0.f, 0.f, 0.f, 0.f}, bonus = 0.f;
-    load4(v + base + c4, v4);
+    const float v4[4] = {bf((uint16_t)vb.x), bf((uint16_t)(vb.x >> 16)), bf((uint16_t)vb.y), bf((uint16_t)(vb.y >> 16))};
+    float acc[4] = {0.f, 0.f, 0.f, 0.f}, bonus = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int key = kq + 16 * i;
-        const float ri = to_float(r[base + key]), ki = to_float(k[base + key]), wi = dec[key];
-        bonus = fmaf(ri * to_float(u[h * HEAD + key]), ki, bonus);
+        const float ri = to_float(rb[i]), ki = to_float(kb[i]), wi = dec[key];
+        bonus = fmaf(ri * to_float(ub[i]), ki, bonus);
         float s[4] = {S[i].x, S[i].y, S[i].z, S[i].w};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -327,7 +352,7 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
         acc[e] += __shfl_xor(acc[e], 32);
     }
     if ((tid & 63) < 16) *reinterpret_cast<float4 *>(&part[tid >> 6][c4]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    __syncthreads();
+    lds_barrier();
     if (tid >= HEAD) return;
     const float y = scale * round_bf16((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]));
     float s = y;
@@ -337,9 +362,7 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
     float q = dy * dy;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) q += __shfl_xor(q, o);
-    const int c = h * HEAD + tid;
-    const float g = to_float(gate[base + tid]);
-    const float z = fmaf(dy * rsqrtf(q * (1.f / HEAD) + eps), to_float(ln_w[c]), to_float(ln_b[c]));
+    const float z = fmaf(dy * rsqrtf(q * (1.f / HEAD) + eps), lnw, lnb);
     out[base + tid] = from_float<bf16>(z * g * sigmoid(g));
 }
 
@@ -351,16 +374,26 @@ __global__ __launch_bounds__(256) void timemix_head(int H, const bf16 *__restric
 // read the weights twice, once half the compute units have one (H12: 56 against 61 us); between, down to 32 workgroups.
 // One or two rows: 8 columns where 16 would leave compute units idle.  Eight wavefronts where the workgroups do not fill
 // the compute units twice over, four (of which several workgroups share a compute unit) otherwise.
-static hipError_t rows_products_launch(hipStream_t s, int rows, int K, const Jobs &jobs) {
+static hipError_t rows_products_launch(hipStream_t s, int rows, int K, Jobs &jobs) {
     int wgs32 = 0, wgs16 = 0, wgs8 = 0;
     bool by32 = true;
     for (int i = 0; i < jobs.count; i++) {
         wgs32 += workgroups<32>(jobs.j[i]); wgs16 += workgroups<16>(jobs.j[i]); wgs8 += workgroups<8>(jobs.j[i]);
         by32 = by32 && (jobs.j[i].k_major || jobs.j[i].n % 32 == 0);
     }
+    auto total = [&](auto columns) {
+        int sum = 0;
+        for (int i = 0; i < MAX_JOBS; i++) {
+            if (i < jobs.count) sum += workgroups<decltype(columns)::value>(jobs.j[i]);
+            jobs.end[i] = i < jobs.count ? sum : INT_MAX;
+        }
+    };
 #define WKV_ROWS(TN, XL, WAVES)                                                                                        \
-    hipLaunchKernelGGL((rows_products<TN, XL, WAVES>), dim3(TN == 32 ? wgs32 : TN == 16 ? wgs16 : wgs8, (rows + TN * XL / 8 - 1) / (TN * XL / 8)), \
-                       dim3(64 * WAVES), 0, s, rows, K, jobs)
+    do {                                                                                                               \
+        total(std::integral_constant<int, TN>());                                                                      \
+        hipLaunchKernelGGL((rows_products<TN, XL, WAVES>), dim3(TN == 32 ? wgs32 : TN == 16 ? wgs16 : wgs8, (rows + TN * XL / 8 - 1) / (TN * XL / 8)), \
+                           dim3(64 * WAVES), 0, s, rows, K, jobs);                                                      \
+    } while (0)
     const int ncu = cu_count();
     if (rows > 32) { if (by32 && wgs32 > ncu / 2) WKV_ROWS(32, 16, 4); else WKV_ROWS(16, 16, 4); }
     else if (rows > 16) {
