@@ -336,6 +336,30 @@ def test_products_of_a_few_rows_of_every_kind(rows, n, K):
         assert bool((err <= 0).all()), (name, err.max().item())
 
 
+@pytest.mark.parametrize("rows", [1, 5, 20, 40])
+@pytest.mark.parametrize("count", [1, 7, 8])
+def test_products_of_a_few_rows_find_their_job(rows, count):
+    """As many jobs as a launch takes, down to a single workgroup each (16 columns; a [k][n] one among them): every workgroup
+    finds its own.  Against 64 bits: the result rounds to bf16 (2^-8 of eight significant bits), fp32 sums of K terms."""
+    import ctypes
+    from rwkv_wkv_hip import _lib
+
+    class Product(ctypes.Structure):
+        _fields_ = [(f, ctypes.c_void_p) for f in ("w", "x", "shift", "mix", "mul", "out")] + [(f, ctypes.c_int) for f in ("n", "k_major", "lerp", "act")]
+    K, g = 256, torch.Generator().manual_seed(rows + count)
+    x = torch.randn(rows, K, generator=g).bfloat16().cuda()
+    ns, k_major = [16, 48, 16, 32, 160, 16, 64, 16][:count], [int(i == 4) for i in range(count)]
+    ws = [torch.randn(*((K, n) if kk else (n, K)), generator=g).bfloat16().cuda() for n, kk in zip(ns, k_major)]
+    outs = [torch.full((8, rows, n), 9.0, device="cuda") if kk else torch.full((rows, n), 9.0, dtype=torch.bfloat16, device="cuda") for n, kk in zip(ns, k_major)]
+    jobs = (Product * count)(*(Product(w.data_ptr(), x.data_ptr(), None, None, None, o.data_ptr(), n, kk, 0, 0) for w, o, n, kk in zip(ws, outs, ns, k_major)))
+    assert _lib.lib().wkv_rows_products(torch.cuda.current_stream().cuda_stream, rows, K, count, jobs) == 0
+    torch.cuda.synchronize()
+    for i, (w, o, kk) in enumerate(zip(ws, outs, k_major)):
+        w, got = (w if kk else w.t()).double(), o.double().sum(0) if kk else o.double()
+        want, sizes = x.double() @ w, x.double().abs() @ w.abs()
+        assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + K * 2 ** -24 * sizes).all()), i
+
+
 @pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("B,H,ffn", [(1, 1, 64), (3, 2, 448), (16, 1, 192), (17, 3, 640), (33, 2, 256), (64, 9, 2016), (65, 1, 128),
                                      (1, 32, 7168), (20, 40, 8960)])
