@@ -39,6 +39,7 @@
 // (S_out = decay o S_in + delta), and every segment's workgroup chains the summaries
 // before it into its first state.  Backward does the same with the state gradient.
 #include "common.h"
+#include "row_offset.h"
 #include <cstddef>
 #include <type_traits>
 
@@ -639,7 +640,7 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
     const __amdgpu_buffer_rsrc_t r_buf = buffer_of(r, 2 * left), k_buf = buffer_of(k, 2 * left), v_buf = buffer_of(v, 2 * left);
     const __amdgpu_buffer_rsrc_t w_buf = buffer_of(wraw, PER_TOKEN_W ? (W16 ? 2 : 4) * left : 0), y_buf = buffer_of(y, y ? 2 * left : 0);
     auto fetch = [&](int sb, Row &x) __attribute__((always_inline)) {          // (tokens past the end: r = k = v = 0)
-        const uint32_t o = ((uint32_t)sb * SB + tok) * C + c4, at = sb < sb1 ? 2 * o : NOWHERE;
+        const uint32_t o = row_offset(sb * SB + tok, Tlen, C, c4), at = sb < sb1 ? 2 * o : NOWHERE;
         x.r = buffer_load8(r_buf, at);
         x.k = buffer_load8(k_buf, at);
         x.v = buffer_load8(v_buf, at);
@@ -1062,7 +1063,7 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     const __amdgpu_buffer_rsrc_t gr_buf = buffer_of(gr, 2 * left), gk_buf = buffer_of(gk, 2 * left), gv_buf = buffer_of(gv, 2 * left);
     const __amdgpu_buffer_rsrc_t gw_buf = buffer_of(gw_tok, PER_TOKEN_W ? (W16 ? 2 : 4) * left : 0);
     auto write_out = [&](int sb, int tok, int c4, int par, int q) __attribute__((always_inline)) {
-        const uint32_t o = ((uint32_t)sb * SB + tok) * C + c4;       // (past the sequence's end: dropped)
+        const uint32_t o = row_offset(sb * SB + tok, Tlen, C, c4);       // (past the sequence's end: dropped)
         auto out = [&](const __amdgpu_buffer_rsrc_t &b, const uint16_t *tile) __attribute__((always_inline)) {
             const uint2 x = *reinterpret_cast<const uint2 *>(&tile[tok * LD + c4]);
             __builtin_amdgcn_raw_buffer_store_b64(dwords2{x.x, x.y}, b, (int)(2 * o), 0, NT_HINT);
@@ -1100,7 +1101,7 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
                     __builtin_amdgcn_raw_buffer_store_b64(dwords2{bf16_pack2(gw4[0], gw4[1]), bf16_pack2(gw4[2], gw4[3])}, gw_buf, (int)(2 * o), 0, NT_HINT);
                 else
                     __builtin_amdgcn_raw_buffer_store_b128(dwords4{__float_as_uint(gw4[0]), __float_as_uint(gw4[1]), __float_as_uint(gw4[2]), __float_as_uint(gw4[3])},
-                                                           gw_buf, (int)(o < left ? 4 * o : NOWHERE), 0, NT_HINT);
+                                                           gw_buf, (int)(4 * o), 0, NT_HINT);
             }
         }
     };

@@ -264,3 +264,35 @@ def test_full_shape_cumsum_decay_helper():
             assert_close(lg(out["r_decay"][b].cpu()), lg(back(tab.r_decay)), 1e-5, f"log r_decay row {b}")
             assert_close(lg(out["k_inv_decay"][b].cpu()), lg(back(tab.k_inv_decay)), 1e-5, f"log k_inv_decay row {b}")
     assert out["log_w"][0, 9, 5].item() == pytest.approx(-5.298317, abs=1e-5)
+
+
+@pytest.mark.parametrize("w16", [False, True])
+def test_missing_tokens_of_the_widest_sequences(w16):
+    """2 tokens of 532 672 heads in bf16: the 62 missing tokens of the step lie so far past the sequence's end that 32-bit byte
+    offsets of them come out inside it again (63 C >= 2^31).  Blocked against token by token, both from the same bf16 inputs:
+    results of two bf16 roundings (2^-8 of the value each way), fp32 ones from sums over 64 keys and 2 tokens whose operands have
+    16 bits as head and remainder (2^-17 each)."""
+    import rwkv_wkv_hip as W
+    B, T, H = 1, 2, 532_672
+    C = 64 * H
+    assert 63 * C >= 1 << 31 and T * C < 1 << 30
+    print(f"case widest v6 T{T} H{H} w16={w16}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    draw = lambda *s: torch.empty(s, device=DEV).normal_(0, 0.5, generator=g)
+    r, k, v, gy, w = (draw(B, T, C).bfloat16() for _ in range(5))
+    u, state = draw(H, 64), 0.2 * draw(B, H, 64, 64)
+
+    def go(algo, w):
+        W.set_algo(algo)
+        try:
+            leaves = [x.clone().requires_grad_(True) for x in (r, k, v, w, u)]
+            y, s = W.WKV_6.apply(B, T, C, H, *leaves, state)
+            return [y.detach(), s.detach(), *torch.autograd.grad(y, leaves, gy)]
+        finally:
+            W.set_algo("auto")
+    got, want = go("chunked", w if w16 else w.float()), go("recurrent", w.float())
+    for name, a, b in zip(("y", "state", "gr", "gk", "gv", "gw", "gu"), got, want):
+        tol = 1e-4 if a.dtype == torch.float32 and name != "gw" else 2e-2
+        rms = b.float().pow(2).mean().sqrt()
+        for x, z in zip(a.flatten().split(1 << 27), b.flatten().split(1 << 27)):
+            assert bool(((x.float() - z.float()).abs() <= tol * (z.float().abs() + rms)).all()), name
