@@ -151,6 +151,13 @@ __device__ __forceinline__ float over_groups(float x) {          // over the fou
 // in registers.  Bound by the matrix pipe: 160 instructions of 32 clocks per SIMD and step.  (With the eight wavefronts
 // that fill two per SIMD, a whole block's preparation per wavefront took 12 k clocks a step, the walk 7 k.)
 constexpr int NT_FWD = 768;
+// Who walks the piece summaries before a segment: the four wavefronts that own the state, while the others prepare the first
+// step, or, where there are more pieces than this and a decay that forgets nothing may have to walk them all, eight wavefronts
+// with half as many loads each, four of which prepare afterwards.  Prompts, four / eight wavefronts / by this rule, us: fp32
+// H4 T300 (4 pieces) 14.8 / 15.5 / 14.4, H12 T777 (12) 18.4 / 19.1 / 18.1, H32 T2048 47.0 / 47.7 / 45.7; H4 T2048 (31) 22.1 / 22.0 /
+// 21.0, H4 T4096 (63) 36.6 / 32.0 / 30.4; with a decay that forgets within a piece, H4 T4096, 21.2 / 20.8 / 20.9.  (The third
+// figures are also without the second step's inputs asked for during the walk.)
+constexpr int LONG_WALK = 16;
 struct FwdTiles {
     float rm[SB * LD], km[SB * LD], v[SB * LD];
     float em[4][HEAD], eb[4][HEAD];      // e^{m}, e^{b-m} per block and key
@@ -218,13 +225,18 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
         store_row_sums(p, sm.rho[2 * q + hf], lane);
         store_plain(&sm.plain[2 * q + hf], m, lane);
     };
+    const float *sp = s_in + (size_t)bh * HEAD * HEAD;
+    const float *pieces = part + (size_t)bh * nseg * m * PART;
+    float *table = sh.step[1].rm;                // the state at the segment's start (not in use yet)
+    const bool long_walk = seg * m > LONG_WALK;
     // (the two roles have loops of their own: in a common one the compiler waits, in either, for what the other may have
     // outstanding)
     if (!chain) {
         fetch(sb0);
+        if (long_walk) chunked::chain_summaries<2>(table, pieces, seg * m - 1, seg * m, -1, sp, threadIdx.x);
         prepare(sb0, sh.step[0]);
-        fetch(min(sb0 + 1, sb1 - 1));
         lds_barrier();
+        fetch(min(sb0 + 1, sb1 - 1));            // (not before the walk is over: its loads would wait behind these)
         if (seg > 0) lds_barrier();              // (the chained state has been read from where the next step's tables go)
         for (int sb = sb0; sb < sb1; sb++) {
             const int par = (sb - sb0) & 1;
@@ -255,10 +267,9 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
     // S[kk][e] = S[key 16kk+4g+e][value 16q+n]
     f4 S[4];
     {
-        const float *sp = s_in + (size_t)bh * HEAD * HEAD;
-        float *table = sh.step[1].rm;            // (not in use yet)
         if (seg > 0) {
-            chunked::chain_summaries<4>(table, part + (size_t)bh * nseg * m * PART, seg * m - 1, seg * m, -1, sp, threadIdx.x);
+            if (long_walk) chunked::chain_summaries<2>(table, pieces, seg * m - 1, seg * m, -1, sp, threadIdx.x);
+            else chunked::chain_summaries<4>(table, pieces, seg * m - 1, seg * m, -1, sp, threadIdx.x);
             lds_barrier();
         }
 #pragma unroll

@@ -816,6 +816,27 @@ def test_f32_blocked(version, dtype, B, H, T, nseg, pps, regime):
         assert (got["gw"].cpu()[hit] == 0).all(), "no gradient where the floor holds"
 
 
+@pytest.mark.parametrize("version,dtype", [(5, torch.float16), (6, torch.float32)])
+@pytest.mark.parametrize("T,nseg,pps", [(17 * 64, 17, 1), (18 * 64 - 5, 18, 1), (22 * 64 + 1, 23, 1), (20 * 64, 10, 1)])
+def test_f32_blocked_long_walks(version, dtype, T, nseg, pps):
+    """A decay that forgets next to nothing and up to 16, 17, 22 and 18 piece summaries before a segment: those up to 16 are walked by the
+    four wavefronts that own the state, more by eight.  The last token's result is half what the first piece left."""
+    from rwkv_wkv_hip import _lib, configs
+    L = _lib.lib()
+    wl = configs.make(1 if version == 5 else 3, B=1, T=T, C=64, H=1, dtype=dtype, seed=6100 + T)
+    wl.tensors["w"].fill_(-7.5)          # a decay of 0.99945 per token
+    print(f"case long walk v{version} T={T} nseg={nseg}", flush=True)
+    assert L.wkv_tune(_lib.TUNE_SEGMENTS, nseg) == 0 and L.wkv_tune(_lib.TUNE_PIECE_STEPS, pps) == 0
+    try:
+        got = run_gpu56(version, wl)
+    finally:
+        assert L.wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0 and L.wkv_tune(_lib.TUNE_PIECE_STEPS, 0) == 0
+    compare(got, run_oracle56(version, wl), 1e-3 if dtype == torch.float32 else 2e-2, f"long walk T{T}")
+    tokens = run_gpu56(version, wl, algo="recurrent")
+    for n in ("state", "gstate"):        # fp32 sums over T tokens in another order: 2^-24 sqrt(T) on average, the worst of 4096 some five times that
+        assert_close(got[n], tokens[n], 1e-4, f"against token by token: {n}")
+
+
 @pytest.mark.parametrize("version", [5, 6])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("name", ["r", "k", "v", "w", "dy"])
