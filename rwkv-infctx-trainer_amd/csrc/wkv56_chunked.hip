@@ -80,6 +80,7 @@ constexpr int NT_F = 256;     // summary passes: 4 wavefronts
 // One 16-deep product, D[m][n] += sum_k A[m][k] B[k][n].  Issued as a 16x16x32 MFMA
 // with a zero upper half: on gfx950 a 16x16x16 MFMA chained on the accumulator of a
 // 16x16x32 one returned corrupted rows in this kernel, and both cost one issue slot.
+// (The rule for one that takes such an accumulator all the same: split_pair().)
 __device__ __forceinline__ f4 mma(s4 a, s4 b, f4 c) {
     const s8 av = {a[0], a[1], a[2], a[3], 0, 0, 0, 0};
     const s8 bv = {b[0], b[1], b[2], b[3], 0, 0, 0, 0};
@@ -110,7 +111,11 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t 
 // The same for a pair of accumulator tiles (rows 4g+e, column n) that go into one product, with the subtraction on the
 // matrix cores: x - hi = x + (-1) hi, exact as on the vector pipe, bit for bit the same results.  Sixteen vector
 // instructions of twenty-four become two MFMAs: a third of the chains' vector work.  `minus`: minus_one().
-// (A non-finite element makes the remainders of its column of both tiles NaN, all of them terms of the sum its own is a term of.)
+// (A non-finite element makes the remainders of its column of its tile NaN, all of them terms of the sum its own is a term of.)
+// These are 16x16x16 MFMAs whose C is the accumulator of 16x16x32 ones, which corrupted rows where one followed the other
+// directly (mma()).  Here none can: each one's B operand is packed by vector instructions from all four registers of its
+// C, so C is complete before the MFMA starts; and its own result is read by vector instructions only, never as
+// another MFMA's C.  Both have to stay so.
 __device__ __forceinline__ s8 pair(s4 a, s4 b) { return s8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 __device__ __forceinline__ s4 minus_one(int g, int n) {
     const int at = n - 4 * g;            // the lane's row holds its -1 at element `at` of its four, if that is one of them
