@@ -148,16 +148,10 @@ __device__ __forceinline__ void scale_split(s4 hi, s4 lo, float4 f, s4 &oh, s4 &
     oh = as_s4(h0, h1);
     ol = as_s4(l0, l1);
 }
-// Result rows leave with the non-temporal hint: they are not read again by these kernels, and left to the default
-// policy they push the inputs that the backward pass reads a second time out of the last-level cache.
+// the last rows of a segment's y (the others leave by buffer stores, NT_HINT)
 __device__ __forceinline__ void store_row(bf16 *p, uint2 v) {
     typedef unsigned int u2 __attribute__((ext_vector_type(2)));
     __builtin_nontemporal_store(u2{v.x, v.y}, reinterpret_cast<u2 *>(p));
-}
-__device__ __forceinline__ void store_row(bf16 *p, const float (&x)[4]) { store_row(p, make_uint2(bf16_pack2(x[0], x[1]), bf16_pack2(x[2], x[3]))); }
-__device__ __forceinline__ void store_row(float *p, const float (&x)[4]) {
-    typedef float f4_ __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(f4_{x[0], x[1], x[2], x[3]}, reinterpret_cast<f4_ *>(p));
 }
 __device__ __forceinline__ float group_sum4(float x) {      // over the 4 lane groups of 16
     x += __shfl_xor(x, 16);
@@ -213,12 +207,14 @@ __device__ __forceinline__ void needed_here(uint2 &a) { asm volatile("" : "+v"(a
 __device__ __forceinline__ void needed_here(float4 &a) { asm volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z), "+v"(a.w)); }
 
 // Access by buffer instructions: what lies at or beyond the range's end reads as 0 and is not written, so that an access
-// that may have to be left out needs no branch (`nowhere`), and the compiler can count the accesses in flight.
+// that may have to be left out needs no branch (NOWHERE), and the compiler can count the accesses in flight.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00027000);
 }
 constexpr uint32_t NOWHERE = 0xfffffff0u;
-constexpr int NT_HINT = 2;          // the non-temporal hint of a buffer store
+// Result rows leave with the non-temporal hint (here that of a buffer store): they are not read again by these kernels, and
+// left to the default policy they push the inputs that the backward pass reads a second time out of the last-level cache.
+constexpr int NT_HINT = 2;
 typedef uint32_t dwords2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dwords4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint2 buffer_load8(__amdgpu_buffer_rsrc_t b, uint32_t at) {
@@ -897,7 +893,8 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
 //                              leave  Q1 = gy S^T  of each block in LDS;
 //             wavefronts  4-7  walk the state gradient backward (value-major copy) and
 //                              leave  Q4 = v G^T;
-//             wavefronts  8-11 walk the key-major copy and keep  kh G  in registers;
+//             wavefronts  8-11 walk the key-major copy and leave  kh G  of three blocks in LDS
+//                              (that of the first, walked last, in registers);
 //             wavefronts 12-15 build, per block, the masked matrices P, P^T and A~ once
 //                              for everybody.
 //   blocks    wavefront (q, w): gr, gk and the decay gradient of block q, keys
