@@ -520,35 +520,36 @@ def test_chunked_forward_backward_matches_oracle(version, T):
 
 
 @pytest.mark.parametrize("version,w16", [(5, False), (6, False), (6, True)])
-@pytest.mark.parametrize("T", [16, 63, 64, 65, 127, 128, 129, 192, 250])
-def test_chunked_steps_in_turn(version, T, w16):
-    """One step, two, three and four, whole and with missing tokens: the register sets used in turn, the accesses that
-    are left out by their address, what each role of the backward does in its own loop.  Without
+@pytest.mark.parametrize("T,nseg", [(16, 1), (63, 1), (64, 1), (65, 1), (127, 1), (128, 1), (129, 1), (192, 1), (250, 1), (129, 0), (192, 0), (250, 0),
+                                    (321, 2), (384, 2), (576, 3)])
+def test_chunked_steps_in_turn(version, T, nseg, w16):
+    """One step, two, three and four walked by a workgroup (nseg = 1), three by each of two and of three (2, 3: 321 tokens with a ragged last
+    step), and whatever the planner makes of these lengths (0): the register sets used in turn, the accesses that
+    are left out by their address, what each role of the backward does in its own loop from step to step.  Without
     autograd (no checkpoints kept) the same bits."""
-    from rwkv_wkv_hip import configs
+    from rwkv_wkv_hip import _lib, configs
+    import rwkv_wkv_hip as W
+    L = _lib.lib()
     B, H = 2, 3
     C = 64 * H
     wl = configs.make(1 if version == 5 else 3, B=B, T=T, C=C, H=H, dtype=torch.bfloat16, seed=90 + T)
     if w16:
         wl.tensors["w"] = wl.tensors["w"].bfloat16()
-    print(f"case steps v{version} T={T} w16={w16}", flush=True)
-    got = run_gpu56(version, wl, algo="chunked")
-    if w16:
-        wl.tensors["w"] = wl.tensors["w"].float()
-    compare(got, run_oracle56(version, wl), 2e-2, f"steps v{version} T{T}")       # bf16 I/O: rtol 2e-2, floor 2e-2 rms
-    # forward without autograd: no checkpoints, same bits
-    import rwkv_wkv_hip as W
-    g = {n: x.to(dev()) for n, x in wl.tensors.items()}
-    if w16:
-        g["w"] = g["w"].bfloat16()
-    W.set_algo("chunked")
+    print(f"case steps v{version} T={T} nseg={nseg} w16={w16}", flush=True)
+    assert L.wkv_tune(_lib.TUNE_SEGMENTS, nseg) == 0
     try:
-        with torch.no_grad():
+        got = run_gpu56(version, wl, algo="chunked")
+        g = {n: x.to(dev()) for n, x in wl.tensors.items()}
+        W.set_algo("chunked")
+        with torch.no_grad():        # no checkpoints
             args = (g["state"], g["r"], g["k"], g["v"], g["w"], g["u"]) if version == 5 else (g["r"], g["k"], g["v"], g["w"], g["u"], g["state"])
             y, s = (W.WKV_5 if version == 5 else W.WKV_6).apply(B, T, C, H, *args)
     finally:
         W.set_algo("auto")
+        assert L.wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0
     assert torch.equal(y, got["y"]) and torch.equal(s, got["state"])
+    wl.tensors["w"] = wl.tensors["w"].float()
+    compare(got, run_oracle56(version, wl), 2e-2, f"steps v{version} T{T} n{nseg}")       # bf16 I/O: rtol 2e-2, floor 2e-2 rms
 
 
 @pytest.mark.parametrize("version", [5, 6])
