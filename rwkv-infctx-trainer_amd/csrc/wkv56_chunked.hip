@@ -1125,12 +1125,15 @@ __global__ __launch_bounds__(NT_B16) void backward16(int bh0, int Tlen, int C, i
     // A loop for each role: in a common one the registers that take the checkpoint in one role and hold the gradient in two
     // others count as awaited in all of them, and those two waited in every step for the results of the step before to be
     // written (one counter covers a wavefront's loads and stores).  With it, the results leaving by buffer stores and two
-    // more blocks of kh G parked in LDS: forward and backward of B8 T4096, WKV6 H40 bf16 decay 983 -> 938 us, WKV5 H32
-    // 549 -> 523 (the forward's part of it some 5 and 12), B1 T4096 H64 fp32 decay 211 -> 203, on one GPU in turn.  Measured and
-    // not kept: the next step's inputs asked for before the chains start in every role (961, 526, 206; left to itself the
-    // compiler asks for them after the chain where that is the long one), the checkpoint asked for where the chain
-    // starts (972, 525, 210), blocks counted from their middle, which spares the builders their factor (943, 531, 205,
-    // but it moves the state gradient's error from 1.6e-6 to 2.3e-6).
+    // more blocks of kh G parked in LDS: forward and backward of B8 T4096, WKV6 H40 bf16 decay 989 -> 946 us, WKV5 H32
+    // 555 -> 527 (the forward's part of it some 5 and 12), B1 T4096 H64 fp32 decay 209 -> 204, on one GPU in turn.  The kernel for
+    // time-invariant decays and ragged lengths, which holds the whole-step and the general way at once, spills 24 registers (11
+    // in one loop) and gains as much all the same: WKV5 B8 H32 T4000 588 -> 557, T1000 158 -> 148, B1 H64 T4000 199 -> 188; per
+    // token it stays 9 % behind the one for whole steps.
+    // Measured and not kept, on a GPU where what is kept read 938, 523 and 203: the next step's inputs asked for before the
+    // chains start in every role (961, 526, 206; left to itself the compiler asks for them after the chain where that is the
+    // long one), the checkpoint asked for where the chain starts (972, 525, 210), blocks counted from their middle, which
+    // spares the builders their factor (943, 531, 205, but it moves the state gradient's error from 1.6e-6 to 2.3e-6).
     auto walk = [&](auto its_role) __attribute__((always_inline)) {
         constexpr int role = decltype(its_role)::value, q = role;
         for (int sb = sb1 - 1; sb >= sb0; sb--) {
