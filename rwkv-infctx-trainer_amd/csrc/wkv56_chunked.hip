@@ -577,7 +577,12 @@ __device__ __forceinline__ void chain_summaries(float *table, const float *__res
 
 // ALL_WHOLE (time-invariant decay only): the sequence is a whole number of 64-token steps, so the general way of
 // a step with missing tokens is left out of the kernel, and with it the registers it keeps alive across the loop.
-template <bool PER_TOKEN_W, bool W16, bool ALL_WHOLE = false>
+// ONE_STEP: the sequence is one step, so what looks ahead, and what keeps the accesses of one step countable in the next, is
+// left out, and missing tokens are not asked for: an access past the range's end moves nothing, but is issued lane by lane
+// all the same, some 0.6 us a workgroup.  Without it / with it, B16 H64, us: WKV6 bf16 decay T16 23.9 / 20.8, T32 26.2 / 23.4, T64
+// 25.4 / 24.5, WKV5 T16 24.2 / 21.4, T56 24.6 / 24.0; B32 T16 46.7 / 40.1 and 46.2 / 40.4.  (Whole steps under a time-invariant
+// decay stay with ALL_WHOLE: T64 22.4.)
+template <bool PER_TOKEN_W, bool W16, bool ALL_WHOLE = false, bool ONE_STEP = false>
 __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, int H, int nseg, int sps, int m,
         const bf16 *__restrict__ r, const bf16 *__restrict__ k, const bf16 *__restrict__ v,
         const void *__restrict__ wraw, const float *__restrict__ u, const float *__restrict__ s_in,
@@ -602,7 +607,7 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
 
     // chain wavefronts: S[j][e] = S[key 32hk+16j+4g+e][value 16wv+n]
     f4 S[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
-    if (seg == 0) {
+    if (ONE_STEP || seg == 0) {
         if (chain) {
             const float *sp = s_in + (size_t)bh * HEAD * HEAD;
 #pragma unroll
@@ -642,6 +647,10 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
     const __amdgpu_buffer_rsrc_t w_buf = buffer_of(wraw, PER_TOKEN_W ? (W16 ? 2 : 4) * left : 0), y_buf = buffer_of(y, y ? 2 * left : 0);
     auto fetch = [&](int sb, Row &x) __attribute__((always_inline)) {          // (tokens past the end: r = k = v = 0)
         const uint32_t o = row_offset(sb * SB + tok, Tlen, C, c4), at = sb < sb1 ? 2 * o : NOWHERE;
+        if (ONE_STEP) {
+            x.r = x.k = x.v = x.w0 = x.w1 = make_uint2(0u, 0u);
+            if (tok >= Tlen) return;
+        }
         x.r = buffer_load8(r_buf, at);
         x.k = buffer_load8(k_buf, at);
         x.v = buffer_load8(v_buf, at);
@@ -661,12 +670,12 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
     bool have_y = false;
     if (tid < HEAD) sm.ub[tid] = u[h * HEAD + tid];
     fetch(sb0, rowA);
-    {      // (as many as a step leaves in flight, so that the wait for the loop's first step is counted as the others are)
+    if (!ONE_STEP) {      // (as many as a step leaves in flight, so that the wait for the loop's first step is counted as the others are)
         __builtin_amdgcn_raw_buffer_store_b64(dwords2{0u, 0u}, y_buf, (int)NOWHERE, 0, 0);
         __builtin_amdgcn_raw_buffer_store_b64(dwords2{0u, 0u}, y_buf, (int)NOWHERE, 0, 0);
         __builtin_amdgcn_raw_buffer_store_b64(dwords2{0u, 0u}, y_buf, (int)NOWHERE, 0, 0);
     }
-    fetch(sb0 + 1, rowB);
+    if (!ONE_STEP) fetch(sb0 + 1, rowB);
     // log w of this lane's token and its running sum inside the wavefront, always one step ahead (see scan_local)
     float lc[4], ic[4];
     auto scan_ahead = [&](int sb, const Row &x) __attribute__((always_inline)) {
@@ -678,7 +687,7 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
         } else {
             lc[0] = l_const.x; lc[1] = l_const.y; lc[2] = l_const.z; lc[3] = l_const.w;
         }
-        if ((sb + 1) * SB > Tlen) {      // (scalar) tokens past the end count as w = 1
+        if (ONE_STEP || (sb + 1) * SB > Tlen) {      // (scalar) tokens past the end count as w = 1
             const bool in = sb * SB + tok < Tlen;
 #pragma unroll
             for (int c = 0; c < 4; c++) lc[c] = in ? lc[c] : 0.f;
@@ -699,7 +708,7 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
             *reinterpret_cast<float4 *>(&sm.ent[q][c4]) = make_float4(exp2_fast(-16.f * lcst[0]), exp2_fast(-16.f * lcst[1]), exp2_fast(-16.f * lcst[2]), exp2_fast(-16.f * lcst[3]));
         }
     }
-    auto whole_step = [&](int sb) { return ALL_WHOLE ? true : !PER_TOKEN_W && (sb + 1) * SB <= Tlen; };       // scalar
+    auto whole_step = [&](int sb) { return ALL_WHOLE ? true : !ONE_STEP && !PER_TOKEN_W && (sb + 1) * SB <= Tlen; };       // scalar
 #pragma unroll
     for (int c = 0; c < 4; c++) lc[c] = ic[c] = 0.f;
     if (!whole_step(sb0)) scan_ahead(sb0, rowA);
@@ -716,7 +725,7 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
             const float kf[4] = {bf_lo(pk.x), bf_hi(pk.x), bf_lo(pk.y), bf_hi(pk.y)};
             const float4 u4 = *reinterpret_cast<const float4 *>(&sm.ub[c4]);
             const float uf[4] = {u4.x, u4.y, u4.z, u4.w};
-            {      // y of the previous step waits in the rh tile: out as full rows, by the lanes that overwrite it next
+            if (!ONE_STEP) {      // y of the previous step waits in the rh tile: out as full rows, by the lanes that overwrite it next
                 const uint2 yv = *reinterpret_cast<const uint2 *>(&sm.rh[tok * LD + c4]);
                 __builtin_amdgcn_raw_buffer_store_b64(dwords2{yv.x, yv.y}, y_buf, (int)(have_y ? 2 * (((uint32_t)(sb - 1) * SB + tok) * C + c4) : NOWHERE), 0, NT_HINT);
             }
@@ -756,13 +765,13 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
         PT_MARK(0)
         lds_barrier();
         PT_MARK(1)
-        {       // the state at the start of this step, 16 bytes per lane and tile, from the wavefronts that own it
+        if (!ONE_STEP || ckpt) {       // the state at the start of this step, 16 bytes per lane and tile, from the wavefronts that own it
             const __amdgpu_buffer_rsrc_t c_buf = buffer_of(ckpt ? ckpt + ck_off + (size_t)sb * HEAD * HEAD : nullptr, ckpt ? HEAD * HEAD * 4 : 0);
             const uint32_t at = chain ? (uint32_t)((wv * 4 + 2 * hk) * 64 + lane) * 16 : NOWHERE;
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dwords4, S[0]), c_buf, (int)at, 0, 0);
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dwords4, S[1]), c_buf, (int)(chain ? at + 1024 : NOWHERE), 0, 0);
         }
-        fetch(sb + 2, cur);     // these loads have two steps to arrive
+        if (!ONE_STEP) fetch(sb + 2, cur);     // these loads have two steps to arrive
 
         if (chain) {
             // ---------------- the state over the four blocks; per block this half's share of rh S
@@ -844,7 +853,7 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
     };
     for (int sb = sb0;;) {          // (left where it ends: a way round the second step would count as a way into the first)
         do_step(sb, rowA, rowB);
-        if (++sb >= sb1) break;
+        if (ONE_STEP || ++sb >= sb1) break;
         do_step(sb, rowB, rowA);
         if (++sb >= sb1) break;
     }
@@ -1688,6 +1697,9 @@ hipError_t init_kernels() {
         if (e == hipSuccess) e = allow((const void *)forward16<true, true>, sizeof(Fwd16Tiles));
         if (e == hipSuccess) e = allow((const void *)forward16<false, false>, sizeof(Fwd16Tiles));
         if (e == hipSuccess) e = allow((const void *)forward16<false, false, true>, sizeof(Fwd16Tiles));
+        if (e == hipSuccess) e = allow((const void *)forward16<true, false, false, true>, sizeof(Fwd16Tiles));
+        if (e == hipSuccess) e = allow((const void *)forward16<true, true, false, true>, sizeof(Fwd16Tiles));
+        if (e == hipSuccess) e = allow((const void *)forward16<false, false, false, true>, sizeof(Fwd16Tiles));
         if (e == hipSuccess) e = allow((const void *)backward16<true, false>, sizeof(Bwd16Tiles));
         if (e == hipSuccess) e = allow((const void *)backward16<true, true>, sizeof(Bwd16Tiles));
         if (e == hipSuccess) e = allow((const void *)backward16<false, false>, sizeof(Bwd16Tiles));
@@ -1727,18 +1739,18 @@ hipError_t forward_launch(hipStream_t s, bool per_token, bool w16, int B, int Tl
     auto launch = [&](int bh0, int n, const SegPlan &x) {
         if (n <= 0) return;
         dim3 grid(n * x.nseg);
-        if (mode == 2)
-            hipLaunchKernelGGL((forward16<true, true>), grid, block16, sizeof(Fwd16Tiles), s, bh0, Tlen, C, H, x.nseg, x.sps, x.m,
-                               rr, kk, vv, w, u, s_in, (bf16 *)y, s_out, ckpt, part, floor_decay);
-        else if (mode == 1)
-            hipLaunchKernelGGL((forward16<true, false>), grid, block16, sizeof(Fwd16Tiles), s, bh0, Tlen, C, H, x.nseg, x.sps, x.m,
-                               rr, kk, vv, w, u, s_in, (bf16 *)y, s_out, ckpt, part, floor_decay);
-        else if (Tlen % SB == 0)
-            hipLaunchKernelGGL((forward16<false, false, true>), grid, block16, sizeof(Fwd16Tiles), s, bh0, Tlen, C, H, x.nseg, x.sps, x.m,
-                               rr, kk, vv, w, u, s_in, (bf16 *)y, s_out, ckpt, part, floor_decay);
-        else
-            hipLaunchKernelGGL((forward16<false, false>), grid, block16, sizeof(Fwd16Tiles), s, bh0, Tlen, C, H, x.nseg, x.sps, x.m,
-                               rr, kk, vv, w, u, s_in, (bf16 *)y, s_out, ckpt, part, floor_decay);
+#define WKV_FORWARD16(...)                                                                                                         \
+    hipLaunchKernelGGL((forward16<__VA_ARGS__>), grid, block16, sizeof(Fwd16Tiles), s, bh0, Tlen, C, H, x.nseg, x.sps, x.m,         \
+                       rr, kk, vv, w, u, s_in, (bf16 *)y, s_out, ckpt, part, floor_decay)
+        if (nsb == 1 && (per_token || Tlen < SB)) {      // (see ONE_STEP)
+            if (mode == 2) WKV_FORWARD16(true, true, false, true);
+            else if (mode == 1) WKV_FORWARD16(true, false, false, true);
+            else WKV_FORWARD16(false, false, false, true);
+        } else if (mode == 2) WKV_FORWARD16(true, true);
+        else if (mode == 1) WKV_FORWARD16(true, false);
+        else if (Tlen % SB == 0) WKV_FORWARD16(false, false, true);
+        else WKV_FORWARD16(false, false);
+#undef WKV_FORWARD16
     };
     prof_begin(KID_CHUNK_FORWARD, s);          // (both groups count as the one forward kernel of the call)
     launch(0, gp.nA, gp.a);

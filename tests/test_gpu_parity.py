@@ -520,13 +520,13 @@ def test_chunked_forward_backward_matches_oracle(version, T):
 
 
 @pytest.mark.parametrize("version,w16", [(5, False), (6, False), (6, True)])
-@pytest.mark.parametrize("T,nseg", [(16, 1), (63, 1), (64, 1), (65, 1), (127, 1), (128, 1), (129, 1), (192, 1), (250, 1), (129, 0), (192, 0), (250, 0),
-                                    (321, 2), (384, 2), (576, 3)])
+@pytest.mark.parametrize("T,nseg", [(2, 1), (15, 1), (16, 1), (17, 1), (48, 1), (63, 1), (64, 1), (65, 1), (127, 1), (128, 1), (129, 1),
+                                    (192, 1), (250, 1), (129, 0), (192, 0), (250, 0), (321, 2), (384, 2), (576, 3)])
 def test_chunked_steps_in_turn(version, T, nseg, w16):
-    """One step, two, three and four walked by a workgroup (nseg = 1), three by each of two and of three (2, 3: 321 tokens with a ragged last
-    step), and whatever the planner makes of these lengths (0): the register sets used in turn, the accesses that
-    are left out by their address, what each role of the backward does in its own loop from step to step.  Without
-    autograd (no checkpoints kept) the same bits."""
+    """One step (which has a forward kernel of its own), two, three and four walked by a workgroup (nseg = 1), three by each of
+    two and of three (2, 3: 321 tokens with a ragged last step), and whatever the planner makes of these lengths (0): the
+    register sets used in turn, the accesses that are left out by their address, what each role of the backward does in its
+    own loop from step to step.  Without autograd (no checkpoints kept) the same bits."""
     from rwkv_wkv_hip import _lib, configs
     import rwkv_wkv_hip as W
     L = _lib.lib()
