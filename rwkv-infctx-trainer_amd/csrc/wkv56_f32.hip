@@ -236,7 +236,7 @@ __global__ __launch_bounds__(NT_FWD) void forward_f32(int bh0, int Tlen, int C, 
         if (long_walk) chunked::chain_summaries<2>(table, pieces, seg * m - 1, seg * m, -1, sp, threadIdx.x);
         prepare(sb0, sh.step[0]);
         lds_barrier();
-        fetch(min(sb0 + 1, sb1 - 1));            // (not before the walk is over: its loads would wait behind these)
+        if (sb0 + 1 < sb1) fetch(sb0 + 1);       // (not before the walk is over: its loads would wait behind these)
         if (seg > 0) lds_barrier();              // (the chained state has been read from where the next step's tables go)
         for (int sb = sb0; sb < sb1; sb++) {
             const int par = (sb - sb0) & 1;
