@@ -742,6 +742,10 @@ __global__ __launch_bounds__(NT_F16) void forward16(int bh0, int Tlen, int C, in
                     khv[c] = kf[c] * exp2_fast(tot[c] - inc[c]);
                 }
             }
+            if (ONE_STEP && !PER_TOKEN_W) {      // (as where two ways meet, the products are rounded before their remainders: scale_split())
+                asm("" : "+v"(rhv[0]), "+v"(rhv[1]), "+v"(rhv[2]), "+v"(rhv[3]));
+                asm("" : "+v"(khv[0]), "+v"(khv[1]), "+v"(khv[2]), "+v"(khv[3]));
+            }
 #pragma unroll
             for (int c = 0; c < 4; c++) p = fmaf(rf[c] * uf[c], kf[c], p);
             uint32_t h0, l0, h1, l1;

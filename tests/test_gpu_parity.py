@@ -552,6 +552,42 @@ def test_chunked_steps_in_turn(version, T, nseg, w16):
     compare(got, run_oracle56(version, wl), 2e-2, f"steps v{version} T{T} n{nseg}")       # bf16 I/O: rtol 2e-2, floor 2e-2 rms
 
 
+@pytest.mark.parametrize("version,w16", [(5, False), (6, False), (6, True)])
+@pytest.mark.parametrize("rest", [2, 17, 40, 63])
+def test_chunked_one_step_is_the_last_step_of_a_longer_sequence(version, w16, rest):
+    """64 tokens and then the rest from the state they leave, each a sequence of one step, against both in one call: the same
+    bits.  (Under a time-invariant decay 64 tokens have a kernel of their own, whose compiler may round a product elsewhere:
+    their keys are zero there and the rest is compared.)"""
+    import rwkv_wkv_hip as W
+    from rwkv_wkv_hip import _lib, configs
+    B, H, T = 2, 3, 64 + rest
+    C = 64 * H
+    wl = configs.make(1 if version == 5 else 3, B=B, T=T, C=C, H=H, dtype=torch.bfloat16, seed=300 + rest)
+    g = {n: x.to(dev()) for n, x in wl.tensors.items()}
+    if w16:
+        g["w"] = g["w"].bfloat16()
+    if version == 5:
+        g["k"][:, :64] = 0
+
+    def call(t0, t1, state):
+        cut = {n: g[n][:, t0:t1].contiguous() for n in ("r", "k", "v")}
+        w = g["w"] if version == 5 else g["w"][:, t0:t1].contiguous()
+        args = (state, cut["r"], cut["k"], cut["v"], w, g["u"]) if version == 5 else (cut["r"], cut["k"], cut["v"], w, g["u"], state)
+        return (W.WKV_5 if version == 5 else W.WKV_6).apply(B, t1 - t0, C, H, *args)
+    W.set_algo("chunked")
+    assert _lib.lib().wkv_tune(_lib.TUNE_SEGMENTS, 1) == 0
+    try:
+        with torch.no_grad():
+            y, s = call(0, T, g["state"])
+            y0, s0 = call(0, 64, g["state"])
+            y1, s1 = call(64, T, s0)
+    finally:
+        assert _lib.lib().wkv_tune(_lib.TUNE_SEGMENTS, 0) == 0
+        W.set_algo("auto")
+    assert version == 5 or torch.equal(y[:, :64], y0)
+    assert torch.equal(y[:, 64:], y1) and torch.equal(s, s1)
+
+
 @pytest.mark.parametrize("version", [5, 6])
 def test_chunked_truncated_bptt_and_floor(version):
     from rwkv_wkv_hip import configs
